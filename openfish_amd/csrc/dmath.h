@@ -179,6 +179,35 @@ OFA_HD double log_1to5_with_cell(float s, float near, LogCell c, const double *s
     return __builtin_fma((double)k, kLn2, lu);
 }
 
+// A third form, for the place where every instruction counts.  The cells are centred on multiples of 1/32
+// and carry the power of two: the entry of a float s is picked by the low seven bits
+// of (exponent, mantissa) rounded to five mantissa bits, which tells c = 2^k (1 + j/32) apart for k = 0 .. 3, so that
+// ln s = lnc + log1p(s * inv - 1) with |s * inv - 1| <= 1/64 (+ 2^-17 when the cell is chosen with an
+// approximation of s) and no exponent is taken apart.  ln 1 comes out as 0 exactly: its cell has inv = 1, lnc = 0.
+constexpr int kLogCentredCells = 128;
+OFA_HD uint32_t log_centred_index(float near) { return ((bits_of(near) + (1u << 17)) >> 18) & (uint32_t)(kLogCentredCells - 1); }
+OFA_HD LogCell log_centred_cell(int i) {
+    const int k = ((i >> 5) + 1) & 3;  // the bits of 1.0f shifted right by 18 end in 96
+    const double c = 1.0 + (i & 31) / 32.0;
+    LogCell x;
+    x.inv = 1.0 / c;  // in (0.5, 1]
+    const bool low = x.inv < 0.70710678118654752;
+    x.lnc = -log_core(low ? 2.0 * x.inv - 1.0 : x.inv - 1.0, (low ? -1 : 0) - k);
+    x.inv = __builtin_ldexp(x.inv, -k);
+    return x;
+}
+OFA_HD double log_centred(float s, LogCell c, const double *series) {
+    const double r = __builtin_fma((double)s, c.inv, -1.0);
+    double q = __builtin_fma(series[0], r, series[1]);
+    q = __builtin_fma(q, r, series[2]);
+    q = __builtin_fma(q, r, series[3]);
+    q = __builtin_fma(q, r, series[4]);
+    q = __builtin_fma(q, r, series[5]);
+    q = __builtin_fma(q, r, -0.5);
+    q = __builtin_fma(q, r, 1.0);
+    return __builtin_fma(q, r, c.lnc);
+}
+
 // RN32(m + ln s) as the CPU path forms it: the sum in double, one rounding.  ln 1 is exactly 0 on
 // the CPU path; the table logarithm returns about 1e-18 there, which would show in a result whose
 // m is zero.

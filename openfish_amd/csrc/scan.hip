@@ -128,60 +128,142 @@ struct LogSeries {
     double e[OFA_EXP_COEF_COUNT];  // exponential: polynomial, rounding shift, log2(e), -ln 2
 };
 struct LogArgs {
-    const ofa::LogCell *cells;
+    const ofa::LogCell *cells;    // 32 cells, for the double arithmetic of all lanes
+    const ofa::LogCell *centred;  // ofa::kLogCentredCells cells, for the second tier
     const double *series;
     const double *expc;
     float *lanes;  // 64 floats of LDS owned by the calling wave (two-tier updates only)
     int hurry = 3;  // the wave's priority during a trip through the second tier
 };
 
-// Two-tier update, second tier.  `value` is the estimate of a lane's update, `unsettled` says
-// that it may differ from the CPU path's result.  A wave usually has none, one or two such
-// lanes, and evaluating the CPU roundings under their execution mask would cost the whole wave
-// the five double exponentials, the running sum and the logarithm one after another.  Instead
-// the unsettled lanes hand their inputs (d_0..d_4 = v_i - m, and m) to groups of eight lanes
-// through LDS: lane 8q+j of group q computes the double exponential of d_j of the q-th unsettled
-// lane, the fp32 running sum travels from lane to lane by DPP row shifts (so lane 8q+4 ends with
-// the CPU path's sum), that lane takes the logarithm, adds m in double and rounds once, and the
-// result returns to its owner through a lane permute.  More than eight unsettled lanes take
-// further trips (only the first few dozen time steps have that many: values are small there and
-// an ulp is tiny; the kernels run those steps with the double arithmetic throughout).
-__device__ __forceinline__ float resolve_unsettled(float value, float sum, bool unsettled, float v0, float v1, float v2,
-                                                   float v3, float v4, float m, const LogArgs &logtab) {
-    uint64_t mask = __builtin_amdgcn_ballot_w64(unsettled);
-    if (mask == 0) return value;
-    // the chunk's other waves wait at the barrier for this one
-    if (logtab.hurry == 3) __builtin_amdgcn_s_setprio(3);
-    else if (logtab.hurry == 2) __builtin_amdgcn_s_setprio(2);
-    else if (logtab.hurry == 1) __builtin_amdgcn_s_setprio(1);
-    const int lane = threadIdx.x & 63;
-    int rank = __builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mask, 0));
-    if (!unsettled) rank = -1;
-    do {  // eight unsettled lanes per trip
-        if ((unsigned)rank < 8u) {
-            float *slot = logtab.lanes + 8 * rank;
-            *reinterpret_cast<float4 *>(slot) = make_float4(v0 - m, v1 - m, v2 - m, v3 - m);
-            *reinterpret_cast<float4 *>(slot + 4) = make_float4(v4 - m, m, sum, 0.f);
-        }
-        const float x = logtab.lanes[lane];  // LDS operations of one wave complete in order
-        // lane 8q+4 will take the logarithm: its table cell is fetched now, chosen with the estimate
-        // of the sum (two lanes up), and arrives while the exponentials are evaluated
-        const float near = dpp<0x102>(x);  // row_shl:2
-        const ofa::LogCell cell = ofa::log_cell_near(near, logtab.cells);
-        const double e = ofa::exp_ldexp((double)x, logtab.expc);
-        float s = (float)e;
+// Two-tier update, second tier: the CPU path's own roundings for the updates whose estimate is unsettled.
+//
+// An instruction costs a wave that is alone on its SIMD about four cycles whatever it does (fp64 and
+// dependent ones included), so a trip through this tier costs what it issues plus its LDS round trips.
+// Three ways, by how many of the wave's updates are unsettled:
+//   one (two waves in three that have any, with one state per lane): served by the whole wave without
+//     LDS.  Its five differences are read into scalar registers and dealt to five lanes, which evaluate
+//     the double exponentials side by side; every lane then forms the fp32 running sum through DPP
+//     broadcasts and takes the logarithm;
+//   several: handed through LDS to rows of 16 lanes, four updates at a time, or with several states per
+//     lane to groups of eight lanes, eight at a time;
+//   many (only the first few hundred time steps have them: values are small there and an ulp is tiny): the
+//     double arithmetic for all lanes at once, which costs about as much as two trips per state of a lane.
+// Backward sweep, T = 1666, together with the loads that are no longer all waited for every eight steps:
+// 1 chunk of 64 states 0.56 -> 0.44 ms, 1 chunk of 256 states 0.78 -> 0.67, 512 chunks of 256 states 0.98 -> 0.86.
+template <int MODE>
+__device__ __forceinline__ void fill_log_tables(ofa::LogCell *cells, ofa::LogCell *centred) {
+    const int tid = threadIdx.x;
+    if (MODE != OFK_SCAN_FAST && tid >= 128 && tid < 160) cells[tid - 128] = ofa::log_cell(tid - 128);
+    if (MODE == OFK_SCAN_TWO_TIER && tid < ofa::kLogCentredCells) centred[tid] = ofa::log_centred_cell(tid);
+}
+
+// lane k of the result: d_k of lane `lane`, for k = 0 .. 4 (d_0 in the other lanes).  v_readlane may read a
+// vector register one instruction after its write (hence the s_nop: the writes are not in sight), and a scalar
+// register that a vector instruction has written may be read by one two instructions later (the order sees to that).
+__device__ __forceinline__ float five_to_lanes(float d0, float d1, float d2, float d3, float d4, int lane) {
+    float x;
+    uint32_t s0, s1, s2, s3, s4;
+    asm("s_nop 0\n\t"
+        "v_readlane_b32 %[s0], %[d0], %[lane]\n\t"
+        "v_readlane_b32 %[s1], %[d1], %[lane]\n\t"
+        "v_readlane_b32 %[s2], %[d2], %[lane]\n\t"
+        "v_readlane_b32 %[s3], %[d3], %[lane]\n\t"
+        "v_readlane_b32 %[s4], %[d4], %[lane]\n\t"
+        "v_mov_b32 %[x], %[s0]\n\t"
+        "v_writelane_b32 %[x], %[s1], 1\n\t"
+        "v_writelane_b32 %[x], %[s2], 2\n\t"
+        "v_writelane_b32 %[x], %[s3], 3\n\t"
+        "v_writelane_b32 %[x], %[s4], 4"
+        : [x] "=&v"(x), [s0] "=&s"(s0), [s1] "=&s"(s1), [s2] "=&s"(s2), [s3] "=&s"(s3), [s4] "=&s"(s4)
+        : [d0] "v"(d0), [d1] "v"(d1), [d2] "v"(d2), [d3] "v"(d3), [d4] "v"(d4), [lane] "s"(lane));
+    return x;
+}
+
+// fp32 running sum of lanes 0 .. 4 of e of the lane's row of 16, rounded after every term, to every lane of
+// the row.  row_newbcast is the one DPP control that 64-bit operations have (their bank mask was seen to be
+// ignored).  e has just been written: two wait states before a DPP operand may read it.
+__device__ __forceinline__ float running_sum_of_five(double e) {
+    double t;
+    float s;
+    const double one = 1.0;
+#define OFK_TERM(K)                                                                           \
+    "v_cvt_f64_f32 %[t], %[s]\n\t"                                                            \
+    "v_fmac_f64_dpp %[t], %[e], %[one] row_newbcast:" #K " row_mask:0xf bank_mask:0xf\n\t"    \
+    "v_cvt_f32_f64 %[s], %[t]\n\t"
+    asm("s_nop 1\n\t"
+        "v_mov_b64_dpp %[t], %[e] row_newbcast:0 row_mask:0xf bank_mask:0xf\n\t"
+        "v_cvt_f32_f64 %[s], %[t]\n\t"
+        OFK_TERM(1) OFK_TERM(2) OFK_TERM(3) OFK_TERM(4)
+        : [t] "=&v"(t), [s] "=&v"(s)
+        : [e] "v"(e), [one] "v"(one));
+#undef OFK_TERM
+    return s;
+}
+
+// The same for groups of eight lanes, to lane 4 of the group only: the sum so far comes from the lane below.
+__device__ __forceinline__ float running_sum_along_eight(double e) {
+    float s = (float)e;
 #pragma unroll
-        for (int k = 0; k < 4; ++k) s = (float)((double)dpp<0x111>(s) + e);  // row_shr:1: the sum so far, from the lane below
-        const float m_of_group = dpp<0x101>(x);  // row_shl:1: lane 8q+4 reads m from lane 8q+5
-        float r = (float)((double)m_of_group + ofa::log_1to5_with_cell(s, near, cell, logtab.series));
-        r = s == 1.0f ? m_of_group : r;  // ln 1 = 0 exactly, as on the CPU path
-        const float mine = __int_as_float(__builtin_amdgcn_ds_bpermute((8 * (rank & 7) + 4) << 2, __float_as_int(r)));
-        if ((unsigned)rank < 8u) value = mine;
-        rank -= 8;
-        mask = __builtin_amdgcn_ballot_w64(rank >= 0);
-    } while (mask != 0);
-    if (logtab.hurry) __builtin_amdgcn_s_setprio(0);
-    return value;
+    for (int k = 0; k < 4; ++k) s = (float)((double)dpp<0x111>(s) + e);  // row_shr:1
+    return s;
+}
+
+// mask[i]: the lanes whose update of state i is unsettled; at least one bit is set
+template <int SPL>
+__device__ __forceinline__ void resolve_unsettled(float (&value)[SPL], const float (&sum)[SPL], const uint64_t (&mask)[SPL],
+                                                  const float (&v)[SPL][5], const float (&m)[SPL], const LogArgs &logtab) {
+    const int lane = threadIdx.x & 63;
+    if (SPL == 1 && (mask[0] & (mask[0] - 1)) == 0) {
+        const int at = __builtin_ctzll(mask[0]);
+        const float near = lane_value(sum[0], at);
+        const ofa::LogCell cell = logtab.centred[ofa::log_centred_index(near)];  // arrives while the exponentials are evaluated
+        const float mm = lane_value(m[0], at);
+        const float x = five_to_lanes(v[0][0] - m[0], v[0][1] - m[0], v[0][2] - m[0], v[0][3] - m[0], v[0][4] - m[0], at);
+        const float s = running_sum_of_five(ofa::exp_ldexp((double)x, logtab.expc));  // in the first row of lanes
+        const float r = lane_value((float)((double)mm + ofa::log_centred(s, cell, logtab.series)), 0);
+        value[0] = lane == at ? r : value[0];
+        return;
+    }
+    int total = 0, rank[SPL];
+#pragma unroll
+    for (int i = 0; i < SPL; ++i) {
+        rank[i] = (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(mask[i] >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mask[i], (uint32_t)total));
+        total += __builtin_amdgcn_readfirstlane(__builtin_popcountll(mask[i]));
+    }
+    constexpr int kSlots = SPL == 1 ? 4 : 8, kStride = 64 / kSlots;  // updates per trip, lanes per update
+    if (total <= 2 * kSlots * SPL - (SPL == 1 ? kSlots : 0)) {
+        for (int first = 0; first < total; first += kSlots) {
+            bool in[SPL];
+#pragma unroll
+            for (int i = 0; i < SPL; ++i) {
+                in[i] = ((mask[i] >> lane) & 1) && (unsigned)(rank[i] - first) < (unsigned)kSlots;
+                if (in[i]) {
+                    float *slot = logtab.lanes + kStride * (rank[i] - first);
+                    *reinterpret_cast<float4 *>(slot) = make_float4(v[i][0] - m[i], v[i][1] - m[i], v[i][2] - m[i], v[i][3] - m[i]);
+                    *reinterpret_cast<float4 *>(slot + 4) = make_float4(v[i][4] - m[i], 0.f, m[i], sum[i]);
+                }
+            }
+            // LDS operations of one wave complete in order
+            const float2 ms = *reinterpret_cast<const float2 *>(logtab.lanes + (lane & -kStride) + 6);
+            const float x = logtab.lanes[lane];
+            const ofa::LogCell cell = logtab.centred[ofa::log_centred_index(ms.y)];  // arrives while the exponentials are evaluated
+            const double e = ofa::exp_ldexp((double)x, logtab.expc);
+            const float s = SPL == 1 ? running_sum_of_five(e) : running_sum_along_eight(e);
+            const float r = (float)((double)ms.x + ofa::log_centred(s, cell, logtab.series));
+#pragma unroll
+            for (int i = 0; i < SPL; ++i) {
+                const float mine = __int_as_float(__builtin_amdgcn_ds_bpermute((kStride * (rank[i] - first) + 4) << 2, __float_as_int(r)));
+                value[i] = in[i] ? mine : value[i];
+            }
+        }
+    } else {
+#pragma unroll
+        for (int i = 0; i < SPL; ++i) {
+            const float r = ofa::lse5_cpu_rounding_tab(v[i][0], v[i][1], v[i][2], v[i][3], v[i][4], m[i], logtab.cells, logtab.series, logtab.expc);
+            value[i] = (mask[i] >> lane) & 1 ? r : value[i];
+        }
+    }
 }
 
 // maximum of three in one instruction (the operands are never NaN here; fmaxf would first quiet
@@ -192,22 +274,44 @@ __device__ __forceinline__ float max3(float a, float b, float c) {
     return r;
 }
 
-// max + log(sum_i exp(v_i - max)), sum taken in the order v0..v4
-template <int MODE>
-__device__ __forceinline__ float lse5(float v0, float v1, float v2, float v3, float v4, const LogArgs &logtab) {
-    const float m = max3(max3(v0, v1, v2), v3, v4);
+// max + log(sum_i exp(v_i - max)) of the SPL states of a lane, sums taken in the order v[.][0] .. v[.][4].
+// With two tiers the states share one test and one branch: reading a comparison's mask and branching on
+// it costs a lone wave about as much as eight other instructions.
+template <int SPL, int MODE>
+__device__ __forceinline__ void lse5_all(float (&out)[SPL], const float (&v)[SPL][5], const LogArgs &logtab) {
+    float m[SPL];
+#pragma unroll
+    for (int i = 0; i < SPL; ++i) m[i] = max3(max3(v[i][0], v[i][1], v[i][2]), v[i][3], v[i][4]);
     if constexpr (MODE == OFK_SCAN_PRECISE) {
-        return ofa::lse5_cpu_rounding_tab(v0, v1, v2, v3, v4, m, logtab.cells, logtab.series, logtab.expc);
+#pragma unroll
+        for (int i = 0; i < SPL; ++i)
+            out[i] = ofa::lse5_cpu_rounding_tab(v[i][0], v[i][1], v[i][2], v[i][3], v[i][4], m[i], logtab.cells, logtab.series, logtab.expc);
     } else if constexpr (MODE == OFK_SCAN_TWO_TIER) {
-        const ofa::Lse5Estimate e = ofa::lse5_estimate(v0, v1, v2, v3, v4, m);
-        return resolve_unsettled(e.value, e.sum, !e.settled, v0, v1, v2, v3, v4, m, logtab);
+        float sum[SPL];
+        uint64_t mask[SPL], any = 0;
+#pragma unroll
+        for (int i = 0; i < SPL; ++i) {
+            const ofa::Lse5Estimate e = ofa::lse5_estimate(v[i][0], v[i][1], v[i][2], v[i][3], v[i][4], m[i]);
+            out[i] = e.value;
+            sum[i] = e.sum;
+            mask[i] = __builtin_amdgcn_ballot_w64(!e.settled);
+            any |= mask[i];
+        }
+        if (any != 0) {
+            // the chunk's other waves wait at the barrier for this one
+            if (logtab.hurry == 3) __builtin_amdgcn_s_setprio(3);
+            else if (logtab.hurry == 1) __builtin_amdgcn_s_setprio(1);
+            resolve_unsettled<SPL>(out, sum, mask, v, m, logtab);
+            __builtin_amdgcn_s_setprio(0);
+        }
     } else {
-        float s = __builtin_amdgcn_exp2f((v0 - m) * kLog2e);
-        s += __builtin_amdgcn_exp2f((v1 - m) * kLog2e);
-        s += __builtin_amdgcn_exp2f((v2 - m) * kLog2e);
-        s += __builtin_amdgcn_exp2f((v3 - m) * kLog2e);
-        s += __builtin_amdgcn_exp2f((v4 - m) * kLog2e);
-        return __builtin_fmaf(__builtin_amdgcn_logf(s), kLn2, m);
+#pragma unroll
+        for (int i = 0; i < SPL; ++i) {
+            float s = __builtin_amdgcn_exp2f((v[i][0] - m[i]) * kLog2e);
+#pragma unroll
+            for (int b = 1; b < 5; ++b) s += __builtin_amdgcn_exp2f((v[i][b] - m[i]) * kLog2e);
+            out[i] = __builtin_fmaf(__builtin_amdgcn_logf(s), kLn2, m[i]);
+        }
     }
 }
 
@@ -370,23 +474,50 @@ struct FloatRun {
     }
 };
 
-template <int I, int SPL, int MODE>
-__device__ __forceinline__ void bwd_update(float (&a)[SPL], const float4 &nx, const BwdRow<SPL> &row, float stay,
-                                           const LogArgs &logtab) {
-    if constexpr (I < SPL) {
-        a[I] = lse5<MODE>(a[I] + stay, row.template add<0, I>(nx.x), row.template add<1, I>(nx.y),
-                          row.template add<2, I>(nx.z), row.template add<3, I>(nx.w), logtab);
-        bwd_update<I + 1, SPL, MODE>(a, nx, row, stay, logtab);
+template <int N, typename F>
+__device__ __forceinline__ void static_for(F &&f) {
+    if constexpr (N > 0) {
+        static_for<N - 1>(f);
+        f(std::integral_constant<int, N - 1>{});
     }
 }
 
-template <int I, int SPL, int MODE>
-__device__ __forceinline__ void fwd_update(float (&f)[SPL], float p0, float p1, float p2, float p3,
-                                           const FwdRow<SPL> &row, float stay, const LogArgs &logtab) {
+// `count` steps, DEPTH of them unrolled per trip: step(k, j, checked) with k = j % DEPTH a
+// compile-time index; in unchecked trips j + DEPTH + SLACK < count holds for every step, i.e.
+// every prefetch DEPTH steps ahead is in range (of a tensor with SLACK rows fewer than steps).
+template <int DEPTH, int SLACK = 0, typename Step>
+__device__ __forceinline__ void pipelined(int count, Step &&step) {
+    int j0 = 0;
+    for (; j0 + 2 * DEPTH + SLACK <= count; j0 += DEPTH)
+        static_for<DEPTH>([&](auto k) { step(k, j0 + (int)k, std::false_type{}); });
+    for (; j0 < count; j0 += DEPTH)
+        static_for<DEPTH>([&](auto k) {
+            if (j0 + (int)k < count) step(k, j0 + (int)k, std::true_type{});
+        });
+}
+
+// the five terms of every state of a lane; the row's registers are free for the next load afterwards
+template <int I, int SPL>
+__device__ __forceinline__ void bwd_terms(float (&v)[SPL][5], const float (&a)[SPL], const float4 &nx, const BwdRow<SPL> &row, float stay) {
     if constexpr (I < SPL) {
-        f[I] = lse5<MODE>(f[I] + stay, row.template add<I, 0>(p0), row.template add<I, 1>(p1),
-                          row.template add<I, 2>(p2), row.template add<I, 3>(p3), logtab);
-        fwd_update<I + 1, SPL, MODE>(f, p0, p1, p2, p3, row, stay, logtab);
+        v[I][0] = a[I] + stay;
+        v[I][1] = row.template add<0, I>(nx.x);
+        v[I][2] = row.template add<1, I>(nx.y);
+        v[I][3] = row.template add<2, I>(nx.z);
+        v[I][4] = row.template add<3, I>(nx.w);
+        bwd_terms<I + 1, SPL>(v, a, nx, row, stay);
+    }
+}
+template <int I, int SPL>
+__device__ __forceinline__ void fwd_terms(float (&v)[SPL][5], const float (&f)[SPL], float p0, float p1, float p2, float p3,
+                                          const FwdRow<SPL> &row, float stay) {
+    if constexpr (I < SPL) {
+        v[I][0] = f[I] + stay;
+        v[I][1] = row.template add<I, 0>(p0);
+        v[I][2] = row.template add<I, 1>(p1);
+        v[I][3] = row.template add<I, 2>(p2);
+        v[I][4] = row.template add<I, 3>(p3);
+        fwd_terms<I + 1, SPL>(v, f, p0, p1, p2, p3, row, stay);
     }
 }
 
@@ -402,62 +533,65 @@ __global__ __launch_bounds__((Shape<S, SPL>::kThreads)) void bwd_scan_kernel(
     constexpr int H = 4 / SPL;  // lanes sharing one quad
     using Vec = BwdVec<S>;
     __shared__ __attribute__((aligned(16))) float vec[Sh::kChunks][2][Vec::kLen];
-    __shared__ __attribute__((aligned(16))) ofa::LogCell logcells[32];
+    __shared__ __attribute__((aligned(16))) ofa::LogCell logcells[32], centred[ofa::kLogCentredCells];
     __shared__ __attribute__((aligned(16))) float tier_lanes[MODE == OFK_SCAN_TWO_TIER ? Sh::kThreads : 64];
     const int tid = threadIdx.x;
-    const LogArgs logtab{logcells, series.c, series.e, tier_lanes + (MODE == OFK_SCAN_TWO_TIER ? (tid & ~63) : 0)};
+    const LogArgs logtab{logcells, centred, series.c, series.e, tier_lanes + (MODE == OFK_SCAN_TWO_TIER ? (tid & ~63) : 0)};
 
-    if (MODE != OFK_SCAN_FAST && tid < 32) logcells[tid] = ofa::log_cell(tid);
+    fill_log_tables<MODE>(logcells, centred);
     const int g = tid / L, l = tid % L;
     const int r = l / H, c0 = (l % H) * SPL;  // own states: r + (c0 + i) * Q
     int n = blockIdx.x * Sh::kChunks + g;
-    const bool live = n < N;
-    if (!live) n = N - 1;
+    if (n >= N) n = N - 1;
 
-    const size_t row_stride = (size_t)N * kCols * S;  // fp16 elements between time steps
-    const _Float16 *sp = scores + (size_t)n * kCols * S + 4 * kCols * r + kLead + c0;
-    float *out = bwd + (size_t)n * (size_t)(T + 1) * S + r + c0 * Q;
+    // Rows are addressed by a base that is the same for the whole workgroup (scalar registers, stepped by
+    // scalar additions) plus a 32-bit offset of the lane.  Lanes past the batch repeat its last chunk, stores included.
+    const ptrdiff_t row_stride = (ptrdiff_t)N * kCols * S;  // fp16 elements between time steps
+    const int first_chunk = blockIdx.x * Sh::kChunks;
+    const unsigned g_eff = (unsigned)(n - first_chunk);
+    const unsigned sc_lane = g_eff * kCols * S + 4 * kCols * r + kLead + c0;
+    const unsigned st_lane = g_eff * (unsigned)(T + 1) * S + r + c0 * Q;
+    const _Float16 *pre = scores + (size_t)first_chunk * kCols * S + (ptrdiff_t)(T - 1) * row_stride;  // next row to fetch
+    float *orow = bwd + ((size_t)first_chunk * (size_t)(T + 1) + T) * S;                              // next row to store
 
     float a[SPL];
 #pragma unroll
-    for (int i = 0; i < SPL; ++i) a[i] = 0.f;
-    if (live) {
-#pragma unroll
-        for (int i = 0; i < SPL; ++i) out[(size_t)T * S + i * Q] = 0.f;
+    for (int i = 0; i < SPL; ++i) {
+        a[i] = 0.f;
+        orow[st_lane + i * Q] = 0.f;
+        vec[g][0][Vec::at(r, c0 + i)] = 0.f;
     }
+    orow -= S;
 
+    // The first rows are fetched without a condition (of a chunk shorter than DEPTH the oldest row again):
+    // were they not, the compiler, which counts loads in flight, would have to assume that a row's load may
+    // be the latest one and let every trip round the loop below wait for all of them.
     BwdRow<SPL> ring[DEPTH];
-#pragma unroll
-    for (int k = 0; k < DEPTH; ++k) {
-        const int t = T - 1 - k;
-        if (t >= 0) ring[k].load(sp + (size_t)t * row_stride);
-    }
-
+    static_for<DEPTH>([&](auto k) {
+        ring[k].load(pre + sc_lane);
+        pre -= (int)k < T - 1 ? row_stride : 0;
+    });
     int buf = 0;
-#pragma unroll
-    for (int i = 0; i < SPL; ++i) vec[g][0][Vec::at(r, c0 + i)] = 0.f;
     __syncthreads();  // the log table is shared by the whole group
 
-    for (int done = 0; done < T; done += DEPTH) {
-#pragma unroll
-        for (int k = 0; k < DEPTH; ++k) {
-            const int t = T - 1 - done - k;
-            if (t >= 0) {
-                const BwdRow<SPL> row = ring[k];
-                if (t - DEPTH >= 0) ring[k].load(sp + (size_t)(t - DEPTH) * row_stride);
-                chunk_sync<Sh::kMultiWave>();
-                const float4 nx = *reinterpret_cast<const float4 *>(&vec[g][buf][Vec::of(4 * r)]);
-                bwd_update<0, SPL, MODE>(a, nx, row, stay, logtab);
-                buf ^= 1;
-#pragma unroll
-                for (int i = 0; i < SPL; ++i) vec[g][buf][Vec::at(r, c0 + i)] = a[i];
-                if (live) {
-#pragma unroll
-                    for (int i = 0; i < SPL; ++i) out[(size_t)t * S + i * Q] = a[i];
-                }
-            }
+    pipelined<DEPTH>(T, [&](auto k, int j, auto checked) {
+        chunk_sync<Sh::kMultiWave>();
+        const float4 nx = *reinterpret_cast<const float4 *>(&vec[g][buf][Vec::of(4 * r)]);
+        float v[SPL][5];
+        bwd_terms<0, SPL>(v, a, nx, ring[k], stay);
+        if (!checked || j + DEPTH < T) {
+            ring[k].load(pre + sc_lane);
+            pre -= row_stride;
         }
-    }
+        lse5_all<SPL, MODE>(a, v, logtab);
+        buf ^= 1;
+#pragma unroll
+        for (int i = 0; i < SPL; ++i) {
+            vec[g][buf][Vec::at(r, c0 + i)] = a[i];
+            orow[st_lane + i * Q] = a[i];
+        }
+        orow -= S;
+    });
 }
 
 // ---------------------------------------------------------------------------
@@ -472,33 +606,39 @@ __global__ __launch_bounds__((Shape<S, SPL>::kThreads)) void fwd_post_kernel(
     constexpr int Q = Sh::kQuarter;
     __shared__ __attribute__((aligned(16))) float vec[Sh::kChunks][2][S];
     __shared__ float part[2][Sh::kChunks][Sh::kChunkWaves];
-    __shared__ __attribute__((aligned(16))) ofa::LogCell logcells[32];
+    __shared__ __attribute__((aligned(16))) ofa::LogCell logcells[32], centred[ofa::kLogCentredCells];
     __shared__ __attribute__((aligned(16))) float tier_lanes[MODE == OFK_SCAN_TWO_TIER ? Sh::kThreads : 64];
     const int tid = threadIdx.x;
     // this sweep runs beside the beam search, whose waves run at priority 3: trips through the second tier
     // at 1 leave that search alone (2048 chunks of 64 states: search 2.50 ms against 2.59 with 3 here)
-    const LogArgs logtab{logcells, series.c, series.e, tier_lanes + (MODE == OFK_SCAN_TWO_TIER ? (tid & ~63) : 0), 1};
+    const LogArgs logtab{logcells, centred, series.c, series.e, tier_lanes + (MODE == OFK_SCAN_TWO_TIER ? (tid & ~63) : 0), 1};
 
-    if (MODE != OFK_SCAN_FAST && tid < 32) logcells[tid] = ofa::log_cell(tid);
+    fill_log_tables<MODE>(logcells, centred);
     const int g = tid / L, l = tid % L;
     const int s0 = SPL * l, q = s0 >> 2;  // own states s0 .. s0+SPL-1, all in quad q
     const int wave = l / 64;  // wave within the chunk
     int n = blockIdx.x * Sh::kChunks + g;
-    const bool live = n < N;
-    if (!live) n = N - 1;
+    if (n >= N) n = N - 1;
 
-    const size_t row_stride = (size_t)N * kCols * S;
-    const _Float16 *sp = scores + (size_t)n * kCols * S + kCols * s0 + kLead;
-    const float *bp = bwd + (size_t)n * (size_t)(T + 1) * S + s0;
-    float *pp = post + (size_t)n * (size_t)(T + 1) * S + s0;
+    // addresses as in bwd_scan_kernel; the first rows are fetched without a condition for the reason given there
+    const ptrdiff_t row_stride = (ptrdiff_t)N * kCols * S;
+    const int first_chunk = blockIdx.x * Sh::kChunks;
+    const unsigned g_eff = (unsigned)(n - first_chunk);
+    const unsigned sc_lane = g_eff * kCols * S + kCols * s0 + kLead;
+    const unsigned st_lane = g_eff * (unsigned)(T + 1) * S + s0;
+    const _Float16 *pre = scores + (size_t)first_chunk * kCols * S;
+    const size_t blk_off = (size_t)first_chunk * (size_t)(T + 1) * S;
+    const float *bpre = bwd + blk_off;
+    float *prow = post + blk_off;
 
     FwdRow<SPL> ring[DEPTH];
     FloatRun<SPL> bring[DEPTH];
-#pragma unroll
-    for (int k = 0; k < DEPTH; ++k) {
-        if (k < T) ring[k].load(sp + (size_t)k * row_stride);
-        if (k <= T) bring[k].load(bp + (size_t)k * S);
-    }
+    static_for<DEPTH>([&](auto k) {
+        ring[k].load(pre + sc_lane);
+        bring[k].load(bpre + st_lane);
+        pre += (int)k < T - 1 ? row_stride : 0;
+        bpre += (int)k < T ? S : 0;
+    });
 
     // Shift of the softmax exponent.  sum_s exp(fwd+bwd) is the same partition function at
     // every time step, and at t = 0 it lies within log(S) of max_s bwd[0][s]; that maximum,
@@ -506,11 +646,9 @@ __global__ __launch_bounds__((Shape<S, SPL>::kThreads)) void fwd_post_kernel(
     // replaces the per-step maximum (the quotient does not depend on the shift).
     float shift;
     {
-        FloatRun<SPL> b0;
-        b0.load(bp);
-        float m = b0.v[0];
+        float m = bring[0].v[0];
 #pragma unroll
-        for (int i = 1; i < SPL; ++i) m = fmaxf(m, b0.v[i]);
+        for (int i = 1; i < SPL; ++i) m = fmaxf(m, bring[0].v[i]);
         m = group_max<Sh::kGroup>(m);
         if constexpr (Sh::kMultiWave) {
             if ((tid & 63) == 0) part[0][g][wave] = m;
@@ -523,61 +661,59 @@ __global__ __launch_bounds__((Shape<S, SPL>::kThreads)) void fwd_post_kernel(
         shift = m - 10.0f;
     }
 
-    float f[SPL];
+    FloatRun<SPL> fv;  // the state vector
+    float (&f)[SPL] = fv.v;
 #pragma unroll
     for (int i = 0; i < SPL; ++i) f[i] = 0.f;
     int buf = 0;
     __syncthreads();  // the log table is shared by the whole group
 
-    for (int done = 0; done <= T; done += DEPTH) {
+    // row j: its posterior, and the state vector goes to the other lanes
+    auto row = [&](const FloatRun<SPL> &bw) {
+        FloatRun<SPL> e;
+        float total = 0.f;
 #pragma unroll
-        for (int k = 0; k < DEPTH; ++k) {
-            const int t = done + k;
-            if (t <= T) {
-                const FwdRow<SPL> row = ring[k];
-                const FloatRun<SPL> bw = bring[k];
-                if (t + DEPTH < T) ring[k].load(sp + (size_t)(t + DEPTH) * row_stride);
-                if (t + DEPTH <= T) bring[k].load(bp + (size_t)(t + DEPTH) * S);
-
-                // posterior of time step t
-                FloatRun<SPL> e;
-                float total = 0.f;
-#pragma unroll
-                for (int i = 0; i < SPL; ++i) {
-                    e.v[i] = __builtin_amdgcn_exp2f(((f[i] + bw.v[i]) - shift) * kLog2e);
-                    total += e.v[i];
-                }
-                total = group_sum<Sh::kGroup>(total);
-
-                FloatRun<SPL> mine;
-#pragma unroll
-                for (int i = 0; i < SPL; ++i) mine.v[i] = f[i];
-                mine.store(&vec[g][buf][s0]);
-                if constexpr (Sh::kMultiWave) {
-                    if ((tid & 63) == 0) part[buf][g][wave] = total;
-                }
-                chunk_sync<Sh::kMultiWave>();
-                if constexpr (Sh::kMultiWave) {
-                    total = part[buf][g][0];
-#pragma unroll
-                    for (int w = 1; w < Sh::kChunkWaves; ++w) total += part[buf][g][w];
-                }
-                const float inv = __builtin_amdgcn_rcpf(total);
-#pragma unroll
-                for (int i = 0; i < SPL; ++i) e.v[i] *= inv;
-                if (live) e.store(pp + (size_t)t * S);
-
-                if (t < T) {
-                    const float p0 = vec[g][buf][q];
-                    const float p1 = vec[g][buf][q + Q];
-                    const float p2 = vec[g][buf][q + 2 * Q];
-                    const float p3 = vec[g][buf][q + 3 * Q];
-                    fwd_update<0, SPL, MODE>(f, p0, p1, p2, p3, row, stay, logtab);
-                    buf ^= 1;
-                }
-            }
+        for (int i = 0; i < SPL; ++i) {
+            e.v[i] = __builtin_amdgcn_exp2f(((f[i] + bw.v[i]) - shift) * kLog2e);
+            total += e.v[i];
         }
-    }
+        total = group_sum<Sh::kGroup>(total);
+        fv.store(&vec[g][buf][s0]);
+        if constexpr (Sh::kMultiWave) {
+            if ((tid & 63) == 0) part[buf][g][wave] = total;
+        }
+        chunk_sync<Sh::kMultiWave>();
+        if constexpr (Sh::kMultiWave) {
+            total = part[buf][g][0];
+#pragma unroll
+            for (int w = 1; w < Sh::kChunkWaves; ++w) total += part[buf][g][w];
+        }
+        const float inv = __builtin_amdgcn_rcpf(total);
+#pragma unroll
+        for (int i = 0; i < SPL; ++i) e.v[i] *= inv;
+        e.store(prow + st_lane);
+        prow += S;
+    };
+    pipelined<DEPTH>(T, [&](auto k, int j, auto checked) {
+        row(bring[k]);
+        const float p0 = vec[g][buf][q], p1 = vec[g][buf][q + Q];
+        const float p2 = vec[g][buf][q + 2 * Q], p3 = vec[g][buf][q + 3 * Q];
+        float v[SPL][5];
+        fwd_terms<0, SPL>(v, f, p0, p1, p2, p3, ring[k], stay);
+        if (!checked || j + DEPTH < T) {
+            ring[k].load(pre + sc_lane);
+            pre += row_stride;
+        }
+        if (!checked || j + DEPTH <= T) {
+            bring[k].load(bpre + st_lane);
+            bpre += S;
+        }
+        lse5_all<SPL, MODE>(f, v, logtab);
+        buf ^= 1;
+    });
+    static_for<DEPTH>([&](auto k) {
+        if (T % DEPTH == (int)k) row(bring[k]);
+    });
 }
 
 // ---------------------------------------------------------------------------
@@ -586,15 +722,21 @@ __global__ __launch_bounds__((Shape<S, SPL>::kThreads)) void fwd_post_kernel(
 // fwd_post_kernel's lanes take the posterior of a row between two steps of the recursion: an
 // exponential, a sum over the wave, a partial sum through LDS, a reciprocal and a store join the
 // chain of dependent operations of every time step, which is what this sweep's duration is made
-// of (it runs beside the beam search with two waves per SIMD; 512 chunks of 256 states: 1.41 ms
-// against 0.95 ms for the backward sweep, which has no such work).  Here a chunk has twice the
+// of.  Here a chunk has twice the
 // lanes: one half runs the recursion alone, the other half reads every row the first half
 // publishes in LDS for its own exchange anyway, and forms that row's posterior one step behind.
 // Every wave takes one block barrier per time step (plus one at the end and two for the shift).
 // Same arithmetic, same results.  (Letting the second half also sum the finished row over every
 // state's neighbours for the quality stage was measured and dropped: the extra LDS traffic slowed
 // the recursion by more, 0.18 ms, than the sums save that stage, 0.09 ms.)
+//
+// Only two rows are in flight per stream: the kernel shares the memory with the beam search, whose rows
+// lie the same N * C * 2 bytes apart, and both together run at the rate a copy reaches.  More rows in
+// flight spread the accesses over more DRAM pages at once and slow both down (512 chunks of 256 states, this
+// kernel / the search beside it: eight rows 1.52 / 2.09 ms, four 1.23 / 1.20, two 1.15 / 1.10).
 // ---------------------------------------------------------------------------
+constexpr int kRolesDepth = 2;
+
 template <int S, int SPL, int DEPTH>
 __global__ __launch_bounds__((2 * (S / SPL))) void fwd_post_roles_kernel(
     const _Float16 *__restrict__ scores, const float *__restrict__ bwd, float *__restrict__ post, int T,
@@ -605,64 +747,61 @@ __global__ __launch_bounds__((2 * (S / SPL))) void fwd_post_roles_kernel(
     static_assert(L % 64 == 0 && RW > 1, "either job owns several whole waves");
     __shared__ __attribute__((aligned(16))) float vec[2][S];
     __shared__ float part[2][RW];
-    __shared__ __attribute__((aligned(16))) ofa::LogCell logcells[32];
+    __shared__ __attribute__((aligned(16))) ofa::LogCell logcells[32], centred[ofa::kLogCentredCells];
     __shared__ __attribute__((aligned(16))) float tier_lanes[L];
     const int tid = threadIdx.x;
     const int posterior = __builtin_amdgcn_readfirstlane(tid / L);
     const int l = tid % L, lane = tid & 63, wave = l / 64;
     // this kernel runs beside the beam search, whose waves run at priority 3: trips through the second
     // tier at 1 leave that search alone (1.17 ms against 1.22 with 3 here) and cost this sweep nothing
-    const LogArgs logtab{logcells, series.c, series.e, tier_lanes + (l & ~63), 1};
-    if (tid < 32) logcells[tid] = ofa::log_cell(tid);
+    const LogArgs logtab{logcells, centred, series.c, series.e, tier_lanes + (l & ~63), 1};
+    fill_log_tables<OFK_SCAN_TWO_TIER>(logcells, centred);
     const int s0 = SPL * l, q = s0 >> 2;  // own states s0 .. s0+SPL-1, all in quad q
     const int n = blockIdx.x;            // one chunk per workgroup
-    const size_t row_stride = (size_t)N * kCols * S;
+    const ptrdiff_t row_stride = (ptrdiff_t)N * kCols * S;
     auto barrier = [] { chunk_sync<true>(); };
 
     if (!posterior) {
-        const _Float16 *sp = scores + (size_t)n * kCols * S + kCols * s0 + kLead;
+        const _Float16 *pre = scores + (size_t)n * kCols * S;
+        const unsigned sc_lane = kCols * s0 + kLead;
         FwdRow<SPL> ring[DEPTH];
-#pragma unroll
-        for (int k = 0; k < DEPTH; ++k) {
-            if (k < T) ring[k].load(sp + (size_t)k * row_stride);
-        }
-        float f[SPL];
+        static_for<DEPTH>([&](auto k) {  // without a condition, as in bwd_scan_kernel
+            ring[k].load(pre + sc_lane);
+            pre += (int)k < T - 1 ? row_stride : 0;
+        });
+        FloatRun<SPL> fv;
+        float (&f)[SPL] = fv.v;
 #pragma unroll
         for (int i = 0; i < SPL; ++i) f[i] = 0.f;
         int buf = 0;
         barrier();  // the other half exchanges the maxima behind the shift
         barrier();
         __syncthreads();  // the log table
-        for (int done = 0; done <= T; done += DEPTH) {
-#pragma unroll
-            for (int k = 0; k < DEPTH; ++k) {
-                const int t = done + k;
-                if (t <= T) {
-                    const FwdRow<SPL> row = ring[k];
-                    if (t + DEPTH < T) ring[k].load(sp + (size_t)(t + DEPTH) * row_stride);
-                    FloatRun<SPL> mine;
-#pragma unroll
-                    for (int i = 0; i < SPL; ++i) mine.v[i] = f[i];
-                    mine.store(&vec[buf][s0]);  // row t
-                    barrier();
-                    if (t < T) {
-                        const float p0 = vec[buf][q], p1 = vec[buf][q + Q];
-                        const float p2 = vec[buf][q + 2 * Q], p3 = vec[buf][q + 3 * Q];
-                        fwd_update<0, SPL, OFK_SCAN_TWO_TIER>(f, p0, p1, p2, p3, row, stay, logtab);
-                        buf ^= 1;
-                    }
-                }
+        pipelined<DEPTH>(T, [&](auto k, int j, auto checked) {
+            fv.store(&vec[buf][s0]);  // row j
+            barrier();
+            const float p0 = vec[buf][q], p1 = vec[buf][q + Q];
+            const float p2 = vec[buf][q + 2 * Q], p3 = vec[buf][q + 3 * Q];
+            float v[SPL][5];
+            fwd_terms<0, SPL>(v, f, p0, p1, p2, p3, ring[k], stay);
+            if (!checked || j + DEPTH < T) {
+                ring[k].load(pre + sc_lane);
+                pre += row_stride;
             }
-        }
+            lse5_all<SPL, OFK_SCAN_TWO_TIER>(f, v, logtab);
+            buf ^= 1;
+        });
+        fv.store(&vec[buf][s0]);  // row T
+        barrier();
         barrier();  // the other half finishes row T
     } else {
-        const float *bp = bwd + (size_t)n * (size_t)(T + 1) * S + s0;
-        float *pp = post + (size_t)n * (size_t)(T + 1) * S + s0;
+        const float *bpre = bwd + (size_t)n * (size_t)(T + 1) * S;
+        float *prow = post + (size_t)n * (size_t)(T + 1) * S;  // row finished next
         FloatRun<SPL> bring[DEPTH];
-#pragma unroll
-        for (int k = 0; k < DEPTH; ++k) {
-            if (k <= T) bring[k].load(bp + (size_t)k * S);
-        }
+        static_for<DEPTH>([&](auto k) {
+            bring[k].load(bpre + s0);
+            bpre += (int)k < T ? S : 0;
+        });
         // Shift of the softmax exponent, as in fwd_post_kernel: max_s bwd[0][s] - 10.
         float shift;
         {
@@ -681,40 +820,40 @@ __global__ __launch_bounds__((2 * (S / SPL))) void fwd_post_roles_kernel(
         __syncthreads();
         FloatRun<SPL> e;  // terms of the row before, waiting for the sum over the waves
         int buf = 0;
-        auto finish_row = [&](int t) {
-            float total = part[t & 1][0];
+        auto finish_row = [&] {  // the row before the one in vec[buf]
+            float total = part[buf ^ 1][0];
 #pragma unroll
-            for (int w = 1; w < RW; ++w) total += part[t & 1][w];
+            for (int w = 1; w < RW; ++w) total += part[buf ^ 1][w];
             const float inv = __builtin_amdgcn_rcpf(total);
 #pragma unroll
             for (int i = 0; i < SPL; ++i) e.v[i] *= inv;
-            e.store(pp + (size_t)t * S);
+            e.store(prow + s0);
+            prow += S;
         };
-        for (int done = 0; done <= T; done += DEPTH) {
+        auto terms = [&](const FloatRun<SPL> &bw) {
+            FloatRun<SPL> fv;
+            fv.load(&vec[buf][s0]);
+            float total = 0.f;
 #pragma unroll
-            for (int k = 0; k < DEPTH; ++k) {
-                const int t = done + k;
-                if (t <= T) {
-                    const FloatRun<SPL> bw = bring[k];
-                    if (t + DEPTH <= T) bring[k].load(bp + (size_t)(t + DEPTH) * S);
-                    barrier();  // row t is in vec[buf], the partial sums of row t - 1 in part[(t - 1) & 1]
-                    if (t > 0) finish_row(t - 1);
-                    FloatRun<SPL> fv;
-                    fv.load(&vec[buf][s0]);
-                    buf ^= 1;
-                    float total = 0.f;
-#pragma unroll
-                    for (int i = 0; i < SPL; ++i) {
-                        e.v[i] = __builtin_amdgcn_exp2f(((fv.v[i] + bw.v[i]) - shift) * kLog2e);
-                        total += e.v[i];
-                    }
-                    total = group_sum<64>(total);
-                    if (lane == 0) part[t & 1][wave] = total;
-                }
+            for (int i = 0; i < SPL; ++i) {
+                e.v[i] = __builtin_amdgcn_exp2f(((fv.v[i] + bw.v[i]) - shift) * kLog2e);
+                total += e.v[i];
             }
-        }
+            total = group_sum<64>(total);
+            if (lane == 0) part[buf][wave] = total;
+            buf ^= 1;
+        };
+        pipelined<DEPTH>(T + 1, [&](auto k, int j, auto checked) {
+            barrier();  // row j is in vec[buf], the partial sums of row j - 1 in part[buf ^ 1]
+            if ((int)k != 0 || j > 0) finish_row();
+            terms(bring[k]);
+            if (!checked || j + DEPTH <= T) {
+                bring[k].load(bpre + s0);
+                bpre += S;
+            }
+        });
         barrier();
-        finish_row(T);
+        finish_row();
     }
 }
 
@@ -748,28 +887,6 @@ struct FusedShape {
     static_assert(kLanes % 64 == 0, "a direction owns whole wavefronts");
 };
 
-template <int N, typename F>
-__device__ __forceinline__ void static_for(F &&f) {
-    if constexpr (N > 0) {
-        static_for<N - 1>(f);
-        f(std::integral_constant<int, N - 1>{});
-    }
-}
-
-// `count` steps, DEPTH of them unrolled per trip: step(k, j, checked) with k = j % DEPTH a
-// compile-time index; in unchecked trips j + DEPTH + SLACK < count holds for every step, i.e.
-// every prefetch DEPTH steps ahead is in range (of a tensor with SLACK rows fewer than steps).
-template <int DEPTH, int SLACK = 0, typename Step>
-__device__ __forceinline__ void pipelined(int count, Step &&step) {
-    int j0 = 0;
-    for (; j0 + 2 * DEPTH + SLACK <= count; j0 += DEPTH)
-        static_for<DEPTH>([&](auto k) { step(k, j0 + (int)k, std::false_type{}); });
-    for (; j0 < count; j0 += DEPTH)
-        static_for<DEPTH>([&](auto k) {
-            if (j0 + (int)k < count) step(k, j0 + (int)k, std::true_type{});
-        });
-}
-
 __device__ __forceinline__ void block_barrier_lds() { chunk_sync<true>(); }
 
 template <int S, int SPL, int DEPTH, int MODE>
@@ -794,12 +911,12 @@ __global__ __launch_bounds__((FusedShape<S, SPL>::kThreads), 4) void scan_post_k
     __shared__ __attribute__((aligned(16))) float vecF[Sh::kChunks][2][S];
     __shared__ float part[Sh::kChunks][2][2][RW];  // [chunk][direction][parity][wave]
     __shared__ float shift_of[Sh::kChunks];
-    __shared__ __attribute__((aligned(16))) ofa::LogCell logcells[32];
+    __shared__ __attribute__((aligned(16))) ofa::LogCell logcells[32], centred[ofa::kLogCentredCells];
     __shared__ __attribute__((aligned(16))) float tier_lanes[MODE == OFK_SCAN_TWO_TIER ? Sh::kThreads : 64];
     const int tid = threadIdx.x;
-    const LogArgs logtab{logcells, series.c, series.e, tier_lanes + (MODE == OFK_SCAN_TWO_TIER ? (tid & ~63) : 0)};
+    const LogArgs logtab{logcells, centred, series.c, series.e, tier_lanes + (MODE == OFK_SCAN_TWO_TIER ? (tid & ~63) : 0)};
 
-    if (MODE != OFK_SCAN_FAST && tid < 32) logcells[tid] = ofa::log_cell(tid);
+    fill_log_tables<MODE>(logcells, centred);
     const int g = tid / Sh::kChunkThreads, u = tid % Sh::kChunkThreads;
     const int forward = __builtin_amdgcn_readfirstlane(u / L);
     const int l = u % L, wave = l / 64;
@@ -856,7 +973,11 @@ __global__ __launch_bounds__((FusedShape<S, SPL>::kThreads), 4) void scan_post_k
                 }
                 step_sync();
                 const float4 nx = *reinterpret_cast<const float4 *>(&vecB[g][buf][VecB::of(4 * r)]);
-                bwd_update<0, SPL, M>(a, nx, row, stay, logtab);
+                {
+                    float v[SPL][5];
+                    bwd_terms<0, SPL>(v, a, nx, row, stay);
+                    lse5_all<SPL, M>(a, v, logtab);
+                }
                 buf ^= 1;
 #pragma unroll
                 for (int i = 0; i < SPL; ++i) vecB[g][buf][VecB::at(r, c0 + i)] = a[i];
@@ -921,7 +1042,11 @@ __global__ __launch_bounds__((FusedShape<S, SPL>::kThreads), 4) void scan_post_k
                 }
                 prow -= S;
                 const float4 nx = *reinterpret_cast<const float4 *>(&vecB[g][buf][VecB::of(4 * r)]);
-                bwd_update<0, SPL, MODE>(a, nx, row, stay, logtab);
+                {
+                    float v[SPL][5];
+                    bwd_terms<0, SPL>(v, a, nx, row, stay);
+                    lse5_all<SPL, MODE>(a, v, logtab);
+                }
                 buf ^= 1;
                 float total;
 #pragma unroll
@@ -996,7 +1121,11 @@ __global__ __launch_bounds__((FusedShape<S, SPL>::kThreads), 4) void scan_post_k
                 step_sync();
                 const float p0 = vecF[g][buf][q], p1 = vecF[g][buf][q + Q];
                 const float p2 = vecF[g][buf][q + 2 * Q], p3 = vecF[g][buf][q + 3 * Q];
-                fwd_update<0, SPL, M>(f, p0, p1, p2, p3, row, stay, logtab);
+                {
+                    float v[SPL][5];
+                    fwd_terms<0, SPL>(v, f, p0, p1, p2, p3, row, stay);
+                    lse5_all<SPL, M>(f, v, logtab);
+                }
                 buf ^= 1;
                 FloatRun<SPL> mine;
 #pragma unroll
@@ -1072,7 +1201,11 @@ __global__ __launch_bounds__((FusedShape<S, SPL>::kThreads), 4) void scan_post_k
                 if (!checked || j + 1 < cnt2) {
                     const float p0 = vecF[g][buf][q], p1 = vecF[g][buf][q + Q];
                     const float p2 = vecF[g][buf][q + 2 * Q], p3 = vecF[g][buf][q + 3 * Q];
-                    fwd_update<0, SPL, MODE>(f, p0, p1, p2, p3, row, stay, logtab);
+                    {
+                    float v[SPL][5];
+                    fwd_terms<0, SPL>(v, f, p0, p1, p2, p3, row, stay);
+                    lse5_all<SPL, MODE>(f, v, logtab);
+                }
                     buf ^= 1;
                     FloatRun<SPL> mine;
 #pragma unroll
@@ -1129,7 +1262,7 @@ int launch_fwd(int mode, const void *scores, const float *bwd, float *post, int 
             // 512 chunks 1.17 ms against 1.41 ms beside the beam search, 1024 chunks 3.5 against 3.1)
             if constexpr (Sh::kMultiWave && 2 * Sh::kLanes <= 1024) {
                 if ((long)N * (2 * Sh::kLanes / 64) <= 4096) {
-                    hipLaunchKernelGGL((fwd_post_roles_kernel<S, SPL, DEPTH>), dim3(N), dim3(2 * Sh::kLanes), 0, st, sc, bwd, post,
+                    hipLaunchKernelGGL((fwd_post_roles_kernel<S, SPL, kRolesDepth>), dim3(N), dim3(2 * Sh::kLanes), 0, st, sc, bwd, post,
                                        T, N, stay, kSeries);
                     break;
                 }
