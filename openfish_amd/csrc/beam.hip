@@ -112,28 +112,27 @@ __device__ __forceinline__ float wave_max(float x) {
     return lane_f(x, 63);
 }
 // What a lane will store for its three candidates once their ranks are known, worked out in the
-// wait states of the wave maximum: a wave that is alone on its SIMD pays a full issue slot (about
-// eight cycles) for every s_nop, so the two idle cycles each rotate-and-max step needs after its
-// source was written are filled with instructions that had to be issued anyway.
+// wait states of the wave maximum: a wave that is alone on its SIMD pays a full issue slot for every
+// s_nop, so the two idle cycles each rotate-and-max step needs after its source was written are filled
+// with instructions that had to be issued anyway.
 //   h0 = crc2(hash, b0), h1 = crc2(hash, b0 + 1) = h0 ^ kTab1   (b0 is even)
 //   info0 = (lo4 + b0) | from, info1 = info0 | 1, infos = state | from | stay bit
-//   rest = candidate score minus its guide term
-// The lane maximum (one v_max3) opens the block and the read of lane 63, where the six steps leave
-// the wave's maximum, closes it, each with its own wait states filled the same way.
+//   rests = the stay's score cs minus its guide term (the steps' scores are still on their way from LDS)
+// The lane maximum of x0, x1, x2 (one v_max3) opens the block and the read of lane 63, where the six
+// steps leave the wave's maximum, closes it.
 struct NextRecords {
     uint32_t h0, h1, info0, info1, infos;
     float rest0, rest1, rests;
 };
-__device__ __forceinline__ float wave_max_beside_records(float c0, float c1, float cs, NextRecords &n, uint32_t hash,
+__device__ __forceinline__ float wave_max_beside_records(float x0, float x1, float x2, NextRecords &n, uint32_t hash,
                                                          uint32_t b0, uint32_t state, uint32_t from_stay,
-                                                         uint32_t lo4b0, uint32_t from, float g0, float g1,
-                                                         float gs) {
+                                                         uint32_t lo4b0, uint32_t from, float cs, float gs) {
     uint32_t t0, t1, best;
     float x;
     asm volatile(
-        "v_max3_f32 %[x], %[c0], %[c1], %[cs]\n\t"
+        "v_max3_f32 %[x], %[x0], %[x1], %[x2]\n\t"
         "v_xor_b32 %[t0], %[hash], %[b0]\n\t"
-        "v_sub_f32 %[r0], %[c0], %[g0]\n\t"
+        "v_or_b32 %[i0], %[lo4b0], %[from]\n\t"
         "v_max_f32_dpp %[x], %[x], %[x] row_ror:8 row_mask:0xf bank_mask:0xf\n\t"
         "v_bfe_i32 %[t1], %[t0], 1, 1\n\t"
         "v_bfe_i32 %[t0], %[t0], 0, 1\n\t"
@@ -145,22 +144,20 @@ __device__ __forceinline__ float wave_max_beside_records(float c0, float c1, flo
         "v_lshrrev_b32 %[t1], 2, %[hash]\n\t"
         "v_max_f32_dpp %[x], %[x], %[x] row_ror:1 row_mask:0xf bank_mask:0xf\n\t"
         "v_xor_b32 %[h0], %[t0], %[t1]\n\t"
-        "v_sub_f32 %[r1], %[c1], %[g1]\n\t"
+        "v_or_b32 %[i1], 1, %[i0]\n\t"
         "v_max_f32_dpp %[x], %[x], %[x] row_bcast:15 row_mask:0xa bank_mask:0xf\n\t"
         "v_xor_b32 %[h1], %[tab1], %[h0]\n\t"
-        "v_sub_f32 %[rs], %[cs], %[gs]\n\t"
-        "v_max_f32_dpp %[x], %[x], %[x] row_bcast:31 row_mask:0xc bank_mask:0xf\n\t"
-        "v_or_b32 %[i0], %[lo4b0], %[from]\n\t"
         "v_or_b32 %[is], %[state], %[fromstay]\n\t"
+        "v_max_f32_dpp %[x], %[x], %[x] row_bcast:31 row_mask:0xc bank_mask:0xf\n\t"
+        "v_sub_f32 %[rs], %[cs], %[gs]\n\t"
+        "s_nop 0\n\t"
         "v_readlane_b32 %[best], %[x], 63\n\t"
-        "v_or_b32 %[i1], 1, %[i0]\n\t"
         "s_nop 0"
         : [x] "=&v"(x), [best] "=&s"(best), [t0] "=&v"(t0), [t1] "=&v"(t1), [h0] "=&v"(n.h0), [h1] "=&v"(n.h1),
-          [i0] "=&v"(n.info0), [i1] "=&v"(n.info1), [is] "=&v"(n.infos), [r0] "=&v"(n.rest0), [r1] "=&v"(n.rest1),
-          [rs] "=&v"(n.rests)
+          [i0] "=&v"(n.info0), [i1] "=&v"(n.info1), [is] "=&v"(n.infos), [rs] "=&v"(n.rests)
         : [hash] "v"(hash), [b0] "v"(b0), [tab1] "s"(kTab1), [tab2] "s"(kTab2), [lo4b0] "v"(lo4b0), [from] "v"(from),
-          [state] "v"(state), [fromstay] "v"(from_stay), [c0] "v"(c0), [c1] "v"(c1), [cs] "v"(cs), [g0] "v"(g0),
-          [g1] "v"(g1), [gs] "v"(gs));
+          [state] "v"(state), [fromstay] "v"(from_stay), [x0] "v"(x0), [x1] "v"(x1), [x2] "v"(x2), [cs] "v"(cs),
+          [gs] "v"(gs));
     return __uint_as_float(best);
 }
 __device__ __forceinline__ int wave_sum_i(int x) {
@@ -173,16 +170,12 @@ __device__ __forceinline__ int wave_sum_i(int x) {
 }
 __device__ __forceinline__ uint64_t ballot(bool p) { return __builtin_amdgcn_ballot_w64(p); }
 // per lane: yes where the lane's bit of a wave-wide mask is set, no elsewhere; the mask goes into
-// the select as it is (a comparison result the wave already holds in scalar registers).
-// The compiler cannot see into these two statements, so it inserts no wait states for them.  None
-// are due: a scalar pair written by a vector comparison may be read as the mask of a select or as
-// a carry by the next vector instruction (the wait states the architecture asks for after such a
-// write concern lane selects of v_readlane/v_writelane, v_div_fmas and memory instructions).  A
-// mask that is to be read by v_readlane or as an address goes through an s_mov first.
+// the select as it is (a comparison result the wave already holds in scalar registers)
 __device__ __forceinline__ int pick_by_bit(uint64_t mask, int yes, int no) {
-    int r;
-    asm("v_cndmask_b32_e64 %0, %1, %2, %3" : "=v"(r) : "v"(no), "v"(yes), "s"(mask));
-    return r;
+    return __builtin_amdgcn_inverse_ballot_w64(mask) ? yes : no;
+}
+__device__ __forceinline__ float pick_by_bit(uint64_t mask, float yes, float no) {
+    return __builtin_amdgcn_inverse_ballot_w64(mask) ? yes : no;
 }
 // x + (the lane's bit of mask), one add-with-carry
 __device__ __forceinline__ int add_bit_of(int x, uint64_t mask) {
@@ -529,10 +522,8 @@ __global__ __launch_bounds__(128 * CPG) void beam_kernel(const _Float16 *__restr
         score = e.rest;
     }
     int state = (int)(info & 1023u);
-    want = crc2_inverse(hash, (uint32_t)state & 3u);
     int w = kW;
     ofk_beam_slot_t *bv = beam + (size_t)n * (size_t)(T + 1) * kW;
-    bv[i] = (ofk_beam_slot_t)state;
 
     // The search is a chain of dependent short instructions; when it shares a SIMD with
     // throughput-bound waves (the forward scan runs at the same time) it should win the
@@ -562,14 +553,29 @@ __global__ __launch_bounds__(128 * CPG) void beam_kernel(const _Float16 *__restr
     // ring addresses: the same in every lane, kept in scalar registers
     const uint32_t ring_s = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uintptr_t)(lds_u32 *)&row_s[0][0]);
     const uint32_t ring_b = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uintptr_t)(lds_u32 *)&row_b[0][0]);
-    auto fetch_row = [&](int tt) {
+    auto wait_row = [&](int tt) {
         while (__builtin_expect(rows_ready <= tt, 0)) {  // the counter is one LDS word: the same value in every lane
             rows_ready = __builtin_amdgcn_readfirstlane(observe(&sh.ready));
             if (rows_ready <= tt) __builtin_amdgcn_s_sleep(1);
         }
+    };
+    // ring addresses of row tt, worked out ahead of the wait for the beam they are used with
+    uint32_t rs, rb;
+    auto locate_row = [&](int tt) {
         const uint32_t slot = (uint32_t)tt % (uint32_t)LR;
-        const uint32_t rs = ring_s + slot * (uint32_t)(2 * COLS * S);  // scalar
-        const uint32_t rb = ring_b + slot * (uint32_t)(4 * S);
+        rs = ring_s + slot * (uint32_t)(2 * COLS * S);
+        rb = ring_b + slot * (uint32_t)(4 * S);
+        asm volatile("" : "+s"(rs), "+s"(rb));
+    };
+    auto fetch_row = [&](int tt) {
+        // hash index of the beam this step starts from; dead lanes file their leftovers apart
+        tagv = ((uint32_t)(tt + 1) << 5) | (uint32_t)i;
+        const uint32_t own = (uint32_t)pick_by_bit(vm, (int)and_or(hash, kBucketBits, idx_base), (int)idx_dump);
+        lds_u32 *own_p = (lds_u32 *)(uintptr_t)own;
+        own_p[0] = hash;
+        own_p[1] = tagv;
+        __builtin_amdgcn_sched_barrier(0);  // the entries go out first, the row is asked for next: `want` takes a while
+        wave_fence();  // one wave's LDS operations are carried out in order: the reads below see every lane's entry
         // scores of the candidates with bases b0, b0 + 1: rs[COLS * (lo4 + b0 + {0,1}) + (COLS - 4) + top];
         // guide terms rb[lo4 + b0 + {0,1}] and rb[state]
         const uint32_t st4 = (uint32_t)state << 2;
@@ -584,23 +590,26 @@ __global__ __launch_bounds__(128 * CPG) void beam_kernel(const _Float16 *__restr
         r1h = *(const lds_u16 *)(uintptr_t)(at_s + 2u * (COLS - 4) + 2u * COLS);
         g01 = lds_load_f2((cand << 2) + rb);
         gst = lds_load_f(st4 + rb);
-        // hash index of the beam this step starts from; dead lanes file their leftovers apart
-        tagv = ((uint32_t)(tt + 1) << 5) | (uint32_t)i;
-        const uint32_t own = (uint32_t)pick_by_bit(vm, (int)and_or(hash, kBucketBits, idx_base), (int)idx_dump);
-        const uint32_t wanted = and_or(want, kBucketBits, idx_base);
-        lds_u32 *own_p = (lds_u32 *)(uintptr_t)own;
-        own_p[0] = hash;
-        own_p[1] = tagv;
-        wave_fence();  // one wave's LDS operations are carried out in order: the reads below see every lane's entry
-        probe = lds_load_u2(wanted);
+        __builtin_amdgcn_sched_barrier(0);
+        want = crc2_inverse(hash, (uint32_t)state & 3u);
+        probe = lds_load_u2(and_or(want, kBucketBits, idx_base));
         mine_back = own_p[1];
     };
+    wait_row(0);
+    locate_row(0);
     fetch_row(0);
     const uint64_t replay_all = (flags & 1) ? ~0ull : 0ull;
+    ofk_beam_slot_t *bv_row = bv;  // row t of the persisted slots
     // One time step.  The last one (LAST) differs in what it hands on (nothing is fetched for a next
     // step, the best survivor goes to slot 0) and is compiled apart, so that the others carry no
     // test for it.
-    auto step = [&](const int t, auto last_tag) {
+    //
+    // The wave is alone on its SIMD: a step costs its instructions, about four cycles each, plus the
+    // LDS round trips and the reads of comparison masks by the scalar unit (about twenty cycles) that
+    // nothing is placed into (about 1370 cycles for 1 chunk of 256 states: 0.93 ms at T = 1666; in the order of the
+    // text, with every wait where its value is first needed, 1.02 ms).  Hence the order below: what does not depend on a round trip is issued
+    // while it is under way, comparisons are issued in groups whose masks are read afterwards.
+    auto step = [&](const int next_t, auto last_tag) {  // next_t - 1 is the time step
         constexpr bool LAST = decltype(last_tag)::value;
         const uint64_t vs = vm & 0x5555555555555555ull;  // the stay candidates sit on the even lanes
         const int lo4 = (state << 2) & (S - 1);
@@ -609,19 +618,16 @@ __global__ __launch_bounds__(128 * CPG) void beam_kernel(const _Float16 *__restr
         float c0 = add_half(r0h, score) + g01.x;
         float c1 = add_half(r1h, score) + g01.y;
         float cs = (score + stay_h) + gst;
-        publish(&sh.consumed, t + 1);  // everything this step needs of row t is in registers
-        const uint32_t gen = (uint32_t)(t + 1) << 5;
+        lds_store_f2(cand_mine, c0, c1);  // for the merges below
+        const uint32_t gen = (uint32_t)next_t << 5;
 
         // which previous element j has hash_j == want_i: off the index if every live element found its
         // own entry intact, else by comparing with every hash
-        uint32_t j;
-        uint64_t mine_mask;  // live even lanes whose stay has a partner
-        const uint64_t stale = (ballot(mine_back != tagv) & vm) | replay_all;
-        if (__builtin_expect(stale == 0, 1)) {
-            const uint32_t d = probe.y - gen;  // below 32: an entry of this generation, and d is its slot
-            mine_mask = ballot(d < 32u) & ballot(probe.x == want) & vs;
-            j = d & 31u;
-        } else {
+        const uint32_t d = probe.y - gen;  // below 32: an entry of this generation, and d is its slot
+        const uint64_t moved = ballot(mine_back != tagv), recent = ballot(d < 32u), equal = ballot(probe.x == want);
+        uint32_t j = d & 31u;
+        uint64_t mine_mask = recent & equal & vs;  // live even lanes whose stay has a partner
+        if (__builtin_expect(((moved & vm) | replay_all) != 0, 0)) {
             // Two live elements in one bucket (or with one hash).  Bit k of m says whether hash k of this
             // half of the beam equals `want`: each comparison is shifted into an accumulator with an
             // add-with-carry (a = 2a + equal), two accumulators so that no instruction waits for the one
@@ -692,7 +698,6 @@ __global__ __launch_bounds__(128 * CPG) void beam_kernel(const _Float16 *__restr
             const uint32_t claimed = sh.claim[claim_at];
             const uint32_t odd = (match & (match - 1u)) | (claimed ^ (uint32_t)i);
             if ((ballot(odd != 0u) & mine_mask) != 0 || (flags & 1)) {
-                lds_store_f2(cand_mine, c0, c1);
                 if (h == 0) sh.stay_score[i] = cs;
                 wave_fence();
                 if (lane == 0) {
@@ -723,112 +728,128 @@ __global__ __launch_bounds__(128 * CPG) void beam_kernel(const _Float16 *__restr
         }
 
         // merge stays with the step spelling the same sequence (src/beam_search.c:281-316).  Every lane
-        // files its two step candidates; a stay with a partner reads the partner's score, folds the
+        // has filed its two step candidates; a stay with a partner reads the partner's score, folds the
         // two, keeps its half of the outcome and overwrites the partner with the other half; every
         // lane reads its step candidates back.  Lanes without a merge go through the same
         // instructions with whatever their registers hold and a dump slot as target: no exec
         // masking on the way.  Conditions are kept as wave-wide masks in scalar registers and combined
         // there; a select takes its mask as it is.
-        if (__builtin_expect(mine_mask != 0, 1)) {
-            lds_store_f2(cand_mine, c0, c1);
-            uint32_t at;  // the partner: step candidate 4j + last base of this element
-            asm("v_lshl_add_u32 %0, %1, 4, %2" : "=v"(at) : "v"(j), "v"(cand_base + (((uint32_t)state & 3u) << 2)));
+        uint32_t at;  // the partner: step candidate 4j + last base of this element
+        asm("v_lshl_add_u32 %0, %1, 4, %2" : "=v"(at) : "v"(j), "v"(cand_base + (((uint32_t)state & 3u) << 2)));
+        wave_fence();
+        const float other = lds_load_f(at);
+        // meanwhile: everything this step needs of row t is in registers; and the slot the traceback
+        // reads is persisted (src/beam_search.c:417-427).  Both halves hold the same element and store the
+        // same slot; slots past the width are never followed by the traceback.
+        bv_row[i] = (ofk_beam_slot_t)info;
+        bv_row += kW;
+        // no wait before this store: the wave's reads of row t are ahead of it in the LDS queue
+        __hip_atomic_store(&sh.consumed, next_t, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        const uint64_t stay_wins = ballot(cs > other) & mine_mask;
+        const uint64_t step_wins = mine_mask & ~stay_wins;
+        const uint32_t target = (uint32_t)pick_by_bit(mine_mask, (int)at, (int)cand_dump);
+        // the fold from hardware exp/log where that provably rounds like the CPU path's double
+        // arithmetic (all but a few merges in a thousand at usual score magnitudes)
+        bool settled;
+        float folded = log_sum_exp_estimate(cs, other, settled);
+        lds_store_f(target, pick_by_bit(step_wins, folded, -FLT_MAX));
+        wave_fence();
+        f32x2 c01 = lds_load_f2(cand_mine);
+        if (__builtin_expect((ballot(!settled) & mine_mask) != 0, 0)) {
+            folded = log_sum_exp(cs, other, lse);
+            lds_store_f(target, pick_by_bit(step_wins, folded, -FLT_MAX));
             wave_fence();
-            const float other = lds_load_f(at);
-            const uint64_t stay_wins = ballot(cs > other) & mine_mask;
-            const uint64_t step_wins = mine_mask & ~stay_wins;
-            // the fold from hardware exp/log where that provably rounds like the CPU path's double
-            // arithmetic (all but a few merges in a thousand at usual score magnitudes)
-            bool settled;
-            float folded = log_sum_exp_estimate(cs, other, settled);
-            if (__builtin_expect((ballot(!settled) & mine_mask) != 0, 0)) folded = log_sum_exp(cs, other, lse);
-            const uint32_t target = (uint32_t)pick_by_bit(mine_mask, (int)at, (int)cand_dump);
-            lds_store_f(target, __int_as_float(pick_by_bit(step_wins, __float_as_int(folded), __float_as_int(-FLT_MAX))));
-            cs = __int_as_float(pick_by_bit(stay_wins, __float_as_int(folded), __float_as_int(cs)));
-            cs = __int_as_float(pick_by_bit(step_wins, __float_as_int(-FLT_MAX), __float_as_int(cs)));
-            wave_fence();
-            const f32x2 c01 = lds_load_f2(cand_mine);
-            c0 = c01.x;
-            c1 = c01.y;
+            c01 = lds_load_f2(cand_mine);
         }
 
         // cut-off (src/beam_search.c:320-381)
         // Dead lanes carry -FLT_MAX as their score, which absorbs whatever is added: their candidates
         // are -FLT_MAX exactly (the stay of an odd lane: -FLT_MAX or -inf, see stay_h).
+        // The best score does not wait for the step candidates to come back: a fold is not below either of
+        // the two scores it joins, so the maximum of the scores before the merges and of the folds is that after them.
+        const float stay_or_fold = pick_by_bit(mine_mask, folded, cs);
+        cs = pick_by_bit(step_wins, -FLT_MAX, stay_or_fold);
         NextRecords next;
-        const float best = wave_max_beside_records(c0, c1, cs, next, hash, (uint32_t)b0, (uint32_t)state, from_stay,
-                                                   (uint32_t)(lo4 + b0), from, g01.x, g01.y, gst);
+        const float best = wave_max_beside_records(c0, c1, stay_or_fold, next, hash, (uint32_t)b0, (uint32_t)state, from_stay,
+                                                   (uint32_t)(lo4 + b0), from, cs, gst);
+        c0 = c01.x;
+        c1 = c01.y;
+        next.rest0 = c0 - g01.x;
+        next.rest1 = c1 - g01.y;
 
-        float cut = best - log_cut;  // may be -FLT_MAX (no cut at all): mask the dead lanes
-        uint64_t k0 = ballot(c0 >= cut) & vm, k1 = ballot(c1 >= cut) & vm, ks = ballot(cs >= cut) & vs;
-        int kept = popc64(k0) + popc64(k1) + popc64(ks);
-        bool overfull = false;  // more candidates than the width pass the final cut (the same in every lane)
-        if (__builtin_expect(kept > kW, 1)) {
+        // Nearly every step has more candidates above the first cut than the width, and goes on to the cut
+        // halfway to the best score: both are counted at once.
+        float lo = best - log_cut;  // may be -FLT_MAX (no cut at all): mask the dead lanes
+        float hi = best;
+        float cut = (lo + hi) / 2.0f;
+        const uint64_t a0 = ballot(c0 >= lo), a1 = ballot(c1 >= lo), as = ballot(cs >= lo);
+        uint64_t k0 = ballot(c0 >= cut), k1 = ballot(c1 >= cut), ks = ballot(cs >= cut);
+        int kept = popc64(a0 & vm) + popc64(a1 & vm) + popc64(as & vs);
+        // kept candidates on lower lanes: masked bit counts
+        auto lower = [&](uint64_t mask, int start) {
+            return (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32),
+                                                  __builtin_amdgcn_mbcnt_lo((uint32_t)mask, (uint32_t)start));
+        };
+        if (__builtin_expect(kept <= kW, 0)) {
+            k0 = a0 & vm;
+            k1 = a1 & vm;
+            ks = as & vs;
+        } else {
             // Bisection between the cut and the best score.  Every cut tried in here lies above
             // (-FLT_MAX + best) / 2, so dead lanes and dropped candidates never pass and the
             // ballots need no mask.  (lo + hi) / 2 is the CPU path's (cut + hi) / 2 or
-            // (cut + lo) / 2: one of the two bounds is the cut just tried.
-            float lo = cut, hi = best;
-            bool found = false;
+            // (cut + lo) / 2: one of the two bounds is the cut just tried.  Both cuts that can come next
+            // are worked out while the masks of the present one are on their way to the scalar unit.
 #pragma unroll
             for (int guess = 2; guess < 10; ++guess) {
+                if (guess > 2) {
+                    k0 = ballot(c0 >= cut);
+                    k1 = ballot(c1 >= cut);
+                    ks = ballot(cs >= cut);
+                }
+                const float next_up = (cut + hi) / 2.0f, next_down = (lo + cut) / 2.0f;
+                kept = popc64(k0) + popc64(k1) + popc64(ks);
+                if ((unsigned)(kept - (kW * 8) / 10) <= (unsigned)(kW - (kW * 8) / 10)) goto cut_found;  // 25..32 kept
                 const bool up = kept > kW;
                 lo = up ? cut : lo;
                 hi = up ? hi : cut;
-                cut = (lo + hi) / 2.0f;
-                k0 = ballot(c0 >= cut);
-                k1 = ballot(c1 >= cut);
-                ks = ballot(cs >= cut);
-                kept = popc64(k0) + popc64(k1) + popc64(ks);
-                if ((unsigned)(kept - (kW * 8) / 10) <= (unsigned)(kW - (kW * 8) / 10)) {  // 25..32 kept
-                    found = true;
-                    break;
-                }
+                cut = up ? next_up : next_down;
             }
-            if (__builtin_expect(!found, 0)) {
-                // The tenth guess: the CPU path moves its bounds once more, tries a cut whose count it
-                // never looks at, and settles for the upper bound, whatever that keeps.
-                hi = kept > kW ? hi : cut;
-                cut = hi;
-                k0 = ballot(c0 >= cut);
-                k1 = ballot(c1 >= cut);
-                ks = ballot(cs >= cut);
-                kept = popc64(k0) + popc64(k1) + popc64(ks);
-                overfull = kept > kW;
-                if (overfull) kept = kW;
+            // The tenth guess: the CPU path moves its bounds once more, tries a cut whose count it
+            // never looks at, and settles for the upper bound, whatever that keeps: of more candidates
+            // than the width the first ones, in candidate order, stay.
+            cut = hi;
+            k0 = ballot(c0 >= cut);
+            k1 = ballot(c1 >= cut);
+            ks = ballot(cs >= cut);
+            kept = popc64(k0) + popc64(k1) + popc64(ks);
+            if (kept > kW) {
+                const int rank0 = lower(k1, lower(k0, 0));
+                const int rank1 = rank0 + (int)((k0 >> lane) & 1);
+                const int ranks = lower(ks, popc64(k0) + popc64(k1));
+                k0 &= ballot(rank0 < kW);
+                k1 &= ballot(rank1 < kW);
+                ks &= ballot(ranks < kW);
+                kept = kW;
             }
         }
+    cut_found:
 
         // survivors in candidate order: steps (i, b) by i then b, then stays by i
+        typedef uint32_t u32x3 __attribute__((ext_vector_type(3)));
+        u32x3 e;
         {
-            // The masks may come straight from vector compares; the selects below are written as
-            // instructions and read them as scalar operands, which a vector instruction may do only two
-            // instructions after a vector instruction wrote them: scalar copies are safe to read at once.
-            asm volatile("s_mov_b64 %0, %0\n\ts_mov_b64 %1, %1\n\ts_mov_b64 %2, %2" : "+s"(k0), "+s"(k1), "+s"(ks));
-            // kept candidates on lower lanes: masked bit counts
-            auto lower = [&](uint64_t mask, int start) {
-                return (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32),
-                                                      __builtin_amdgcn_mbcnt_lo((uint32_t)mask, (uint32_t)start));
-            };
             // k0, k1 and ks hold this lane's own verdicts at its bit (dead lanes and the stays of the odd
             // lanes never pass): the masks select directly, nothing is compared again
             const int rank0 = lower(k1, lower(k0, 0));
             const int rank1 = add_bit_of(rank0, k0);
             const int ranks = lower(ks, popc64(k0) + popc64(k1));
             // every lane stores all three of its candidates, the ones that are dropped into its own dump
-            // slot: no exec masking on the path from the cut-off to the next beam.  Kept candidates
-            // beyond the width exist only after the ten-guess exit of the bisection; a branch that is
-            // almost never taken sends them to the dump slot as well.
+            // slot: no exec masking on the path from the cut-off to the next beam
             const int dump = kW + lane;
-            int slot0 = pick_by_bit(k0, rank0, dump);
-            int slot1 = pick_by_bit(k1, rank1, dump);
-            int slots = pick_by_bit(ks, ranks, dump);
-            if (__builtin_expect(overfull, 0)) {
-                asm volatile("");  // keeps this a branch instead of three selects on every step
-                slot0 = slot0 >= kW ? dump : slot0;
-                slot1 = slot1 >= kW ? dump : slot1;
-                slots = slots >= kW ? dump : slots;
-            }
+            const int slot0 = pick_by_bit(k0, rank0, dump);
+            const int slot1 = pick_by_bit(k1, rank1, dump);
+            const int slots = pick_by_bit(ks, ranks, dump);
             if constexpr (LAST) {
                 // the last beam is ranked by its candidate scores (src/beam_search.c:398-414)
                 next.rest0 = c0;
@@ -836,7 +857,6 @@ __global__ __launch_bounds__(128 * CPG) void beam_kernel(const _Float16 *__restr
                 next.rests = cs;
             }
             const uint32_t elem_base = (uint32_t)(uintptr_t)(lds_u32 *)&sh.elem[0].hash;
-            typedef uint32_t u32x3 __attribute__((ext_vector_type(3)));
             auto put = [&](int slot, uint32_t hsh, uint32_t inf, float rst) {
                 uint32_t at_elem;
                 asm("v_lshl_add_u32 %0, %1, 4, %2" : "=v"(at_elem) : "v"(slot), "v"(elem_base));
@@ -850,44 +870,41 @@ __global__ __launch_bounds__(128 * CPG) void beam_kernel(const _Float16 *__restr
             put(slot1, next.h1, next.info1, next.rest1);
             put(slots, hash, next.infos, next.rests);
             wave_fence();
+            // every lane reads its slot; slots past the new width hold leftovers: they count as dead through
+            // their score and persist as zero, which is what the CPU path's untouched slots hold (a beam
+            // cut below 1 empties the beam, and the traceback then walks such slots)
+            e = *(const LDS_AS u32x3 *)(uintptr_t)(elem_base + 16u * (uint32_t)i);
         }
         w = kept;
         vm = w > 0 ? ~0ull >> (64 - 2 * w) : 0ull;  // (the best candidate is always kept: w is zero only after NaN scores)
-        // every lane reads its slot; slots past the new width hold leftovers: they count as dead through
-        // their score and persist as zero, which is what the CPU path's untouched slots hold (a beam
-        // cut below 1 empties the beam, and the traceback then walks such slots)
-        {
-            typedef uint32_t u32x3 __attribute__((ext_vector_type(3)));
-            const u32x3 e = *(const LDS_AS u32x3 *)(uintptr_t)((uint32_t)(uintptr_t)(lds_u32 *)&sh.elem[0].hash + 16u * (uint32_t)i);
-            hash = e.x;
-            info = (uint32_t)pick_by_bit(vm, (int)e.z, 0);
-            score = __int_as_float(pick_by_bit(vm, __float_as_int(__uint_as_float(e.y)), __float_as_int(-FLT_MAX)));
+        if constexpr (!LAST) {
+            wait_row(next_t);
+            locate_row(next_t);
+            __builtin_amdgcn_sched_barrier(0);
         }
+        hash = e.x;
+        info = (uint32_t)pick_by_bit(vm, (int)e.z, 0);
+        score = pick_by_bit(vm, __uint_as_float(e.y), -FLT_MAX);
         state = (int)(info & 1023u);
-        want = crc2_inverse(hash, (uint32_t)state & 3u);
-        if constexpr (!LAST) fetch_row(t + 1);
+        if constexpr (!LAST) fetch_row(next_t);
 
         // last block: the best survivor goes to slot 0 (src/beam_search.c:398-414)
         if constexpr (LAST) {
             const bool in = i < w;
             const float top_score = wave_max(score);
-            const uint64_t at = ballot(in && h == 0 && score == top_score);
-            const int arg_lane = (top_score > -FLT_MAX && at != 0) ? __builtin_ctzll(at) : 0;  // an even lane
+            const uint64_t at_top = ballot(in && h == 0 && score == top_score);
+            const int arg_lane = (top_score > -FLT_MAX && at_top != 0) ? __builtin_ctzll(at_top) : 0;  // an even lane
             const int arg = arg_lane >> 1;
             if (arg != 0) {
                 const uint32_t in0 = lane_u(info, 0), ina = lane_u(info, arg_lane);
                 if (i == 0) info = ina;
                 if (i == arg) info = in0;
             }
+            bv_row[i] = (ofk_beam_slot_t)info;
         }
-
-        // persist the slot (src/beam_search.c:417-427); the guide term was dropped again by the lane
-        // that held the candidate, which had the term at hand.  Both halves hold the same element
-        // and store the same slot; slots past the width are never followed by the traceback
-        bv[(size_t)(t + 1) * kW + i] = (ofk_beam_slot_t)info;
     };
-    for (int t = 0; t < T - 1; ++t) step(t, std::false_type{});
-    step(T - 1, std::true_type{});
+    for (int next_t = 1; next_t < T; ++next_t) step(next_t, std::false_type{});
+    step(T, std::true_type{});
 
     // ---- traceback from slot 0 of the last block (src/beam_search.c:432-439) ----
     // Followed one row at a time the walk is a chain of T dependent LDS reads.  It is done per block
