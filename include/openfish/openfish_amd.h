@@ -171,7 +171,8 @@ void openfish_amd_decode_wait(const openfish_gpubuf_t *gpubuf, const uint8_t **m
 
 enum openfish_amd_stage {
     OPENFISH_AMD_STAGE_BWD = 0,   /* backward scan kernel (0 when both scans ran as one kernel) */
-    OPENFISH_AMD_STAGE_FWD = 1,   /* forward + posterior kernel (0 when both scans ran as one kernel) */
+    OPENFISH_AMD_STAGE_FWD = 1,   /* forward + posterior kernel (0 when both scans ran as one kernel; equal to the
+                                   * next where they ran within the beam search's kernel) */
     OPENFISH_AMD_STAGE_BEAM = 2,  /* beam search + traceback kernel */
     OPENFISH_AMD_STAGE_SEQ = 3,   /* quality + sequence kernel */
     OPENFISH_AMD_STAGE_TOTAL = 4, /* first launch to last kernel end, device side */

@@ -36,6 +36,7 @@
 #include <type_traits>
 
 #include "kernels.h"
+#include "lse5.h"
 
 namespace {
 
@@ -78,10 +79,6 @@ __device__ __forceinline__ uint32_t crc32_word(uint32_t crc, uint32_t word) {
     return crc;
 }
 
-template <int CTRL>
-__device__ __forceinline__ float dpp(float x) {
-    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), CTRL, 0xF, 0xF, true));
-}
 __device__ __forceinline__ float lane_f(float x, int lane) {
     return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(x), lane));
 }
@@ -322,11 +319,14 @@ struct RowRegs {
 };
 
 
-template <int S>
+// FWD is the number of waves per chunk that run the forward recursion beside the search (0: the search alone).
+template <int S, int FWD>
 struct BeamCfg {
     static constexpr int kBits = S == 64 ? 6 : S == 256 ? 8 : 10;
-    static constexpr int kLdsRows = S >= 1024 ? 3 : S >= 256 ? 4 : 6;  // LDS ring depth
-    static constexpr int kRegRows = S >= 1024 ? 3 : 6;  // rows in flight in registers (3 or 6)
+    // two waves of recursion at 256 states is the choice for two workgroups per compute unit: 80 KB of LDS each
+    static constexpr bool kDense = FWD == 2;
+    static constexpr int kLdsRows = FWD == 0 ? (S >= 1024 ? 3 : S >= 256 ? 4 : 6) : (kDense ? 3 : 4);  // LDS ring depth
+    static constexpr int kRegRows = S >= 1024 ? (FWD == 0 ? 3 : 2) : (kDense ? 3 : 6);  // rows in flight in registers (2, 3 or 6)
 };
 
 // one beam element as handed from one time step to the next: three words of a 16-byte slot, written
@@ -350,30 +350,87 @@ struct BeamShared {
 
 // LDS of one chunk.  Score rows are kept as the caller lays them out: COLS = 4 transitions per
 // state, or 5 with an unused blank first.
-template <int S, int COLS>
-struct BeamRing {
-    _Float16 row_s[BeamCfg<S>::kLdsRows][COLS * S];
-    float row_b[BeamCfg<S>::kLdsRows][S];
+template <int S, int COLS, int FWD>
+struct __attribute__((aligned(16))) BeamRing {
+    _Float16 row_s[BeamCfg<S, FWD>::kLdsRows][COLS * S];
+    float row_b[BeamCfg<S, FWD>::kLdsRows][S];
 };
 // Buckets of the hash index of one chunk (8 bytes each: hash, generation << 5 | slot).  With w
 // live elements two of them share a bucket in about w^2 / (2 * buckets) of the time steps.
-template <int S, int CPG>
+template <int S, int CPG, int FWD>
 struct BeamIdx {
-    static constexpr int kBuckets = (S >= 1024 || CPG > 2) ? 2048 : 4096;
+    static constexpr int kBuckets = (S >= 1024 || CPG > 2 || BeamCfg<S, FWD>::kDense) ? 2048 : 4096;
 };
-template <int S, int COLS>
+// What the forward recursion and the posterior of a chunk share.
+constexpr int kVecRows = 4;  // two would do (see beam_kernel); four let the posterior lag (1024 chunks of 256 states: 2.66 ms against 2.78)
+template <int S, int FWD>
+struct __attribute__((aligned(16))) FwdLds {
+    int published[FWD < 4 ? 4 : FWD];  // rows of the state vector each wave of the recursion has written
+    int taken;                         // rows the posterior's wave has read
+    int pad[3];
+    float vec[kVecRows][S];                   // row t in vec[t % kVecRows]
+    float tier_lanes[64 * FWD];
+};
+template <int S>
+struct FwdLds<S, 0> {};
+struct FwdTables {
+    ofa::LogCell cells[32], centred[ofa::kLogCentredCells];
+};
+struct NoTables {};
+template <int S, int COLS, int FWD>
 struct __attribute__((aligned(16))) BeamLds {
-    BeamRing<S, COLS> ring;
+    BeamRing<S, COLS, FWD> ring;
     BeamShared sh;
     uint2 idx_dump[64];  // where a dead lane files its leftovers instead of a bucket of the index
+    FwdLds<S, FWD> fwd;
 };
 // All LDS of a workgroup, one object: the index tables come first and each is aligned to its
 // size, so that a bucket's address is (hash & bits) | table, one instruction.
-template <int S, int CPG, int COLS>
-struct __attribute__((aligned(BeamIdx<S, CPG>::kBuckets * 8))) BeamGroupLds {
-    uint2 idx[CPG][BeamIdx<S, CPG>::kBuckets];
-    BeamLds<S, COLS> chunk[CPG];
+template <int S, int CPG, int COLS, int FWD>
+struct __attribute__((aligned(16))) BeamGroupLds {
+    uint2 idx[CPG][BeamIdx<S, CPG, FWD>::kBuckets];
+    BeamLds<S, COLS, FWD> chunk[CPG];
     double lse[OFK_LSE_DOUBLES];  // coefficient table of the folds, one copy per workgroup
+    typename std::conditional<FWD == 0, NoTables, FwdTables>::type logs;
+};
+
+// The scores of one lane's states for one step of the recursion, read from a row in LDS: fp16 pairs in
+// 32-bit words.  Five-column rows are read in aligned words (a state's transitions start at a word or in the
+// middle of one, by its parity) and shifted into place.
+template <int SPL, int COLS>
+struct LdsRow {
+    uint32_t w[2 * SPL];
+    __device__ __forceinline__ void load(const _Float16 *row, int s0) {
+        const uint32_t *p = reinterpret_cast<const uint32_t *>(row);
+        if constexpr (COLS == 4) {
+            p += 2 * s0;
+            if constexpr (SPL == 1) {
+                const uint2 x = *reinterpret_cast<const uint2 *>(p);
+                w[0] = x.x; w[1] = x.y;
+            } else {
+#pragma unroll
+                for (int i = 0; i < SPL / 2; ++i) {
+                    const uint4 x = reinterpret_cast<const uint4 *>(p)[i];
+                    w[4 * i] = x.x; w[4 * i + 1] = x.y; w[4 * i + 2] = x.z; w[4 * i + 3] = x.w;
+                }
+            }
+        } else if constexpr (SPL == 1) {
+            p += (5 * s0 + 1) >> 1;
+            const uint32_t a = p[0], b = p[1], c = p[s0 & 1 ? 1 : 2], by = s0 & 1 ? 0u : 16u;
+            w[0] = __builtin_amdgcn_alignbit(b, a, by);
+            w[1] = __builtin_amdgcn_alignbit(c, b, by);
+        } else {
+            p += (5 * s0) >> 1;  // s0 is even
+#pragma unroll
+            for (int i = 0; i < SPL / 2; ++i) {
+                const uint32_t a = p[5 * i], b = p[5 * i + 1], c = p[5 * i + 2];
+                w[4 * i] = __builtin_amdgcn_alignbit(b, a, 16);
+                w[4 * i + 1] = __builtin_amdgcn_alignbit(c, b, 16);
+                w[4 * i + 2] = p[5 * i + 3];
+                w[4 * i + 3] = p[5 * i + 4];
+            }
+        }
+    }
 };
 
 
@@ -382,26 +439,54 @@ struct __attribute__((aligned(BeamIdx<S, CPG>::kBuckets * 8))) BeamGroupLds {
 // to pile onto two SIMDs.  With two chunks a group is four waves, two of them searching;
 // with four chunks it is eight waves and every SIMD holds exactly one search wave and one
 // loader, which is what a batch of more than two chunks per compute unit needs.
-template <int S, int CPG, int COLS>
-__global__ __launch_bounds__(128 * CPG) void beam_kernel(const _Float16 *__restrict__ scores,
-                                                   const float *__restrict__ bwd,
+//
+// FWD > 0: the forward recursion and the posterior of the same chunks run in the same workgroup and read the
+// rows the loader has put into LDS, so that scores and bwd cross HBM once for both.  As two kernels side by
+// side they were bound by that traffic at large batches (1024 chunks of 256 states with five columns: 13.9 GB
+// in 2.98 ms, what a copy reaches; 256 of 1024 states the same in 2.84); here 7.9 GB take 2.54 and 1.74 ms,
+// bound by the vector ALUs and by a step's chain of round trips.
+//   search | posterior | FWD waves of recursion | loader
+// There is no barrier after the set-up: the waves of a chunk hand rows over through counters in LDS.  A wave of
+// the recursion writes its part of row t + 1 of the state vector and then its counter (a wave's LDS operations
+// are carried out in order), and starts on a row once all counters of its chunk have reached it.  Row t + 1
+// takes the place of row t + 1 - kVecRows, which the other waves of the recursion have read if they have
+// published row t (kVecRows >= 2), and the posterior's wave if it says so.  The loader refills a ring slot when
+// search, recursion and posterior are all past it.  A wave only waits for rows that the others can produce
+// without it: loader row t for consumers past row t - LR, recursion step t for row t of the ring and of the vector
+// and the posterior past row t + 1 - kVecRows, the posterior's row t for row t of the vector.  So all waits end.
+// Priorities: search 3, recursion 2 (3 in the second tier), posterior 1; with the recursion at 0 it takes 3 to 5 %
+// more at large batches, with the search below the recursion 256 states lose 0.2 ms at 512 chunks.
+//
+// FWD: one state per lane (4 waves) with one workgroup of two chunks on a compute unit.  Above 512 chunks of 256
+// states two workgroups share a unit (80 KB of LDS, 96 registers per lane): two states per lane and smaller
+// rings.  1024 states: two per lane, one chunk per workgroup (four per lane: 2.15 ms against 1.74 at 256 chunks).
+template <int S, int CPG, int COLS, int FWD>
+constexpr int kBeamThreads = 64 * CPG * (FWD == 0 ? 2 : FWD + 3);
+template <int S, int CPG, int COLS, int FWD>
+__global__ __launch_bounds__((kBeamThreads<S, CPG, COLS, FWD>), (BeamCfg<S, FWD>::kDense ? 5 : 1)) void beam_kernel(const _Float16 *__restrict__ scores,
+                                                   const float *__restrict__ bwd, float *__restrict__ post,
                                                    ofk_beam_slot_t *__restrict__ beam,
                                                    int32_t *__restrict__ states, uint8_t *__restrict__ moves,
                                                    int T, int N, float log_cut, float stay, int flags,
-                                                   const double *__restrict__ lse_table) {
-    using Cfg = BeamCfg<S>;
+                                                   const double *__restrict__ lse_table, LogSeries series) {
+    using Cfg = BeamCfg<S, FWD>;
     constexpr int BITS = Cfg::kBits;
     constexpr int LR = Cfg::kLdsRows;
     constexpr int RR = Cfg::kRegRows;
 
     constexpr int kGroupChunks = CPG;
-    __shared__ BeamGroupLds<S, CPG, COLS> all;
+    // bytes, so that the size is not rounded up to the alignment the index tables want
+    __shared__ __attribute__((aligned(BeamIdx<S, CPG, FWD>::kBuckets * 8))) unsigned char
+        lds_bytes[sizeof(BeamGroupLds<S, CPG, COLS, FWD>)];
+    auto &all = *reinterpret_cast<BeamGroupLds<S, CPG, COLS, FWD> *>(lds_bytes);
     auto &lds = all.chunk;
     auto &lse = all.lse;
 
-    // waves 0 .. kGroupChunks-1 search, the others load; wave k and wave k + kGroupChunks share a chunk
-    const int wave = (int)(threadIdx.x >> 6);
-    const int member = wave % kGroupChunks;
+    // waves 0 .. kGroupChunks-1 search, the last kGroupChunks load; between them those of the forward sweep
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    constexpr int kFirstFwd = 2 * kGroupChunks, kFirstLoader = kGroupChunks * (FWD == 0 ? 1 : FWD + 2);
+    const bool recursion = FWD > 0 && wave >= kFirstFwd && wave < kFirstLoader;
+    const int member = recursion ? (wave - kFirstFwd) / (FWD > 0 ? FWD : 1) : wave % kGroupChunks;
     const int n = blockIdx.x * kGroupChunks + member;
     const int lane = threadIdx.x & 63;
     auto &row_s = lds[member].ring.row_s;
@@ -414,13 +499,125 @@ __global__ __launch_bounds__(128 * CPG) void beam_kernel(const _Float16 *__restr
     if (wave < kGroupChunks && lane == 0) {
         sh.ready = 0;
         sh.consumed = 0;
+        if constexpr (FWD > 0) {
+            for (int x = 0; x < (FWD < 4 ? 4 : FWD); ++x) lds[member].fwd.published[x] = 0;
+            lds[member].fwd.taken = 0;
+        }
     }
-    for (int x = (int)threadIdx.x; x < OFK_LSE_DOUBLES; x += 128 * CPG) lse[x] = lse_table[x];
+    if constexpr (FWD > 0) {
+        static_assert(kBeamThreads<S, CPG, COLS, FWD> >= 160, "the tables are filled by the first 160 threads");
+        fill_log_tables<OFK_SCAN_TWO_TIER>(all.logs.cells, all.logs.centred);
+        static_assert(ofa::kLogCentredCells <= 160, "one cell per thread");
+    }
+    for (int x = (int)threadIdx.x; x < OFK_LSE_DOUBLES; x += kBeamThreads<S, CPG, COLS, FWD>) lse[x] = lse_table[x];
     // the hash index starts empty: no entry may look like one of a real generation (tags start at 1 << 5)
-    for (int x = (int)threadIdx.x; x < kGroupChunks * BeamIdx<S, CPG>::kBuckets; x += 128 * CPG) (&all.idx[0][0])[x] = make_uint2(0u, 0u);
+    for (int x = (int)threadIdx.x; x < kGroupChunks * BeamIdx<S, CPG, FWD>::kBuckets; x += kBeamThreads<S, CPG, COLS, FWD>) (&all.idx[0][0])[x] = make_uint2(0u, 0u);
     __syncthreads();
     if (n >= N) return;  // odd batch: the last group has one chunk
 
+    if constexpr (FWD > 0) {
+        auto &fw = lds[member].fwd;
+        // whether every wave of the recursion has written row t of the state vector: a lane reads one counter
+        auto row_published = [&](int t) {
+            const int rows = __hip_atomic_load(&fw.published[lane & (FWD - 1)], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+            return ballot(rows <= t) == 0;
+        };
+        if (recursion) {
+            // ---- one wave of the forward recursion (same arithmetic as fwd_post_roles_kernel) ----
+            constexpr int SPL = S / (64 * FWD), Q = S / 4;
+            const int w = (wave - kFirstFwd) % FWD;
+            const int s0 = SPL * (64 * w + lane), q = s0 >> 2;
+            const LogArgs logtab{all.logs.cells, all.logs.centred, series.c, series.e, fw.tier_lanes + 64 * w, 3};
+            __builtin_amdgcn_s_setprio(2);
+            float f[SPL];
+#pragma unroll
+            for (int k = 0; k < SPL; ++k) f[k] = 0.f;
+            int rows_ready = 0, rows_taken = 0, slot = 0;
+            auto publish_row = [&](int t) {
+#pragma unroll
+                for (int k = 0; k < SPL; ++k) fw.vec[t % kVecRows][s0 + k] = f[k];
+                wave_fence();
+                __hip_atomic_store(&fw.published[w], t + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+            };
+            publish_row(0);
+            for (int t = 0; t < T; ++t) {
+                while (rows_ready <= t) {
+                    rows_ready = __builtin_amdgcn_readfirstlane(observe(&sh.ready));
+                    if (rows_ready <= t) __builtin_amdgcn_s_sleep(1);
+                }
+                LdsRow<SPL, COLS> row;
+                row.load(row_s[slot], s0);
+                slot = slot + 1 == LR ? 0 : slot + 1;
+                while (rows_taken < t + 2 - kVecRows) {  // rows 0 .. t - 1: row t + 1 goes where row t - 1 was
+                    rows_taken = __builtin_amdgcn_readfirstlane(observe(&fw.taken));
+                    if (rows_taken < t + 2 - kVecRows) __builtin_amdgcn_s_sleep(1);
+                }
+                if constexpr (FWD > 1) {
+                    while (!row_published(t)) {}
+                } else {
+                    wave_fence();
+                }
+                const float *vec = fw.vec[t % kVecRows];
+                const float p0 = vec[q], p1 = vec[q + Q], p2 = vec[q + 2 * Q], p3 = vec[q + 3 * Q];
+                float v[SPL][5];
+#pragma unroll
+                for (int k = 0; k < SPL; ++k) {
+                    v[k][0] = f[k] + stay;
+                    v[k][1] = ::add_half<0>(row.w[2 * k], p0);
+                    v[k][2] = ::add_half<1>(row.w[2 * k], p1);
+                    v[k][3] = ::add_half<0>(row.w[2 * k + 1], p2);
+                    v[k][4] = ::add_half<1>(row.w[2 * k + 1], p3);
+                }
+                lse5_all<SPL, OFK_SCAN_TWO_TIER>(f, v, logtab);
+                __builtin_amdgcn_s_setprio(2);  // a trip through the second tier leaves it at 0
+                publish_row(t + 1);
+            }
+            return;
+        }
+        if (wave >= kGroupChunks && wave < kFirstFwd) {
+            // ---- posterior: softmax over the states of fwd[t] + bwd[t], t = 0 .. T ----
+            __builtin_amdgcn_s_setprio(1);
+            constexpr int G = S / 256;  // pieces of four states per lane
+            static_assert(G >= 1, "a lane holds at least four states");
+            float4 b[G];
+            float top = -FLT_MAX;
+#pragma unroll
+            for (int g = 0; g < G; ++g) {
+                b[g] = *reinterpret_cast<const float4 *>(bw_n + 256 * g + 4 * lane);
+                top = fmaxf(top, fmaxf(fmaxf(b[g].x, b[g].y), fmaxf(b[g].z, b[g].w)));
+            }
+            const float shift = group_max<64>(top) - 10.0f;  // as in fwd_post_kernel
+            float *prow = post + (size_t)n * (size_t)(T + 1) * S + 4 * lane;
+            int slot = 0;
+            for (int t = 0; t <= T; ++t) {
+                while (!row_published(t)) __builtin_amdgcn_s_sleep(2);
+                float4 e[G];
+#pragma unroll
+                for (int g = 0; g < G; ++g) {
+                    e[g] = *reinterpret_cast<const float4 *>(&fw.vec[t % kVecRows][256 * g + 4 * lane]);
+                    if (t > 0) b[g] = *reinterpret_cast<const float4 *>(&row_b[slot][256 * g + 4 * lane]);
+                }
+                if (t > 0) slot = slot + 1 == LR ? 0 : slot + 1;
+                publish(&fw.taken, t + 1);
+                float total = 0.f;
+#pragma unroll
+                for (int g = 0; g < G; ++g) {
+                    e[g].x = __builtin_amdgcn_exp2f(((e[g].x + b[g].x) - shift) * kLog2e);
+                    e[g].y = __builtin_amdgcn_exp2f(((e[g].y + b[g].y) - shift) * kLog2e);
+                    e[g].z = __builtin_amdgcn_exp2f(((e[g].z + b[g].z) - shift) * kLog2e);
+                    e[g].w = __builtin_amdgcn_exp2f(((e[g].w + b[g].w) - shift) * kLog2e);
+                    total += (e[g].x + e[g].y) + (e[g].z + e[g].w);
+                }
+                const float inv = __builtin_amdgcn_rcpf(group_sum<64>(total));
+#pragma unroll
+                for (int g = 0; g < G; ++g)
+                    *reinterpret_cast<float4 *>(prow + 256 * g) = make_float4(e[g].x * inv, e[g].y * inv, e[g].z * inv, e[g].w * inv);
+                prow += S;
+            }
+            return;
+        }
+    }
     if (wave >= kGroupChunks) {
         // ---- loader wave: row t = (scores[t], bwd[t+1]) into ring slot t % LR ----
         // The ring is spelled out as named registers (not an array indexed by a loop that
@@ -437,7 +634,25 @@ __global__ __launch_bounds__(128 * CPG) void beam_kernel(const _Float16 *__restr
             if (t < T) {
                 // the ring is full most of the time (a search step takes about 3000 cycles): poll
                 // seldom, the rows in registers and in the ring leave ample slack for waking up late
-                while (t - observe(&sh.consumed) >= LR) __builtin_amdgcn_s_sleep(8);
+                if constexpr (FWD == 0) {
+                    while (t - observe(&sh.consumed) >= LR) __builtin_amdgcn_s_sleep(8);
+                } else {
+                    // the recursion is done with row p of scores once it has published row p + 1 of its vector,
+                    // the posterior with row p of bwd (bwd[p + 1]) once it has taken row p + 1
+                    auto slots_free = [&] {
+                        int low = observe(&sh.consumed);
+                        const auto &fw = lds[member].fwd;
+                        const int taken = observe(const_cast<int *>(&fw.taken)) - 1;
+                        low = low < taken ? low : taken;
+#pragma unroll
+                        for (int x = 0; x < FWD; ++x) {
+                            const int done = observe(const_cast<int *>(&fw.published[x])) - 1;
+                            low = low < done ? low : done;
+                        }
+                        return low;
+                    };
+                    while (t >= LR && t - slots_free() >= LR) __builtin_amdgcn_s_sleep(2);
+                }
                 const int slot = t % LR;
                 rs.store(reinterpret_cast<char *>(row_s[slot]), lane);
                 rb.store(reinterpret_cast<char *>(row_b[slot]), lane);
@@ -447,7 +662,7 @@ __global__ __launch_bounds__(128 * CPG) void beam_kernel(const _Float16 *__restr
         };
         fetch(s0, g0, 0);
         fetch(s1, g1, 1);
-        fetch(s2, g2, 2);
+        if constexpr (RR >= 3) fetch(s2, g2, 2);
         if constexpr (RR == 6) {
             fetch(s3, g3, 3);
             fetch(s4, g4, 4);
@@ -456,7 +671,7 @@ __global__ __launch_bounds__(128 * CPG) void beam_kernel(const _Float16 *__restr
         for (int t0 = 0; t0 < T; t0 += RR) {
             hand_over(s0, g0, t0);
             hand_over(s1, g1, t0 + 1);
-            hand_over(s2, g2, t0 + 2);
+            if constexpr (RR >= 3) hand_over(s2, g2, t0 + 2);
             if constexpr (RR == 6) {
                 hand_over(s3, g3, t0 + 3);
                 hand_over(s4, g4, t0 + 4);
@@ -469,7 +684,7 @@ __global__ __launch_bounds__(128 * CPG) void beam_kernel(const _Float16 *__restr
     // ---- search wave ----
     const int i = lane >> 1;  // lanes 2i and 2i+1 hold element i; candidate order is lane order
     const int h = lane & 1;
-    constexpr int kBuckets = BeamIdx<S, CPG>::kBuckets;
+    constexpr int kBuckets = BeamIdx<S, CPG, FWD>::kBuckets;
     constexpr uint32_t kBucketBits = (uint32_t)(kBuckets - 1) << 3;  // hash bits that address an 8-byte bucket
     typedef __attribute__((address_space(3))) uint32_t lds_u32;
     // LDS addresses of this chunk's index table (a multiple of its size) and of this lane's spare entry
@@ -921,7 +1136,7 @@ __global__ __launch_bounds__(128 * CPG) void beam_kernel(const _Float16 *__restr
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
     {
         constexpr int RB = 128;  // rows per block
-        static_assert(2 * RB * kW * (int)sizeof(ofk_beam_slot_t) <= BeamIdx<S, CPG>::kBuckets * 8, "two blocks fit the index");
+        static_assert(2 * RB * kW * (int)sizeof(ofk_beam_slot_t) <= BeamIdx<S, CPG, FWD>::kBuckets * 8, "two blocks fit the index");
         int32_t *st_out = states + (size_t)n * T;
         uint8_t *mv_out = moves + (size_t)n * T;
         const uint32_t buf0 = idx_base;  // two buffers of RB rows of 64 bytes, row 127 the newest of a block
@@ -1027,15 +1242,28 @@ int launch_beam(const void *scores, const float *bwd, ofk_beam_slot_t *beam, int
     // where the LDS of four chunks fits (64 and 256 states)
     if constexpr (S <= 256) {
         if (N > OFK_SPARSE_SEARCH_MAX_CHUNKS) {
-            hipLaunchKernelGGL((beam_kernel<S, 4, COLS>), dim3((N + 3) / 4), dim3(512), 0, st,
-                               static_cast<const _Float16 *>(scores), bwd, beam, states, moves, T, N, log_cut,
-                               stay, flags, lse_table);
+            hipLaunchKernelGGL((beam_kernel<S, 4, COLS, 0>), dim3((N + 3) / 4), dim3(512), 0, st,
+                               static_cast<const _Float16 *>(scores), bwd, nullptr, beam, states, moves, T, N, log_cut,
+                               stay, flags, lse_table, LogSeries{});
             return (int)hipGetLastError();
         }
     }
-    hipLaunchKernelGGL((beam_kernel<S, 2, COLS>), dim3((N + 1) / 2), dim3(256), 0, st,
-                           static_cast<const _Float16 *>(scores), bwd, beam, states, moves, T, N, log_cut, stay,
-                           flags, lse_table);
+    hipLaunchKernelGGL((beam_kernel<S, 2, COLS, 0>), dim3((N + 1) / 2), dim3(256), 0, st,
+                           static_cast<const _Float16 *>(scores), bwd, nullptr, beam, states, moves, T, N, log_cut, stay,
+                           flags, lse_table, LogSeries{});
+    return (int)hipGetLastError();
+}
+
+const LogSeries kSeries = {OFA_LOG_SERIES, OFA_EXP_COEFS};
+
+// search, forward recursion and posterior in one workgroup: CPG chunks of it, FWD waves of recursion each
+template <int S, int CPG, int COLS, int FWD>
+int launch_beam_forward(const void *scores, const float *bwd, float *post, ofk_beam_slot_t *beam, int32_t *states,
+                        uint8_t *moves, int T, int N, float log_cut, float stay, int flags, const double *lse_table,
+                        hipStream_t st) {
+    hipLaunchKernelGGL((beam_kernel<S, CPG, COLS, FWD>), dim3((N + CPG - 1) / CPG), dim3(kBeamThreads<S, CPG, COLS, FWD>), 0, st,
+                       static_cast<const _Float16 *>(scores), bwd, post, beam, states, moves, T, N, log_cut, stay, flags,
+                       lse_table, kSeries);
     return (int)hipGetLastError();
 }
 
@@ -1133,4 +1361,25 @@ extern "C" int ofk_beam_search(const void *scores, const float *bwd, ofk_beam_sl
     hipStream_t st = static_cast<hipStream_t>(stream);
     return dispatch_beam(scores, bwd, beam, states, moves, T, N, state_len, columns, log_beam_cut, stay, flags,
                          lse_table, st);
+}
+
+extern "C" int ofk_beam_search_forward(const void *scores, const float *bwd, float *post, ofk_beam_slot_t *beam,
+                                       int32_t *states, uint8_t *moves, int T, int N, int state_len, int columns,
+                                       float log_beam_cut, float stay, const double *lse_table, int flags, void *stream) {
+    if (!scores || !bwd || !post || !beam || !states || !moves || !lse_table || T < 1 || N < 1) return OFK_BAD_ARGS;
+    if ((reinterpret_cast<uintptr_t>(scores) | reinterpret_cast<uintptr_t>(bwd) | reinterpret_cast<uintptr_t>(post) |
+         reinterpret_cast<uintptr_t>(beam)) & 15u)
+        return OFK_BAD_ARGS;
+    hipStream_t st = static_cast<hipStream_t>(stream);
+#define OFK_FORWARD(S, CPG, COLS, FWD) \
+    return launch_beam_forward<S, CPG, COLS, FWD>(scores, bwd, post, beam, states, moves, T, N, log_beam_cut, stay, flags, lse_table, st)
+    const bool dense = N > OFK_SPARSE_SEARCH_MAX_CHUNKS;
+    switch (state_len * 8 + columns) {
+        case 4 * 8 + 4: if (dense) OFK_FORWARD(256, 2, 4, 2); OFK_FORWARD(256, 2, 4, 4);
+        case 4 * 8 + 5: if (dense) OFK_FORWARD(256, 2, 5, 2); OFK_FORWARD(256, 2, 5, 4);
+        case 5 * 8 + 4: OFK_FORWARD(1024, 1, 4, 8);
+        case 5 * 8 + 5: OFK_FORWARD(1024, 1, 5, 8);
+        default: return OFK_BAD_ARGS;
+    }
+#undef OFK_FORWARD
 }

@@ -55,6 +55,12 @@ int ofk_scan_posterior(const void *scores, float *bwd, float *post, int T, int N
 int ofk_beam_search(const void *scores, const float *bwd, ofk_beam_slot_t *beam, int32_t *states,
                     uint8_t *moves, int T, int N, int state_len, int columns, float log_beam_cut, float stay,
                     const double *lse_table, int flags, void *stream);
+/* The search together with the forward sweep and the posterior of the same chunks, one kernel that reads
+ * scores and bwd once for both (256 and 1024 states): the results of ofk_beam_search and of
+ * ofk_fwd_post_scan with the two-tier arithmetic. */
+int ofk_beam_search_forward(const void *scores, const float *bwd, float *post, ofk_beam_slot_t *beam, int32_t *states,
+                            uint8_t *moves, int T, int N, int state_len, int columns, float log_beam_cut, float stay,
+                            const double *lse_table, int flags, void *stream);
 /* The same search with the beam slots and the table in a static device array of the library
  * (OFK_STATIC_SLOT_BYTES of slots: N * (T + 1) * 64 bytes must fit, else OFK_TOO_LARGE and nothing
  * is launched).  ofk_beam_search_static_prepare sets the array up on the current device (looks up

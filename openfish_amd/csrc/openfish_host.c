@@ -136,7 +136,8 @@ typedef struct {
     int timed;
     int pending;           /* a decode has been enqueued and not yet waited for */
     int pend_T, pend_N, pend_sums;    /* its shape */
-    int pend_split;        /* how its scans were queued (which events were recorded) */
+    int pend_split;        /* how its scans were queued (which events were recorded): 0 one kernel, 1 two, 2 the forward
+                            * sweep within the beam search's kernel */
     int scan_mode;         /* OFK_SCAN_*: arithmetic of the scans of this gpubuf's decodes */
     int scan_spl;          /* states per lane of the scans, 0 = chosen from the batch size */
     int debug_flags;       /* bit 0: serial replay of the beam search's merges; bit 1: colliding seed hashes */
@@ -366,26 +367,57 @@ static int split_by_default(int N, int state_len) {
     return state_len <= 4 && (long)N * states_of(state_len) <= 512L * 256L;
 }
 
+/* Whether the forward sweep and the posterior run within the beam search's kernel, after the backward sweep.
+ * Scores and bwd then cross HBM once for both, which is what large batches are bound by; small ones are bound by
+ * the search's own chain, which is a little shorter beside a separate kernel.  Whole decodes, ms, T = 1666, the
+ * better of the other two arrangements | merged:
+ *    256 states:  403 chunks (T = 1201) 1.62 | 1.69,  512 chunks 2.29 | 2.36,  1024 chunks, five columns 4.99 | 4.59
+ *   1024 states:  37 chunks (T = 833) 1.98 | 1.81,  256 chunks, five columns 4.58 | 3.47
+ * A decode that is enqueued shares the machine with others: two of 512 chunks of 256 states at a time took
+ * 4.4 ms with four streams in the process, 5.4 with twelve, whose sweeps then wait in each other's hardware queues
+ * (one kernel on one stream has no second stream to wait for), merged 3.96 either way.
+ * Batches of fewer than 16 chunks of 1024 states keep the one kernel, 64 states their split sweeps (a chunk's
+ * rows are small, the search alone is the longest stage). */
+static int merged_by_default(const ofa_gpubuf_t *g, int N, int state_len, int enqueued) {
+    if (g->split_scans >= 0 || g->scan_mode != OFK_SCAN_TWO_TIER || g->scan_spl != 0) return 0;
+    if (state_len == 4) return enqueued || N > OFK_SPARSE_SEARCH_MAX_CHUNKS;
+    return state_len == 5 && N >= 16;
+}
+
 /* Queue one decode on the gpubuf's streams, results into its pinned staging buffer; returns
  * without waiting for the GPU. */
 static void enqueue_decode(ofa_gpubuf_t *g, const int T, const int N, const int C, const void *scores_TNC,
-                           const int state_len, const openfish_opt_t *options) {
+                           const int state_len, const openfish_opt_t *options, const int enqueued) {
     const float stay = options->blank_score; /* as the reference GPU path, src/decode_hip.hip:120 */
     const size_t nt = (size_t)N * (size_t)T;
 
     join_null_stream(g);
     HIP_OK(hipEventRecord(g->ev[EV_START], g->s_main));
     const int cols = columns_of(C, state_len);
-    g->pend_split = g->split_scans < 0 ? split_by_default(N, state_len) : g->split_scans;
+    const int merged = merged_by_default(g, N, state_len, enqueued);
+    g->pend_split = merged ? 2 : (g->split_scans < 0 ? split_by_default(N, state_len) : g->split_scans);
     /* only where the search leaves the machine idle, and not with 1024 states, whose search waits for
      * memory and was measured to take half as long again beside the extra kernel */
     /* With split scans the posteriors are complete when the forward kernel ends.  With 64 states that is
      * well before the search does (0.83 against 1.13 ms at 512 chunks), and the sums (0.21 ms) fit in
      * between; with 256 states the two end together and the sequence stage gathers by itself. */
     const int sums_fit = g->path_sums != NULL && N <= OFK_SPARSE_SEARCH_MAX_CHUNKS;
-    const int use_sums = sums_fit && (!g->pend_split || state_len == 3);
+    const int use_sums = sums_fit && !merged && (!g->pend_split || state_len == 3);
     g->pend_sums = use_sums;
-    if (!g->pend_split) {
+    if (merged) {
+        /* backward sweep, then the search with the forward sweep and the posterior in its workgroups */
+        launch_ok(ofk_bwd_scan(scores_TNC, g->pub.bwd_NTC, T, N, state_len, cols, stay, g->scan_mode, g->scan_spl, g->s_main),
+                  "bwd_scan");
+        HIP_OK(hipEventRecord(g->ev[EV_BWD_END], g->s_main));
+        HIP_OK(hipEventRecord(g->ev[EV_BEAM_START], g->s_main));
+        launch_ok(ofk_beam_search_forward(scores_TNC, g->pub.bwd_NTC, g->pub.post_NTC, (ofk_beam_slot_t *)g->pub.beam_vector,
+                                          (int32_t *)g->pub.states, g->pub.moves, T, N, state_len, cols,
+                                          log_beam_cut(options), stay, g->lse_table, g->debug_flags, g->s_main),
+                  "beam_search_forward");
+        HIP_OK(hipEventRecord(g->ev[EV_BEAM_END], g->s_main));
+        HIP_OK(hipStreamWaitEvent(g->s_side, g->ev[EV_BEAM_END], 0));
+        HIP_OK(hipMemcpyAsync(g->h_out, g->pub.moves, nt, hipMemcpyDeviceToHost, g->s_side));
+    } else if (!g->pend_split) {
         /* both sweeps and the posterior in one kernel, then the beam search, all on one stream */
         launch_ok(ofk_scan_posterior(scores_TNC, g->pub.bwd_NTC, g->pub.post_NTC, T, N, state_len, cols, stay, g->scan_mode,
                                      g->scan_spl, g->s_main), "scan_posterior");
@@ -461,7 +493,7 @@ void openfish_decode_gpu(const int T, const int N, const int C, void *scores_TNC
     const size_t nt = (size_t)N * (size_t)T;
     OPENFISH_LOG_TRACE("scores tensor dim: %d, %d, %d", T, N, C);
 
-    enqueue_decode(g, T, N, C, scores_TNC, state_len, options);
+    enqueue_decode(g, T, N, C, scores_TNC, state_len, options, 0);
     alloc_outputs(T, N, moves, sequence, qstring);
     HIP_OK(hipStreamSynchronize(g->s_side));
     memcpy(*moves, g->h_out, nt);
@@ -476,7 +508,7 @@ void openfish_amd_decode_enqueue(int T, int N, int C, const void *scores_TNC, in
                                  const openfish_opt_t *options, const openfish_gpubuf_t *gpubuf) {
     check_scores(T, N, C, scores_TNC, state_len, options);
     ofa_gpubuf_t *g = checked(gpubuf, T, N, state_len);
-    enqueue_decode(g, T, N, C, scores_TNC, state_len, options);
+    enqueue_decode(g, T, N, C, scores_TNC, state_len, options, 1);
 }
 
 void openfish_amd_decode_wait(const openfish_gpubuf_t *gpubuf, const uint8_t **moves, const char **sequence,
@@ -501,7 +533,8 @@ int openfish_amd_last_timings(const openfish_gpubuf_t *gpubuf, float *ms, int n)
     if (!g->timed || !ms || n < 1) return 0;
     if (g->pend_split) {
         HIP_OK(hipEventElapsedTime(&g->ms[OPENFISH_AMD_STAGE_BWD], g->ev[EV_START], g->ev[EV_BWD_END]));
-        HIP_OK(hipEventElapsedTime(&g->ms[OPENFISH_AMD_STAGE_FWD], g->ev[EV_BWD_END], g->ev[EV_FWD_END]));
+        HIP_OK(hipEventElapsedTime(&g->ms[OPENFISH_AMD_STAGE_FWD], g->ev[EV_BWD_END],
+                                    g->ev[g->pend_split == 2 ? EV_BEAM_END : EV_FWD_END])); /* merged: one kernel with the search */
         g->ms[OPENFISH_AMD_STAGE_SCAN] = 0.0f;
     } else {
         g->ms[OPENFISH_AMD_STAGE_BWD] = g->ms[OPENFISH_AMD_STAGE_FWD] = 0.0f;

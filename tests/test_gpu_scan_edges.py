@@ -28,3 +28,33 @@ def test_short_chunks(api, state_len, N, columns):  # noqa: F811
             bwd, post = stage_scans(api, s16, state_len, 2.0, "two_tier", fused)
             assert np.array_equal(bwd, ref["bwd"]), (T, fused)
             close(post, ref["post"])
+
+
+@pytest.mark.parametrize("columns", [4, 5])
+@pytest.mark.parametrize("state_len,T,N,enqueue", [(4, 1, 3, True), (4, 2, 1, True), (4, 37, 4, True), (4, 3, 513, False),
+                                                   (4, 41, 515, False), (5, 1, 16, False), (5, 2, 17, False),
+                                                   (5, 38, 19, False)])
+def test_forward_sweep_within_the_search_gives_the_oracle_s_tensors(api, state_len, T, N, enqueue, columns):
+    """the default of an enqueued decode and of large batches: forward sweep and posterior in the beam search's
+    workgroups, fed from its LDS rings; chunks shorter than the rings and batches that leave a workgroup half full"""
+    S = 4 ** state_len
+    s16 = synth.crf_scores(T, N, state_len, seed=T + N + state_len)
+    given = s16
+    if columns == 5:
+        given = np.full((T, N, S, 5), np.nan, np.float16)
+        given[..., 1:] = s16.reshape(T, N, S, 4)
+        given = given.reshape(T, N, 5 * S)
+    ref = O.decode(s16.astype(np.float32), state_len, {}, nthreads=8)
+    sc = api.upload_scores_to_hip(given)
+    gb = api.GpuBuf(T, N, state_len)
+    api.lib().openfish_amd_memset(gb.handle.contents.post_NTC, 0xff, N * (T + 1) * S * 4)
+    if enqueue:
+        api.openfish_amd_decode_enqueue(T, N, columns * S, sc, state_len, api.DECODER_INIT(), gb)
+        mv, sq, _ = api.openfish_amd_decode_wait(gb)
+    else:
+        mv, sq, _ = api.openfish_decode_gpu(T, N, columns * S, sc, state_len, api.DECODER_INIT(), gb)
+    t = gb.timings()
+    assert t["scan"] == 0 and t["path_sums"] == 0 and t["fwd_post"] > 0
+    assert np.array_equal(gb.tensor("bwd_NTC"), ref["bwd"])
+    close(gb.tensor("post_NTC"), ref["post"])
+    assert np.array_equal(mv, ref["moves"]) and np.array_equal(sq, ref["sequence"])
