@@ -1,6 +1,7 @@
 // Beam search over CRF scores, gfx950.
 //
-// Every chunk is served by two wavefronts of a workgroup.  The loader wave streams the
+// Every chunk is served by two wavefronts of a workgroup (with the forward sweep in it, beam_kernel
+// with FWD > 0, by several more).  The loader wave streams the
 // rows the search needs (scores[t] as fp16 and bwd[t+1] as fp32) from HBM into an LDS
 // ring, several rows ahead; the search wave runs the search with the 32-wide beam
 // resident in registers/LDS.  The two communicate through two LDS counters (rows ready /
@@ -217,7 +218,7 @@ __device__ __forceinline__ void wave_fence() {
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-// Hand-over of LDS rows between the two waves of a workgroup.  The fences name the
+// Hand-over of LDS rows between the waves of a workgroup.  The fences name the
 // local address space only: they wait for outstanding LDS operations, not for the
 // global loads and stores each wave keeps in flight.
 __device__ __forceinline__ void publish(int *flag, int value) {

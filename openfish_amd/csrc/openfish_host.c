@@ -361,10 +361,13 @@ static void join_null_stream(ofa_gpubuf_t *g) {
  *   1024 states:   64 chunks 16.6k | 16.9k, 256 chunks 57.7k | 55.2k
  * Up to 512 chunks of 256 states (or as many states in all with 64 per chunk) the beam search, one
  * wave per chunk, is the longest stage and leaves most of the machine idle: the forward sweep and the
- * posterior fit beside it.  Beyond that the search fills the compute units itself and the one
- * kernel, which has the shorter scan stage at every size, wins. */
+ * posterior fit beside it.  Beyond that the search's workgroups hold four chunks, and compute units
+ * that got none take the forward sweep: split stays ahead of both one-kernel forms up to three chunks per unit
+ * of 256 states (ms, one kernel for the scans | forward within the search | split:
+ * 520 chunks 3.82 | 3.97 | 2.97, 700 chunks, five columns 4.17 | 4.29 | 3.81, 840 of them 4.96 | 4.46 | 4.99, 1024 5.09 | 4.60 | 4.99). */
+#define OFA_SPLIT_MAX_CHUNKS_256 768
 static int split_by_default(int N, int state_len) {
-    return state_len <= 4 && (long)N * states_of(state_len) <= 512L * 256L;
+    return state_len == 3 ? N <= 2048 : state_len == 4 && N <= OFA_SPLIT_MAX_CHUNKS_256;
 }
 
 /* Whether the forward sweep and the posterior run within the beam search's kernel, after the backward sweep.
@@ -380,7 +383,7 @@ static int split_by_default(int N, int state_len) {
  * rows are small, the search alone is the longest stage). */
 static int merged_by_default(const ofa_gpubuf_t *g, int N, int state_len, int enqueued) {
     if (g->split_scans >= 0 || g->scan_mode != OFK_SCAN_TWO_TIER || g->scan_spl != 0) return 0;
-    if (state_len == 4) return enqueued || N > OFK_SPARSE_SEARCH_MAX_CHUNKS;
+    if (state_len == 4) return enqueued || N > OFA_SPLIT_MAX_CHUNKS_256;
     return state_len == 5 && N >= 16;
 }
 

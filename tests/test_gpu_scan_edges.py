@@ -31,8 +31,8 @@ def test_short_chunks(api, state_len, N, columns):  # noqa: F811
 
 
 @pytest.mark.parametrize("columns", [4, 5])
-@pytest.mark.parametrize("state_len,T,N,enqueue", [(4, 1, 3, True), (4, 2, 1, True), (4, 37, 4, True), (4, 3, 513, False),
-                                                   (4, 41, 515, False), (5, 1, 16, False), (5, 2, 17, False),
+@pytest.mark.parametrize("state_len,T,N,enqueue", [(4, 1, 3, True), (4, 2, 1, True), (4, 37, 4, True), (4, 3, 513, True),
+                                                   (4, 41, 515, True), (4, 5, 769, False), (5, 1, 16, False), (5, 2, 17, False),
                                                    (5, 38, 19, False)])
 def test_forward_sweep_within_the_search_gives_the_oracle_s_tensors(api, state_len, T, N, enqueue, columns):
     """the default of an enqueued decode and of large batches: forward sweep and posterior in the beam search's
