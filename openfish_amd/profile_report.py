@@ -56,7 +56,8 @@ def short(name):
             if fn in ("scan_post_kernel", "bwd_scan_kernel", "fwd_post_kernel") and len(a) >= 4:
                 return "%s<S=%s,SPL=%s,DEPTH=%s,%s>" % (fn, a[0], a[1], a[2], SCAN_MODES.get(a[3], a[3]))
             if fn == "beam_kernel" and len(a) >= 3:
-                return "beam_kernel<S=%s,chunks/group=%s,columns=%s>" % (a[0], a[1], a[2])
+                forward = ",forward waves=%s" % a[3] if len(a) >= 4 and a[3] != "0" else ""
+                return "beam_kernel<S=%s,chunks/group=%s,columns=%s%s>" % (a[0], a[1], a[2], forward)
             return "%s<%s>" % (fn, ",".join(a)) if a else fn
     return name[:60]
 
