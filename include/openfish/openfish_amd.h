@@ -206,14 +206,15 @@ int openfish_amd_last_timings(const openfish_gpubuf_t *gpubuf, float *ms, int n)
  *   is found by the search's own duplicate detection; for tests against a CPU search seeded
  *   the same way, never for real decoding.
  * split scans: 0 runs both scans and the posterior as one kernel, then the beam search; 1 runs the
- *   backward scan, then the forward scan + posterior on a second stream beside the beam search.
+ *   backward scan, then the forward scan + posterior on a second stream beside the beam search; 2 runs
+ *   the backward scan, then the forward scan + posterior in the beam search's own workgroups.
  *   Same results.  The second hides the forward scan beneath the beam search, which pays while that
- *   search, one wavefront per chunk, leaves the machine idle.  A negative value, the default, lets
- *   every call choose between these and a third, the forward scan + posterior in the beam search's own
- *   workgroups, which reads scores and bwd once for both: the third from 16 chunks of 1024 states and
- *   above 768 of 256, and for enqueued decodes of 256 states; split for up to 768 chunks of 256 states
- *   (2048 of 64); one kernel for what is left.  The third has the default arithmetic only and is not
- *   taken when the states per lane are set.
+ *   search, one wavefront per chunk, leaves the machine idle; the third reads scores and bwd once for
+ *   both.  It exists for 256 and 1024 states with the default arithmetic and its own states per lane; a
+ *   decode that asks for it elsewhere gets the library's choice of the other two.  A negative value, the
+ *   default, lets every call choose: the third from 16 chunks of 1024 states and above 768 of 256, and
+ *   for enqueued decodes of 256 states; split for up to 768 chunks of 256 states (2048 of 64); one kernel
+ *   for what is left.
  */
 void openfish_amd_gpubuf_set_scan_mode(const openfish_gpubuf_t *gpubuf, int scan_mode);
 void openfish_amd_gpubuf_set_split_scans(const openfish_gpubuf_t *gpubuf, int split);

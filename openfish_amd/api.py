@@ -26,6 +26,8 @@ STAGES = ("bwd", "fwd_post", "beam", "sequence", "total", "scan", "path_sums")
 # enum openfish_amd_scan_mode
 SCAN_TWO_TIER, SCAN_PRECISE, SCAN_FAST = 0, 1, 2
 SCAN_MODES = {"two_tier": SCAN_TWO_TIER, "precise": SCAN_PRECISE, "fast": SCAN_FAST}
+# the third value of set_split_scans: forward scan and posterior in the beam search's own workgroups
+SCANS_MERGED = 2
 
 
 class openfish_opt_t(C.Structure):
@@ -205,8 +207,9 @@ class GpuBuf:
 
     def set_split_scans(self, split):
         """True: backward scan, then forward scan + posterior beside the beam search; False: both
-        scans as one kernel; None: the library chooses per call (the default)"""
-        _L.openfish_amd_gpubuf_set_split_scans(self.handle, -1 if split is None else (1 if split else 0))
+        scans as one kernel; 2 (SCANS_MERGED): forward scan + posterior within the beam search's kernel;
+        None: the library chooses per call (the default)"""
+        _L.openfish_amd_gpubuf_set_split_scans(self.handle, -1 if split is None else int(split))
 
     def set_scan_states_per_lane(self, spl):
         _L.openfish_amd_gpubuf_set_scan_states_per_lane(self.handle, int(spl))

@@ -121,6 +121,10 @@ void openfish_amd_lse_table(double *out) { build_lse_table(out); }
 enum { EV_JOIN, EV_START, EV_BWD_END, EV_BEAM_START, EV_BEAM_END, EV_FWD_END, EV_SEQ_START, EV_SEQ_END, EV_SUMS_START, EV_SUMS_END, EV_COUNT };
 /* with both sweeps in one kernel EV_BWD_END marks its end and EV_FWD_END is not recorded */
 
+/* arrangements of the scans: both sweeps in one kernel; backward sweep, then forward sweep beside the beam search;
+ * backward sweep, then forward sweep within the beam search's kernel */
+enum { ARR_ONE = 0, ARR_SPLIT = 1, ARR_MERGED = 2 };
+
 typedef struct {
     openfish_gpubuf_t pub; /* first: the pointer handed to callers is this struct */
     unsigned long long magic;
@@ -136,13 +140,11 @@ typedef struct {
     int timed;
     int pending;           /* a decode has been enqueued and not yet waited for */
     int pend_T, pend_N, pend_sums;    /* its shape */
-    int pend_split;        /* how its scans were queued (which events were recorded): 0 one kernel, 1 two, 2 the forward
-                            * sweep within the beam search's kernel */
+    int pend_split;        /* how its scans were queued (which events were recorded): ARR_* */
     int scan_mode;         /* OFK_SCAN_*: arithmetic of the scans of this gpubuf's decodes */
     int scan_spl;          /* states per lane of the scans, 0 = chosen from the batch size */
     int debug_flags;       /* bit 0: serial replay of the beam search's merges; bit 1: colliding seed hashes */
-    int split_scans;       /* 1: backward sweep, then forward sweep beside the beam search; 0: both sweeps in one
-                            * kernel; -1 (default): chosen per call by split_by_default() */
+    int split_scans;       /* the arrangement asked for: ARR_*, or -1 (default): chosen per call */
     ofk_phred_table_t phred; /* thresholds for (phred_shift, phred_scale) */
     float phred_shift, phred_scale;
     int phred_valid;
@@ -381,10 +383,19 @@ static int split_by_default(int N, int state_len) {
  * (one kernel on one stream has no second stream to wait for), merged 3.96 either way.
  * Batches of fewer than 16 chunks of 1024 states keep the one kernel, 64 states their split sweeps (a chunk's
  * rows are small, the search alone is the longest stage). */
-static int merged_by_default(const ofa_gpubuf_t *g, int N, int state_len, int enqueued) {
-    if (g->split_scans >= 0 || g->scan_mode != OFK_SCAN_TWO_TIER || g->scan_spl != 0) return 0;
+static int merged_by_default(int N, int state_len, int enqueued) {
     if (state_len == 4) return enqueued || N > OFA_SPLIT_MAX_CHUNKS_256;
     return state_len == 5 && N >= 16;
+}
+
+/* the arrangement of one decode: what the gpubuf asks for, or by the rules above.  The merged kernel exists for 256 and
+ * 1024 states with the default arithmetic and its own states per lane only; asked for elsewhere it gives way to the
+ * choice among the other two. */
+static int arrangement_of(const ofa_gpubuf_t *g, int N, int state_len, int enqueued) {
+    const int can_merge = state_len >= 4 && g->scan_mode == OFK_SCAN_TWO_TIER && g->scan_spl == 0;
+    if (g->split_scans == ARR_ONE || g->split_scans == ARR_SPLIT) return g->split_scans;
+    if (can_merge && (g->split_scans == ARR_MERGED || merged_by_default(N, state_len, enqueued))) return ARR_MERGED;
+    return split_by_default(N, state_len) ? ARR_SPLIT : ARR_ONE;
 }
 
 /* Queue one decode on the gpubuf's streams, results into its pinned staging buffer; returns
@@ -397,17 +408,16 @@ static void enqueue_decode(ofa_gpubuf_t *g, const int T, const int N, const int 
     join_null_stream(g);
     HIP_OK(hipEventRecord(g->ev[EV_START], g->s_main));
     const int cols = columns_of(C, state_len);
-    const int merged = merged_by_default(g, N, state_len, enqueued);
-    g->pend_split = merged ? 2 : (g->split_scans < 0 ? split_by_default(N, state_len) : g->split_scans);
-    /* only where the search leaves the machine idle, and not with 1024 states, whose search waits for
-     * memory and was measured to take half as long again beside the extra kernel */
-    /* With split scans the posteriors are complete when the forward kernel ends.  With 64 states that is
+    g->pend_split = arrangement_of(g, N, state_len, enqueued);
+    /* Sums only where the search leaves the machine idle, and not with 1024 states, whose search waits for
+     * memory and was measured to take half as long again beside the extra kernel.
+     * With split scans the posteriors are complete when the forward kernel ends.  With 64 states that is
      * well before the search does (0.83 against 1.13 ms at 512 chunks), and the sums (0.21 ms) fit in
      * between; with 256 states the two end together and the sequence stage gathers by itself. */
     const int sums_fit = g->path_sums != NULL && N <= OFK_SPARSE_SEARCH_MAX_CHUNKS;
-    const int use_sums = sums_fit && !merged && (!g->pend_split || state_len == 3);
+    const int use_sums = sums_fit && (g->pend_split == ARR_ONE || (g->pend_split == ARR_SPLIT && state_len == 3));
     g->pend_sums = use_sums;
-    if (merged) {
+    if (g->pend_split == ARR_MERGED) {
         /* backward sweep, then the search with the forward sweep and the posterior in its workgroups */
         launch_ok(ofk_bwd_scan(scores_TNC, g->pub.bwd_NTC, T, N, state_len, cols, stay, g->scan_mode, g->scan_spl, g->s_main),
                   "bwd_scan");
@@ -420,7 +430,7 @@ static void enqueue_decode(ofa_gpubuf_t *g, const int T, const int N, const int 
         HIP_OK(hipEventRecord(g->ev[EV_BEAM_END], g->s_main));
         HIP_OK(hipStreamWaitEvent(g->s_side, g->ev[EV_BEAM_END], 0));
         HIP_OK(hipMemcpyAsync(g->h_out, g->pub.moves, nt, hipMemcpyDeviceToHost, g->s_side));
-    } else if (!g->pend_split) {
+    } else if (g->pend_split == ARR_ONE) {
         /* both sweeps and the posterior in one kernel, then the beam search, all on one stream */
         launch_ok(ofk_scan_posterior(scores_TNC, g->pub.bwd_NTC, g->pub.post_NTC, T, N, state_len, cols, stay, g->scan_mode,
                                      g->scan_spl, g->s_main), "scan_posterior");
@@ -534,10 +544,10 @@ int openfish_amd_last_timings(const openfish_gpubuf_t *gpubuf, float *ms, int n)
     ofa_gpubuf_t *g = (ofa_gpubuf_t *)gpubuf;
     if (!g || g->magic != OFA_MAGIC) die("gpubuf was not created by openfish_gpubuf_init");
     if (!g->timed || !ms || n < 1) return 0;
-    if (g->pend_split) {
+    if (g->pend_split != ARR_ONE) {
         HIP_OK(hipEventElapsedTime(&g->ms[OPENFISH_AMD_STAGE_BWD], g->ev[EV_START], g->ev[EV_BWD_END]));
         HIP_OK(hipEventElapsedTime(&g->ms[OPENFISH_AMD_STAGE_FWD], g->ev[EV_BWD_END],
-                                    g->ev[g->pend_split == 2 ? EV_BEAM_END : EV_FWD_END])); /* merged: one kernel with the search */
+                                    g->ev[g->pend_split == ARR_MERGED ? EV_BEAM_END : EV_FWD_END])); /* merged: one kernel with the search */
         g->ms[OPENFISH_AMD_STAGE_SCAN] = 0.0f;
     } else {
         g->ms[OPENFISH_AMD_STAGE_BWD] = g->ms[OPENFISH_AMD_STAGE_FWD] = 0.0f;
@@ -784,7 +794,7 @@ void openfish_amd_gpubuf_set_scan_mode(const openfish_gpubuf_t *gpubuf, int scan
 }
 
 void openfish_amd_gpubuf_set_split_scans(const openfish_gpubuf_t *gpubuf, int split) {
-    owned(gpubuf)->split_scans = split < 0 ? -1 : (split ? 1 : 0);
+    owned(gpubuf)->split_scans = split < 0 ? -1 : split == 2 ? ARR_MERGED : split ? ARR_SPLIT : ARR_ONE;
 }
 
 void openfish_amd_gpubuf_set_scan_states_per_lane(const openfish_gpubuf_t *gpubuf, int spl) {

@@ -35,8 +35,7 @@ def test_short_chunks(api, state_len, N, columns):  # noqa: F811
                                                    (4, 41, 515, True), (4, 5, 769, False), (5, 1, 16, False), (5, 2, 17, False),
                                                    (5, 38, 19, False)])
 def test_forward_sweep_within_the_search_gives_the_oracle_s_tensors(api, state_len, T, N, enqueue, columns):
-    """the default of an enqueued decode and of large batches: forward sweep and posterior in the beam search's
-    workgroups, fed from its LDS rings; chunks shorter than the rings and batches that leave a workgroup half full"""
+    """forward sweep and posterior in the beam search's workgroups, fed from its LDS rings; chunks shorter than the rings and batches that leave a workgroup half full"""
     S = 4 ** state_len
     s16 = synth.crf_scores(T, N, state_len, seed=T + N + state_len)
     given = s16
@@ -47,6 +46,7 @@ def test_forward_sweep_within_the_search_gives_the_oracle_s_tensors(api, state_l
     ref = O.decode(s16.astype(np.float32), state_len, {}, nthreads=8)
     sc = api.upload_scores_to_hip(given)
     gb = api.GpuBuf(T, N, state_len)
+    gb.set_split_scans(api.SCANS_MERGED)
     api.lib().openfish_amd_memset(gb.handle.contents.post_NTC, 0xff, N * (T + 1) * S * 4)
     if enqueue:
         api.openfish_amd_decode_enqueue(T, N, columns * S, sc, state_len, api.DECODER_INIT(), gb)
