@@ -152,8 +152,8 @@ void openfish_amd_decode_from_tensors(int T, int N, int C, const void *scores, i
  * synchronisations and three host allocations per call) is enqueue + wait + a copy
  * into fresh malloc'd buffers.
  *
- * openfish_amd_decode_enqueue queues every kernel and the copies of the results into
- * the gpubuf's pinned host buffer, ordered after work already queued on the null
+ * openfish_amd_decode_enqueue queues every kernel (the last one writes the results into
+ * the gpubuf's pinned host buffer), ordered after work already queued on the null
  * stream, and returns without waiting.  The scores must stay valid and unchanged until
  * the wait returns.  A gpubuf holds one enqueued decode at a time.
  *

@@ -86,10 +86,11 @@ typedef struct {
     float thr[OFK_PHRED_STEPS];
 } ofk_phred_table_t;
 
-/* path_sums: NULL, or what ofk_path_sums left for these posteriors (post is then not read). */
+/* path_sums: NULL, or what ofk_path_sums left for these posteriors (post is then not read).
+ * moves_out: NULL, or N * T bytes (pinned host memory) that get a copy of moves. */
 int ofk_sequence(const float *post, int32_t *states, const uint8_t *moves, float *qual_data,
                  float *base_probs, float *total_probs, char *sequence, char *qstring, int T, int N,
-                 int state_len, const ofk_phred_table_t *phred, const float *path_sums, void *stream);
+                 int state_len, const ofk_phred_table_t *phred, const float *path_sums, uint8_t *moves_out, void *stream);
 /* sums[n][t][s], N x T x states floats: posterior of state s at row t + 1 of chunk n plus that of its
  * distinct one-base shifts, fp32 sums in the CPU path's order (src/beam_search.c:441-463), for every
  * state: the input of a block's quality whichever state the path then takes. */
@@ -104,6 +105,11 @@ int ofk_copy(void *dst, const void *src, size_t bytes, void *stream);
 int ofk_rotary_emb(void *x, const float *sin_buf, const float *cos_buf, int batch, int seqlen,
                    int nheads, int rotary_half, long stride_batch, long stride_seq, long stride_head,
                    void *stream);
+
+/* One lane that waits, for 100 us at most, for mark[0] and stores to mark[1] whether it came (waits = 1), or one
+ * that sets mark[0] (waits = 0).  Launched in this order on two streams they tell whether the streams run side by
+ * side.  mark: two ints of pinned host memory as the device addresses it, zero before the launches. */
+int ofk_meet(int *mark, int waits, void *stream);
 
 /* Worst errors of v_exp_f32 over every fp32 in [-160, 0] (relative, results in the normal range)
  * and of v_log_f32 over every fp32 in [1, 2), [2, 4), [4, 5.01] (absolute), against double

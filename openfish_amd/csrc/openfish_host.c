@@ -13,6 +13,7 @@
 #include <errno.h>
 #include <float.h>
 #include <math.h>
+#include <pthread.h>
 #include <stdarg.h>
 #include <stdio.h>
 #include <stdlib.h>
@@ -118,7 +119,7 @@ void openfish_amd_lse_table(double *out) { build_lse_table(out); }
 
 #define OFA_MAGIC 0x6f66616d64677075ull /* "ofamdgpu" */
 
-enum { EV_JOIN, EV_START, EV_BWD_END, EV_BEAM_START, EV_BEAM_END, EV_FWD_END, EV_SEQ_START, EV_SEQ_END, EV_SUMS_START, EV_SUMS_END, EV_COUNT };
+enum { EV_JOIN, EV_START, EV_BWD_END, EV_BEAM_START, EV_BEAM_END, EV_FWD_END, EV_SEQ_START, EV_SEQ_END, EV_SUMS_START, EV_SUMS_END, EV_MOVES, EV_COUNT };
 /* with both sweeps in one kernel EV_BWD_END marks its end and EV_FWD_END is not recorded */
 
 /* arrangements of the scans: both sweeps in one kernel; backward sweep, then forward sweep beside the beam search;
@@ -134,12 +135,14 @@ typedef struct {
     unsigned char *h_out;  /* pinned host memory for moves | sequence | qstring */
     unsigned char *d_out;  /* the same memory as the device addresses it */
     double *lse_table;     /* device copy of the log(1 + e^-gap) table */
-    hipStream_t s_main, s_side;
+    hipStream_t s_main, s_side; /* shared with other gpubufs of the device, see take_lanes */
+    int device;
     hipEvent_t ev[EV_COUNT];
     float ms[OPENFISH_AMD_STAGE_COUNT];
     int timed;
     int pending;           /* a decode has been enqueued and not yet waited for */
     int pend_T, pend_N, pend_sums;    /* its shape */
+    int pend_copy;         /* its moves travel by a copy on the side lane */
     int pend_split;        /* how its scans were queued (which events were recorded): ARR_* */
     int scan_mode;         /* OFK_SCAN_*: arithmetic of the scans of this gpubuf's decodes */
     int scan_spl;          /* states per lane of the scans, 0 = chosen from the batch size */
@@ -156,6 +159,81 @@ static int states_of(int state_len) { return 1 << (2 * state_len); }
 
 static void check_state_len(int state_len) {
     if (state_len < 3 || state_len > 5) die("state_len must be 3, 4 or 5 (64, 256 or 1024 states)");
+}
+
+/* ---- streams ----------------------------------------------------------------
+ *
+ * A process has a handful of hardware queues (four unless the environment says otherwise, one of them the null
+ * stream's) and the runtime deals its streams round them; kernels of one queue run one after another whatever
+ * streams they are on, and what waits for an event holds up all that is behind it in its queue.  With two streams
+ * per gpubuf, created without regard to that, one gpubuf in four or so had both in one queue (its split decodes ran
+ * the forward sweep after the search: 512 chunks of 256 states 2.55 ms instead of 2.24, 37 of 1024 states with
+ * T = 833 2.29 instead of 1.70), and two batches in flight could share one queue (512 chunks each: 4.35 ms for the
+ * two instead of 3.67) or one of them the null stream's, which every decode starts with a look at.
+ *
+ * So the gpubufs of a device share three streams in three queues, none of them the null stream's: two for the
+ * kernels of a decode, which the gpubufs take in turn, and one for what runs beside them (forward
+ * sweeps, sums, copies).  Nothing in the API tells the queue of a stream, but it stays the same for its life: every
+ * new stream is tried against the null stream and those found before it (ofk_meet, 0.03 ms a try), and held if it
+ * will not do, so that the next goes elsewhere.  Where three queues are not to be found (fewer allowed, or too busy to
+ * start two kernels within the time of a try) the gpubufs make do with what there is; only speed depends on it.
+ * The streams are created with a device's first gpubuf and destroyed with its last.  Waits of the host are for events
+ * of the decode in question, never for a stream. */
+#define OFA_LANES 3
+#define OFA_LANE_TRIES 8
+#define OFA_MAX_DEVICES 64
+enum { LANE_MAIN = 0, LANE_SIDE = 1, LANE_MAIN_TOO = 2 }; /* in the order in which the queues are found */
+typedef struct {
+    hipStream_t stream[OFA_LANES];
+    int gpubufs; /* that use them */
+    int turn;    /* which main lane the next gpubuf gets */
+} ofa_lanes_t;
+static ofa_lanes_t g_lanes[OFA_MAX_DEVICES];
+static pthread_mutex_t g_lanes_mutex = PTHREAD_MUTEX_INITIALIZER;
+
+static int run_side_by_side(hipStream_t a, hipStream_t b, volatile int *h_mark, int *d_mark) {
+    h_mark[0] = h_mark[1] = 0;
+    launch_ok(ofk_meet(d_mark, 1, a), "meet");
+    launch_ok(ofk_meet(d_mark, 0, b), "meet");
+    HIP_OK(hipStreamSynchronize(a));
+    HIP_OK(hipStreamSynchronize(b));
+    return h_mark[1];
+}
+
+/* mark: eight bytes of pinned memory, as host and device address them */
+static void find_lanes(ofa_lanes_t *l, volatile int *h_mark, int *d_mark) {
+    hipStream_t other[OFA_LANE_TRIES];
+    int found = 0, others = 0;
+    while (found < OFA_LANES && found + others < OFA_LANE_TRIES) {
+        hipStream_t s;
+        HIP_OK(hipStreamCreateWithFlags(&s, hipStreamNonBlocking));
+        int apart = run_side_by_side(NULL, s, h_mark, d_mark);
+        for (int i = 0; apart && i < found; ++i) apart = run_side_by_side(l->stream[i], s, h_mark, d_mark);
+        if (apart) l->stream[found++] = s;
+        else other[others++] = s;
+    }
+    while (found < OFA_LANES) l->stream[found++] = other[--others];
+    while (others > 0) HIP_OK(hipStreamDestroy(other[--others]));
+}
+
+static void take_lanes(ofa_gpubuf_t *g) {
+    HIP_OK(hipGetDevice(&g->device));
+    if (g->device < 0 || g->device >= OFA_MAX_DEVICES) die("gpubuf: device number out of range");
+    ofa_lanes_t *l = &g_lanes[g->device];
+    pthread_mutex_lock(&g_lanes_mutex);
+    if (l->gpubufs++ == 0) find_lanes(l, (volatile int *)g->h_out, (int *)g->d_out);
+    g->s_main = l->stream[l->turn ? LANE_MAIN_TOO : LANE_MAIN];
+    l->turn = !l->turn;
+    g->s_side = l->stream[LANE_SIDE];
+    pthread_mutex_unlock(&g_lanes_mutex);
+}
+
+static void give_lanes_back(ofa_gpubuf_t *g) {
+    ofa_lanes_t *l = &g_lanes[g->device];
+    pthread_mutex_lock(&g_lanes_mutex);
+    if (--l->gpubufs == 0)
+        for (int i = 0; i < OFA_LANES; ++i) HIP_OK(hipStreamDestroy(l->stream[i]));
+    pthread_mutex_unlock(&g_lanes_mutex);
 }
 
 openfish_gpubuf_t *openfish_gpubuf_init(const int T, const int N, const int state_len) {
@@ -191,7 +269,7 @@ openfish_gpubuf_t *openfish_gpubuf_init(const int T, const int N, const int stat
         *field[i] = sz[i] ? p : NULL;
         p += round_up(sz[i]);
     }
-    HIP_OK(hipHostMalloc((void **)&g->h_out, 3 * nt, hipHostMallocDefault));
+    HIP_OK(hipHostMalloc((void **)&g->h_out, 3 * nt < 64 ? 64 : 3 * nt, hipHostMallocDefault));
     HIP_OK(hipHostGetDevicePointer((void **)&g->d_out, g->h_out, 0));
     {
         double tab[OFK_LSE_DOUBLES];
@@ -199,10 +277,15 @@ openfish_gpubuf_t *openfish_gpubuf_init(const int T, const int N, const int stat
         HIP_OK(hipMalloc((void **)&g->lse_table, sizeof tab));
         HIP_OK(hipMemcpy(g->lse_table, tab, sizeof tab, hipMemcpyHostToDevice));
     }
-    HIP_OK(hipStreamCreateWithFlags(&g->s_main, hipStreamNonBlocking));
-    HIP_OK(hipStreamCreateWithFlags(&g->s_side, hipStreamNonBlocking));
+    take_lanes(g);
     for (int i = 0; i < EV_COUNT; ++i) HIP_OK(hipEventCreate(&g->ev[i]));
     return &g->pub;
+}
+
+/* until every kernel and copy of the enqueued decode is done */
+static void wait_for_decode(ofa_gpubuf_t *g) {
+    if (g->pend_copy) HIP_OK(hipEventSynchronize(g->ev[EV_MOVES]));
+    HIP_OK(hipEventSynchronize(g->ev[EV_SEQ_END])); /* the main lane has waited for what ran on the side lane */
 }
 
 void openfish_gpubuf_free(openfish_gpubuf_t *gpubuf) {
@@ -210,12 +293,10 @@ void openfish_gpubuf_free(openfish_gpubuf_t *gpubuf) {
     if (!g) return;
     if (g->magic != OFA_MAGIC) die("gpubuf was not created by openfish_gpubuf_init");
     if (g->pending) { /* an enqueued decode still reads and writes these buffers */
-        HIP_OK(hipStreamSynchronize(g->s_side));
-        HIP_OK(hipStreamSynchronize(g->s_main));
+        wait_for_decode(g);
     }
     for (int i = 0; i < EV_COUNT; ++i) HIP_OK(hipEventDestroy(g->ev[i]));
-    HIP_OK(hipStreamDestroy(g->s_main));
-    HIP_OK(hipStreamDestroy(g->s_side));
+    give_lanes_back(g);
     HIP_OK(hipHostFree(g->h_out));
     HIP_OK(hipFree(g->lse_table));
     HIP_OK(hipFree(g->slab));
@@ -343,8 +424,9 @@ static void fetch_outputs(ofa_gpubuf_t *g, int T, int N, uint8_t **moves, char *
     HIP_OK(hipMemcpyAsync(g->h_out, g->pub.moves, nt, hipMemcpyDeviceToHost, g->s_main));
     HIP_OK(hipMemcpyAsync(g->h_out + nt, g->pub.sequence, nt, hipMemcpyDeviceToHost, g->s_main));
     HIP_OK(hipMemcpyAsync(g->h_out + 2 * nt, g->pub.qstring, nt, hipMemcpyDeviceToHost, g->s_main));
+    HIP_OK(hipEventRecord(g->ev[EV_MOVES], g->s_main));
     alloc_outputs(T, N, moves, sequence, qstring);
-    HIP_OK(hipStreamSynchronize(g->s_main));
+    HIP_OK(hipEventSynchronize(g->ev[EV_MOVES]));
     memcpy(*moves, g->h_out, nt);
     memcpy(*sequence, g->h_out + nt, nt);
     memcpy(*qstring, g->h_out + 2 * nt, nt);
@@ -428,8 +510,6 @@ static void enqueue_decode(ofa_gpubuf_t *g, const int T, const int N, const int 
                                           log_beam_cut(options), stay, g->lse_table, g->debug_flags, g->s_main),
                   "beam_search_forward");
         HIP_OK(hipEventRecord(g->ev[EV_BEAM_END], g->s_main));
-        HIP_OK(hipStreamWaitEvent(g->s_side, g->ev[EV_BEAM_END], 0));
-        HIP_OK(hipMemcpyAsync(g->h_out, g->pub.moves, nt, hipMemcpyDeviceToHost, g->s_side));
     } else if (g->pend_split == ARR_ONE) {
         /* both sweeps and the posterior in one kernel, then the beam search, all on one stream */
         launch_ok(ofk_scan_posterior(scores_TNC, g->pub.bwd_NTC, g->pub.post_NTC, T, N, state_len, cols, stay, g->scan_mode,
@@ -449,10 +529,6 @@ static void enqueue_decode(ofa_gpubuf_t *g, const int T, const int N, const int 
             launch_ok(ofk_path_sums(g->pub.post_NTC, g->path_sums, T, N, state_len, g->s_side), "path_sums");
             HIP_OK(hipEventRecord(g->ev[EV_SUMS_END], g->s_side));
         }
-        /* the moves are final once the beam search is: they travel while the sequence stage runs */
-        HIP_OK(hipStreamWaitEvent(g->s_side, g->ev[EV_BEAM_END], 0));
-        HIP_OK(hipMemcpyAsync(g->h_out, g->pub.moves, nt, hipMemcpyDeviceToHost, g->s_side));
-        if (use_sums) HIP_OK(hipStreamWaitEvent(g->s_main, g->ev[EV_SUMS_END], 0));
     } else {
         launch_ok(ofk_bwd_scan(scores_TNC, g->pub.bwd_NTC, T, N, state_len, cols, stay, g->scan_mode, g->scan_spl, g->s_main),
                   "bwd_scan");
@@ -476,11 +552,20 @@ static void enqueue_decode(ofa_gpubuf_t *g, const int T, const int N, const int 
             launch_ok(ofk_path_sums(g->pub.post_NTC, g->path_sums, T, N, state_len, g->s_side), "path_sums");
             HIP_OK(hipEventRecord(g->ev[EV_SUMS_END], g->s_side));
         }
-        /* the moves are final once the beam search is: they travel while the sequence stage runs */
+    }
+
+    /* The moves are final once the beam search is.  Of a blocking decode they travel, and the host takes them, while
+     * the sequence stage runs.  Of an enqueued one nobody waits for them: that stage writes them to the host itself
+     * (0.02 ms), because a copy that waits for the search would hold up the forward sweep of the next decode behind
+     * it on the side lane (two batches of 16 chunks of 64 states in flight: 2.14 ms with the copies, 1.63 without). */
+    g->pend_copy = !enqueued;
+    if (g->pend_copy) {
         HIP_OK(hipStreamWaitEvent(g->s_side, g->ev[EV_BEAM_END], 0));
         HIP_OK(hipMemcpyAsync(g->h_out, g->pub.moves, nt, hipMemcpyDeviceToHost, g->s_side));
-        HIP_OK(hipStreamWaitEvent(g->s_main, g->ev[use_sums ? EV_SUMS_END : EV_FWD_END], 0));
+        HIP_OK(hipEventRecord(g->ev[EV_MOVES], g->s_side));
     }
+    if (use_sums) HIP_OK(hipStreamWaitEvent(g->s_main, g->ev[EV_SUMS_END], 0));
+    else if (g->pend_split == ARR_SPLIT) HIP_OK(hipStreamWaitEvent(g->s_main, g->ev[EV_FWD_END], 0));
 
     HIP_OK(hipEventRecord(g->ev[EV_SEQ_START], g->s_main));
     /* The last kernel writes bases and qualities straight into the pinned host memory (N * T bytes
@@ -490,7 +575,7 @@ static void enqueue_decode(ofa_gpubuf_t *g, const int T, const int N, const int 
      * are filled by the stage-level entry points only. */
     launch_ok(ofk_sequence(g->pub.post_NTC, (int32_t *)g->pub.states, g->pub.moves, g->pub.qual_data,
                            g->pub.base_probs, g->pub.total_probs, (char *)g->d_out + nt, (char *)g->d_out + 2 * nt, T, N,
-                           state_len, phred_for(g, options), use_sums ? g->path_sums : NULL, g->s_main), "sequence");
+                           state_len, phred_for(g, options), use_sums ? g->path_sums : NULL, enqueued ? g->d_out : NULL, g->s_main), "sequence");
     HIP_OK(hipEventRecord(g->ev[EV_SEQ_END], g->s_main));
     g->pending = 1;
     g->pend_T = T;
@@ -508,9 +593,9 @@ void openfish_decode_gpu(const int T, const int N, const int C, void *scores_TNC
 
     enqueue_decode(g, T, N, C, scores_TNC, state_len, options, 0);
     alloc_outputs(T, N, moves, sequence, qstring);
-    HIP_OK(hipStreamSynchronize(g->s_side));
+    HIP_OK(hipEventSynchronize(g->ev[EV_MOVES]));
     memcpy(*moves, g->h_out, nt);
-    HIP_OK(hipStreamSynchronize(g->s_main));
+    HIP_OK(hipEventSynchronize(g->ev[EV_SEQ_END]));
     memcpy(*sequence, g->h_out + nt, nt);
     memcpy(*qstring, g->h_out + 2 * nt, nt);
     g->pending = 0;
@@ -531,8 +616,7 @@ void openfish_amd_decode_wait(const openfish_gpubuf_t *gpubuf, const uint8_t **m
     if (!g->pending) die("decode_wait: nothing was enqueued on this gpubuf");
     if (!moves || !sequence || !qstring) die("decode_wait: output pointer is NULL");
     const size_t nt = (size_t)g->pend_N * (size_t)g->pend_T;
-    HIP_OK(hipStreamSynchronize(g->s_side));
-    HIP_OK(hipStreamSynchronize(g->s_main));
+    wait_for_decode(g);
     *moves = g->h_out;
     *sequence = (const char *)g->h_out + nt;
     *qstring = (const char *)g->h_out + 2 * nt;
@@ -646,7 +730,7 @@ void openfish_amd_sequence(int T, int N, int state_len, const openfish_opt_t *op
     ofa_gpubuf_t *g = checked(gpubuf, T, N, state_len);
     launch_ok(ofk_sequence(post, (int32_t *)g->pub.states, g->pub.moves, g->pub.qual_data, g->pub.base_probs,
                            g->pub.total_probs, g->pub.sequence, g->pub.qstring, T, N, state_len,
-                           phred_for(g, options), NULL, NULL), "sequence");
+                           phred_for(g, options), NULL, NULL, NULL), "sequence");
     HIP_OK(hipStreamSynchronize(0));
 }
 
@@ -670,7 +754,7 @@ void openfish_amd_decode_from_tensors(int T, int N, int C, const void *scores, i
     }
     launch_ok(ofk_sequence(post, (int32_t *)g->pub.states, g->pub.moves, g->pub.qual_data, g->pub.base_probs,
                            g->pub.total_probs, g->pub.sequence, g->pub.qstring, T, N, state_len,
-                           phred_for(g, options), sums, g->s_main), "sequence");
+                           phred_for(g, options), sums, NULL, g->s_main), "sequence");
     fetch_outputs(g, T, N, moves, sequence, qstring);
 }
 

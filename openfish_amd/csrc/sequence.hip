@@ -24,7 +24,7 @@ __global__ __launch_bounds__(kThreads) void sequence_kernel(
     const float *__restrict__ post, int32_t *__restrict__ states, const uint8_t *__restrict__ moves,
     float *__restrict__ qual_data, float *__restrict__ base_probs, float *__restrict__ total_probs,
     char *__restrict__ sequence, char *__restrict__ qstring, int T, ofk_phred_table_t phred,
-    const float *__restrict__ path_sums) {
+    const float *__restrict__ path_sums, uint8_t *__restrict__ moves_out) {
     extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
     float *s_prob = reinterpret_cast<float *>(lds);        // [T] called-base probability
     float *s_wrong = s_prob + T;                           // [T] probability of each other base
@@ -71,7 +71,9 @@ __global__ __launch_bounds__(kThreads) void sequence_kernel(
         s_prob[t] = prob;
         s_wrong[t] = wrong;
         s_base[t] = (unsigned char)base;
-        s_move[t] = mv_n[t];
+        const uint8_t move = mv_n[t];
+        s_move[t] = move;
+        if (moves_out) moves_out[(size_t)n * T + t] = move;
         float4 q;
         q.x = base == 0 ? prob : wrong;
         q.y = base == 1 ? prob : wrong;
@@ -263,7 +265,7 @@ int launch_path_sums(const float *post, float *sums, int T, int N, hipStream_t s
 template <int S>
 int launch_sequence(const float *post, int32_t *states, const uint8_t *moves, float *qual_data,
                     float *base_probs, float *total_probs, char *sequence, char *qstring, int T, int N,
-                    const ofk_phred_table_t &phred, const float *path_sums, hipStream_t st) {
+                    const ofk_phred_table_t &phred, const float *path_sums, uint8_t *moves_out, hipStream_t st) {
     const size_t lds = (size_t)T * (4 + 4 + 1 + 1) + (size_t)(T + 1) * 4;
     if (lds > 64 * 1024) {  // beyond the default limit of dynamic LDS; the compute unit has 160 KB
         const hipError_t rc = hipFuncSetAttribute(reinterpret_cast<const void *>(&sequence_kernel<S>),
@@ -271,7 +273,7 @@ int launch_sequence(const float *post, int32_t *states, const uint8_t *moves, fl
         if (rc != hipSuccess) return (int)rc;
     }
     hipLaunchKernelGGL((sequence_kernel<S>), dim3(N), dim3(kThreads), lds, st, post, states, moves, qual_data,
-                       base_probs, total_probs, sequence, qstring, T, phred, path_sums);
+                       base_probs, total_probs, sequence, qstring, T, phred, path_sums, moves_out);
     return (int)hipGetLastError();
 }
 
@@ -291,7 +293,8 @@ extern "C" int ofk_path_sums(const float *post, float *sums, int T, int N, int s
 
 extern "C" int ofk_sequence(const float *post, int32_t *states, const uint8_t *moves, float *qual_data,
                             float *base_probs, float *total_probs, char *sequence, char *qstring, int T, int N,
-                            int state_len, const ofk_phred_table_t *phred, const float *path_sums, void *stream) {
+                            int state_len, const ofk_phred_table_t *phred, const float *path_sums, uint8_t *moves_out,
+                            void *stream) {
     // the per-chunk tables live in LDS: 14 bytes per time step
     if ((!post && !path_sums) || !states || !moves || !qual_data || !base_probs || !total_probs || !sequence || !qstring ||
         !phred || T < 1 || T > OFK_MAX_T || N < 1)
@@ -299,9 +302,9 @@ extern "C" int ofk_sequence(const float *post, int32_t *states, const uint8_t *m
     if (reinterpret_cast<uintptr_t>(qual_data) & 15u) return OFK_BAD_ARGS;
     hipStream_t st = static_cast<hipStream_t>(stream);
     switch (state_len) {
-        case 3: return launch_sequence<64>(post, states, moves, qual_data, base_probs, total_probs, sequence, qstring, T, N, *phred, path_sums, st);
-        case 4: return launch_sequence<256>(post, states, moves, qual_data, base_probs, total_probs, sequence, qstring, T, N, *phred, path_sums, st);
-        case 5: return launch_sequence<1024>(post, states, moves, qual_data, base_probs, total_probs, sequence, qstring, T, N, *phred, path_sums, st);
+        case 3: return launch_sequence<64>(post, states, moves, qual_data, base_probs, total_probs, sequence, qstring, T, N, *phred, path_sums, moves_out, st);
+        case 4: return launch_sequence<256>(post, states, moves, qual_data, base_probs, total_probs, sequence, qstring, T, N, *phred, path_sums, moves_out, st);
+        case 5: return launch_sequence<1024>(post, states, moves, qual_data, base_probs, total_probs, sequence, qstring, T, N, *phred, path_sums, moves_out, st);
         default: return OFK_BAD_ARGS;
     }
 }
