@@ -241,28 +241,72 @@ __device__ __forceinline__ void pipelined(int count, Step &&step) {
         });
 }
 
-// the five terms of every state of a lane; the row's registers are free for the next load afterwards
+// the five terms of one state of a lane, and of every one; the row's registers are free for the next load afterwards
 template <int I, int SPL>
-__device__ __forceinline__ void bwd_terms(float (&v)[SPL][5], const float (&a)[SPL], const float4 &nx, const BwdRow<SPL> &row, float stay) {
-    if constexpr (I < SPL) {
-        v[I][0] = a[I] + stay;
-        v[I][1] = row.template add<0, I>(nx.x);
-        v[I][2] = row.template add<1, I>(nx.y);
-        v[I][3] = row.template add<2, I>(nx.z);
-        v[I][4] = row.template add<3, I>(nx.w);
-        bwd_terms<I + 1, SPL>(v, a, nx, row, stay);
-    }
+__device__ __forceinline__ void bwd_terms_of(float (&v)[5], const float (&a)[SPL], const float4 &nx, const BwdRow<SPL> &row, float stay) {
+    v[0] = a[I] + stay;
+    v[1] = row.template add<0, I>(nx.x);
+    v[2] = row.template add<1, I>(nx.y);
+    v[3] = row.template add<2, I>(nx.z);
+    v[4] = row.template add<3, I>(nx.w);
 }
 template <int I, int SPL>
+__device__ __forceinline__ void fwd_terms_of(float (&v)[5], const float (&f)[SPL], float p0, float p1, float p2, float p3,
+                                             const FwdRow<SPL> &row, float stay) {
+    v[0] = f[I] + stay;
+    v[1] = row.template add<I, 0>(p0);
+    v[2] = row.template add<I, 1>(p1);
+    v[3] = row.template add<I, 2>(p2);
+    v[4] = row.template add<I, 3>(p3);
+}
+template <int SPL>
+__device__ __forceinline__ void bwd_terms(float (&v)[SPL][5], const float (&a)[SPL], const float4 &nx, const BwdRow<SPL> &row, float stay) {
+    static_for<SPL>([&](auto i) { bwd_terms_of<i, SPL>(v[i], a, nx, row, stay); });
+}
+template <int SPL>
 __device__ __forceinline__ void fwd_terms(float (&v)[SPL][5], const float (&f)[SPL], float p0, float p1, float p2, float p3,
                                           const FwdRow<SPL> &row, float stay) {
-    if constexpr (I < SPL) {
-        v[I][0] = f[I] + stay;
-        v[I][1] = row.template add<I, 0>(p0);
-        v[I][2] = row.template add<I, 1>(p1);
-        v[I][3] = row.template add<I, 2>(p2);
-        v[I][4] = row.template add<I, 3>(p3);
-        fwd_terms<I + 1, SPL>(v, f, p0, p1, p2, p3, row, stay);
+    static_for<SPL>([&](auto i) { fwd_terms_of<i, SPL>(v[i], f, p0, p1, p2, p3, row, stay); });
+}
+
+// A step of the kernel that holds both sweeps and is capped at 128 registers.  Of four states to a lane the terms are
+// not kept for a common second tier (as in the separate sweeps, which may use 256 registers): that spilled inside the
+// loops.  One state after another in the backward sweep and two and two in the forward one needs no scratch with 256
+// states, and with 1024 only between the phases.  Scans of 2048 chunks of 256 states, T = 1666: 6.87 ms all four
+// together, 5.8 now (five columns 7.87, 5.8); 512 chunks of 1024 states 6.14, 5.4; with the batch spread over twice the
+// lanes 6.07, 6.15 and 5.82.
+template <int SPL, int MODE>
+__device__ __forceinline__ void bwd_update(float (&a)[SPL], const float4 &nx, const BwdRow<SPL> &row, float stay, const LogArgs &logtab) {
+    if constexpr (SPL < 4) {
+        float v[SPL][5];
+        bwd_terms(v, a, nx, row, stay);
+        lse5_all<SPL, MODE>(a, v, logtab);
+    } else {
+        static_for<SPL>([&](auto i) {
+            float v[1][5], out[1];
+            bwd_terms_of<i, SPL>(v[0], a, nx, row, stay);
+            lse5_all<1, MODE>(out, v, logtab);
+            a[i] = out[0];
+        });
+    }
+}
+template <int SPL, int MODE>
+__device__ __forceinline__ void fwd_update(float (&f)[SPL], float p0, float p1, float p2, float p3, const FwdRow<SPL> &row, float stay,
+                                           const LogArgs &logtab) {
+    if constexpr (SPL < 4) {
+        float v[SPL][5];
+        fwd_terms(v, f, p0, p1, p2, p3, row, stay);
+        lse5_all<SPL, MODE>(f, v, logtab);
+    } else {
+        static_for<SPL / 2>([&](auto h) {
+            constexpr int i = 2 * h;
+            float v[2][5], out[2];
+            fwd_terms_of<i, SPL>(v[0], f, p0, p1, p2, p3, row, stay);
+            fwd_terms_of<i + 1, SPL>(v[1], f, p0, p1, p2, p3, row, stay);
+            lse5_all<2, MODE>(out, v, logtab);
+            f[i] = out[0];
+            f[i + 1] = out[1];
+        });
     }
 }
 
@@ -323,7 +367,7 @@ __global__ __launch_bounds__((Shape<S, SPL>::kThreads)) void bwd_scan_kernel(
         chunk_sync<Sh::kMultiWave>();
         const float4 nx = *reinterpret_cast<const float4 *>(&vec[g][buf][Vec::of(4 * r)]);
         float v[SPL][5];
-        bwd_terms<0, SPL>(v, a, nx, ring[k], stay);
+        bwd_terms(v, a, nx, ring[k], stay);
         if (!checked || j + DEPTH < T) {
             ring[k].load(pre + sc_lane);
             pre -= row_stride;
@@ -444,7 +488,7 @@ __global__ __launch_bounds__((Shape<S, SPL>::kThreads)) void fwd_post_kernel(
         const float p0 = vec[g][buf][q], p1 = vec[g][buf][q + Q];
         const float p2 = vec[g][buf][q + 2 * Q], p3 = vec[g][buf][q + 3 * Q];
         float v[SPL][5];
-        fwd_terms<0, SPL>(v, f, p0, p1, p2, p3, ring[k], stay);
+        fwd_terms(v, f, p0, p1, p2, p3, ring[k], stay);
         if (!checked || j + DEPTH < T) {
             ring[k].load(pre + sc_lane);
             pre += row_stride;
@@ -528,7 +572,7 @@ __global__ __launch_bounds__((2 * (S / SPL))) void fwd_post_roles_kernel(
             const float p0 = vec[buf][q], p1 = vec[buf][q + Q];
             const float p2 = vec[buf][q + 2 * Q], p3 = vec[buf][q + 3 * Q];
             float v[SPL][5];
-            fwd_terms<0, SPL>(v, f, p0, p1, p2, p3, ring[k], stay);
+            fwd_terms(v, f, p0, p1, p2, p3, ring[k], stay);
             if (!checked || j + DEPTH < T) {
                 ring[k].load(pre + sc_lane);
                 pre += row_stride;
@@ -718,11 +762,7 @@ __global__ __launch_bounds__((FusedShape<S, SPL>::kThreads), 4) void scan_post_k
                 }
                 step_sync();
                 const float4 nx = *reinterpret_cast<const float4 *>(&vecB[g][buf][VecB::of(4 * r)]);
-                {
-                    float v[SPL][5];
-                    bwd_terms<0, SPL>(v, a, nx, row, stay);
-                    lse5_all<SPL, M>(a, v, logtab);
-                }
+                bwd_update<SPL, M>(a, nx, row, stay, logtab);
                 buf ^= 1;
 #pragma unroll
                 for (int i = 0; i < SPL; ++i) vecB[g][buf][VecB::at(r, c0 + i)] = a[i];
@@ -787,11 +827,7 @@ __global__ __launch_bounds__((FusedShape<S, SPL>::kThreads), 4) void scan_post_k
                 }
                 prow -= S;
                 const float4 nx = *reinterpret_cast<const float4 *>(&vecB[g][buf][VecB::of(4 * r)]);
-                {
-                    float v[SPL][5];
-                    bwd_terms<0, SPL>(v, a, nx, row, stay);
-                    lse5_all<SPL, MODE>(a, v, logtab);
-                }
+                bwd_update<SPL, MODE>(a, nx, row, stay, logtab);
                 buf ^= 1;
                 float total;
 #pragma unroll
@@ -866,11 +902,7 @@ __global__ __launch_bounds__((FusedShape<S, SPL>::kThreads), 4) void scan_post_k
                 step_sync();
                 const float p0 = vecF[g][buf][q], p1 = vecF[g][buf][q + Q];
                 const float p2 = vecF[g][buf][q + 2 * Q], p3 = vecF[g][buf][q + 3 * Q];
-                {
-                    float v[SPL][5];
-                    fwd_terms<0, SPL>(v, f, p0, p1, p2, p3, row, stay);
-                    lse5_all<SPL, M>(f, v, logtab);
-                }
+                fwd_update<SPL, M>(f, p0, p1, p2, p3, row, stay, logtab);
                 buf ^= 1;
                 FloatRun<SPL> mine;
 #pragma unroll
@@ -946,11 +978,7 @@ __global__ __launch_bounds__((FusedShape<S, SPL>::kThreads), 4) void scan_post_k
                 if (!checked || j + 1 < cnt2) {
                     const float p0 = vecF[g][buf][q], p1 = vecF[g][buf][q + Q];
                     const float p2 = vecF[g][buf][q + 2 * Q], p3 = vecF[g][buf][q + 3 * Q];
-                    {
-                    float v[SPL][5];
-                    fwd_terms<0, SPL>(v, f, p0, p1, p2, p3, row, stay);
-                    lse5_all<SPL, MODE>(f, v, logtab);
-                }
+                    fwd_update<SPL, MODE>(f, p0, p1, p2, p3, row, stay, logtab);
                     buf ^= 1;
                     FloatRun<SPL> mine;
 #pragma unroll
@@ -1100,6 +1128,10 @@ int states_per_lane(int S, int N, bool backward, int forced) {
 #ifndef OFK_DEPTH_FUSED_1024
 #define OFK_DEPTH_FUSED_1024 3
 #endif
+// four states to a lane (2048 and more chunks of 256 states): a row more would not fit the 128 registers
+#ifndef OFK_DEPTH_FUSED_WIDE
+#define OFK_DEPTH_FUSED_WIDE 3
+#endif
 #define OFK_DISPATCH(BACKWARD, LAUNCH, ...)                                                    \
     switch (state_len * 8 + states_per_lane(1 << (2 * state_len), N, BACKWARD, lanes_asked(mode, spl))) { \
         case 3 * 8 + 4: return LAUNCH<64, 4, OFK_DEPTH>(__VA_ARGS__);                          \
@@ -1140,7 +1172,7 @@ static int scan_posterior(const void *scores, float *bwd, float *post, int T, in
             if ((size_t)N * kCols * S * 2 < ((size_t)4 << 20))
                 return launch_fused<64, 1, OFK_DEPTH>(mode, scores, bwd, post, T, N, stay, st);
             return launch_fused<64, 1, OFK_DEPTH_FUSED>(mode, scores, bwd, post, T, N, stay, st);
-        case 4 * 8 + 4: return launch_fused<256, 4, OFK_DEPTH_FUSED>(mode, scores, bwd, post, T, N, stay, st);
+        case 4 * 8 + 4: return launch_fused<256, 4, OFK_DEPTH_FUSED_WIDE>(mode, scores, bwd, post, T, N, stay, st);
         case 4 * 8 + 2: return launch_fused<256, 2, OFK_DEPTH_FUSED>(mode, scores, bwd, post, T, N, stay, st);
         case 4 * 8 + 1: return launch_fused<256, 1, OFK_DEPTH_FUSED>(mode, scores, bwd, post, T, N, stay, st);
         case 5 * 8 + 4: return launch_fused<1024, 4, OFK_DEPTH_FUSED_1024>(mode, scores, bwd, post, T, N, stay, st);
