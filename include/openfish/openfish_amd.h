@@ -84,7 +84,7 @@ void openfish_amd_fwd_post_scan(int T, int N, int C, const void *scores, int sta
                                 float stay_score, int scan_mode, const float *bwd, float *post);
 
 /*
- * Both scans and the posterior in one kernel (what openfish_decode_gpu runs by default): the
+ * Both scans and the posterior in one kernel (one of the arrangements of openfish_decode_gpu): the
  * backward and the forward recursion of a chunk advance side by side and meet in the middle of
  * the chunk.  Same tensors as openfish_amd_bwd_scan followed by openfish_amd_fwd_post_scan.
  */
@@ -212,14 +212,24 @@ int openfish_amd_last_timings(const openfish_gpubuf_t *gpubuf, float *ms, int n)
  *   search, one wavefront per chunk, leaves the machine idle; the third reads scores and bwd once for
  *   both.  It exists for 256 and 1024 states with the default arithmetic and its own states per lane; a
  *   decode that asks for it elsewhere gets the library's choice of the other two.  A negative value, the
- *   default, lets every call choose: the third from 16 chunks of 1024 states and above 768 of 256, and
- *   for enqueued decodes of 256 states; split for up to 768 chunks of 256 states (2048 of 64); one kernel
- *   for what is left.
+ *   default, lets every call choose (openfish_amd_scan_arrangement).
  */
 void openfish_amd_gpubuf_set_scan_mode(const openfish_gpubuf_t *gpubuf, int scan_mode);
 void openfish_amd_gpubuf_set_split_scans(const openfish_gpubuf_t *gpubuf, int split);
 void openfish_amd_gpubuf_set_scan_states_per_lane(const openfish_gpubuf_t *gpubuf, int spl);
 void openfish_amd_gpubuf_set_debug_flags(const openfish_gpubuf_t *gpubuf, int flags);
+
+/*
+ * The arrangement of the scans that a decode of this shape takes where the gpubuf leaves the choice to the
+ * library, with the default arithmetic and states per lane: 0, 1 or 2 as openfish_amd_gpubuf_set_split_scans
+ * numbers them.  enqueued: 0 for openfish_decode_gpu, 1 for openfish_amd_decode_enqueue.  Host-only.
+ *   64 states: 1 up to 2048 chunks, 0 beyond.
+ *   256 states: blocking 1 up to 512 chunks (five columns: 463), 2 for five columns up to 512, 1 up to 768,
+ *     2 beyond; enqueued 2 up to 512, 1 up to 640, 2 beyond.
+ *   1024 states: blocking 1 up to 160 chunks and from 257 to 320, 2 elsewhere, or 0 where chunks are shorter
+ *     than 128 steps and there are not 257 to 320 of them; enqueued 2, or 0 up to 160 chunks shorter than that.
+ */
+int openfish_amd_scan_arrangement(int T, int N, int C, int state_len, int enqueued);
 
 /*
  * The 49 miss-probability thresholds behind the phred characters for one

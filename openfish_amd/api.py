@@ -94,6 +94,7 @@ _SIGS = {
     "openfish_amd_gpubuf_set_debug_flags": (None, [_bufp, _i]),
     "openfish_amd_gpubuf_set_scan_mode": (None, [_bufp, _i]),
     "openfish_amd_gpubuf_set_scan_states_per_lane": (None, [_bufp, _i]),
+    "openfish_amd_scan_arrangement": (_i, [_i, _i, _i, _i, _i]),
     "openfish_amd_lse_table": (None, [C.POINTER(C.c_double)]),
     "openfish_amd_phred_table": (None, [_f, _f, C.POINTER(C.c_float)]),
     "openfish_amd_probe_hw_math": (None, [C.POINTER(C.c_double), C.POINTER(C.c_uint)]),
@@ -324,6 +325,11 @@ def upload_scores_to_hip(scores_half):
     """host fp16 [T][N][C] -> DeviceBuffer (reference upload_scores_to_hip)"""
     a = np.ascontiguousarray(scores_half, dtype=np.float16)
     return DeviceBuffer.from_host(a)
+
+
+def scan_arrangement(T, N, Cc, state_len, enqueued=False):
+    """the library's choice for a decode of this shape: 0 one kernel, 1 split, 2 merged"""
+    return int(_L.openfish_amd_scan_arrangement(T, N, Cc, state_len, 1 if enqueued else 0))
 
 
 def phred_table(q_scale, q_shift):

@@ -2,11 +2,12 @@
  * Host side of the MI355X decoder: the public openfish entry points and the
  * stage-level C-ABI, in C, above the kernel launchers of kernels.h.
  *
- * One decode is   bwd scan -> { beam search || fwd+posterior scan } -> sequence   on two streams
- * (the beam search needs only scores and bwd, the posterior only feeds the quality stage, reference
- * src/beam_search.c:193,450) while the beam search leaves the machine idle, and   scans + posterior
- * (one kernel) -> { beam search || per-state sums of posteriors } -> sequence   for larger batches and
- * 1024 states; every call chooses unless the gpubuf says which (split_by_default).  The sequence stage
+ * One decode is one of three arrangements of the same stages (the beam search needs only scores and bwd, the
+ * posterior only feeds the quality stage, reference src/beam_search.c:193,450):
+ *   split    bwd scan -> { beam search || fwd scan + posterior } -> sequence
+ *   merged   bwd scan -> beam search with the fwd scan and the posterior in its workgroups -> sequence
+ *   one      both scans + posterior in one kernel -> { beam search || per-state sums of posteriors } -> sequence
+ * Every call chooses (arrangement_by_default) unless the gpubuf says which.  The sequence stage
  * writes bases and qualities into pinned host memory itself.  Errors follow the reference convention
  * (reference src/hip_utils.h:11-28, src/error.h:44-72): message on stderr, then exit.
  */
@@ -438,46 +439,72 @@ static void join_null_stream(ofa_gpubuf_t *g) {
     HIP_OK(hipStreamWaitEvent(g->s_main, g->ev[EV_JOIN], 0));
 }
 
-/* Which arrangement of the scans a blocking decode finishes sooner with, as measured on whole
- * decodes (T = 1666; chunks/s with one kernel | split):
- *     64 states:  512 chunks 248k | 260k, 2048 chunks 418k | 485k
- *    256 states:  128 chunks  57k |  61k,  512 chunks 180k | 195k, 1024 chunks 215k | 206k, 2048 chunks 223k | 207k
- *   1024 states:   64 chunks 16.6k | 16.9k, 256 chunks 57.7k | 55.2k
- * Up to 512 chunks of 256 states (or as many states in all with 64 per chunk) the beam search, one
- * wave per chunk, is the longest stage and leaves most of the machine idle: the forward sweep and the
- * posterior fit beside it.  Beyond that the search's workgroups hold four chunks, and compute units
- * that got none take the forward sweep: split stays ahead of both one-kernel forms up to three chunks per unit
- * of 256 states (ms, one kernel for the scans | forward within the search | split:
- * 520 chunks 3.82 | 3.97 | 2.97, 700 chunks, five columns 4.17 | 4.29 | 3.81, 840 of them 4.96 | 4.46 | 4.99, 1024 5.09 | 4.60 | 4.99). */
-#define OFA_SPLIT_MAX_CHUNKS_256 768
-static int split_by_default(int N, int state_len) {
-    return state_len == 3 ? N <= 2048 : state_len == 4 && N <= OFA_SPLIT_MAX_CHUNKS_256;
+/* Which arrangement of the scans a decode finishes soonest with.  What bounds them, after the backward sweep:
+ *   split   the longer of the search's chain and of the bytes that search and forward sweep move side by side, per
+ *           chunk and step 4C + 12S: fp16 scores and fp32 bwd twice, the posterior once;
+ *   merged  the chain of the kernel that holds both, three quarters of those bytes or less; the chain is longer than
+ *           the search's alone (256 states by 5 %, 1024 by 16 to 40 %), twice that with two rounds of workgroups;
+ *   one     both sweeps of a chunk side by side from its two ends, then the search: the longest, with the fewest launches.
+ * Whole blocking calls, ms, one | split | merged, T = 1666 unless stated, inputs and arrangements in turn; in all of them
+ * the forward sweep of the split decodes was seen to run beside the search.
+ *   1024 states: 16 chunks, T = 833 1.95 | 1.69 | 1.80;  37, T = 833 1.98 | 1.71 | 1.82;  128 3.76 | 3.15 | 3.34;
+ *                160 3.81 | 3.19 | 3.38;  168 3.81 | 4.26 | 3.40;  192 3.87 | 4.28 | 3.39;  256 4.26 | 4.34 | 3.46;
+ *                257 6.91 | 5.10 | 5.69;  320 6.95 | 5.63 | 5.79;  336 7.03 | 5.82 | 5.86;  400 7.28 | 7.74 | 6.03;
+ *                five columns: 160 3.90 | 3.18 | 3.40;  256 4.55 | 4.80 | 3.54;  257 7.15 | 5.44 | 5.72;
+ *                288 7.27 | 5.78 | 5.89;  304 7.30 | 5.95 | 5.90;  320 7.36 | 6.11 | 5.88;
+ *                T = 833: 320 3.80 | 3.11 | 3.11;  T = 400: 320 1.89 | 1.58 | 1.67;
+ *                T = 100: 16 0.352 | 0.363 | 0.380;  256 0.392 | 0.467 | 0.401;  352 0.621 | 0.643 | 0.613;  512 0.648 | 0.829 | 0.708;
+ *                T = 128: 16 0.425 | 0.422 | 0.440;  512 0.797 | 0.971 | 0.823;  T = 200: 16 0.586 | 0.563 | 0.593
+ *    256 states: 403 2.63 | 2.14 | 2.20;  512 2.77 | 2.26 | 2.31;  520 3.77 | 2.64 | 3.93;  700 4.09 | 3.71 | 4.25;
+ *                768 4.18 | 3.79 | 4.31;  800 4.62 | 4.41 | 4.52;  1024 4.84 | 5.03 | 4.84;
+ *                five columns: 456 2.77 | 2.24 | 2.27;  472 2.80 | 2.30 | 2.28;  488 2.83 | 2.42 | 2.33;  512 2.90 | 2.57 | 2.34;
+ *                768 4.34 | 4.15 | 4.42;  784 4.70 | 4.63 | 4.51;  1024 5.03 | 5.54 | 4.93
+ *     64 states: 16 1.83 | 1.58;  512 2.03 | 1.76;  2048 4.37 | 3.61
+ * Hence the lines: up to 160 chunks of 1024 states the search (two chunks to a unit) and the forward sweep (one) find
+ * compute units of their own; above 256 merged takes a second round of workgroups, split does so only above 320; chunks
+ * shorter than 128 steps are decided by launches and set-up.  Up to 512 chunks of 256 states the chain of split is
+ * shorter, while its bytes fit beneath the chain, 3.8 MB a step; above, the search's workgroups hold four chunks, a unit
+ * that has one of them in the merged kernel takes 2.5 ms whatever the others do, and split has units left for the
+ * forward sweep up to three chunks to a unit.
+ *
+ * A decode that is enqueued shares the machine with others; two at a time, one | split | merged:
+ *   1024 states: 16, T = 833 1.99 | 2.48 | 1.84;  128 4.32 | 5.01 | 3.89;  256 five columns 8.44 | 8.55 | 6.40;
+ *                320 10.27 | 10.07 | 8.16;  16, T = 100 0.38 | 0.50 | 0.41
+ *    256 states: 128 2.64 | 2.35 | 2.07;  512 5.34 | 4.65 | 3.78;  520 5.69 | 4.78 | 5.70;  640 five columns 6.77 | 6.03 | 6.17;
+ *                700 6.60 | 6.21 | 6.13 (one alone 3.83 | 3.24 | 4.05);  704 five columns 6.93 | 6.73 | 6.41;  768 five columns 7.45 | 7.07 | 6.57
+ *     64 states: 512 3.19 | 2.75;  2048 8.10 | 6.91
+ *
+ * The merged kernel exists for 256 and 1024 states with the default arithmetic and its own states per lane; without it
+ * (can_merge = 0) 1024 states keep the one kernel and 256 states the split sweeps where they are ahead of it. */
+static int arrangement_by_default(int T, int N, int C, int state_len, int enqueued, int can_merge) {
+    const size_t step_bytes = (size_t)N * (4 * (size_t)C + 12 * (size_t)states_of(state_len)); /* of split */
+    switch (state_len) {
+        case 3: return N <= 2048 ? ARR_SPLIT : ARR_ONE;
+        case 4:
+            if (!can_merge) return N <= 768 ? ARR_SPLIT : ARR_ONE;
+            if (N <= 512) return enqueued || step_bytes > 3800000 ? ARR_MERGED : ARR_SPLIT;
+            return N <= (enqueued ? 640 : 768) ? ARR_SPLIT : ARR_MERGED;
+        default:
+            if (!can_merge) return ARR_ONE;
+            if (enqueued) return T < 128 && N <= 160 ? ARR_ONE : ARR_MERGED;
+            if (N > 256 && N <= 320) return ARR_SPLIT;
+            if (T < 128) return ARR_ONE;
+            return N <= 160 ? ARR_SPLIT : ARR_MERGED;
+    }
 }
 
-/* Whether the forward sweep and the posterior run within the beam search's kernel, after the backward sweep.
- * Scores and bwd then cross HBM once for both, which is what large batches are bound by; small ones are bound by
- * the search's own chain, which is a little shorter beside a separate kernel.  Whole decodes, ms, T = 1666, the
- * better of the other two arrangements | merged:
- *    256 states:  403 chunks (T = 1201) 1.62 | 1.69,  512 chunks 2.29 | 2.36,  1024 chunks, five columns 4.99 | 4.59
- *   1024 states:  37 chunks (T = 833) 1.98 | 1.81,  256 chunks, five columns 4.58 | 3.47
- * A decode that is enqueued shares the machine with others: two of 512 chunks of 256 states at a time took
- * 4.4 ms with four streams in the process, 5.4 with twelve, whose sweeps then wait in each other's hardware queues
- * (one kernel on one stream has no second stream to wait for), merged 3.96 either way.
- * Batches of fewer than 16 chunks of 1024 states keep the one kernel, 64 states their split sweeps (a chunk's
- * rows are small, the search alone is the longest stage). */
-static int merged_by_default(int N, int state_len, int enqueued) {
-    if (state_len == 4) return enqueued || N > OFA_SPLIT_MAX_CHUNKS_256;
-    return state_len == 5 && N >= 16;
+int openfish_amd_scan_arrangement(int T, int N, int C, int state_len, int enqueued) {
+    check_state_len(state_len);
+    return arrangement_by_default(T, N, C, state_len, enqueued, state_len >= 4);
 }
 
-/* the arrangement of one decode: what the gpubuf asks for, or by the rules above.  The merged kernel exists for 256 and
- * 1024 states with the default arithmetic and its own states per lane only; asked for elsewhere it gives way to the
- * choice among the other two. */
-static int arrangement_of(const ofa_gpubuf_t *g, int N, int state_len, int enqueued) {
+/* the arrangement of one decode: what the gpubuf asks for, or by the rule above.  Merged asked for where it does not
+ * exist gives way to the choice among the other two. */
+static int arrangement_of(const ofa_gpubuf_t *g, int T, int N, int C, int state_len, int enqueued) {
     const int can_merge = state_len >= 4 && g->scan_mode == OFK_SCAN_TWO_TIER && g->scan_spl == 0;
     if (g->split_scans == ARR_ONE || g->split_scans == ARR_SPLIT) return g->split_scans;
-    if (can_merge && (g->split_scans == ARR_MERGED || merged_by_default(N, state_len, enqueued))) return ARR_MERGED;
-    return split_by_default(N, state_len) ? ARR_SPLIT : ARR_ONE;
+    if (g->split_scans == ARR_MERGED && can_merge) return ARR_MERGED;
+    return arrangement_by_default(T, N, C, state_len, enqueued, can_merge);
 }
 
 /* Queue one decode on the gpubuf's streams, results into its pinned staging buffer; returns
@@ -490,7 +517,7 @@ static void enqueue_decode(ofa_gpubuf_t *g, const int T, const int N, const int 
     join_null_stream(g);
     HIP_OK(hipEventRecord(g->ev[EV_START], g->s_main));
     const int cols = columns_of(C, state_len);
-    g->pend_split = arrangement_of(g, N, state_len, enqueued);
+    g->pend_split = arrangement_of(g, T, N, C, state_len, enqueued);
     /* Sums only where the search leaves the machine idle, and not with 1024 states, whose search waits for
      * memory and was measured to take half as long again beside the extra kernel.
      * With split scans the posteriors are complete when the forward kernel ends.  With 64 states that is
