@@ -366,10 +366,9 @@ struct BeamIdx {
 constexpr int kVecRows = 4;  // two would do (see beam_kernel); four let the posterior lag (1024 chunks of 256 states: 2.66 ms against 2.78)
 template <int S, int FWD>
 struct __attribute__((aligned(16))) FwdLds {
-    int published[FWD < 4 ? 4 : FWD];  // rows of the state vector each wave of the recursion has written
-    int taken;                         // rows the posterior's wave has read
-    int pad[3];
-    float vec[kVecRows][S];                   // row t in vec[t % kVecRows]
+    int published[FWD];  // rows of the state vector each wave of the recursion has written
+    int taken;           // rows the posterior's wave has read
+    __attribute__((aligned(16))) float vec[kVecRows][S];  // row t in vec[t % kVecRows]
     float tier_lanes[64 * FWD];
 };
 template <int S>
@@ -501,7 +500,7 @@ __global__ __launch_bounds__((kBeamThreads<S, CPG, COLS, FWD>), (BeamCfg<S, FWD>
         sh.ready = 0;
         sh.consumed = 0;
         if constexpr (FWD > 0) {
-            for (int x = 0; x < (FWD < 4 ? 4 : FWD); ++x) lds[member].fwd.published[x] = 0;
+            for (int x = 0; x < FWD; ++x) lds[member].fwd.published[x] = 0;
             lds[member].fwd.taken = 0;
         }
     }
@@ -516,6 +515,7 @@ __global__ __launch_bounds__((kBeamThreads<S, CPG, COLS, FWD>), (BeamCfg<S, FWD>
     __syncthreads();
     if (n >= N) return;  // odd batch: the last group has one chunk
 
+    static_assert((FWD & (FWD - 1)) == 0 && FWD <= 64, "a lane reads one wave's counter");
     if constexpr (FWD > 0) {
         auto &fw = lds[member].fwd;
         // whether every wave of the recursion has written row t of the state vector: a lane reads one counter
@@ -554,11 +554,7 @@ __global__ __launch_bounds__((kBeamThreads<S, CPG, COLS, FWD>), (BeamCfg<S, FWD>
                     rows_taken = __builtin_amdgcn_readfirstlane(observe(&fw.taken));
                     if (rows_taken < t + 2 - kVecRows) __builtin_amdgcn_s_sleep(1);
                 }
-                if constexpr (FWD > 1) {
-                    while (!row_published(t)) {}
-                } else {
-                    wave_fence();
-                }
+                while (!row_published(t)) {}
                 const float *vec = fw.vec[t % kVecRows];
                 const float p0 = vec[q], p1 = vec[q + Q], p2 = vec[q + 2 * Q], p3 = vec[q + 3 * Q];
                 float v[SPL][5];

@@ -156,30 +156,8 @@ OFA_HD double log_1to5_tab(float s, const LogCell *table, const double *series) 
     return __builtin_fma((double)k, kLn2, lu);
 }
 
-// The same logarithm with the table cell (and the power of two) taken from an approximation
-// `near` of s, |near / s - 1| < 2^-18, so that the cell can be fetched before s is known: with k the
-// exponent of `near` and c its cell, ln s = k ln2 + ln c + log1p(s 2^-k / c - 1), and the argument of
-// log1p stays within 1/64 + 2^-17 in magnitude whichever side of a cell (or binade) boundary s itself
-// falls on: the ninth power, the first one the series drops, stays below 2^-56.
-OFA_HD LogCell log_cell_near(float near, const LogCell *table) { return table[(bits_of(near) >> 18) & 31u]; }
-OFA_HD double log_1to5_with_cell(float s, float near, LogCell c, const double *series) {
-    const int k = (int)(bits_of(near) >> 23) - 127;
-    const double u = __builtin_ldexp((double)s, -k);
-    const double r = __builtin_fma(u, c.inv, -1.0);
-    double q = series[0];
-    q = __builtin_fma(q, r, series[1]);
-    q = __builtin_fma(q, r, series[2]);
-    q = __builtin_fma(q, r, series[3]);
-    q = __builtin_fma(q, r, series[4]);
-    q = __builtin_fma(q, r, series[5]);
-    q = __builtin_fma(q, r, -0.5);
-    q = __builtin_fma(q, r, 1.0);
-    const double lu = __builtin_fma(q, r, c.lnc);
-    const double kLn2 = 0.69314718055994530942;
-    return __builtin_fma((double)k, kLn2, lu);
-}
-
-// A third form, for the place where every instruction counts.  The cells are centred on multiples of 1/32
+// A second form, for the place where every instruction counts, with the table cell taken from an approximation
+// `near` of s, |near / s - 1| < 2^-18, so that it can be fetched before s is known.  The cells are centred on multiples of 1/32
 // and carry the power of two: the entry of a float s is picked by the low seven bits
 // of (exponent, mantissa) rounded to five mantissa bits, which tells c = 2^k (1 + j/32) apart for k = 0 .. 3, so that
 // ln s = lnc + log1p(s * inv - 1) with |s * inv - 1| <= 1/64 (+ 2^-17 when the cell is chosen with an

@@ -34,17 +34,17 @@ double max_abs_err_log_tab(const float *s, long n) {
     return worst;
 }
 
-// largest absolute error of the logarithm whose table cell comes from a neighbour `near` of s
+// largest absolute error of the second tier's logarithm, whose table cell comes from a neighbour `near` of s
 // (s moved by up to `ulps` fp32 steps either way), against logl
 double max_abs_err_log_near(const float *s, long n, int ulps) {
-    ofa::LogCell table[32];
-    for (int i = 0; i < 32; ++i) table[i] = ofa::log_cell(i);
+    ofa::LogCell table[ofa::kLogCentredCells];
+    for (int i = 0; i < ofa::kLogCentredCells; ++i) table[i] = ofa::log_centred_cell(i);
     double worst = 0;
     for (long i = 0; i < n; ++i) {
         for (int d = -ulps; d <= ulps; d += (ulps > 0 ? ulps : 1)) {
             const float near = ofa::float_of(ofa::bits_of(s[i]) + (uint32_t)d);
             if (!(near >= 1.0f)) continue;
-            const double got = ofa::log_1to5_with_cell(s[i], near, ofa::log_cell_near(near, table), kSeries);
+            const double got = ofa::log_centred(s[i], table[ofa::log_centred_index(near)], kSeries);
             const double err = (double)fabsl((long double)got - logl((long double)s[i]));
             if (err > worst) worst = err;
         }
