@@ -39,7 +39,7 @@ HBM_PEAK_GBS = 8000.0
 TRAFFIC_FILE = os.path.join(ROOT, "profiles", "traffic.json")
 
 
-def measured_traffic(workload, N, columns, kernel):
+def measured_traffic(workload, N, columns, kernel, arrangement):
     """HBM bytes per launch of one kernel as rocprofv3 counted them (FETCH_SIZE + WRITE_SIZE, each
     scaled by the plain copy kernel's reading of the same counter): read from the summary the
     profiling script wrote (profiles/traffic.json); None where that run has not been made"""
@@ -49,7 +49,25 @@ def measured_traffic(workload, N, columns, kernel):
     except (OSError, ValueError):
         return None
     entry = table.get("%s_n%d_c%d" % (workload, N, columns), {}).get(kernel)
-    return None if entry is None else int(round(entry["hbm_bytes"]))
+    if entry is None or (kernel == "beam" and ("forward waves" in entry["kernel"]) != (arrangement == "merged")):
+        return None
+    return int(round(entry["hbm_bytes"]))
+
+
+# as the library numbers them
+SCANS = ("one", "split", "merged")
+SCANS_TEXT = {"one": "both scans and the posterior as one kernel, then the beam search",
+              "split": "backward scan, then forward scan + posterior on a second stream beside the beam search",
+              "merged": "backward scan, then forward scan + posterior within the beam search's kernel"}
+
+
+def arrangement_run(api, asked, mean, shape, scan_mode, states_per_lane, enqueued=False):
+    """what a decode ran with: what was asked for, or the library's choice"""
+    if mean is not None and mean["scan"] > 0:
+        return "one"
+    choice = asked if asked is not None else api.scan_arrangement(*shape, enqueued)
+    can_merge = shape[3] >= 4 and scan_mode == "two_tier" and states_per_lane == 0
+    return "merged" if choice == 2 and can_merge else "split"
 
 
 def algorithmic_bytes(state_len, T, N, columns=4):
@@ -66,6 +84,7 @@ def algorithmic_bytes(state_len, T, N, columns=4):
         "path_sums": N * 2 * T * S * 4,               # read the posteriors of T rows, write a sum per state
     }
     need["scan"] = need["bwd"] + need["fwd_post"]     # both scans + posterior as one kernel: the same minimum
+    need["beam_merged"] = need["beam"] + N * vec      # search, forward scan and posterior over one reading of the rows
     return need
 
 
@@ -95,7 +114,7 @@ def cpu_baseline(s16, state_len, opt_kw, sample_chunks):
 
 
 def cpu_baseline_config1(seed):
-    """BASELINE's first configuration, the one the reference runs on the CPU: fast model (state_len 3,
+    """the smallest configuration, the one the reference runs on the CPU: fast model (state_len 3,
     64 states), T=1666, N=16 chunks, fp32 scores (the fp16-rounded values of the generator), beam 32,
     beam cut 100, blank 2.0, q_shift 0, q_scale 1, on 8 threads, the thread count of the reference's
     own driver (src/main.c:287)"""
@@ -170,7 +189,8 @@ def timed_decodes(api, gpubuf, call_args, steps):
 
 
 def scan_stage(need, mean):
-    """scans + posterior: one kernel (`scan`) or the two split kernels (`bwd`, `fwd_post`)"""
+    """scans + posterior: one kernel (`scan`) or the two split kernels (`bwd`, `fwd_post`); not for a forward scan
+    within the beam search's kernel, whose time is not the scans' alone"""
     ms = mean["scan"] + mean["bwd"] + mean["fwd_post"]
     gbs = need["scan"] / 1e9 / (ms / 1e3)
     return {"ms": round(ms, 4), "algorithmic_GB": round(need["scan"] / 1e9, 4), "GBps": round(gbs, 1),
@@ -188,9 +208,9 @@ def main():
                     help="scores per state and time step: 4 (what the reference consumes) or 5 (a blank column first, "
                          "C = 5 * 4^state_len as the network emits it)")
     ap.add_argument("--scan-mode", default="two_tier", choices=("two_tier", "precise", "fast"))
-    ap.add_argument("--scans", default="auto", choices=("auto", "one", "split"),
+    ap.add_argument("--scans", default="auto", choices=("auto",) + SCANS,
                     help="arrangement of the scans: both as one kernel, or the backward scan and then the forward scan "
-                         "beside the beam search; auto (the default): the library chooses per call")
+                         "beside the beam search or within its kernel; auto (the default): the library chooses per call")
     ap.add_argument("--split-scans", action="store_const", dest="scans", const="split", help="the same as --scans split")
     ap.add_argument("--states-per-lane", type=int, default=0, choices=(0, 1, 2, 4),
                     help="force the scans' states per lane (0: the library chooses)")
@@ -240,7 +260,7 @@ def main():
     del made, device_input
     gpubuf = api.GpuBuf(T, N, state_len)
     gpubuf.set_scan_mode(a.scan_mode)
-    asked = {"auto": None, "one": False, "split": True}[a.scans]
+    asked = None if a.scans == "auto" else SCANS.index(a.scans)
     gpubuf.set_split_scans(asked)
     gpubuf.set_scan_states_per_lane(a.states_per_lane)
     call = (T, N, C, scores, state_len, opt)
@@ -258,6 +278,10 @@ def main():
     ms_per_step, mean = timed_decodes(api, gpubuf, call, a.steps)
 
     need = algorithmic_bytes(state_len, T, N, a.columns)
+    ran = arrangement_run(api, asked, mean, (T, N, C, state_len), a.scan_mode, a.states_per_lane)
+    if ran == "merged":  # one kernel: its time is the beam search's, its bytes both stages'
+        mean["fwd_post"] = 0.0
+        need["beam"] = need["beam_merged"]
     stages = {}
     for k in ("scan", "bwd", "fwd_post", "beam", "sequence", "path_sums"):  # path_sums runs beside the beam search
         if mean[k] > 0:
@@ -273,39 +297,38 @@ def main():
         stages["beam_and_" + beside + "_side_by_side"] = {
             "ms": round(window_ms, 4), "algorithmic_GB": round(gb, 4), "GBps": round(gb / (window_ms / 1e3), 1),
             "frac_of_hbm_peak": round(gb / (window_ms / 1e3) / HBM_PEAK_GBS, 4)}
-    stages["scan_plus_posterior"] = scan_stage(need, mean)
-    scan_gbs = stages["scan_plus_posterior"]["GBps"]
+    if ran != "merged":
+        stages["scan_plus_posterior"] = scan_stage(need, mean)
     dominant = max((k for k in ("scan", "bwd", "fwd_post", "beam", "sequence") if k in stages), key=lambda k: stages[k]["ms"])
     roofline = {"bound": "hbm", "kernel": dominant, "achieved": stages[dominant]["GBps"], "peak": HBM_PEAK_GBS,
                 "unit": "GB/s", "frac": round(stages[dominant]["GBps"] / HBM_PEAK_GBS, 4),
-                "traffic": measured_traffic(a.workload, N, a.columns, dominant)}
+                "traffic": measured_traffic(a.workload, N, a.columns, dominant, ran)}
 
     # side measurements on the same batch (never `value`): the other arrangement of the scans, and the
     # hardware-exp/log scan arithmetic (not parity-grade)
-    def side(split, mode, note):
-        gpubuf.set_split_scans(split)
+    def side(scans, mode, note):
+        gpubuf.set_split_scans(scans)
         gpubuf.set_scan_mode(mode)
         api.openfish_decode_gpu_discard(*call, gpubuf)
         ms, mn = timed_decodes(api, gpubuf, call, a.alt_steps)
         gpubuf.set_split_scans(asked)
         gpubuf.set_scan_mode(a.scan_mode)
+        apart = arrangement_run(api, scans, mn, (T, N, C, state_len), mode, a.states_per_lane) != "merged"
         return {"chunks_per_s": round(N / (ms / 1e3), 1), "ms_per_step": round(ms, 4),
                 "stage_ms": {k: round(v, 4) for k, v in mn.items() if v > 0},
-                "scan_plus_posterior": scan_stage(need, mn), "note": note}
+                "scan_plus_posterior": scan_stage(need, mn) if apart else None, "note": note}
 
     other_split, fast_mode = None, None
     if a.alt_steps > 0:
-        ran_split = mean["scan"] == 0  # what the timed calls ran with, asked for or chosen by the library
-        other_split = side(not ran_split, a.scan_mode,
-                           "split scans: backward scan, then forward scan + posterior on a second stream beside the beam search"
-                           if not ran_split else "both scans and the posterior as one kernel, then the beam search")
+        other = "split" if ran == "one" else "one"
+        other_split = side(SCANS.index(other), a.scan_mode, SCANS_TEXT[other])
         if a.scan_mode != "fast":
             fast_mode = side(asked, "fast",
                              "scans with v_exp_f32/v_log_f32 only: bwd within 2 ulp, a few posteriors per ten million "
                              "beyond 1e-3 relative; outside the acceptance bar, shown as the memory-bound floor of the kernels")
 
     # the same scores as the network emits them, five columns per state with a blank first (the layout
-    # BASELINE's configurations name), read in place; its algorithmic bytes count C = 5 * 4^state_len
+    # the full benchmark configurations have), read in place; its algorithmic bytes count C = 5 * 4^state_len
     five_columns = None
     if five is not None:
         scores5 = api.upload_scores_to_hip(five)
@@ -313,9 +336,11 @@ def main():
         call5 = (T, N, 5 * S, scores5, state_len, opt)
         api.openfish_decode_gpu_discard(*call5, gpubuf)
         ms5, mn5 = timed_decodes(api, gpubuf, call5, a.alt_steps)
+        ran5 = arrangement_run(api, asked, mn5, (T, N, 5 * S, state_len), a.scan_mode, a.states_per_lane)
         five_columns = {"C": 5 * S, "chunks_per_s": round(N / (ms5 / 1e3), 1), "ms_per_step": round(ms5, 4),
                         "stage_ms": {k: round(v, 4) for k, v in mn5.items() if v > 0},
-                        "scan_plus_posterior": scan_stage(algorithmic_bytes(state_len, T, N, 5), mn5),
+                        "scan_plus_posterior": scan_stage(algorithmic_bytes(state_len, T, N, 5), mn5) if ran5 != "merged" else None,
+                        "scans": SCANS_TEXT[ran5],
                         "note": "the same batch with five fp16 columns per state (blank first, never read), default settings"}
         scores5.free()
 
@@ -357,7 +382,8 @@ def main():
         dst.free()
     if copy_gbs:
         stages["device_copy_GBps"] = round(copy_gbs, 1)
-        stages["scan_plus_posterior"]["frac_of_device_copy"] = round(scan_gbs / copy_gbs, 4)
+        if "scan_plus_posterior" in stages:
+            stages["scan_plus_posterior"]["frac_of_device_copy"] = round(stages["scan_plus_posterior"]["GBps"] / copy_gbs, 4)
 
     opt_kw = dict(beam_cut=100.0, blank_score=2.0, q_shift=q_shift, q_scale=q_scale)
     cpu = cpu_baseline(s16, state_len, opt_kw, min(a.cpu_sample, N)) if a.cpu_sample > 0 else None
@@ -372,7 +398,7 @@ def main():
         "vs_baseline": None, "dtype": "f32" if a.scan_mode == "fast" else "f32+f64", "data": "synthetic",
         "config": {"workload": "%s: state_len %d, S=%d, C=%d fp16 TNC (%d columns per state), T=%d, N=%d, beam 32, "
                                "beam_cut 100, blank 2.0" % (a.workload, state_len, S, C, a.columns, T, N),
-                   "scan_mode": a.scan_mode, "scans": "one kernel" if mean["scan"] > 0 else "two kernels (backward, then forward + posterior beside the beam search)",
+                   "scan_mode": a.scan_mode, "scans": SCANS_TEXT[ran],
                    "seed": a.seed},
         "roofline": roofline, "stages": stages, "other_scan_arrangement": other_split, "fast_scan_mode": fast_mode,
         "five_columns": five_columns, "two_in_flight": overlap, "cpu_baseline": cpu, "cpu_baseline_config1": cpu1,

@@ -31,9 +31,11 @@
 // up as a 5e-4 relative difference of a posterior.  Two-tier is the default for
 // that reason; fast exists for measurements.
 //
-// Kernels: bwd_scan_kernel and fwd_post_kernel are the two sweeps one after the other;
-// scan_post_kernel runs both sweeps of a chunk in one workgroup, from both ends of the
-// chunk towards the middle and on to the other end, and is what a decode uses.
+// Kernels: bwd_scan_kernel is the backward sweep; fwd_post_kernel and fwd_post_roles_kernel are the
+// forward sweep with the posterior, for a decode that runs it beside the beam search (the third place
+// for it, within the search's kernel, is in beam.hip); scan_post_kernel runs both sweeps of a chunk in one
+// workgroup, from both ends of the chunk towards the middle and on to the other end.  Which of them a
+// decode uses is decided by its shape (openfish_host.c).
 #include <hip/hip_runtime.h>
 
 #include <type_traits>

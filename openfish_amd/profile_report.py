@@ -48,7 +48,7 @@ def template_ints(name):
 
 def short(name):
     for fn in ("scan_post_kernel", "bwd_scan_kernel", "fwd_post_roles_kernel", "fwd_post_kernel", "beam_kernel",
-               "sequence_kernel", "path_sums_kernel", "copy_kernel", "rotary_vec8_kernel", "rotary_kernel"):
+               "sequence_kernel", "path_sums_kernel", "copy_kernel", "meet_kernel", "rotary_vec8_kernel", "rotary_kernel"):
         if fn in name:
             a = template_ints(name)
             if fn == "fwd_post_roles_kernel" and len(a) >= 3:
@@ -201,9 +201,10 @@ def main():
                 ("%.2f" % (d.get("SQ_INSTS_VALU_FMA_F64", 0.0) / (waves * steps))) if (steps and waves and stage_of(k) in ("scan", "bwd", "fwd_post")) else "-"))
         if a.steps_per_wave:
             out.append("\nfp64 FMA per wave and time step = SQ_INSTS_VALU_FMA_F64 / (waves x T): the second tier of the default "
-                       "arithmetic is the only user of fp64 in the scans besides the 32 warm-up steps of either sweep (70 fp64 "
-                       "FMA per wave and step there); one trip through it is 23 fp64 FMA, so the figure, less the warm-up's "
-                       "share, over 23 is the number of trips per wave-level update.")
+                       "arithmetic is the only user of fp64 in the scans, but for the 32 warm-up steps of either sweep in the "
+                       "kernel that holds both (70 fp64 FMA per wave, state of a lane and step).  A trip through it is 25 fp64 "
+                       "FMA with one state to a lane and 21 with more; where many lanes need it (the first few hundred steps) "
+                       "it takes 70 for every state of a lane at once.")
 
     log = first(os.path.join(base, "trace.log"))
     if log:
