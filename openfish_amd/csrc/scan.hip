@@ -63,8 +63,11 @@ __device__ __forceinline__ void chunk_sync() {
     if constexpr (MULTIWAVE) {
         // Only LDS traffic has to be ordered across the barrier.  __syncthreads() would also
         // wait for every global load and store in flight, i.e. drain the prefetch ring at
-        // every time step.
+        // every time step.  The wait for this wave's own LDS writes is spelled out: the one that the
+        // fence stands for is dropped by the compiler where a loop begins with the barrier and
+        // nothing is under way when the loop is entered, although every trip round it ends with a write.
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+        __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0), the other counters unlimited
         __builtin_amdgcn_s_barrier();
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
     } else {
