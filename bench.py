@@ -61,11 +61,11 @@ SCANS_TEXT = {"one": "both scans and the posterior as one kernel, then the beam 
               "merged": "backward scan, then forward scan + posterior within the beam search's kernel"}
 
 
-def arrangement_run(api, asked, mean, shape, scan_mode, states_per_lane, enqueued=False):
+def arrangement_run(api, asked, mean, shape, scan_mode, states_per_lane):
     """what a decode ran with: what was asked for, or the library's choice"""
-    if mean is not None and mean["scan"] > 0:
+    if mean["scan"] > 0:
         return "one"
-    choice = asked if asked is not None else api.scan_arrangement(*shape, enqueued)
+    choice = asked if asked is not None else api.scan_arrangement(*shape)
     can_merge = shape[3] >= 4 and scan_mode == "two_tier" and states_per_lane == 0
     return "merged" if choice == 2 and can_merge else "split"
 

@@ -222,14 +222,18 @@ void openfish_amd_gpubuf_set_debug_flags(const openfish_gpubuf_t *gpubuf, int fl
 /*
  * The arrangement of the scans that a decode of this shape takes where the gpubuf leaves the choice to the
  * library, with the default arithmetic and states per lane: 0, 1 or 2 as openfish_amd_gpubuf_set_split_scans
- * numbers them.  enqueued: 0 for openfish_decode_gpu, 1 for openfish_amd_decode_enqueue.  Host-only.
+ * numbers them.  shared: 1 for openfish_amd_decode_enqueue, and for openfish_decode_gpu while another decode is
+ * under way on the device (another thread's, or an enqueued one that has not been waited for); 0 otherwise.
+ * moves, sequence and bwd do not depend on the arrangement; the sum below a posterior is taken in another order, which
+ * moves a quality character by one step now and then (up to three in ten thousand).  Callers that decode from several
+ * threads and want the same characters every time fix the arrangement.  Host-only.
  *   64 states: 1 up to 2048 chunks, 0 beyond.
- *   256 states: blocking 1 up to 512 chunks (five columns: 463), 2 for five columns up to 512, 1 up to 768,
- *     2 beyond; enqueued 2 up to 512, 1 up to 640, 2 beyond.
- *   1024 states: blocking 1 up to 160 chunks and from 257 to 320, 2 elsewhere, or 0 where chunks are shorter
- *     than 128 steps and there are not 257 to 320 of them; enqueued 2, or 0 up to 160 chunks shorter than that.
+ *   256 states: alone 1 up to 512 chunks (five columns: 463), 2 for five columns up to 512, 1 up to 768,
+ *     2 beyond; shared 2 up to 512, 1 up to 640, 2 beyond.
+ *   1024 states: alone 1 up to 160 chunks and from 257 to 320, 2 elsewhere, or 0 where chunks are shorter
+ *     than 128 steps and there are not 257 to 320 of them; shared 2, or 0 up to 160 chunks shorter than that.
  */
-int openfish_amd_scan_arrangement(int T, int N, int C, int state_len, int enqueued);
+int openfish_amd_scan_arrangement(int T, int N, int C, int state_len, int shared);
 
 /*
  * The 49 miss-probability thresholds behind the phred characters for one

@@ -327,9 +327,10 @@ def upload_scores_to_hip(scores_half):
     return DeviceBuffer.from_host(a)
 
 
-def scan_arrangement(T, N, Cc, state_len, enqueued=False):
-    """the library's choice for a decode of this shape: 0 one kernel, 1 split, 2 merged"""
-    return int(_L.openfish_amd_scan_arrangement(T, N, Cc, state_len, 1 if enqueued else 0))
+def scan_arrangement(T, N, Cc, state_len, shared=False):
+    """the library's choice for a decode of this shape: 0 one kernel, 1 split, 2 merged; shared: enqueued, or while
+    another decode is under way"""
+    return int(_L.openfish_amd_scan_arrangement(T, N, Cc, state_len, 1 if shared else 0))
 
 
 def phred_table(q_scale, q_shift):

@@ -136,8 +136,9 @@ typedef struct {
     unsigned char *h_out;  /* pinned host memory for moves | sequence | qstring */
     unsigned char *d_out;  /* the same memory as the device addresses it */
     double *lse_table;     /* device copy of the log(1 + e^-gap) table */
-    hipStream_t s_main, s_side; /* shared with other gpubufs of the device, see take_lanes */
     int device;
+    hipStream_t s_main, s_side; /* of the decode under way; shared with other gpubufs of the device, see take_main_lane */
+    int main_lane, side_lane; /* side_lane -1: none */
     hipEvent_t ev[EV_COUNT];
     float ms[OPENFISH_AMD_STAGE_COUNT];
     int timed;
@@ -172,9 +173,9 @@ static void check_state_len(int state_len) {
  * T = 833 2.29 instead of 1.70), and two batches in flight could share one queue (512 chunks each: 4.35 ms for the
  * two instead of 3.67) or one of them the null stream's, which every decode starts with a look at.
  *
- * So the gpubufs of a device share three streams in three queues, none of them the null stream's: two for the
- * kernels of a decode, which the gpubufs take in turn, and one for what runs beside them (forward
- * sweeps, sums, copies).  Nothing in the API tells the queue of a stream, but it stays the same for its life: every
+ * So the gpubufs of a device share three streams in three queues, none of them the null stream's.  A decode takes the
+ * least loaded for its kernels and, for what runs beside them (forward sweep, sums, a copy), the least loaded of the
+ * other two.  Nothing in the API tells the queue of a stream, but it stays the same for its life: every
  * new stream is tried against the null stream and those found before it (ofk_meet, 0.03 ms a try), and held if it
  * will not do, so that the next goes elsewhere.  Where three queues are not to be found (fewer allowed, or too busy to
  * start two kernels within the time of a try) the gpubufs make do with what there is; only speed depends on it.
@@ -183,11 +184,11 @@ static void check_state_len(int state_len) {
 #define OFA_LANES 3
 #define OFA_LANE_TRIES 8
 #define OFA_MAX_DEVICES 64
-enum { LANE_MAIN = 0, LANE_SIDE = 1, LANE_MAIN_TOO = 2 }; /* in the order in which the queues are found */
 typedef struct {
     hipStream_t stream[OFA_LANES];
-    int gpubufs; /* that use them */
-    int turn;    /* which main lane the next gpubuf gets */
+    int load[OFA_LANES]; /* 2 for every decode whose kernels are there, 1 for every one with something beside them */
+    int last;            /* where the last decode's kernels went */
+    int gpubufs;         /* that use them */
 } ofa_lanes_t;
 static ofa_lanes_t g_lanes[OFA_MAX_DEVICES];
 static pthread_mutex_t g_lanes_mutex = PTHREAD_MUTEX_INITIALIZER;
@@ -217,23 +218,62 @@ static void find_lanes(ofa_lanes_t *l, volatile int *h_mark, int *d_mark) {
     while (others > 0) HIP_OK(hipStreamDestroy(other[--others]));
 }
 
-static void take_lanes(ofa_gpubuf_t *g) {
+static void open_lanes(ofa_gpubuf_t *g) {
     HIP_OK(hipGetDevice(&g->device));
     if (g->device < 0 || g->device >= OFA_MAX_DEVICES) die("gpubuf: device number out of range");
     ofa_lanes_t *l = &g_lanes[g->device];
     pthread_mutex_lock(&g_lanes_mutex);
     if (l->gpubufs++ == 0) find_lanes(l, (volatile int *)g->h_out, (int *)g->d_out);
-    g->s_main = l->stream[l->turn ? LANE_MAIN_TOO : LANE_MAIN];
-    l->turn = !l->turn;
-    g->s_side = l->stream[LANE_SIDE];
     pthread_mutex_unlock(&g_lanes_mutex);
 }
 
-static void give_lanes_back(ofa_gpubuf_t *g) {
+static void close_lanes(ofa_gpubuf_t *g) {
     ofa_lanes_t *l = &g_lanes[g->device];
     pthread_mutex_lock(&g_lanes_mutex);
     if (--l->gpubufs == 0)
         for (int i = 0; i < OFA_LANES; ++i) HIP_OK(hipStreamDestroy(l->stream[i]));
+    pthread_mutex_unlock(&g_lanes_mutex);
+}
+
+/* the least loaded lane other than `taken`, of equals the first after `last` */
+static int least_loaded(const ofa_lanes_t *l, int last, int taken) {
+    int best = -1;
+    for (int k = 1; k <= OFA_LANES; ++k) {
+        const int i = (last + k) % OFA_LANES;
+        if (i != taken && (best < 0 || l->load[i] < l->load[best])) best = i;
+    }
+    return best;
+}
+
+/* A lane for the kernels of a decode.  Returns whether another decode is under way on the device. */
+static int take_main_lane(ofa_gpubuf_t *g) {
+    ofa_lanes_t *l = &g_lanes[g->device];
+    pthread_mutex_lock(&g_lanes_mutex);
+    int others = 0;
+    for (int i = 0; i < OFA_LANES; ++i) others |= l->load[i] > 0;
+    g->main_lane = l->last = least_loaded(l, l->last, -1);
+    g->side_lane = -1;
+    l->load[g->main_lane] += 2;
+    g->s_main = l->stream[g->main_lane];
+    pthread_mutex_unlock(&g_lanes_mutex);
+    return others;
+}
+
+/* another one for what runs beside them */
+static void take_side_lane(ofa_gpubuf_t *g) {
+    ofa_lanes_t *l = &g_lanes[g->device];
+    pthread_mutex_lock(&g_lanes_mutex);
+    g->side_lane = least_loaded(l, g->main_lane, g->main_lane);
+    l->load[g->side_lane] += 1;
+    g->s_side = l->stream[g->side_lane];
+    pthread_mutex_unlock(&g_lanes_mutex);
+}
+
+static void leave_lanes(ofa_gpubuf_t *g) {
+    ofa_lanes_t *l = &g_lanes[g->device];
+    pthread_mutex_lock(&g_lanes_mutex);
+    l->load[g->main_lane] -= 2;
+    if (g->side_lane >= 0) l->load[g->side_lane] -= 1;
     pthread_mutex_unlock(&g_lanes_mutex);
 }
 
@@ -278,7 +318,7 @@ openfish_gpubuf_t *openfish_gpubuf_init(const int T, const int N, const int stat
         HIP_OK(hipMalloc((void **)&g->lse_table, sizeof tab));
         HIP_OK(hipMemcpy(g->lse_table, tab, sizeof tab, hipMemcpyHostToDevice));
     }
-    take_lanes(g);
+    open_lanes(g);
     for (int i = 0; i < EV_COUNT; ++i) HIP_OK(hipEventCreate(&g->ev[i]));
     return &g->pub;
 }
@@ -287,6 +327,7 @@ openfish_gpubuf_t *openfish_gpubuf_init(const int T, const int N, const int stat
 static void wait_for_decode(ofa_gpubuf_t *g) {
     if (g->pend_copy) HIP_OK(hipEventSynchronize(g->ev[EV_MOVES]));
     HIP_OK(hipEventSynchronize(g->ev[EV_SEQ_END])); /* the main lane has waited for what ran on the side lane */
+    leave_lanes(g);
 }
 
 void openfish_gpubuf_free(openfish_gpubuf_t *gpubuf) {
@@ -297,7 +338,7 @@ void openfish_gpubuf_free(openfish_gpubuf_t *gpubuf) {
         wait_for_decode(g);
     }
     for (int i = 0; i < EV_COUNT; ++i) HIP_OK(hipEventDestroy(g->ev[i]));
-    give_lanes_back(g);
+    close_lanes(g);
     HIP_OK(hipHostFree(g->h_out));
     HIP_OK(hipFree(g->lse_table));
     HIP_OK(hipFree(g->slab));
@@ -428,6 +469,7 @@ static void fetch_outputs(ofa_gpubuf_t *g, int T, int N, uint8_t **moves, char *
     HIP_OK(hipEventRecord(g->ev[EV_MOVES], g->s_main));
     alloc_outputs(T, N, moves, sequence, qstring);
     HIP_OK(hipEventSynchronize(g->ev[EV_MOVES]));
+    leave_lanes(g);
     memcpy(*moves, g->h_out, nt);
     memcpy(*sequence, g->h_out + nt, nt);
     memcpy(*qstring, g->h_out + 2 * nt, nt);
@@ -467,7 +509,7 @@ static void join_null_stream(ofa_gpubuf_t *g) {
  * that has one of them in the merged kernel takes 2.5 ms whatever the others do, and split has units left for the
  * forward sweep up to three chunks to a unit.
  *
- * A decode that is enqueued shares the machine with others; two at a time, one | split | merged:
+ * A decode that is enqueued, or finds another one under way, shares the machine; two at a time, one | split | merged:
  *   1024 states: 16, T = 833 1.99 | 2.48 | 1.84;  128 4.32 | 5.01 | 3.89;  256 five columns 8.44 | 8.55 | 6.40;
  *                320 10.27 | 10.07 | 8.16;  16, T = 100 0.38 | 0.50 | 0.41
  *    256 states: 128 2.64 | 2.35 | 2.07;  512 5.34 | 4.65 | 3.78;  520 5.69 | 4.78 | 5.70;  640 five columns 6.77 | 6.03 | 6.17;
@@ -476,35 +518,35 @@ static void join_null_stream(ofa_gpubuf_t *g) {
  *
  * The merged kernel exists for 256 and 1024 states with the default arithmetic and its own states per lane; without it
  * (can_merge = 0) 1024 states keep the one kernel and 256 states the split sweeps where they are ahead of it. */
-static int arrangement_by_default(int T, int N, int C, int state_len, int enqueued, int can_merge) {
+static int arrangement_by_default(int T, int N, int C, int state_len, int shared, int can_merge) {
     const size_t step_bytes = (size_t)N * (4 * (size_t)C + 12 * (size_t)states_of(state_len)); /* of split */
     switch (state_len) {
         case 3: return N <= 2048 ? ARR_SPLIT : ARR_ONE;
         case 4:
             if (!can_merge) return N <= 768 ? ARR_SPLIT : ARR_ONE;
-            if (N <= 512) return enqueued || step_bytes > 3800000 ? ARR_MERGED : ARR_SPLIT;
-            return N <= (enqueued ? 640 : 768) ? ARR_SPLIT : ARR_MERGED;
+            if (N <= 512) return shared || step_bytes > 3800000 ? ARR_MERGED : ARR_SPLIT;
+            return N <= (shared ? 640 : 768) ? ARR_SPLIT : ARR_MERGED;
         default:
             if (!can_merge) return ARR_ONE;
-            if (enqueued) return T < 128 && N <= 160 ? ARR_ONE : ARR_MERGED;
+            if (shared) return T < 128 && N <= 160 ? ARR_ONE : ARR_MERGED;
             if (N > 256 && N <= 320) return ARR_SPLIT;
             if (T < 128) return ARR_ONE;
             return N <= 160 ? ARR_SPLIT : ARR_MERGED;
     }
 }
 
-int openfish_amd_scan_arrangement(int T, int N, int C, int state_len, int enqueued) {
+int openfish_amd_scan_arrangement(int T, int N, int C, int state_len, int shared) {
     check_state_len(state_len);
-    return arrangement_by_default(T, N, C, state_len, enqueued, state_len >= 4);
+    return arrangement_by_default(T, N, C, state_len, shared, state_len >= 4);
 }
 
 /* the arrangement of one decode: what the gpubuf asks for, or by the rule above.  Merged asked for where it does not
  * exist gives way to the choice among the other two. */
-static int arrangement_of(const ofa_gpubuf_t *g, int T, int N, int C, int state_len, int enqueued) {
+static int arrangement_of(const ofa_gpubuf_t *g, int T, int N, int C, int state_len, int shared) {
     const int can_merge = state_len >= 4 && g->scan_mode == OFK_SCAN_TWO_TIER && g->scan_spl == 0;
     if (g->split_scans == ARR_ONE || g->split_scans == ARR_SPLIT) return g->split_scans;
     if (g->split_scans == ARR_MERGED && can_merge) return ARR_MERGED;
-    return arrangement_by_default(T, N, C, state_len, enqueued, can_merge);
+    return arrangement_by_default(T, N, C, state_len, shared, can_merge);
 }
 
 /* Queue one decode on the gpubuf's streams, results into its pinned staging buffer; returns
@@ -514,18 +556,23 @@ static void enqueue_decode(ofa_gpubuf_t *g, const int T, const int N, const int 
     const float stay = options->blank_score; /* as the reference GPU path, src/decode_hip.hip:120 */
     const size_t nt = (size_t)N * (size_t)T;
 
-    join_null_stream(g);
-    HIP_OK(hipEventRecord(g->ev[EV_START], g->s_main));
     const int cols = columns_of(C, state_len);
-    g->pend_split = arrangement_of(g, T, N, C, state_len, enqueued);
+    const int others = take_main_lane(g), shared = others || enqueued;
+    g->pend_split = arrangement_of(g, T, N, C, state_len, shared);
     /* Sums only where the search leaves the machine idle, and not with 1024 states, whose search waits for
      * memory and was measured to take half as long again beside the extra kernel.
      * With split scans the posteriors are complete when the forward kernel ends.  With 64 states that is
      * well before the search does (0.83 against 1.13 ms at 512 chunks), and the sums (0.21 ms) fit in
-     * between; with 256 states the two end together and the sequence stage gathers by itself. */
+     * between; with 256 states the two end together and the sequence stage gathers by itself, as it does where
+     * another decode waits for the side lane (four decodes of 256 chunks of 64 states: 4.19 ms with sums, 3.69 without;
+     * the results have the same bits). */
     const int sums_fit = g->path_sums != NULL && N <= OFK_SPARSE_SEARCH_MAX_CHUNKS;
-    const int use_sums = sums_fit && (g->pend_split == ARR_ONE || (g->pend_split == ARR_SPLIT && state_len == 3));
+    const int use_sums = sums_fit && (g->pend_split == ARR_ONE || (g->pend_split == ARR_SPLIT && state_len == 3 && !others));
     g->pend_sums = use_sums;
+    g->pend_copy = !shared;
+    if (g->pend_split == ARR_SPLIT || use_sums || g->pend_copy) take_side_lane(g);
+    join_null_stream(g);
+    HIP_OK(hipEventRecord(g->ev[EV_START], g->s_main));
     if (g->pend_split == ARR_MERGED) {
         /* backward sweep, then the search with the forward sweep and the posterior in its workgroups */
         launch_ok(ofk_bwd_scan(scores_TNC, g->pub.bwd_NTC, T, N, state_len, cols, stay, g->scan_mode, g->scan_spl, g->s_main),
@@ -581,11 +628,10 @@ static void enqueue_decode(ofa_gpubuf_t *g, const int T, const int N, const int 
         }
     }
 
-    /* The moves are final once the beam search is.  Of a blocking decode they travel, and the host takes them, while
-     * the sequence stage runs.  Of an enqueued one nobody waits for them: that stage writes them to the host itself
-     * (0.02 ms), because a copy that waits for the search would hold up the forward sweep of the next decode behind
+    /* The moves are final once the beam search is.  Of a decode that has the device to itself they travel, and
+     * the host takes them, while the sequence stage runs.  Otherwise that stage writes them to the host itself (0.02 ms),
+     * because a copy that waits for the search would hold up another decode's forward sweep behind
      * it on the side lane (two batches of 16 chunks of 64 states in flight: 2.14 ms with the copies, 1.63 without). */
-    g->pend_copy = !enqueued;
     if (g->pend_copy) {
         HIP_OK(hipStreamWaitEvent(g->s_side, g->ev[EV_BEAM_END], 0));
         HIP_OK(hipMemcpyAsync(g->h_out, g->pub.moves, nt, hipMemcpyDeviceToHost, g->s_side));
@@ -602,7 +648,7 @@ static void enqueue_decode(ofa_gpubuf_t *g, const int T, const int N, const int 
      * are filled by the stage-level entry points only. */
     launch_ok(ofk_sequence(g->pub.post_NTC, (int32_t *)g->pub.states, g->pub.moves, g->pub.qual_data,
                            g->pub.base_probs, g->pub.total_probs, (char *)g->d_out + nt, (char *)g->d_out + 2 * nt, T, N,
-                           state_len, phred_for(g, options), use_sums ? g->path_sums : NULL, enqueued ? g->d_out : NULL, g->s_main), "sequence");
+                           state_len, phred_for(g, options), use_sums ? g->path_sums : NULL, g->pend_copy ? NULL : g->d_out, g->s_main), "sequence");
     HIP_OK(hipEventRecord(g->ev[EV_SEQ_END], g->s_main));
     g->pending = 1;
     g->pend_T = T;
@@ -620,9 +666,12 @@ void openfish_decode_gpu(const int T, const int N, const int C, void *scores_TNC
 
     enqueue_decode(g, T, N, C, scores_TNC, state_len, options, 0);
     alloc_outputs(T, N, moves, sequence, qstring);
-    HIP_OK(hipEventSynchronize(g->ev[EV_MOVES]));
-    memcpy(*moves, g->h_out, nt);
-    HIP_OK(hipEventSynchronize(g->ev[EV_SEQ_END]));
+    if (g->pend_copy) {
+        HIP_OK(hipEventSynchronize(g->ev[EV_MOVES]));
+        memcpy(*moves, g->h_out, nt);
+    }
+    wait_for_decode(g);
+    if (!g->pend_copy) memcpy(*moves, g->h_out, nt);
     memcpy(*sequence, g->h_out + nt, nt);
     memcpy(*qstring, g->h_out + 2 * nt, nt);
     g->pending = 0;
@@ -768,6 +817,7 @@ void openfish_amd_decode_from_tensors(int T, int N, int C, const void *scores, i
     check_scores(T, N, C, scores, state_len, options);
     if (!moves || !sequence || !qstring) die("decode: output pointer is NULL");
     ofa_gpubuf_t *g = checked(gpubuf, T, N, state_len);
+    take_main_lane(g);
     join_null_stream(g);
     launch_ok(ofk_beam_search(scores, bwd, (ofk_beam_slot_t *)g->pub.beam_vector, (int32_t *)g->pub.states,
                               g->pub.moves, T, N, state_len, columns_of(C, state_len), log_beam_cut(options),

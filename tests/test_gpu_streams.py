@@ -8,6 +8,7 @@ import numpy as np
 import pytest
 
 from openfish_amd import synth
+from test_gpu_parity import qstring_close
 from test_gpu_scan_options import api  # noqa: F401
 
 pytestmark = pytest.mark.gpu
@@ -38,12 +39,12 @@ def test_forward_sweep_runs_beside_the_search_in_every_gpubuf(api, scores):  # n
     assert max(ratios) < 1.25, ratios
 
 
-@pytest.mark.parametrize("others", [0, 1, 2, 3])
-def test_two_batches_in_flight_run_side_by_side(api, scores, others):  # noqa: F811
-    """two decodes of 64 chunks together take 1.1 times as long as one, and twice as long where they share a queue or one
-    sits in the null stream's"""
+@pytest.mark.parametrize("batches,others", [(2, 0), (2, 1), (2, 2), (2, 3), (3, 0), (3, 1)])
+def test_batches_in_flight_run_side_by_side(api, scores, batches, others):  # noqa: F811
+    """two or three decodes of 64 chunks together take 1.1 to 1.2 times as long as one, and twice as long where two of them
+    share a queue or one sits in the null stream's"""
     kept = [api.GpuBuf(32, 1, 3) for _ in range(others)]
-    bufs = [api.GpuBuf(T, N, STATE_LEN) for _ in range(2)]
+    bufs = [api.GpuBuf(T, N, STATE_LEN) for _ in range(batches)]
 
     def ms(which):
         best = 1e9
@@ -57,14 +58,15 @@ def test_two_batches_in_flight_run_side_by_side(api, scores, others):  # noqa: F
         return best * 1e3
 
     ms(bufs)
-    one, two = ms(bufs[:1]), ms(bufs)
-    assert two < 1.5 * one, (one, two)
+    one, together = ms(bufs[:1]), ms(bufs)
+    assert together < 1.6 * one, (one, together)
     del kept
 
 
 def test_gpubufs_made_used_and_freed_by_several_threads(api, scores):  # noqa: F811
     """the streams that gpubufs share come and go with them: threads that make, use and free gpubufs at the same time, down to
-    none and up again, all get the results of a single one"""
+    none and up again, all get the results of a single one (the quality characters within their bound: a decode that finds
+    another under way takes another arrangement, whose posteriors are summed in another order)"""
     def decode():
         gb = api.GpuBuf(T, N, STATE_LEN)
         out = api.openfish_decode_gpu(T, N, 4 * S, scores, STATE_LEN, api.DECODER_INIT(), gb)
@@ -76,12 +78,16 @@ def test_gpubufs_made_used_and_freed_by_several_threads(api, scores):  # noqa: F
     def work():
         api.lib().set_device_hip(0)
         for _ in range(5):
-            if not all(np.array_equal(a, b) for a, b in zip(decode(), want)):
-                wrong.append(1)
+            try:
+                mv, sq, qs = decode()
+                assert np.array_equal(mv, want[0]) and np.array_equal(sq, want[1])
+                qstring_close(qs, want[2], mv)
+            except Exception as e:  # an exception in a thread would otherwise pass silently
+                wrong.append(e)
 
     threads = [threading.Thread(target=work) for _ in range(3)]
     for th in threads:
         th.start()
     for th in threads:
         th.join()
-    assert not wrong
+    assert not wrong, wrong
