@@ -504,7 +504,8 @@ static void join_null_stream(ofa_gpubuf_t *g) {
  *     64 states: 16 1.83 | 1.58;  512 2.03 | 1.76;  2048 4.37 | 3.61
  * Hence the lines: up to 160 chunks of 1024 states the search (two chunks to a unit) and the forward sweep (one) find
  * compute units of their own; above 256 merged takes a second round of workgroups, split does so only above 320; chunks
- * shorter than 128 steps are decided by launches and set-up.  Up to 512 chunks of 256 states the chain of split is
+ * shorter than 128 steps are decided by launches and set-up (from 16 to 256 of them no arrangement is ahead by more than
+ * 0.03 ms, and they take that of longer ones).  Up to 512 chunks of 256 states the chain of split is
  * shorter, while its bytes fit beneath the chain, 3.8 MB a step; above, the search's workgroups hold four chunks, a unit
  * that has one of them in the merged kernel takes 2.5 ms whatever the others do, and split has units left for the
  * forward sweep up to three chunks to a unit.
@@ -528,10 +529,9 @@ static int arrangement_by_default(int T, int N, int C, int state_len, int shared
             return N <= (shared ? 640 : 768) ? ARR_SPLIT : ARR_MERGED;
         default:
             if (!can_merge) return ARR_ONE;
-            if (shared) return T < 128 && N <= 160 ? ARR_ONE : ARR_MERGED;
-            if (N > 256 && N <= 320) return ARR_SPLIT;
-            if (T < 128) return ARR_ONE;
-            return N <= 160 ? ARR_SPLIT : ARR_MERGED;
+            if (T < 128 && (N < 16 || (N > 320 && !shared))) return ARR_ONE;
+            if (shared) return ARR_MERGED;
+            return N <= 160 || (N > 256 && N <= 320) ? ARR_SPLIT : ARR_MERGED;
     }
 }
 
