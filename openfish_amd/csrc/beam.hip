@@ -535,12 +535,15 @@ __global__ __launch_bounds__((kBeamThreads<S, CPG, COLS, FWD>), (BeamCfg<S, FWD>
 #pragma unroll
             for (int k = 0; k < SPL; ++k) f[k] = 0.f;
             int rows_ready = 0, rows_taken = 0, slot = 0;
-            auto publish_row = [&](int t) {
+            auto write_row = [&](int t) {
 #pragma unroll
                 for (int k = 0; k < SPL; ++k) fw.vec[t % kVecRows][s0 + k] = f[k];
+            };
+            auto publish_row = [&](int t) {
                 wave_fence();
                 __hip_atomic_store(&fw.published[w], t + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
             };
+            write_row(0);
             publish_row(0);
             for (int t = 0; t < T; ++t) {
                 while (rows_ready <= t) {
@@ -566,7 +569,7 @@ __global__ __launch_bounds__((kBeamThreads<S, CPG, COLS, FWD>), (BeamCfg<S, FWD>
                     v[k][3] = ::add_half<0>(row.w[2 * k + 1], p2);
                     v[k][4] = ::add_half<1>(row.w[2 * k + 1], p3);
                 }
-                lse5_all<SPL, OFK_SCAN_TWO_TIER>(f, v, logtab);
+                lse5_all<SPL, OFK_SCAN_TWO_TIER>(f, v, logtab, [&] { write_row(t + 1); }, [](bool) {});
                 __builtin_amdgcn_s_setprio(2);  // a trip through the second tier leaves it at 0
                 publish_row(t + 1);
             }

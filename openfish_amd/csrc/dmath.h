@@ -61,7 +61,7 @@ OFA_HD float float_of(uint32_t u) {
      0x1.ffffffffffe17p-2,  0x1.000000000001dp+0,  6755399441055744.0,    1.4426950408889634074,         \
      -0.69314718055994530942}
 #define OFA_EXP_COEF_COUNT 13
-OFA_HD double exp_reduced(double r, const double *c) {
+OFA_HD double exp_reduced(double r, const double *c, double unit = 1.0) {
     double p = c[0];
     p = __builtin_fma(p, r, c[1]);
     p = __builtin_fma(p, r, c[2]);
@@ -72,7 +72,7 @@ OFA_HD double exp_reduced(double r, const double *c) {
     p = __builtin_fma(p, r, c[7]);
     p = __builtin_fma(p, r, c[8]);
     p = __builtin_fma(p, r, c[9]);
-    return __builtin_fma(p, r, 1.0);
+    return __builtin_fma(p, r, unit);
 }
 
 // e^x for a double x (|x| < 1e9: the integer part of x*log2(e) is read from 32 bits); the scans
@@ -80,12 +80,13 @@ OFA_HD double exp_reduced(double r, const double *c) {
 // One-step argument reduction r = x - n ln2 with ln2 rounded to double: its error, |n| 2^-54
 // relative to e^x, is |n| 2^(-54-|n|/0.69..) relative to 1, and the sums these exponentials
 // enter are at least 1 (one term of every sum is e^0).  The scaling by 2^n is a true ldexp,
-// which underflows to zero by itself.
-OFA_HD double exp_ldexp(double x, const double *c) {
+// which underflows to zero by itself.  A `unit` of 1 + u moves the result by a factor between 1 + 0.7 u and 1 + 1.42 u
+// at no cost.
+OFA_HD double exp_ldexp(double x, const double *c, double unit = 1.0) {
     const double t = __builtin_fma(x, c[11], c[10]);
     const double n = t - c[10];
     const double r = __builtin_fma(n, c[12], x);  // |r| <= ln2/2 (+ 1e-14)
-    const double p = exp_reduced(r, c);
+    const double p = exp_reduced(r, c, unit);
     return __builtin_ldexp(p, (int)(uint32_t)bits_of(t));
 }
 OFA_HD double exp_nonpos_ldexp(float d, const double *c) { return exp_ldexp((double)d, c); }
@@ -267,30 +268,45 @@ OFA_HD float log2_hw(float x) {
 
 struct Lse5Estimate {
     float value;
-    float sum;  // the fp32 estimate of the sum of exponentials, within 1e-6 (relative) of the CPU path's
+    float sum;   // the fp32 estimate of the sum of exponentials, within 1e-6 (relative) of the CPU path's
+    float half;  // h: half an ulp of `value`, of the smaller neighbour's binade for a power of two
     bool settled;
 };
-OFA_HD Lse5Estimate lse5_estimate(float v0, float v1, float v2, float v3, float v4, float m) {
+// the estimate, and apart from it the verdict, which a kernel need not have before it hands the estimate on
+struct Lse5Value {
+    float value, sum, l2;
+};
+OFA_HD Lse5Value lse5_value(float v0, float v1, float v2, float v3, float v4, float m) {
     const float kLog2e = 1.44269504088896340736f, kLn2 = 0.69314718055994530942f;
     float s = exp2_hw((v0 - m) * kLog2e);
     s += exp2_hw((v1 - m) * kLog2e);
     s += exp2_hw((v2 - m) * kLog2e);
     s += exp2_hw((v3 - m) * kLog2e);
     s += exp2_hw((v4 - m) * kLog2e);
-    const float kEps0 = 8.68e-7f, kEpsMu = 5.21e-7f, kEps1 = 6.42e-8f;
-    const float l2 = log2_hw(s);
-    Lse5Estimate e;
+    Lse5Value e;
     e.sum = s;
-    e.value = __builtin_fmaf(l2, kLn2, m);
-    const float rho = __builtin_fmaf(l2, kLn2, -(e.value - m));
-    const uint32_t rb = bits_of(e.value);
+    e.l2 = log2_hw(s);
+    e.value = __builtin_fmaf(e.l2, kLn2, m);
+    return e;
+}
+OFA_HD Lse5Estimate lse5_verdict(Lse5Value x, float m) {
+    const float kLn2 = 0.69314718055994530942f;
+    const float kEps0 = 8.68e-7f, kEpsMu = 5.21e-7f, kEps1 = 6.42e-8f;
+    Lse5Estimate e;
+    e.value = x.value;
+    e.sum = x.sum;
+    const float rho = __builtin_fmaf(x.l2, kLn2, -(x.value - m));
+    const uint32_t rb = bits_of(x.value);
     // exponent field of the float below |r~|, lowered by 24; where that wraps, the sign bit survives the mask
-    const float h = float_of(((rb & 0x7fffffffu) - ((24u << 23) + 1u)) & 0xff800000u);
-    const uint32_t sb = bits_of(s) + 16u;
+    e.half = float_of(((rb & 0x7fffffffu) - ((24u << 23) + 1u)) & 0xff800000u);
+    const uint32_t sb = bits_of(x.sum) + 16u;
     const float mu = float_of((sb & 0x007fffffu) | 0x3f000000u);
     const float eps = __builtin_fmaf(mu, -kEpsMu, __builtin_fmaf(float_of(sb & 0x7f800000u), kEps1, kEps0));
-    e.settled = h - __builtin_fabsf(rho) > eps;
+    e.settled = e.half - __builtin_fabsf(rho) > eps;
     return e;
+}
+OFA_HD Lse5Estimate lse5_estimate(float v0, float v1, float v2, float v3, float v4, float m) {
+    return lse5_verdict(lse5_value(v0, v1, v2, v3, v4, m), m);
 }
 
 // the scan update in two tiers: the estimate where it is settled, the CPU roundings elsewhere

@@ -280,38 +280,39 @@ __device__ __forceinline__ void fwd_terms(float (&v)[SPL][5], const float (&f)[S
 // states, and with 1024 only between the phases.  Scans of 2048 chunks of 256 states, T = 1666: 6.87 ms all four
 // together, 5.8 now (five columns 7.87, 5.8); 512 chunks of 1024 states 6.14, 5.4; with the batch spread over twice the
 // lanes 6.07, 6.15 and 5.82.
-template <int SPL, int MODE>
-__device__ __forceinline__ void bwd_update(float (&a)[SPL], const float4 &nx, const BwdRow<SPL> &row, float stay, const LogArgs &logtab) {
+// `publish` writes the new values to LDS (lse5_all says when; with four states to a lane once all of them are there).
+template <int SPL, int MODE, typename Publish>
+__device__ __forceinline__ void bwd_update(float (&a)[SPL], const float4 &nx, const BwdRow<SPL> &row, float stay, const LogArgs &logtab,
+                                           Publish &&publish) {
     if constexpr (SPL < 4) {
         float v[SPL][5];
         bwd_terms(v, a, nx, row, stay);
-        lse5_all<SPL, MODE>(a, v, logtab);
+        lse5_all<SPL, MODE>(a, v, logtab, publish, [](bool) {});
     } else {
         static_for<SPL>([&](auto i) {
             float v[1][5], out[1];
             bwd_terms_of<i, SPL>(v[0], a, nx, row, stay);
-            lse5_all<1, MODE>(out, v, logtab);
+            lse5_all<1, MODE, true>(out, v, logtab, [] {}, [](bool) {});
             a[i] = out[0];
         });
+        publish();
     }
 }
-template <int SPL, int MODE>
+template <int SPL, int MODE, typename Publish>
 __device__ __forceinline__ void fwd_update(float (&f)[SPL], float p0, float p1, float p2, float p3, const FwdRow<SPL> &row, float stay,
-                                           const LogArgs &logtab) {
+                                           const LogArgs &logtab, Publish &&publish) {
     if constexpr (SPL < 4) {
         float v[SPL][5];
         fwd_terms(v, f, p0, p1, p2, p3, row, stay);
-        lse5_all<SPL, MODE>(f, v, logtab);
+        lse5_all<SPL, MODE>(f, v, logtab, publish, [](bool) {});
     } else {
-        static_for<SPL / 2>([&](auto h) {
-            constexpr int i = 2 * h;
-            float v[2][5], out[2];
+        static_for<SPL>([&](auto i) {
+            float v[1][5], out[1];
             fwd_terms_of<i, SPL>(v[0], f, p0, p1, p2, p3, row, stay);
-            fwd_terms_of<i + 1, SPL>(v[1], f, p0, p1, p2, p3, row, stay);
-            lse5_all<2, MODE>(out, v, logtab);
+            lse5_all<1, MODE, true>(out, v, logtab, [] {}, [](bool) {});
             f[i] = out[0];
-            f[i + 1] = out[1];
         });
+        publish();
     }
 }
 
@@ -346,7 +347,7 @@ __global__ __launch_bounds__((Shape<S, SPL>::kThreads)) void bwd_scan_kernel(
     const unsigned sc_lane = g_eff * kCols * S + 4 * kCols * r + kLead + c0;
     const unsigned st_lane = g_eff * (unsigned)(T + 1) * S + r + c0 * Q;
     const _Float16 *pre = scores + (size_t)first_chunk * kCols * S + (ptrdiff_t)(T - 1) * row_stride;  // next row to fetch
-    float *orow = bwd + ((size_t)first_chunk * (size_t)(T + 1) + T) * S;                              // next row to store
+    float *orow = bwd + ((size_t)first_chunk * (size_t)(T + 1) + T) * S;                              // row stored last
 
     float a[SPL];
 #pragma unroll
@@ -355,7 +356,6 @@ __global__ __launch_bounds__((Shape<S, SPL>::kThreads)) void bwd_scan_kernel(
         orow[st_lane + i * Q] = 0.f;
         vec[g][0][Vec::at(r, c0 + i)] = 0.f;
     }
-    orow -= S;
 
     // The first rows are fetched without a condition (of a chunk shorter than DEPTH the oldest row again):
     // were they not, the compiler, which counts loads in flight, would have to assume that a row's load may
@@ -368,23 +368,49 @@ __global__ __launch_bounds__((Shape<S, SPL>::kThreads)) void bwd_scan_kernel(
     int buf = 0;
     __syncthreads();  // the log table is shared by the whole group
 
+    // The chain of a step: LDS read, terms, estimate, LDS write (and the barrier).  The verdict on the estimates is formed
+    // while the write is under way, the row's store and the loads ahead are issued while the verdict's mask is (lse5_all);
+    // where a chunk is one wave, the next step's read is asked for as soon as the values are written.
+    auto neighbours = [&](int b) { return *reinterpret_cast<const float4 *>(&vec[g][b][Vec::of(4 * r)]); };
+    constexpr bool kBehindRead = SPL == 1;
+    float4 nx;
+    if constexpr (!Sh::kMultiWave) {
+        chunk_sync<false>();
+        nx = neighbours(0);
+    }
     pipelined<DEPTH>(T, [&](auto k, int j, auto checked) {
-        chunk_sync<Sh::kMultiWave>();
-        const float4 nx = *reinterpret_cast<const float4 *>(&vec[g][buf][Vec::of(4 * r)]);
+        if constexpr (Sh::kMultiWave) {
+            chunk_sync<true>();
+            nx = neighbours(buf);
+        }
+        const BwdRow<SPL> row = ring[k];
+        auto load_ahead = [&] {
+            if (!checked || j + DEPTH < T) {
+                ring[k].load(pre + sc_lane);
+                pre -= row_stride;
+            }
+        };
+        if constexpr (kBehindRead) {
+            __builtin_amdgcn_sched_barrier(0);
+            load_ahead();
+            __builtin_amdgcn_sched_barrier(0);
+        }
         float v[SPL][5];
-        bwd_terms(v, a, nx, ring[k], stay);
-        if (!checked || j + DEPTH < T) {
-            ring[k].load(pre + sc_lane);
-            pre -= row_stride;
-        }
-        lse5_all<SPL, MODE>(a, v, logtab);
+        bwd_terms(v, a, nx, row, stay);
         buf ^= 1;
-#pragma unroll
-        for (int i = 0; i < SPL; ++i) {
-            vec[g][buf][Vec::at(r, c0 + i)] = a[i];
-            orow[st_lane + i * Q] = a[i];
-        }
         orow -= S;
+        lse5_all<SPL, MODE>(a, v, logtab, [&] {
+#pragma unroll
+            for (int i = 0; i < SPL; ++i) vec[g][buf][Vec::at(r, c0 + i)] = a[i];
+            if constexpr (!Sh::kMultiWave) {
+                chunk_sync<false>();
+                nx = neighbours(buf);
+            }
+        }, [&](bool first) {
+#pragma unroll
+            for (int i = 0; i < SPL; ++i) orow[st_lane + i * Q] = a[i];
+            if (!kBehindRead && first) load_ahead();
+        });
     });
 }
 
@@ -460,9 +486,10 @@ __global__ __launch_bounds__((Shape<S, SPL>::kThreads)) void fwd_post_kernel(
 #pragma unroll
     for (int i = 0; i < SPL; ++i) f[i] = 0.f;
     int buf = 0;
+    fv.store(&vec[g][0][s0]);
     __syncthreads();  // the log table is shared by the whole group
 
-    // row j: its posterior, and the state vector goes to the other lanes
+    // row j: its posterior; the state vector, written by the update before, becomes visible to the other lanes
     auto row = [&](const FloatRun<SPL> &bw) {
         FloatRun<SPL> e;
         float total = 0.f;
@@ -472,7 +499,6 @@ __global__ __launch_bounds__((Shape<S, SPL>::kThreads)) void fwd_post_kernel(
             total += e.v[i];
         }
         total = group_sum<Sh::kGroup>(total);
-        fv.store(&vec[g][buf][s0]);
         if constexpr (Sh::kMultiWave) {
             if ((tid & 63) == 0) part[buf][g][wave] = total;
         }
@@ -502,8 +528,8 @@ __global__ __launch_bounds__((Shape<S, SPL>::kThreads)) void fwd_post_kernel(
             bring[k].load(bpre + st_lane);
             bpre += S;
         }
-        lse5_all<SPL, MODE>(f, v, logtab);
         buf ^= 1;
+        lse5_all<SPL, MODE>(f, v, logtab, [&] { fv.store(&vec[g][buf][s0]); }, [](bool) {});
     });
     static_for<DEPTH>([&](auto k) {
         if (T % DEPTH == (int)k) row(bring[k]);
@@ -568,24 +594,24 @@ __global__ __launch_bounds__((2 * (S / SPL))) void fwd_post_roles_kernel(
 #pragma unroll
         for (int i = 0; i < SPL; ++i) f[i] = 0.f;
         int buf = 0;
+        fv.store(&vec[0][s0]);  // row 0
         barrier();  // the other half exchanges the maxima behind the shift
         barrier();
         __syncthreads();  // the log table
         pipelined<DEPTH>(T, [&](auto k, int j, auto checked) {
-            fv.store(&vec[buf][s0]);  // row j
             barrier();
             const float p0 = vec[buf][q], p1 = vec[buf][q + Q];
             const float p2 = vec[buf][q + 2 * Q], p3 = vec[buf][q + 3 * Q];
             float v[SPL][5];
             fwd_terms(v, f, p0, p1, p2, p3, ring[k], stay);
-            if (!checked || j + DEPTH < T) {
-                ring[k].load(pre + sc_lane);
-                pre += row_stride;
-            }
-            lse5_all<SPL, OFK_SCAN_TWO_TIER>(f, v, logtab);
             buf ^= 1;
+            lse5_all<SPL, OFK_SCAN_TWO_TIER>(f, v, logtab, [&] { fv.store(&vec[buf][s0]); }, [&](bool first) {  // row j + 1
+                if (first && (!checked || j + DEPTH < T)) {
+                    ring[k].load(pre + sc_lane);
+                    pre += row_stride;
+                }
+            });
         });
-        fv.store(&vec[buf][s0]);  // row T
         barrier();
         barrier();  // the other half finishes row T
     } else {
@@ -710,7 +736,7 @@ __global__ __launch_bounds__((FusedShape<S, SPL>::kThreads), 4) void scan_post_k
     const int tid = threadIdx.x;
     const LogArgs logtab{logcells, centred, series.c, series.e, tier_lanes + (MODE == OFK_SCAN_TWO_TIER ? (tid & ~63) : 0)};
 
-    fill_log_tables<MODE>(logcells, centred);
+    fill_log_tables<MODE, MODE == OFK_SCAN_TWO_TIER>(logcells, centred);  // the first steps of either sweep take the always-double arithmetic
     const int g = tid / Sh::kChunkThreads, u = tid % Sh::kChunkThreads;
     const int forward = __builtin_amdgcn_readfirstlane(u / L);
     const int l = u % L, wave = l / 64;
@@ -767,10 +793,11 @@ __global__ __launch_bounds__((FusedShape<S, SPL>::kThreads), 4) void scan_post_k
                 }
                 step_sync();
                 const float4 nx = *reinterpret_cast<const float4 *>(&vecB[g][buf][VecB::of(4 * r)]);
-                bwd_update<SPL, M>(a, nx, row, stay, logtab);
                 buf ^= 1;
+                bwd_update<SPL, M>(a, nx, row, stay, logtab, [&] {
 #pragma unroll
-                for (int i = 0; i < SPL; ++i) vecB[g][buf][VecB::at(r, c0 + i)] = a[i];
+                    for (int i = 0; i < SPL; ++i) vecB[g][buf][VecB::at(r, c0 + i)] = a[i];
+                });
                 if (live) {
 #pragma unroll
                     for (int i = 0; i < SPL; ++i) orow[st_lane + i * Q] = a[i];
@@ -832,12 +859,14 @@ __global__ __launch_bounds__((FusedShape<S, SPL>::kThreads), 4) void scan_post_k
                 }
                 prow -= S;
                 const float4 nx = *reinterpret_cast<const float4 *>(&vecB[g][buf][VecB::of(4 * r)]);
-                bwd_update<SPL, MODE>(a, nx, row, stay, logtab);
                 buf ^= 1;
+                bwd_update<SPL, MODE>(a, nx, row, stay, logtab, [&] {
+#pragma unroll
+                    for (int i = 0; i < SPL; ++i) vecB[g][buf][VecB::at(r, c0 + i)] = a[i];
+                });
                 float total;
 #pragma unroll
                 for (int i = 0; i < SPL; ++i) {
-                    vecB[g][buf][VecB::at(r, c0 + i)] = a[i];
                     e_prev[i] = __builtin_amdgcn_exp2f(((fv[i] + a[i]) - shift) * kLog2e);
                     total = i ? total + e_prev[i] : e_prev[i];
                 }
@@ -876,6 +905,12 @@ __global__ __launch_bounds__((FusedShape<S, SPL>::kThreads), 4) void scan_post_k
             vecF[g][0][s0 + i] = 0.f;
         }
         int buf = 0;
+        auto hand_on = [&] {  // the state vector, to the other lanes
+            FloatRun<SPL> mine;
+#pragma unroll
+            for (int i = 0; i < SPL; ++i) mine.v[i] = f[i];
+            mine.store(&vecF[g][buf][s0]);
+        };
         FwdRow<SPL> ring[DEPTH];
         __syncthreads();
 
@@ -907,12 +942,8 @@ __global__ __launch_bounds__((FusedShape<S, SPL>::kThreads), 4) void scan_post_k
                 step_sync();
                 const float p0 = vecF[g][buf][q], p1 = vecF[g][buf][q + Q];
                 const float p2 = vecF[g][buf][q + 2 * Q], p3 = vecF[g][buf][q + 3 * Q];
-                fwd_update<SPL, M>(f, p0, p1, p2, p3, row, stay, logtab);
                 buf ^= 1;
-                FloatRun<SPL> mine;
-#pragma unroll
-                for (int i = 0; i < SPL; ++i) mine.v[i] = f[i];
-                mine.store(&vecF[g][buf][s0]);
+                fwd_update<SPL, M>(f, p0, p1, p2, p3, row, stay, logtab, hand_on);
             });
         };
         const int warm = MODE == OFK_SCAN_TWO_TIER ? (cnt1 < kWarmup ? cnt1 : kWarmup) : 0;
@@ -983,12 +1014,8 @@ __global__ __launch_bounds__((FusedShape<S, SPL>::kThreads), 4) void scan_post_k
                 if (!checked || j + 1 < cnt2) {
                     const float p0 = vecF[g][buf][q], p1 = vecF[g][buf][q + Q];
                     const float p2 = vecF[g][buf][q + 2 * Q], p3 = vecF[g][buf][q + 3 * Q];
-                    fwd_update<SPL, MODE>(f, p0, p1, p2, p3, row, stay, logtab);
                     buf ^= 1;
-                    FloatRun<SPL> mine;
-#pragma unroll
-                    for (int i = 0; i < SPL; ++i) mine.v[i] = f[i];
-                    mine.store(&vecF[g][buf][s0]);
+                    fwd_update<SPL, MODE>(f, p0, p1, p2, p3, row, stay, logtab, hand_on);
                 }
             });
         }
@@ -1135,7 +1162,7 @@ int states_per_lane(int S, int N, bool backward, int forced) {
 #endif
 // four states to a lane (2048 and more chunks of 256 states): a row more would not fit the 128 registers
 #ifndef OFK_DEPTH_FUSED_WIDE
-#define OFK_DEPTH_FUSED_WIDE 3
+#define OFK_DEPTH_FUSED_WIDE 2
 #endif
 #define OFK_DISPATCH(BACKWARD, LAUNCH, ...)                                                    \
     switch (state_len * 8 + states_per_lane(1 << (2 * state_len), N, BACKWARD, lanes_asked(mode, spl))) { \

@@ -58,3 +58,27 @@ def test_forward_sweep_within_the_search_gives_the_oracle_s_tensors(api, state_l
     assert np.array_equal(gb.tensor("bwd_NTC"), ref["bwd"])
     close(gb.tensor("post_NTC"), ref["post"])
     assert np.array_equal(mv, ref["moves"]) and np.array_equal(sq, ref["sequence"])
+
+
+# mean and spread of the scores, stay score, time steps: state values that hover about zero; that fall through negative
+# powers of two; that rise past 2^19, where half an ulp is beyond what the proofs of estimates allow for; coarse ulps from the start
+@pytest.mark.parametrize("mean,spread,stay,T", [(-1.65, 0.5, -1.65, 150), (-21.0, 3.0, -19.0, 220), (2600.0, 3.0, 2600.0, 230),
+                                                (30000.0, 2000.0, 30000.0, 40), (-30000.0, 8.0, -30000.0, 40), (0.0, 12.0, 2.0, 120)])
+@pytest.mark.parametrize("state_len,N", [(3, 3), (4, 2), (5, 1)])
+def test_estimates_are_settled_right_at_every_magnitude(api, state_len, N, mean, spread, stay, T):  # noqa: F811
+    """bwd bit for bit the oracle's, posteriors bit for bit those of the always-double arithmetic"""
+    S = 4 ** state_len
+    rng = np.random.default_rng(17 + T)
+    s16 = np.clip(rng.normal(mean, spread, (T, N, 4 * S)), -65000, 65000).astype(np.float16)
+    O.set_scan_stay(stay)
+    try:
+        ref_bwd, _, _ = O.scans(s16.astype(np.float32), state_len)
+    finally:
+        O.set_scan_stay()
+    got = {}
+    for fused in (False, True):
+        for mode in ("two_tier", "precise"):
+            bwd, post = stage_scans(api, s16, state_len, stay, api.SCAN_MODES[mode], fused)
+            assert np.array_equal(bwd, ref_bwd), (fused, mode)
+            got[fused, mode] = post
+        assert np.array_equal(got[fused, "two_tier"], got[fused, "precise"], equal_nan=True)
