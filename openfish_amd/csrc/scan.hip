@@ -1121,8 +1121,7 @@ bool aligned16(const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15u) ==
 
 // States per lane: the largest of {4, 2, 1} (fewest lanes, least LDS traffic per state)
 // that still gives every SIMD of the device (256 CUs x 4) a wave; small batches are
-// spread thinner.  1024 states at one state per lane would need 1024-thread groups
-// with a barrier per step, so that size stops at 2.
+// spread thinner.  1024 states stop at 2, except in the backward sweep (bwd_scan below).
 // The sweeps of the smaller models measure faster with two waves per SIMD (hac, 512 chunks:
 // backward 1.29 ms against 1.33 ms; forward + posterior beside the beam search 1.41 ms against
 // 1.61 ms, which is 13 000 chunks/s of a whole decode).
@@ -1218,6 +1217,12 @@ static int bwd_scan(const void *scores, float *bwd, int T, int N, int state_len,
     if (!scores || !bwd || T < 1 || N < 1 || !aligned16(scores) || !aligned16(bwd)) return OFK_BAD_ARGS;
     if (state_len < 3 || state_len > 5) return OFK_BAD_ARGS;
     hipStream_t st = static_cast<hipStream_t>(stream);
+    // Up to a chunk for every compute unit, 1024 states take one state to a lane, sixteen waves: four waves on a SIMD fill each
+    // other's waits, and a wave with half as many updates has the second tier's single trip more often (ms, two states to a
+    // lane | one: 37 chunks, T = 833 0.76 | 0.67; 256, T = 1666 1.45 | 1.32; 9, T = 64 0.091 | 0.078).  Two such workgroups do
+    // not fit a unit (257 chunks, T = 400 0.55 | 0.71; 512 0.68 | 0.75; 1024, T = 300 1.05 | 1.15).
+    if (state_len == 5 && mode == OFK_SCAN_TWO_TIER && spl == 0 && N <= 256)
+        return launch_bwd<1024, 1, OFK_DEPTH_1024>(mode, scores, bwd, T, N, stay, st);
     OFK_DISPATCH(true, launch_bwd, mode, scores, bwd, T, N, stay, st)
 }
 

@@ -82,3 +82,17 @@ def test_estimates_are_settled_right_at_every_magnitude(api, state_len, N, mean,
             assert np.array_equal(bwd, ref_bwd), (fused, mode)
             got[fused, mode] = post
         assert np.array_equal(got[fused, "two_tier"], got[fused, "precise"], equal_nan=True)
+
+
+@pytest.mark.parametrize("T,N", [(1, 256), (9, 255), (9, 257)])
+@pytest.mark.parametrize("columns", [4, 5])
+def test_backward_sweep_of_1024_states_on_either_side_of_a_chunk_per_unit(api, T, N, columns):  # noqa: F811
+    four = synth.crf_scores(T, N, 5, seed=N + T)
+    given = four
+    if columns == 5:
+        given = np.full((T, N, 1024, 5), np.nan, np.float16)
+        given[..., 1:] = four.reshape(T, N, 1024, 4)
+        given = given.reshape(T, N, 5 * 1024)
+    ref_bwd, _, _ = O.scans(four.astype(np.float32), 5)
+    bwd, _ = stage_scans(api, given, 5, 2.0, "two_tier", False)
+    assert np.array_equal(bwd, ref_bwd)
