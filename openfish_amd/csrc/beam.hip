@@ -529,7 +529,7 @@ __global__ __launch_bounds__((kBeamThreads<S, CPG, COLS, FWD>), (BeamCfg<S, FWD>
             constexpr int SPL = S / (64 * FWD), Q = S / 4;
             const int w = (wave - kFirstFwd) % FWD;
             const int s0 = SPL * (64 * w + lane), q = s0 >> 2;
-            const LogArgs logtab{all.logs.cells, all.logs.centred, series.c, series.e, fw.tier_lanes + 64 * w, 3};
+            const LogArgs logtab{all.logs.cells, all.logs.centred, series.c, series.e, fw.tier_lanes + 64 * w, 3, 2};
             __builtin_amdgcn_s_setprio(2);
             float f[SPL];
 #pragma unroll
@@ -570,7 +570,6 @@ __global__ __launch_bounds__((kBeamThreads<S, CPG, COLS, FWD>), (BeamCfg<S, FWD>
                     v[k][4] = ::add_half<1>(row.w[2 * k + 1], p3);
                 }
                 lse5_all<SPL, OFK_SCAN_TWO_TIER>(f, v, logtab, [&] { write_row(t + 1); }, [](bool) {});
-                __builtin_amdgcn_s_setprio(2);  // a trip through the second tier leaves it at 0
                 publish_row(t + 1);
             }
             return;

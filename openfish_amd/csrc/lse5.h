@@ -76,6 +76,7 @@ struct LogArgs {
     const double *expc;
     float *lanes;  // 64 floats of LDS owned by the calling wave (two-tier updates only)
     int hurry = 3;  // the wave's priority during a trip through the second tier
+    int rest = 0;   // and outside
     double unit = certificate_unit();
 };
 
@@ -163,6 +164,14 @@ __device__ __forceinline__ float running_sum_along_eight(double e) {
 #pragma unroll
     for (int k = 0; k < 4; ++k) s = (float)((double)dpp<0x111>(s) + e);  // row_shr:1
     return dpp<0x00>(s);                                                 // quad_perm:[0,0,0,0]
+}
+
+// the argument is a constant wherever this is inlined
+__device__ __forceinline__ void set_priority(int level) {
+    if (level == 0) __builtin_amdgcn_s_setprio(0);
+    else if (level == 1) __builtin_amdgcn_s_setprio(1);
+    else if (level == 2) __builtin_amdgcn_s_setprio(2);
+    else __builtin_amdgcn_s_setprio(3);
 }
 
 // a value that is the same in every lane, kept in a scalar register so that what is decided by it is decided there
@@ -345,13 +354,12 @@ __device__ __forceinline__ void lse5_all(float (&out)[SPL], const float (&v)[SPL
         for (int i = 0; i < SPL; ++i) any |= mask[i];
         if (any != 0) {
             // the chunk's other waves wait at the barrier for this one
-            if (logtab.hurry == 3) __builtin_amdgcn_s_setprio(3);
-            else if (logtab.hurry == 1) __builtin_amdgcn_s_setprio(1);
+            if (logtab.hurry != logtab.rest) set_priority(logtab.hurry);
             if (resolve_unsettled<SPL, COMPACT>(out, sum, half, mask, v, m, logtab)) {
                 publish();
                 beside(false);
             }
-            __builtin_amdgcn_s_setprio(0);
+            if (logtab.hurry != logtab.rest) set_priority(logtab.rest);
         }
     } else {
 #pragma unroll

@@ -572,9 +572,11 @@ __global__ __launch_bounds__((2 * (S / SPL))) void fwd_post_roles_kernel(
     const int tid = threadIdx.x;
     const int posterior = __builtin_amdgcn_readfirstlane(tid / L);
     const int l = tid % L, lane = tid & 63, wave = l / 64;
-    // this kernel runs beside the beam search, whose waves run at priority 3: trips through the second
-    // tier at 1 leave that search alone (1.17 ms against 1.22 with 3 here) and cost this sweep nothing
-    const LogArgs logtab{logcells, centred, series.c, series.e, tier_lanes + (l & ~63), 1};
+    // This kernel runs beside the beam search, whose waves run at priority 3, which trips through the second tier leave
+    // alone.  The recursion, which is the chain, goes before the posterior (512 chunks of 256 states: 1.02 ms against 1.14
+    // with both at 0, search beside it 1.09 against 1.11).
+    const LogArgs logtab{logcells, centred, series.c, series.e, tier_lanes + (l & ~63), 2, 1};
+    if (!posterior) __builtin_amdgcn_s_setprio(1);
     fill_log_tables<OFK_SCAN_TWO_TIER>(logcells, centred);
     const int s0 = SPL * l, q = s0 >> 2;  // own states s0 .. s0+SPL-1, all in quad q
     const int n = blockIdx.x;            // one chunk per workgroup
