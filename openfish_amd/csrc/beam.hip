@@ -114,23 +114,23 @@ __device__ __forceinline__ float wave_max(float x) {
 // s_nop, so the two idle cycles each rotate-and-max step needs after its source was written are filled
 // with instructions that had to be issued anyway.
 //   h0 = crc2(hash, b0), h1 = crc2(hash, b0 + 1) = h0 ^ kTab1   (b0 is even)
-//   info0 = (lo4 + b0) | from, info1 = info0 | 1, infos = state | from | stay bit
-//   rests = the stay's score cs minus its guide term (the steps' scores are still on their way from LDS)
-// The lane maximum of x0, x1, x2 (one v_max3) opens the block and the read of lane 63, where the six
-// steps leave the wave's maximum, closes it.
+//   info0 = (st4 & state_mask) | b0 | from, info1 = info0 | 1, infos = state | from | stay bit
+//   cs = the stay's score after the merges, rests = cs minus its guide term (the steps' scores are still on their way from LDS)
+// The lane maximum of x0, x1 and the stay's (one v_max3) opens the block; the read of lane 63, where the six steps leave the
+// wave's maximum, wants one instruction between itself and the last of them, and the vector unit two before it uses what was read.
 struct NextRecords {
     uint32_t h0, h1, info0, info1, infos;
     float rest0, rest1, rests;
 };
-__device__ __forceinline__ float wave_max_beside_records(float x0, float x1, float x2, NextRecords &n, uint32_t hash,
-                                                         uint32_t b0, uint32_t state, uint32_t from_stay,
-                                                         uint32_t lo4b0, uint32_t from, float cs, float gs) {
+__device__ __forceinline__ float wave_max_beside_records(float x0, float x1, float stay_or_fold, NextRecords &n, float &cs, uint32_t hash,
+                                                         uint32_t b0, uint32_t state, uint32_t from_stay, uint32_t st4,
+                                                         uint32_t state_mask, uint32_t from, uint64_t step_wins, float lowest, float gs) {
     uint32_t t0, t1, best;
     float x;
     asm volatile(
         "v_max3_f32 %[x], %[x0], %[x1], %[x2]\n\t"
         "v_xor_b32 %[t0], %[hash], %[b0]\n\t"
-        "v_or_b32 %[i0], %[lo4b0], %[from]\n\t"
+        "v_and_or_b32 %[i0], %[st4], %[mask], %[b0]\n\t"
         "v_max_f32_dpp %[x], %[x], %[x] row_ror:8 row_mask:0xf bank_mask:0xf\n\t"
         "v_bfe_i32 %[t1], %[t0], 1, 1\n\t"
         "v_bfe_i32 %[t0], %[t0], 0, 1\n\t"
@@ -142,20 +142,20 @@ __device__ __forceinline__ float wave_max_beside_records(float x0, float x1, flo
         "v_lshrrev_b32 %[t1], 2, %[hash]\n\t"
         "v_max_f32_dpp %[x], %[x], %[x] row_ror:1 row_mask:0xf bank_mask:0xf\n\t"
         "v_xor_b32 %[h0], %[t0], %[t1]\n\t"
-        "v_or_b32 %[i1], 1, %[i0]\n\t"
+        "v_or_b32 %[i0], %[i0], %[from]\n\t"
         "v_max_f32_dpp %[x], %[x], %[x] row_bcast:15 row_mask:0xa bank_mask:0xf\n\t"
         "v_xor_b32 %[h1], %[tab1], %[h0]\n\t"
-        "v_or_b32 %[is], %[state], %[fromstay]\n\t"
+        "v_or_b32 %[i1], 1, %[i0]\n\t"
         "v_max_f32_dpp %[x], %[x], %[x] row_bcast:31 row_mask:0xc bank_mask:0xf\n\t"
-        "v_sub_f32 %[rs], %[cs], %[gs]\n\t"
-        "s_nop 0\n\t"
+        "v_cndmask_b32 %[cs], %[x2], %[lowest], %[wins]\n\t"
         "v_readlane_b32 %[best], %[x], 63\n\t"
-        "s_nop 0"
+        "v_or_b32 %[is], %[state], %[fromstay]\n\t"
+        "v_sub_f32 %[rs], %[cs], %[gs]"
         : [x] "=&v"(x), [best] "=&s"(best), [t0] "=&v"(t0), [t1] "=&v"(t1), [h0] "=&v"(n.h0), [h1] "=&v"(n.h1),
-          [i0] "=&v"(n.info0), [i1] "=&v"(n.info1), [is] "=&v"(n.infos), [rs] "=&v"(n.rests)
-        : [hash] "v"(hash), [b0] "v"(b0), [tab1] "s"(kTab1), [tab2] "s"(kTab2), [lo4b0] "v"(lo4b0), [from] "v"(from),
-          [state] "v"(state), [fromstay] "v"(from_stay), [x0] "v"(x0), [x1] "v"(x1), [x2] "v"(x2), [cs] "v"(cs),
-          [gs] "v"(gs));
+          [i0] "=&v"(n.info0), [i1] "=&v"(n.info1), [is] "=&v"(n.infos), [rs] "=&v"(n.rests), [cs] "=&v"(cs)
+        : [hash] "v"(hash), [b0] "v"(b0), [tab1] "s"(kTab1), [tab2] "s"(kTab2), [st4] "v"(st4), [mask] "s"(state_mask),
+          [from] "v"(from), [state] "v"(state), [fromstay] "v"(from_stay), [x0] "v"(x0), [x1] "v"(x1), [x2] "v"(stay_or_fold),
+          [wins] "s"(step_wins), [lowest] "v"(lowest), [gs] "v"(gs));
     return __uint_as_float(best);
 }
 __device__ __forceinline__ int wave_sum_i(int x) {
@@ -206,10 +206,13 @@ __device__ __forceinline__ void lds_store_f2(uint32_t at, float a, float b) {
 }
 __device__ __forceinline__ void lds_store_f(uint32_t at, float a) { *(LDS_AS float *)(uintptr_t)at = a; }
 // (x & bits) | base in one instruction
-__device__ __forceinline__ uint32_t and_or(uint32_t x, uint32_t bits, uint32_t base) {
-    uint32_t r;
-    asm("v_and_or_b32 %0, %1, %2, %3" : "=v"(r) : "v"(x), "s"(bits), "v"(base));
-    return r;
+__device__ __forceinline__ uint32_t and_or(uint32_t x, uint32_t bits, uint32_t base) { return (x & bits) | base; }
+// The LDS address of an object as a plain number that the compiler keeps in a register: where it can see the constant, it works
+// the address out again at every use and tests it for the null of a flat pointer.
+__device__ __forceinline__ uint32_t lds_address(const void *p) {
+    uint32_t at = (uint32_t)(uintptr_t)(const LDS_AS uint32_t *)p;
+    asm volatile("" : "+v"(at));
+    return at;
 }
 
 __device__ __forceinline__ void wave_fence() {
@@ -260,9 +263,9 @@ __device__ __forceinline__ float log_sum_exp(float x, float y, const double *tab
 // together 3.64; the bound used is 4.0.  (The two hardware figures are measured on the device at
 // hand, over every fp32 input of their ranges, by tests/test_gpu_hw_math.py.)  The result is settled when the distance from the
 // unrounded sum to the nearer rounding boundary of the result exceeds that bound (the residual of
-// the fused multiply-add, taken exactly with a second one).  Half an ulp is read from the exponent
-// of the next smaller float, which for a power of two is the binade below, where its nearer
-// boundary lies; results that are zero or below 2^-102 in magnitude never count as settled.
+// the fused multiply-add, taken exactly with a second one).  Half an ulp is 2^-24 of the binade of the
+// float below r in magnitude (r (1 - 2^-24), rounded: for a power of two it lies in the binade below, where its nearer
+// boundary is; every other float stays in its own); results below 2^-102 in magnitude never count as settled.
 __device__ __forceinline__ float log_sum_exp_estimate(float x, float y, bool &settled) {
     const float gap = fabsf(x - y);
     const float top = x > y ? x : y;
@@ -271,9 +274,8 @@ __device__ __forceinline__ float log_sum_exp_estimate(float x, float y, bool &se
     const float kLn2 = 0.69314718055994530942f;
     const float r = __builtin_fmaf(l2, kLn2, top);
     const float rho = __builtin_fmaf(l2, kLn2, -(r - top));
-    const uint32_t rb = __float_as_uint(r);
-    const float half_ulp = __uint_as_float(((rb & 0x7fffffffu) - ((24u << 23) + 1u)) & 0xff800000u);
-    settled = half_ulp - fabsf(rho) > 4.0f * 5.9604644775390625e-8f;
+    const float binade = __uint_as_float(__float_as_uint(r * 0x1.fffffep-1f) & 0x7f800000u);
+    settled = __builtin_fmaf(binade, 0x1p-24f, -fabsf(rho)) > 4.0f * 0x1p-24f;
     return r;
 }
 
@@ -687,8 +689,8 @@ __global__ __launch_bounds__((kBeamThreads<S, CPG, COLS, FWD>), (BeamCfg<S, FWD>
     constexpr uint32_t kBucketBits = (uint32_t)(kBuckets - 1) << 3;  // hash bits that address an 8-byte bucket
     typedef __attribute__((address_space(3))) uint32_t lds_u32;
     // LDS addresses of this chunk's index table (a multiple of its size) and of this lane's spare entry
-    const uint32_t idx_base = (uint32_t)(uintptr_t)(lds_u32 *)&all.idx[member][0].x;
-    const uint32_t idx_dump = (uint32_t)(uintptr_t)(lds_u32 *)&lds[member].idx_dump[lane].x;
+    const uint32_t idx_base = lds_address(&all.idx[member][0]);
+    const uint32_t idx_dump = lds_address(&lds[member].idx_dump[lane]);
 
     // seeding: the 32 best states of bwd[0] in ascending state order (src/beam_search.c:151-175)
     {
@@ -750,7 +752,8 @@ __global__ __launch_bounds__((kBeamThreads<S, CPG, COLS, FWD>), (BeamCfg<S, FWD>
     const uint32_t from = (uint32_t)i << 10, from_stay = from | (1u << 15);  // the element's index as "prev" of its candidates
     int rows_ready = 0;  // last value seen of the loader's counter; it is usually several rows ahead
     const int b0 = 2 * h;
-    const uint32_t cand_base = (uint32_t)(uintptr_t)(lds_u32 *)&sh.cand[0];
+    const uint32_t cand_base = lds_address(&sh.cand[0]);
+    const uint32_t elem_base = lds_address(&sh.elem[0]);
     const uint32_t cand_mine = cand_base + 8u * (uint32_t)lane;           // candidates 4i+b0, 4i+b0+1
     const uint32_t cand_dump = cand_base + 4u * (uint32_t)(4 * kW + lane);  // where a stay without a partner writes
     // What a time step reads from LDS depends only on the beam it starts from, so it is
@@ -820,13 +823,12 @@ __global__ __launch_bounds__((kBeamThreads<S, CPG, COLS, FWD>), (BeamCfg<S, FWD>
     //
     // The wave is alone on its SIMD: a step costs its instructions, about four cycles each, plus the
     // LDS round trips and the reads of comparison masks by the scalar unit (about twenty cycles) that
-    // nothing is placed into (about 1370 cycles for 1 chunk of 256 states: 0.93 ms at T = 1666; in the order of the
+    // nothing is placed into (about 1310 cycles for 1 chunk of 64 or 256 states: 0.94 ms at T = 1666; in the order of the
     // text, with every wait where its value is first needed, 1.02 ms).  Hence the order below: what does not depend on a round trip is issued
     // while it is under way, comparisons are issued in groups whose masks are read afterwards.
     auto step = [&](const int next_t, auto last_tag) {  // next_t - 1 is the time step
         constexpr bool LAST = decltype(last_tag)::value;
         const uint64_t vs = vm & 0x5555555555555555ull;  // the stay candidates sit on the even lanes
-        const int lo4 = (state << 2) & (S - 1);
         // (score + transition) + guide, the CPU path's order of additions; the fp16 transition is
         // converted inside the first addition
         float c0 = add_half(r0h, score) + g01.x;
@@ -982,10 +984,9 @@ __global__ __launch_bounds__((kBeamThreads<S, CPG, COLS, FWD>), (BeamCfg<S, FWD>
         // The best score does not wait for the step candidates to come back: a fold is not below either of
         // the two scores it joins, so the maximum of the scores before the merges and of the folds is that after them.
         const float stay_or_fold = pick_by_bit(mine_mask, folded, cs);
-        cs = pick_by_bit(step_wins, -FLT_MAX, stay_or_fold);
         NextRecords next;
-        const float best = wave_max_beside_records(c0, c1, stay_or_fold, next, hash, (uint32_t)b0, (uint32_t)state, from_stay,
-                                                   (uint32_t)(lo4 + b0), from, cs, gst);
+        const float best = wave_max_beside_records(c0, c1, stay_or_fold, next, cs, hash, (uint32_t)b0, (uint32_t)state, from_stay,
+                                                   (uint32_t)state << 2, (uint32_t)(S - 1), from, step_wins, -FLT_MAX, gst);
         c0 = c01.x;
         c1 = c01.y;
         next.rest0 = c0 - g01.x;
@@ -1004,50 +1005,72 @@ __global__ __launch_bounds__((kBeamThreads<S, CPG, COLS, FWD>), (BeamCfg<S, FWD>
             return (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32),
                                                   __builtin_amdgcn_mbcnt_lo((uint32_t)mask, (uint32_t)start));
         };
+        int steps_kept = popc64(k0) + popc64(k1);  // of `kept` those that are steps
         if (__builtin_expect(kept <= kW, 0)) {
             k0 = a0 & vm;
             k1 = a1 & vm;
             ks = as & vs;
+            steps_kept = popc64(k0) + popc64(k1);
         } else {
             // Bisection between the cut and the best score.  Every cut tried in here lies above
             // (-FLT_MAX + best) / 2, so dead lanes and dropped candidates never pass and the
             // ballots need no mask.  (lo + hi) / 2 is the CPU path's (cut + hi) / 2 or
-            // (cut + lo) / 2: one of the two bounds is the cut just tried.  Both cuts that can come next
-            // are worked out while the masks of the present one are on their way to the scalar unit.
-#pragma unroll
-            for (int guess = 2; guess < 10; ++guess) {
-                if (guess > 2) {
-                    k0 = ballot(c0 >= cut);
-                    k1 = ballot(c1 >= cut);
-                    ks = ballot(cs >= cut);
-                }
-                const float next_up = (cut + hi) / 2.0f, next_down = (lo + cut) / 2.0f;
-                kept = popc64(k0) + popc64(k1) + popc64(ks);
-                if ((unsigned)(kept - (kW * 8) / 10) <= (unsigned)(kW - (kW * 8) / 10)) goto cut_found;  // 25..32 kept
+            // (cut + lo) / 2: one of the two bounds is the cut just tried.  Two guesses in a row settle most steps; they
+            // are nested and not left by jumps, for which the compiler builds a ladder of blocks that costs as much as a guess.
+            float next_up, next_down;  // both cuts that can come next, worked out while the masks travel to the scalar unit
+            auto look_ahead = [&] {
+                next_up = (cut + hi) / 2.0f;
+                next_down = (lo + cut) / 2.0f;
+                asm volatile("" : "+v"(next_up), "+v"(next_down));
+            };
+            auto next_guess = [&] {
                 const bool up = kept > kW;
                 lo = up ? cut : lo;
                 hi = up ? hi : cut;
                 cut = up ? next_up : next_down;
-            }
-            // The tenth guess: the CPU path moves its bounds once more, tries a cut whose count it
-            // never looks at, and settles for the upper bound, whatever that keeps: of more candidates
-            // than the width the first ones, in candidate order, stay.
-            cut = hi;
-            k0 = ballot(c0 >= cut);
-            k1 = ballot(c1 >= cut);
-            ks = ballot(cs >= cut);
-            kept = popc64(k0) + popc64(k1) + popc64(ks);
-            if (kept > kW) {
-                const int rank0 = lower(k1, lower(k0, 0));
-                const int rank1 = rank0 + (int)((k0 >> lane) & 1);
-                const int ranks = lower(ks, popc64(k0) + popc64(k1));
-                k0 &= ballot(rank0 < kW);
-                k1 &= ballot(rank1 < kW);
-                ks &= ballot(ranks < kW);
-                kept = kW;
+            };
+            auto count = [&] {
+                k0 = ballot(c0 >= cut);
+                k1 = ballot(c1 >= cut);
+                ks = ballot(cs >= cut);
+                look_ahead();
+                steps_kept = popc64(k0) + popc64(k1);
+                kept = steps_kept + popc64(ks);
+            };
+            auto too_many_or_few = [&] { return (unsigned)(kept - (kW * 8) / 10) > (unsigned)(kW - (kW * 8) / 10); };  // not 25..32
+            look_ahead();
+            kept = steps_kept + popc64(ks);
+            if (too_many_or_few()) {
+                next_guess();
+                count();
+                if (too_many_or_few()) {
+                    next_guess();
+                    count();
+                    if (too_many_or_few()) {
+                        // The tenth guess: the CPU path moves its bounds once more, tries a cut whose count it
+                        // never looks at, and settles for the upper bound, whatever that keeps: of more candidates
+                        // than the width the first ones, in candidate order, stay.
+#pragma unroll 1
+                        for (int guess = 5;; ++guess) {
+                            next_guess();
+                            if (guess == 10) cut = hi;
+                            count();
+                            if (!too_many_or_few() || guess == 10) break;
+                        }
+                        if (kept > kW) {
+                            const int rank0 = lower(k1, lower(k0, 0));
+                            const int rank1 = rank0 + (int)((k0 >> lane) & 1);
+                            const int ranks = lower(ks, steps_kept);
+                            k0 &= ballot(rank0 < kW);
+                            k1 &= ballot(rank1 < kW);
+                            ks &= ballot(ranks < kW);
+                            kept = kW;
+                            steps_kept = popc64(k0) + popc64(k1);
+                        }
+                    }
+                }
             }
         }
-    cut_found:
 
         // survivors in candidate order: steps (i, b) by i then b, then stays by i
         typedef uint32_t u32x3 __attribute__((ext_vector_type(3)));
@@ -1057,7 +1080,7 @@ __global__ __launch_bounds__((kBeamThreads<S, CPG, COLS, FWD>), (BeamCfg<S, FWD>
             // lanes never pass): the masks select directly, nothing is compared again
             const int rank0 = lower(k1, lower(k0, 0));
             const int rank1 = add_bit_of(rank0, k0);
-            const int ranks = lower(ks, popc64(k0) + popc64(k1));
+            const int ranks = lower(ks, steps_kept);
             // every lane stores all three of its candidates, the ones that are dropped into its own dump
             // slot: no exec masking on the path from the cut-off to the next beam
             const int dump = kW + lane;
@@ -1070,8 +1093,7 @@ __global__ __launch_bounds__((kBeamThreads<S, CPG, COLS, FWD>), (BeamCfg<S, FWD>
                 next.rest1 = c1;
                 next.rests = cs;
             }
-            const uint32_t elem_base = (uint32_t)(uintptr_t)(lds_u32 *)&sh.elem[0].hash;
-            auto put = [&](int slot, uint32_t hsh, uint32_t inf, float rst) {
+                        auto put = [&](int slot, uint32_t hsh, uint32_t inf, float rst) {
                 uint32_t at_elem;
                 asm("v_lshl_add_u32 %0, %1, 4, %2" : "=v"(at_elem) : "v"(slot), "v"(elem_base));
                 u32x3 rec;

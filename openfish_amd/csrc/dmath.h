@@ -247,9 +247,9 @@ OFA_HD float lse5_cpu_rounding_tab(float v0, float v1, float v2, float v3, float
 // to one rounding: r~ - m is exact by Sterbenz' lemma once |m| >= 3.3, and smaller |m| are
 // never settled because half an ulp of r~ is then below eps) and h = half an ulp of r~, the
 // distance from x~ to the nearer boundary is at least h - |rho|.  A power of two has its lower
-// boundary only a quarter of its ulp away: h is read from the exponent of the next smaller
-// float, which is the binade below exactly for powers of two, so that one comparison serves
-// every case.  Values below 2^-102 (zero included) come out with h <= 0 and are never settled.
+// boundary only a quarter of its ulp away: h is taken from the binade of the next smaller
+// float, which is the one below exactly for powers of two, so that one comparison serves
+// every case.  Values below 2^-102 (zero included) have an h below eps and are never settled.
 // ---------------------------------------------------------------------------------------------
 OFA_HD float exp2_hw(float x) {
 #if defined(__HIP_DEVICE_COMPILE__)
@@ -296,13 +296,13 @@ OFA_HD Lse5Estimate lse5_verdict(Lse5Value x, float m) {
     e.value = x.value;
     e.sum = x.sum;
     const float rho = __builtin_fmaf(x.l2, kLn2, -(x.value - m));
-    const uint32_t rb = bits_of(x.value);
-    // exponent field of the float below |r~|, lowered by 24; where that wraps, the sign bit survives the mask
-    e.half = float_of(((rb & 0x7fffffffu) - ((24u << 23) + 1u)) & 0xff800000u);
+    // 2^24 h: the binade of the float below |r~|, which |r~| (1 - 2^-24) is for a power of two; every other float stays in its own
+    const float binade = float_of(bits_of(x.value * 0x1.fffffep-1f) & 0x7f800000u);
+    e.half = binade * 0x1p-24f;
     const uint32_t sb = bits_of(x.sum) + 16u;
     const float mu = float_of((sb & 0x007fffffu) | 0x3f000000u);
     const float eps = __builtin_fmaf(mu, -kEpsMu, __builtin_fmaf(float_of(sb & 0x7f800000u), kEps1, kEps0));
-    e.settled = e.half - __builtin_fabsf(rho) > eps;
+    e.settled = __builtin_fmaf(binade, 0x1p-24f, -__builtin_fabsf(rho)) > eps;
     return e;
 }
 OFA_HD Lse5Estimate lse5_estimate(float v0, float v1, float v2, float v3, float v4, float m) {
