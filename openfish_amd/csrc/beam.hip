@@ -362,7 +362,8 @@ struct __attribute__((aligned(16))) BeamRing {
 // live elements two of them share a bucket in about w^2 / (2 * buckets) of the time steps.
 template <int S, int CPG, int FWD>
 struct BeamIdx {
-    static constexpr int kBuckets = (S >= 1024 || CPG > 2 || BeamCfg<S, FWD>::kDense) ? 2048 : 4096;
+    static constexpr bool kLone = CPG == 1 && FWD == 0;  // a compute unit's LDS for one chunk
+    static constexpr int kBuckets = kLone ? (S >= 1024 ? 8192 : 16384) : (S >= 1024 || CPG > 2 || BeamCfg<S, FWD>::kDense) ? 2048 : 4096;
 };
 // What the forward recursion and the posterior of a chunk share.
 constexpr int kVecRows = 4;  // two would do (see beam_kernel); four let the posterior lag (1024 chunks of 256 states: 2.66 ms against 2.78)
@@ -463,7 +464,7 @@ struct LdsRow {
 // states two workgroups share a unit (80 KB of LDS, 96 registers per lane): two states per lane and smaller
 // rings.  1024 states: two per lane, one chunk per workgroup (four per lane: 2.15 ms against 1.74 at 256 chunks).
 template <int S, int CPG, int COLS, int FWD>
-constexpr int kBeamThreads = 64 * CPG * (FWD == 0 ? 2 : FWD + 3);
+constexpr int kBeamThreads = BeamIdx<S, CPG, FWD>::kLone ? 256 : 64 * CPG * (FWD == 0 ? 2 : FWD + 3);  // a lone chunk: two waves more for the set-up
 template <int S, int CPG, int COLS, int FWD>
 __global__ __launch_bounds__((kBeamThreads<S, CPG, COLS, FWD>), (BeamCfg<S, FWD>::kDense ? 5 : 1)) void beam_kernel(const _Float16 *__restrict__ scores,
                                                    const float *__restrict__ bwd, float *__restrict__ post,
@@ -513,9 +514,11 @@ __global__ __launch_bounds__((kBeamThreads<S, CPG, COLS, FWD>), (BeamCfg<S, FWD>
     }
     for (int x = (int)threadIdx.x; x < OFK_LSE_DOUBLES; x += kBeamThreads<S, CPG, COLS, FWD>) lse[x] = lse_table[x];
     // the hash index starts empty: no entry may look like one of a real generation (tags start at 1 << 5)
-    for (int x = (int)threadIdx.x; x < kGroupChunks * BeamIdx<S, CPG, FWD>::kBuckets; x += kBeamThreads<S, CPG, COLS, FWD>) (&all.idx[0][0])[x] = make_uint2(0u, 0u);
+    for (int x = (int)threadIdx.x; x < kGroupChunks * BeamIdx<S, CPG, FWD>::kBuckets / 2; x += kBeamThreads<S, CPG, COLS, FWD>)
+        reinterpret_cast<uint4 *>(&all.idx[0][0])[x] = make_uint4(0u, 0u, 0u, 0u);
     __syncthreads();
     if (n >= N) return;  // odd batch: the last group has one chunk
+    if (BeamIdx<S, CPG, FWD>::kLone && wave > kFirstLoader) return;
 
     static_assert((FWD & (FWD - 1)) == 0 && FWD <= 64, "a lane reads one wave's counter");
     if constexpr (FWD > 0) {
@@ -1260,7 +1263,18 @@ int launch_beam(const void *scores, const float *bwd, ofk_beam_slot_t *beam, int
                 uint8_t *moves, int T, int N, float log_cut, float stay, int flags, const double *lse_table,
                 hipStream_t st) {
     // 256 compute units: up to 512 chunks fit two to a unit; larger batches go four to a group
-    // where the LDS of four chunks fits (64 and 256 states)
+    // where the LDS of four chunks fits (64 and 256 states).  Few chunks have a unit each: two searches on one wait for each
+    // other's LDS operations, and with the LDS to itself a chunk has an index so large that one step in forty instead of
+    // one in ten meets two elements in a bucket.  Search, two to a unit | one, T = 1666 (1024 states 833), ms: 64 states, 1 chunk
+    // 0.943 | 0.929, 16 1.033 | 0.936, 200 1.051 | 0.974; 256 states, 16 1.024 | 0.941, 200 1.042 | 1.002; 1024 states, 37
+    // 0.565 | 0.490, 100 0.577 | 0.504, 160 (split: units are short) 0.74 | 1.0.  Such a group leaves no room for a second on its unit, hence
+    // the smaller bound where other decodes may be under way: three of them (a lane each) find units for all their chunks.
+    const int units = (flags & OFK_SEARCH_ALONE) ? 256 : 64;
+    if (N <= (S >= 1024 ? units / 2 : units)) {
+        hipLaunchKernelGGL((beam_kernel<S, 1, COLS, 0>), dim3(N), dim3(kBeamThreads<S, 1, COLS, 0>), 0, st, static_cast<const _Float16 *>(scores), bwd,
+                           nullptr, beam, states, moves, T, N, log_cut, stay, flags, lse_table, LogSeries{});
+        return (int)hipGetLastError();
+    }
     if constexpr (S <= 256) {
         if (N > OFK_SPARSE_SEARCH_MAX_CHUNKS) {
             hipLaunchKernelGGL((beam_kernel<S, 4, COLS, 0>), dim3((N + 3) / 4), dim3(512), 0, st,
@@ -1270,8 +1284,8 @@ int launch_beam(const void *scores, const float *bwd, ofk_beam_slot_t *beam, int
         }
     }
     hipLaunchKernelGGL((beam_kernel<S, 2, COLS, 0>), dim3((N + 1) / 2), dim3(256), 0, st,
-                           static_cast<const _Float16 *>(scores), bwd, nullptr, beam, states, moves, T, N, log_cut, stay,
-                           flags, lse_table, LogSeries{});
+                       static_cast<const _Float16 *>(scores), bwd, nullptr, beam, states, moves, T, N, log_cut, stay,
+                       flags, lse_table, LogSeries{});
     return (int)hipGetLastError();
 }
 

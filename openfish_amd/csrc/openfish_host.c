@@ -558,6 +558,7 @@ static void enqueue_decode(ofa_gpubuf_t *g, const int T, const int N, const int 
 
     const int cols = columns_of(C, state_len);
     const int others = take_main_lane(g), shared = others || enqueued;
+    const int search_flags = g->debug_flags | (shared ? 0 : OFK_SEARCH_ALONE);
     g->pend_split = arrangement_of(g, T, N, C, state_len, shared);
     /* Sums only where the search leaves the machine idle, and not with 1024 states, whose search waits for
      * memory and was measured to take half as long again beside the extra kernel.
@@ -592,7 +593,7 @@ static void enqueue_decode(ofa_gpubuf_t *g, const int T, const int N, const int 
         HIP_OK(hipEventRecord(g->ev[EV_BEAM_START], g->s_main));
         launch_ok(ofk_beam_search(scores_TNC, g->pub.bwd_NTC, (ofk_beam_slot_t *)g->pub.beam_vector,
                                   (int32_t *)g->pub.states, g->pub.moves, T, N, state_len, cols, log_beam_cut(options),
-                                  stay, g->lse_table, g->debug_flags, g->s_main), "beam_search");
+                                  stay, g->lse_table, search_flags, g->s_main), "beam_search");
         HIP_OK(hipEventRecord(g->ev[EV_BEAM_END], g->s_main));
         /* The search keeps one wave per chunk busy and leaves the rest of the machine idle: beside
          * it, on the second stream, the posteriors that a block's quality is made of are summed for
@@ -614,7 +615,7 @@ static void enqueue_decode(ofa_gpubuf_t *g, const int T, const int N, const int 
         HIP_OK(hipEventRecord(g->ev[EV_BEAM_START], g->s_main));
         launch_ok(ofk_beam_search(scores_TNC, g->pub.bwd_NTC, (ofk_beam_slot_t *)g->pub.beam_vector,
                                   (int32_t *)g->pub.states, g->pub.moves, T, N, state_len, cols, log_beam_cut(options),
-                                  stay, g->lse_table, g->debug_flags, g->s_main), "beam_search");
+                                  stay, g->lse_table, search_flags, g->s_main), "beam_search");
         HIP_OK(hipEventRecord(g->ev[EV_BEAM_END], g->s_main));
 
         HIP_OK(hipStreamWaitEvent(g->s_side, g->ev[EV_BWD_END], 0));
