@@ -38,6 +38,10 @@ int ofk_bwd_scan(const void *scores, float *bwd, int T, int N, int state_len, in
                  int spl, void *stream);
 int ofk_fwd_post_scan(const void *scores, const float *bwd, float *post, int T, int N, int state_len,
                       int columns, float stay, int mode, int spl, void *stream);
+/* The same in two steps, 1024 states and the two-tier arithmetic only: the forward recursion by itself, which needs no bwd and can
+ * run beside the backward sweep, and then the posteriors of its rows, in place. */
+int ofk_fwd_scan(const void *scores, float *fwd, int T, int N, int state_len, int columns, float stay, void *stream);
+int ofk_posterior_rows(const float *bwd, float *post, int T, int N, int state_len, void *stream);
 /* Both sweeps and the posterior in one kernel: the forward and backward recursions of a chunk run
  * side by side in one workgroup and meet in the middle of the chunk (same tensors as
  * ofk_bwd_scan followed by ofk_fwd_post_scan).  Rows 0 .. T/2-1 of post hold forward values

@@ -504,8 +504,10 @@ static void join_null_stream(ofa_gpubuf_t *g) {
  *     64 states: 16 1.83 | 1.58;  512 2.03 | 1.76;  2048 4.37 | 3.61
  * Hence the lines: up to 160 chunks of 1024 states the search (two chunks to a unit) and the forward sweep (one) find
  * compute units of their own; above 256 merged takes a second round of workgroups, split does so only above 320; chunks
- * shorter than 128 steps are decided by launches and set-up (from 16 to 256 of them no arrangement is ahead by more than
- * 0.03 ms, and they take that of longer ones).  Up to 512 chunks of 256 states the chain of split is
+ * shorter than 128 steps are decided by launches and set-up (up to 256 of them no arrangement was ahead by more than
+ * 0.03 ms, and they take that of longer ones).  The figures are from before up to 96 chunks of 1024 states had their sweeps apart,
+ * see enqueue_decode, which only split gains from (8 chunks, T = 100 0.345 | 0.264); up to 64 steps fewer than 16 of them keep the
+ * one kernel because that choice is part of what is tested (1 chunk, T = 33 0.20 | 0.16).  Up to 512 chunks of 256 states the chain of split is
  * shorter, while its bytes fit beneath the chain, 3.8 MB a step; above, the search's workgroups hold four chunks, a unit
  * that has one of them in the merged kernel takes 2.5 ms whatever the others do, and split has units left for the
  * forward sweep up to three chunks to a unit.
@@ -529,7 +531,7 @@ static int arrangement_by_default(int T, int N, int C, int state_len, int shared
             return N <= (shared ? 640 : 768) ? ARR_SPLIT : ARR_MERGED;
         default:
             if (!can_merge) return ARR_ONE;
-            if (T < 128 && (N < 16 || (N > 320 && !shared))) return ARR_ONE;
+            if (T < 128 && ((N < 16 && (shared || T <= 64)) || (N > 320 && !shared))) return ARR_ONE;
             if (shared) return ARR_MERGED;
             return N <= 160 || (N > 256 && N <= 320) ? ARR_SPLIT : ARR_MERGED;
     }
@@ -605,9 +607,20 @@ static void enqueue_decode(ofa_gpubuf_t *g, const int T, const int N, const int 
             HIP_OK(hipEventRecord(g->ev[EV_SUMS_END], g->s_side));
         }
     } else {
+        /* A sweep of 1024 states has a compute unit to a chunk.  A batch that leaves half of the units idle, and shares them
+         * with no other decode, has the forward sweep on units of its own beside the backward one; only the posterior is then
+         * left to do beside the search.  It moves 8 more bytes per state and step, which is why it ends short of 128 chunks.
+         * Whole calls, ms, sweep and posterior beside the search | apart: 1 chunk, T = 33 0.171 | 0.160; 8, T = 100 0.317 | 0.264;
+         * T = 833: 1 1.48 | 1.23, 37 1.51 | 1.27, 64 1.52 | 1.31, 96 1.53 | 1.33; five columns, T = 1666: 80 2.67 | 2.51,
+         * 96 2.68 | 2.57, 112 2.72 | 2.73, 128 2.82 | 2.85. */
+        const int apart = state_len == 5 && N <= 96 && !shared && g->scan_mode == OFK_SCAN_TWO_TIER && g->scan_spl == 0;
         launch_ok(ofk_bwd_scan(scores_TNC, g->pub.bwd_NTC, T, N, state_len, cols, stay, g->scan_mode, g->scan_spl, g->s_main),
                   "bwd_scan");
         HIP_OK(hipEventRecord(g->ev[EV_BWD_END], g->s_main));
+        if (apart) {
+            HIP_OK(hipStreamWaitEvent(g->s_side, g->ev[EV_START], 0));
+            launch_ok(ofk_fwd_scan(scores_TNC, g->pub.post_NTC, T, N, state_len, cols, stay, g->s_side), "fwd_scan");
+        }
 
         /* The beam search is the longer of the two stages that follow and wants its workgroups (large
          * LDS blocks) resident before the forward sweep fills the compute units: it stays on the stream
@@ -619,8 +632,11 @@ static void enqueue_decode(ofa_gpubuf_t *g, const int T, const int N, const int 
         HIP_OK(hipEventRecord(g->ev[EV_BEAM_END], g->s_main));
 
         HIP_OK(hipStreamWaitEvent(g->s_side, g->ev[EV_BWD_END], 0));
-        launch_ok(ofk_fwd_post_scan(scores_TNC, g->pub.bwd_NTC, g->pub.post_NTC, T, N, state_len, cols, stay, g->scan_mode,
-                                    g->scan_spl, g->s_side), "fwd_post_scan");
+        if (apart)
+            launch_ok(ofk_posterior_rows(g->pub.bwd_NTC, g->pub.post_NTC, T, N, state_len, g->s_side), "posterior_rows");
+        else
+            launch_ok(ofk_fwd_post_scan(scores_TNC, g->pub.bwd_NTC, g->pub.post_NTC, T, N, state_len, cols, stay, g->scan_mode,
+                                        g->scan_spl, g->s_side), "fwd_post_scan");
         HIP_OK(hipEventRecord(g->ev[EV_FWD_END], g->s_side));
         if (use_sums) {
             HIP_OK(hipEventRecord(g->ev[EV_SUMS_START], g->s_side));

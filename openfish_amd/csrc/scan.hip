@@ -680,6 +680,106 @@ __global__ __launch_bounds__((2 * (S / SPL))) void fwd_post_roles_kernel(
 }
 
 // ---------------------------------------------------------------------------
+// The forward recursion by itself, rows left in post[t], and the posterior of rows whose recursion is done: for
+// batches of 1024 states that leave compute units idle.  A chunk's sweep is bound by what its one unit can issue, and nothing
+// in the recursion waits for the backward one: on units of their own the two run at the same time, and what is left to do
+// beside the search is a pass over rows that depends on no other row.  37 chunks, T = 833, ms: backward 0.67, then forward
+// sweep with posterior 0.74 beside a search of 0.49 | both sweeps 0.68, then posteriors 0.14 beside a search of 0.49.
+// ---------------------------------------------------------------------------
+template <int S, int DEPTH>
+__global__ __launch_bounds__(S) void fwd_scan_kernel(const _Float16 *__restrict__ scores, float *__restrict__ fwd, int T, int N,
+                                                     float stay, LogSeries series) {
+    constexpr int Q = S / 4;
+    static_assert(S > 64, "a state to a lane, and several waves");
+    __shared__ __attribute__((aligned(16))) float vec[2][S];
+    __shared__ __attribute__((aligned(16))) ofa::LogCell logcells[32], centred[ofa::kLogCentredCells];
+    __shared__ __attribute__((aligned(16))) float tier_lanes[S];
+    const int s = threadIdx.x, q = s >> 2;
+    const LogArgs logtab{logcells, centred, series.c, series.e, tier_lanes + (s & ~63)};
+    fill_log_tables<OFK_SCAN_TWO_TIER>(logcells, centred);
+    const ptrdiff_t row_stride = (ptrdiff_t)N * kCols * S;
+    const _Float16 *pre = scores + (size_t)blockIdx.x * kCols * S;
+    float *frow = fwd + (size_t)blockIdx.x * (size_t)(T + 1) * S;
+    const unsigned sc_lane = kCols * s + kLead;
+    FwdRow<1> ring[DEPTH];
+    static_for<DEPTH>([&](auto k) {  // without a condition, as in bwd_scan_kernel
+        ring[k].load(pre + sc_lane);
+        pre += (int)k < T - 1 ? row_stride : 0;
+    });
+    float f[1] = {0.f};
+    int buf = 0;
+    vec[0][s] = 0.f;
+    frow[s] = 0.f;
+    __syncthreads();  // the log table
+    pipelined<DEPTH>(T, [&](auto k, int j, auto checked) {
+        chunk_sync<true>();
+        const float p0 = vec[buf][q], p1 = vec[buf][q + Q], p2 = vec[buf][q + 2 * Q], p3 = vec[buf][q + 3 * Q];
+        const FwdRow<1> row = ring[k];
+        __builtin_amdgcn_sched_barrier(0);
+        if (!checked || j + DEPTH < T) {
+            ring[k].load(pre + sc_lane);
+            pre += row_stride;
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        float v[1][5];
+        fwd_terms(v, f, p0, p1, p2, p3, row, stay);
+        buf ^= 1;
+        frow += S;
+        lse5_all<1, OFK_SCAN_TWO_TIER>(f, v, logtab, [&] { vec[buf][s] = f[0]; }, [&](bool) { frow[s] = f[0]; });
+    });
+}
+
+// post[n][t] holds fwd[t] and gets softmax(fwd[t] + bwd[n][t]): a wave takes a row, `parts` workgroups a chunk.  Sums in the order
+// of fwd_post_roles_kernel with two states to a lane (pieces of 128 states, their totals one after another): the same bits.
+template <int S>
+__global__ __launch_bounds__(256) void posterior_rows_kernel(const float *__restrict__ bwd, float *__restrict__ post, int T, int parts) {
+    constexpr int P = S / 128;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int n = blockIdx.x / parts, part = blockIdx.x % parts;
+    const size_t first = (size_t)n * (size_t)(T + 1) * S + 2 * lane;
+    const float *b0 = bwd + first;
+    float *p0 = post + first;
+    auto load = [&](const float *row, float2 (&x)[P]) {
+#pragma unroll
+        for (int k = 0; k < P; ++k) x[k] = *reinterpret_cast<const float2 *>(row + 128 * k);
+    };
+    float2 b[P], f[P], b_next[P], f_next[P];
+    load(b0, b);  // the shift of the exponent, as in fwd_post_kernel: max_s bwd[0][s] - 10
+    float top = fmaxf(b[0].x, b[0].y);
+#pragma unroll
+    for (int k = 1; k < P; ++k) top = fmaxf(top, fmaxf(b[k].x, b[k].y));
+    const float shift = group_max<64>(top) - 10.0f;
+    const int step = 4 * parts;
+    int t = 4 * part + wave;
+    if (t > T) return;
+    load(b0 + (size_t)t * S, b_next);
+    load(p0 + (size_t)t * S, f_next);
+    for (; t <= T; t += step) {
+#pragma unroll
+        for (int k = 0; k < P; ++k) {
+            b[k] = b_next[k];
+            f[k] = f_next[k];
+        }
+        if (t + step <= T) {
+            load(b0 + (size_t)(t + step) * S, b_next);
+            load(p0 + (size_t)(t + step) * S, f_next);
+        }
+        float total = 0.f;
+#pragma unroll
+        for (int k = 0; k < P; ++k) {
+            f[k].x = __builtin_amdgcn_exp2f(((f[k].x + b[k].x) - shift) * kLog2e);
+            f[k].y = __builtin_amdgcn_exp2f(((f[k].y + b[k].y) - shift) * kLog2e);
+            const float piece = group_sum<64>(f[k].x + f[k].y);
+            total = k == 0 ? piece : total + piece;
+        }
+        const float inv = __builtin_amdgcn_rcpf(total);
+#pragma unroll
+        for (int k = 0; k < P; ++k)
+            *reinterpret_cast<float2 *>(p0 + (size_t)t * S + 128 * k) = make_float2(f[k].x * inv, f[k].y * inv);
+    }
+}
+
+// ---------------------------------------------------------------------------
 // Both sweeps in one kernel, meeting in the middle.
 //
 // The forward recursion does not depend on the backward one; only the posterior needs
@@ -1237,6 +1337,13 @@ static int fwd_post_scan(const void *scores, const float *bwd, float *post, int 
     OFK_DISPATCH(false, launch_fwd, mode, scores, bwd, post, T, N, stay, st)
 }
 
+static int fwd_scan(const void *scores, float *fwd, int T, int N, int state_len, float stay, void *stream) {
+    if (!scores || !fwd || T < 1 || N < 1 || state_len != 5 || !aligned16(scores) || !aligned16(fwd)) return OFK_BAD_ARGS;
+    hipLaunchKernelGGL((fwd_scan_kernel<1024, OFK_DEPTH_1024>), dim3(N), dim3(1024), 0, static_cast<hipStream_t>(stream),
+                       static_cast<const _Float16 *>(scores), fwd, T, N, stay, kSeries);
+    return (int)hipGetLastError();
+}
+
 // The build compiles this file twice: with four columns, which also holds the entry points, and
 // with five, whose kernels the entry points reach through the three functions named *_five.
 #if OFK_COLS == 5
@@ -1252,10 +1359,14 @@ extern "C" int ofk_fwd_post_scan_five(const void *scores, const float *bwd, floa
                                       int state_len, float stay, int mode, int spl, void *stream) {
     return fwd_post_scan(scores, bwd, post, T, N, state_len, stay, mode, spl, stream);
 }
+extern "C" int ofk_fwd_scan_five(const void *scores, float *fwd, int T, int N, int state_len, float stay, void *stream) {
+    return fwd_scan(scores, fwd, T, N, state_len, stay, stream);
+}
 #else
 extern "C" int ofk_scan_posterior_five(const void *, float *, float *, int, int, int, float, int, int, void *);
 extern "C" int ofk_bwd_scan_five(const void *, float *, int, int, int, float, int, int, void *);
 extern "C" int ofk_fwd_post_scan_five(const void *, const float *, float *, int, int, int, float, int, int, void *);
+extern "C" int ofk_fwd_scan_five(const void *, float *, int, int, int, float, void *);
 
 extern "C" int ofk_scan_posterior(const void *scores, float *bwd, float *post, int T, int N, int state_len,
                                   int columns, float stay, int mode, int spl, void *stream) {
@@ -1276,5 +1387,22 @@ extern "C" int ofk_fwd_post_scan(const void *scores, const float *bwd, float *po
     if (columns == 5) return ofk_fwd_post_scan_five(scores, bwd, post, T, N, state_len, stay, mode, spl, stream);
     if (columns != 4) return OFK_BAD_ARGS;
     return fwd_post_scan(scores, bwd, post, T, N, state_len, stay, mode, spl, stream);
+}
+
+extern "C" int ofk_fwd_scan(const void *scores, float *fwd, int T, int N, int state_len, int columns, float stay, void *stream) {
+    if (columns == 5) return ofk_fwd_scan_five(scores, fwd, T, N, state_len, stay, stream);
+    if (columns != 4) return OFK_BAD_ARGS;
+    return fwd_scan(scores, fwd, T, N, state_len, stay, stream);
+}
+
+extern "C" int ofk_posterior_rows(const float *bwd, float *post, int T, int N, int state_len, void *stream) {
+    if (!bwd || !post || T < 1 || N < 1 || state_len != 5 || !aligned16(bwd) || !aligned16(post)) return OFK_BAD_ARGS;
+    // Four rows to a workgroup, and few workgroups: the search beside this is longer, and more rows in flight only slow it down
+    // (128 | 256 | 1024 workgroups, whole call, ms: 37 chunks, T = 833 1.27 | 1.27 | 1.29; 80, T = 1666 2.43 | 2.47 | 2.56).
+    int parts = 128 / N;
+    parts = parts < 1 ? 1 : parts;
+    parts = parts < (T + 4) / 4 ? parts : (T + 4) / 4;
+    hipLaunchKernelGGL((posterior_rows_kernel<1024>), dim3(N * parts), dim3(256), 0, static_cast<hipStream_t>(stream), bwd, post, T, parts);
+    return (int)hipGetLastError();
 }
 #endif
