@@ -2,10 +2,11 @@
 //
 // Follows the CPU path (reference src/beam_search.c:441-496 for the quality of a
 // block, src/beam_search.c:49-99 and src/decode_cpu.c:218-225 for the sequence):
-//   1. every time step in parallel: posterior of the path k-mer plus its distinct
+//   1. and 2. a running sum of the moves gives every time step its base position, and the
+//      bases of the sequence;
+//   3. every time step in parallel: posterior of the path k-mer plus its distinct
 //      one-base shifts (fp32 sums in the CPU path's order), clamped, to the power 0.4;
-//   2. a block-wide prefix sum of the moves gives every time step its base position;
-//   3. every base in parallel: the fp32 sums over its dwell are taken in time order,
+//   4. every base in parallel: the fp32 sums over its dwell are taken in time order,
 //      exactly as the serial loop takes them, then the phred character follows.
 // pow is evaluated in double and rounded once to fp32.  The phred character is a
 // step function of the miss probability 1 - base/total; its 49 thresholds are
@@ -17,102 +18,161 @@
 
 namespace {
 
-constexpr int kThreads = 256;
+// The characters of a chunk lie at any address; their copy in LDS lies at the same distance from a multiple of 16, so that whole
+// 16-byte pieces move by one store a lane.  Bytes [lo, hi) of the chunk, by the lanes of `lanes` (lane 0 .. lanes - 1).
+__device__ __forceinline__ void copy_out(unsigned char *dst, const unsigned char *lds, int lo, int hi, int lane, int lanes) {
+    const int skew = (int)(reinterpret_cast<uintptr_t>(dst) & 15u);
+    const int first = (lo + skew + 15) & ~15, last = (hi + skew) & ~15;  // whole pieces, counted from dst - skew
+    unsigned char *d = dst - skew;
+    const unsigned char *l = lds - skew;
+    for (int i = first + 16 * lane; i < last; i += 16 * lanes)
+        *reinterpret_cast<uint4 *>(d + i) = *reinterpret_cast<const uint4 *>(l + i);
+    const int head_end = first < hi + skew ? first : hi + skew;
+    const int tail = last > head_end ? last : head_end;
+    for (int i = lo + skew + lane; i < head_end; i += lanes) d[i] = l[i];
+    for (int i = tail + lane; i < hi + skew; i += lanes) d[i] = l[i];
+}
 
-template <int S>
+// LDS of a chunk: two 4-byte tables, a 2-byte one and three of bytes with room for their skews.
+constexpr size_t sequence_lds(int T) {
+    const size_t t16 = ((size_t)T + 15) & ~(size_t)15;
+    return 4 * t16 + 4 * (t16 + 16) + 2 * t16 + 3 * (t16 + 16);
+}
+
+// What bounds it: up to a chunk per compute unit the waits of its few dependent rounds of memory accesses, above that the sectors
+// that the posteriors are gathered from (0.69 GB with 512 chunks of 256 states, 0.13 ms at 5.3 TB/s).  All that does not need
+// the posteriors comes first: base positions, the characters of the sequence and the zeros behind both strings, which one wave
+// then writes to their place (host memory, in a decode) while the others gather.  What is left after the gathers is a base's
+// character.  Inside decodes, ms, against gathers first, bytes last and one at a time, 256 lanes: 1 chunk of 64 states 0.021 ->
+// 0.014; 512 of 256 states 0.167 -> 0.130, 1024 of them 0.328 -> 0.263; 256 of 1024 0.103 -> 0.084.
+template <int S, int kThreads>
 __global__ __launch_bounds__(kThreads) void sequence_kernel(
     const float *__restrict__ post, int32_t *__restrict__ states, const uint8_t *__restrict__ moves,
     float *__restrict__ qual_data, float *__restrict__ base_probs, float *__restrict__ total_probs,
     char *__restrict__ sequence, char *__restrict__ qstring, int T, ofk_phred_table_t phred,
     const float *__restrict__ path_sums, uint8_t *__restrict__ moves_out) {
+    constexpr int kWaves = kThreads / 64;
+    constexpr int kGather = kThreads - 64;  // the last wave writes the finished bytes
+    static_assert(OFK_MAX_T <= 128 * 64, "two counts of moves to a lane");
     extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
-    float *s_prob = reinterpret_cast<float *>(lds);        // [T] called-base probability
-    float *s_wrong = s_prob + T;                           // [T] probability of each other base
-    int *s_start = reinterpret_cast<int *>(s_wrong + T);   // [T+1] first time step of base p
-    unsigned char *s_base = reinterpret_cast<unsigned char *>(s_start + T + 1);  // [T]
-    unsigned char *s_move = s_base + T;                    // [T]
-    __shared__ int s_scan[kThreads];
-
+    __shared__ int s_count[128];  // moves of every 64 time steps
+    const int t16 = (T + 15) & ~15;
     const int n = blockIdx.x;
-    const int tid = threadIdx.x;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const size_t first = (size_t)n * T;
+    unsigned char *out_seq = reinterpret_cast<unsigned char *>(sequence) + first;
+    unsigned char *out_qual = reinterpret_cast<unsigned char *>(qstring) + first;
+    unsigned char *out_moves = moves_out + first;
+    float *s_prob = reinterpret_cast<float *>(lds);                        // [T] called-base probability
+    int *s_start = reinterpret_cast<int *>(s_prob + t16);                  // [T+1] first time step of base p
+    uint16_t *s_state = reinterpret_cast<uint16_t *>(s_start + t16 + 16);  // [T]
+    unsigned char *bytes = reinterpret_cast<unsigned char *>(s_state + t16);
+    unsigned char *s_seq = bytes + (reinterpret_cast<uintptr_t>(out_seq) & 15u);                    // [T]
+    unsigned char *s_qual = bytes + t16 + 16 + (reinterpret_cast<uintptr_t>(out_qual) & 15u);       // [T]
+    unsigned char *s_move = bytes + 2 * (t16 + 16) + (reinterpret_cast<uintptr_t>(out_moves) & 15u);  // [T]
+
     const float *post_n = post + (size_t)n * (size_t)(T + 1) * S;
-    int32_t *st_n = states + (size_t)n * T;
-    const uint8_t *mv_n = moves + (size_t)n * T;
+    int32_t *st_n = states + first;
+    const uint8_t *mv_n = moves + first;
 
-    // 1. quality of every block
-    for (int t = tid; t < T; t += kThreads) {
-        const int st = st_n[t];
-        const int base = st & 3;
-        st_n[t] = base;
-        float prob;
-        if (path_sums) {  // the sum below, taken for every state by path_sums_kernel: one read instead of nine
-            prob = path_sums[((size_t)n * T + t) * S + st];
-        } else {
-            const float *p = post_n + (size_t)(t + 1) * S;
-            prob = p[st];
-            int nb[8];
-#pragma unroll
-            for (int b = 0; b < 4; ++b) {
-                nb[2 * b] = (st >> 2) + (S / 4) * b;
-                nb[2 * b + 1] = ((st << 2) & (S - 1)) + b;
-            }
-#pragma unroll
-            for (int k = 0; k < 8; ++k) {
-                bool fresh = nb[k] != st;
-#pragma unroll
-                for (int m = 0; m < k; ++m) fresh = fresh && nb[m] != nb[k];
-                if (fresh) prob += p[nb[k]];
-            }
+    // 1. moves of every 64 time steps
+    const int pieces = (T + 63) / 64;
+    for (int e = wave; e < pieces; e += kWaves) {
+        const int t = 64 * e + lane;
+        uint8_t move = 0;
+        if (t < T) {
+            const int st = st_n[t];
+            move = mv_n[t];
+            s_state[t] = (uint16_t)st;
+            s_move[t] = move;
+            st_n[t] = st & 3;
         }
-        if (prob > 1.0f) prob = 1.0f;
-        else if (prob < 0.0f) prob = 0.0f;
-        prob = (float)pow((double)prob, (double)0.4f);
-        const float wrong = (1.0f - prob) / 3.0f;
-        s_prob[t] = prob;
-        s_wrong[t] = wrong;
-        s_base[t] = (unsigned char)base;
-        const uint8_t move = mv_n[t];
-        s_move[t] = move;
-        if (moves_out) moves_out[(size_t)n * T + t] = move;
-        float4 q;
-        q.x = base == 0 ? prob : wrong;
-        q.y = base == 1 ? prob : wrong;
-        q.z = base == 2 ? prob : wrong;
-        q.w = base == 3 ? prob : wrong;
-        reinterpret_cast<float4 *>(qual_data)[(size_t)n * T + t] = q;
+        const uint64_t mask = __ballot(move != 0);
+        if (lane == 0) s_count[e] = __popcll(mask);
     }
     __syncthreads();
 
-    // 2. base position of every time step: inclusive prefix sum of the moves, minus one
-    const int seg = (T + kThreads - 1) / kThreads;
-    const int t_lo = tid * seg < T ? tid * seg : T;
-    const int t_hi = t_lo + seg < T ? t_lo + seg : T;
-    int mine = 0;
-    for (int t = t_lo; t < t_hi; ++t) mine += s_move[t];
-    s_scan[tid] = mine;
-    __syncthreads();
-    for (int d = 1; d < kThreads; d <<= 1) {
-        const int add = tid >= d ? s_scan[tid - d] : 0;
-        __syncthreads();
-        s_scan[tid] += add;
-        __syncthreads();
+    // 2. base position of every time step, and what follows from the path alone.  Every wave takes the running sum of
+    // the counts by itself: lane i those of pieces i and 64 + i.
+    int low = lane < pieces ? s_count[lane] : 0, high = 64 + lane < pieces ? s_count[64 + lane] : 0;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+        const int l = __shfl_up(low, d), h = __shfl_up(high, d);
+        low += lane >= d ? l : 0;
+        high += lane >= d ? h : 0;
     }
-    const int seq_len = s_scan[kThreads - 1];
-    {
-        int pos = s_scan[tid] - mine;  // bases emitted before this segment
-        for (int t = t_lo; t < t_hi; ++t) {
-            if (s_move[t]) s_start[pos++] = t;
+    high += __builtin_amdgcn_readlane(low, 63);
+    const int seq_len = __builtin_amdgcn_readlane(high, 63);
+    for (int e = wave; e < pieces; e += kWaves) {
+        const int t = 64 * e + lane;
+        const bool begins = t < T && s_move[t] != 0;
+        const uint64_t mask = __ballot(begins);
+        const int before = e == 0 ? 0 : e <= 64 ? __builtin_amdgcn_readlane(low, e - 1) : __builtin_amdgcn_readlane(high, e - 65);
+        if (begins) {
+            const int pos = before + (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mask, 0u));
+            s_start[pos] = t;
+            s_seq[pos] = "ACGT"[s_state[t] & 3];
         }
-        if (tid == 0) s_start[seq_len] = T;
+        if (t < T && t >= seq_len) {
+            s_seq[t] = 0;
+            s_qual[t] = 0;
+        }
+    }
+    if (tid == 0) s_start[seq_len] = T;
+    __syncthreads();
+
+    // 3. one wave writes what is known, the others take the quality of every block
+    if (wave == kWaves - 1) {
+        copy_out(out_seq, s_seq, 0, T, lane, 64);
+        copy_out(out_qual, s_qual, seq_len, T, lane, 64);
+        if (moves_out) copy_out(out_moves, s_move, 0, T, lane, 64);
+    } else {
+        for (int t = tid; t < T; t += kGather) {
+            const int st = s_state[t];
+            const int base = st & 3;
+            float prob;
+            if (path_sums) {  // the sum below, taken for every state by path_sums_kernel: one read instead of nine
+                prob = path_sums[(first + t) * S + st];
+            } else {
+                const float *p = post_n + (size_t)(t + 1) * S;
+                prob = p[st];
+                int nb[8];
+#pragma unroll
+                for (int b = 0; b < 4; ++b) {
+                    nb[2 * b] = (st >> 2) + (S / 4) * b;
+                    nb[2 * b + 1] = ((st << 2) & (S - 1)) + b;
+                }
+                float x[8];  // all in flight together
+#pragma unroll
+                for (int k = 0; k < 8; ++k) x[k] = p[nb[k]];
+#pragma unroll
+                for (int k = 0; k < 8; ++k) {
+                    bool fresh = nb[k] != st;
+#pragma unroll
+                    for (int m = 0; m < k; ++m) fresh = fresh && nb[m] != nb[k];
+                    const float with = prob + x[k];
+                    prob = fresh ? with : prob;
+                }
+            }
+            if (prob > 1.0f) prob = 1.0f;
+            else if (prob < 0.0f) prob = 0.0f;
+            prob = (float)pow((double)prob, (double)0.4f);
+            const float wrong = (1.0f - prob) / 3.0f;
+            s_prob[t] = prob;
+            float4 q;
+            q.x = base == 0 ? prob : wrong;
+            q.y = base == 1 ? prob : wrong;
+            q.z = base == 2 ? prob : wrong;
+            q.w = base == 3 ? prob : wrong;
+            reinterpret_cast<float4 *>(qual_data)[first + t] = q;
+        }
     }
     __syncthreads();
 
-    // 3. one base per thread
+    // 4. one base per thread
     for (int p = tid; p < T; p += kThreads) {
-        const size_t o = (size_t)n * T + p;
+        const size_t o = first + p;
         if (p >= seq_len) {
-            sequence[o] = 0;
-            qstring[o] = 0;
             base_probs[o] = 0.f;
             total_probs[o] = 0.f;
             continue;
@@ -120,8 +180,8 @@ __global__ __launch_bounds__(kThreads) void sequence_kernel(
         const int t0 = s_start[p], t1 = s_start[p + 1];
         float bp = 0.f, tp = 0.f;
         for (int t = t0; t < t1; ++t) {
-            const float prob = s_prob[t], wrong = s_wrong[t];
-            const int base = s_base[t];
+            const float prob = s_prob[t], wrong = (1.0f - prob) / 3.0f;
+            const int base = s_state[t] & 3;
             bp += prob;
             tp += base == 0 ? prob : wrong;
             tp += base == 1 ? prob : wrong;
@@ -133,11 +193,12 @@ __global__ __launch_bounds__(kThreads) void sequence_kernel(
 #pragma unroll
         for (int j = 0; j < OFK_PHRED_STEPS; ++j) ch -= miss >= phred.thr[j] ? 1 : 0;
         if (miss != miss) ch = 0;
-        sequence[o] = "ACGT"[s_base[t0]];
-        qstring[o] = (char)ch;
+        s_qual[p] = (unsigned char)ch;
         base_probs[o] = -10.0f * (float)log10((double)miss);  // diagnostic copy, not used for the character
         total_probs[o] = tp;
     }
+    __syncthreads();
+    copy_out(out_qual, s_qual, 0, seq_len, tid, kThreads);
 }
 
 
@@ -262,19 +323,34 @@ int launch_path_sums(const float *post, float *sums, int T, int N, hipStream_t s
     return (int)hipGetLastError();
 }
 
+template <int S, int kThreads>
+int launch_sequence_with(const float *post, int32_t *states, const uint8_t *moves, float *qual_data,
+                         float *base_probs, float *total_probs, char *sequence, char *qstring, int T, int N,
+                         const ofk_phred_table_t &phred, const float *path_sums, uint8_t *moves_out, hipStream_t st) {
+    const size_t lds = sequence_lds(T);
+    if (lds > 64 * 1024 - 1024) {  // beyond the default limit of dynamic LDS; the compute unit has 160 KB
+        const hipError_t rc = hipFuncSetAttribute(reinterpret_cast<const void *>(&sequence_kernel<S, kThreads>),
+                                                  hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+        if (rc != hipSuccess) return (int)rc;
+    }
+    hipLaunchKernelGGL((sequence_kernel<S, kThreads>), dim3(N), dim3(kThreads), lds, st, post, states, moves, qual_data,
+                       base_probs, total_probs, sequence, qstring, T, phred, path_sums, moves_out);
+    return (int)hipGetLastError();
+}
+
 template <int S>
 int launch_sequence(const float *post, int32_t *states, const uint8_t *moves, float *qual_data,
                     float *base_probs, float *total_probs, char *sequence, char *qstring, int T, int N,
                     const ofk_phred_table_t &phred, const float *path_sums, uint8_t *moves_out, hipStream_t st) {
-    const size_t lds = (size_t)T * (4 + 4 + 1 + 1) + (size_t)(T + 1) * 4;
-    if (lds > 64 * 1024) {  // beyond the default limit of dynamic LDS; the compute unit has 160 KB
-        const hipError_t rc = hipFuncSetAttribute(reinterpret_cast<const void *>(&sequence_kernel<S>),
-                                                  hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-        if (rc != hipSuccess) return (int)rc;
-    }
-    hipLaunchKernelGGL((sequence_kernel<S>), dim3(N), dim3(kThreads), lds, st, post, states, moves, qual_data,
-                       base_probs, total_probs, sequence, qstring, T, phred, path_sums, moves_out);
-    return (int)hipGetLastError();
+    // Up to a chunk per compute unit a time step has a lane of its own, or two share one: the rounds of memory accesses are what
+    // is waited for.  Beyond, two workgroups of half the size fill a unit and one's gathers run beside the other's characters.
+    // 1024 | 512 | 256 lanes, us: 16 chunks of 64 states 14 | 17 | 25, 256 of 1024 84 | 86 | 92, 512 of 256 131 | 129 | 145, 1024 of 256
+    // 270 | 263 | 283.
+    if (N <= 256)
+        return launch_sequence_with<S, 1024>(post, states, moves, qual_data, base_probs, total_probs, sequence, qstring, T, N, phred,
+                                             path_sums, moves_out, st);
+    return launch_sequence_with<S, 512>(post, states, moves, qual_data, base_probs, total_probs, sequence, qstring, T, N, phred,
+                                        path_sums, moves_out, st);
 }
 
 }  // namespace
@@ -295,7 +371,7 @@ extern "C" int ofk_sequence(const float *post, int32_t *states, const uint8_t *m
                             float *base_probs, float *total_probs, char *sequence, char *qstring, int T, int N,
                             int state_len, const ofk_phred_table_t *phred, const float *path_sums, uint8_t *moves_out,
                             void *stream) {
-    // the per-chunk tables live in LDS: 14 bytes per time step
+    // the per-chunk tables live in LDS: 13 bytes per time step
     if ((!post && !path_sums) || !states || !moves || !qual_data || !base_probs || !total_probs || !sequence || !qstring ||
         !phred || T < 1 || T > OFK_MAX_T || N < 1)
         return OFK_BAD_ARGS;
