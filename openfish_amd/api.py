@@ -161,11 +161,21 @@ def _device_to_host(ptr, dtype, shape):
     return out
 
 
+class _Malloced:
+    """what the C API returned by malloc, for numpy to look at; freed with the last array that does"""
+
+    def __init__(self, address, shape, free=_libc.free):
+        self._address, self._free = address, free
+        self.__array_interface__ = {"data": (address, False), "shape": shape, "typestr": "|u1", "version": 3}
+
+    def __del__(self):
+        self._free(self._address)
+
+
 def _take(ptr, N, T):
-    """copy one malloc'd [N][T] byte buffer returned by the C API and free it"""
-    a = np.ctypeslib.as_array(C.cast(ptr, C.POINTER(C.c_uint8)), shape=(N, T)).copy()
-    _libc.free(ptr)
-    return a
+    """one malloc'd [N][T] byte buffer returned by the C API, as the array that owns it.  A copy of the three, after
+    the decode has ended, touches new pages: 0.2 ms with 1024 chunks of 1666 steps, 0.08 with 512."""
+    return np.asarray(_Malloced(ptr.value, (N, T)))
 
 
 class GpuBuf:
