@@ -40,7 +40,7 @@ constexpr size_t sequence_lds(int T) {
 }
 
 // What bounds it: up to a chunk per compute unit the waits of its few dependent rounds of memory accesses, above that the sectors
-// that the posteriors are gathered from (0.69 GB with 512 chunks of 256 states, 0.13 ms at 5.3 TB/s).  All that does not need
+// that the posteriors are gathered from (0.59 GB with 512 chunks of 256 states, 0.13 ms at 4.5 TB/s).  All that does not need
 // the posteriors comes first: base positions, the characters of the sequence and the zeros behind both strings, which one wave
 // then writes to their place (host memory, in a decode) while the others gather.  What is left after the gathers is a base's
 // character.  Inside decodes, ms, against gathers first, bytes last and one at a time, 256 lanes: 1 chunk of 64 states 0.021 ->
