@@ -97,7 +97,7 @@ def main():
 
     base, args = a.out_dir, a.bench_args
     out = ["# %s\n" % a.title,
-           "Commands (on the GPU box, from the repository root, one rocprofv3 run per pass; `A` = `%s`):\n" % args,
+           "Commands (from the repository root, one rocprofv3 run per pass; `A` = `%s`):\n" % args,
            "```",
            "rocprofv3 --kernel-trace --stats --output-format csv -d OUT/trace -o t -- python3 bench.py A",
            "rocprofv3 --pmc FETCH_SIZE --output-format csv -d OUT/fetch -o f -- python3 bench.py A",
