@@ -166,11 +166,11 @@ def rotary_bench(a):
         "scaling": "weak", "vs_baseline": None, "dtype": "f32", "data": "synthetic",
         "config": {"workload": "rotary: batch 500, seqlen 833, 8 heads x 64, rotary_half 32 (half x, fp32 sin/cos); "
                                "time of the synchronous call, launch and sync included"},
-        "roofline": {"bound": "hbm", "kernel": "rotary_vec8", "achieved": round(gbs, 1), "peak": HBM_PEAK_GBS,
+        "roofline": {"bound": "hbm", "kernel": "rotary_rows", "achieved": round(gbs, 1), "peak": HBM_PEAK_GBS,
                      "unit": "GB/s", "frac": round(gbs / HBM_PEAK_GBS, 4),
-                     # measured: 0.426 GB written, 0.220 GB fetched -- about half of the tensor the
+                     # measured: 0.426 GB written, 0.214 GB fetched -- about half of the tensor the
                      # previous call wrote is still in the 256 MB last-level cache
-                     "traffic": 647000000},
+                     "traffic": 641000000},
         "cpu_baseline": None}))
 
 

@@ -48,7 +48,8 @@ def template_ints(name):
 
 def short(name):
     for fn in ("scan_post_kernel", "bwd_scan_kernel", "fwd_post_roles_kernel", "fwd_post_kernel", "beam_kernel",
-               "sequence_kernel", "path_sums_kernel", "copy_kernel", "meet_kernel", "rotary_vec8_kernel", "rotary_kernel"):
+               "sequence_kernel", "path_sums_kernel", "copy_kernel", "meet_kernel", "fwd_scan_kernel", "posterior_rows_kernel",
+               "rotary_rows_kernel", "rotary_vec8_kernel", "rotary_narrow_kernel"):
         if fn in name:
             a = template_ints(name)
             if fn == "fwd_post_roles_kernel" and len(a) >= 3:
