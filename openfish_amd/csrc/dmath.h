@@ -212,7 +212,7 @@ OFA_HD float lse5_cpu_rounding_tab(float v0, float v1, float v2, float v3, float
 // Two-tier evaluation.  lse5_estimate computes the same quantity with the fp32 hardware
 // exponential and logarithm and decides whether its rounded result is certain to be the fp32
 // number the CPU path (reference src/decode_cpu.c:45-49) produces.  Where it is not certain
-// ("unsettled"), the caller evaluates lse5_cpu_rounding_tab instead.
+// ("unsettled"), the caller proves it or takes the CPU path's own steps (lse5_bounds below).
 //
 // With d_i = v_i - m (fp32, as on the CPU path) the CPU path's result is RN32(m + ln s_cpu),
 // s_cpu the fp32 running sum of the double exponentials.  The estimate forms
@@ -289,6 +289,8 @@ OFA_HD Lse5Value lse5_value(float v0, float v1, float v2, float v3, float v4, fl
     e.value = __builtin_fmaf(e.l2, kLn2, m);
     return e;
 }
+// 2^24 h of a result: the binade of the float below |r~|, which |r~| (1 - 2^-24) is for a power of two; every other float stays in its own
+OFA_HD float lse5_binade(float value) { return float_of(bits_of(value * 0x1.fffffep-1f) & 0x7f800000u); }
 OFA_HD Lse5Estimate lse5_verdict(Lse5Value x, float m) {
     const float kLn2 = 0.69314718055994530942f;
     const float kEps0 = 8.68e-7f, kEpsMu = 5.21e-7f, kEps1 = 6.42e-8f;
@@ -296,8 +298,7 @@ OFA_HD Lse5Estimate lse5_verdict(Lse5Value x, float m) {
     e.value = x.value;
     e.sum = x.sum;
     const float rho = __builtin_fmaf(x.l2, kLn2, -(x.value - m));
-    // 2^24 h: the binade of the float below |r~|, which |r~| (1 - 2^-24) is for a power of two; every other float stays in its own
-    const float binade = float_of(bits_of(x.value * 0x1.fffffep-1f) & 0x7f800000u);
+    const float binade = lse5_binade(x.value);
     e.half = binade * 0x1p-24f;
     const uint32_t sb = bits_of(x.sum) + 16u;
     const float mu = float_of((sb & 0x007fffffu) | 0x3f000000u);
@@ -309,12 +310,45 @@ OFA_HD Lse5Estimate lse5_estimate(float v0, float v1, float v2, float v3, float 
     return lse5_verdict(lse5_value(v0, v1, v2, v3, v4, m), m);
 }
 
-// the scan update in two tiers: the estimate where it is settled, the CPU roundings elsewhere
-OFA_HD float lse5_two_tier(float v0, float v1, float v2, float v3, float v4, float m, const LogCell *table,
+// ---------------------------------------------------------------------------------------------
+// Unsettled estimates are right all but one or two times in a hundred, so they are proven before anything is worked
+// out again.  With q = r~ - m and h as above, both exact in fp32, the CPU path rounds m + ln s_cpu to r~ if
+//   e^(q-h) < s_cpu < e^(q+h).
+// The boundaries are drawn in by 2^-32.5 or more (exp_ldexp's `unit`).  That covers the rounding of m + ln s_cpu to double on
+// the CPU path, at most 2^-34 for h <= 2^-6, and the error of the exponentials here, 2^-50.
+// From h = 2^-19 up q - h and q + h are exact: multiples of h, and not above 2 in magnitude.  Outside h = 2^-19 .. 2^-6
+// (|r~| up to 32 or above 2^19) nothing is proven: the lower boundary is a NaN, which no sum is above.
+// ---------------------------------------------------------------------------------------------
+constexpr double kProofLowerUnit = 1.0 + 0x1p-32, kProofUpperUnit = 1.0 - 0x1p-32;
+struct Lse5Bounds {
+    float lower, upper;  // logarithms, against m
+};
+OFA_HD Lse5Bounds lse5_bounds(float value, float half, float m) {
+    const float q = value - m;
+    const uint32_t h = bits_of(half);
+    Lse5Bounds b;
+    b.lower = h - 0x36000000u <= 0x3c800000u - 0x36000000u ? q - half : __builtin_nanf("");
+    b.upper = q + half;
+    return b;
+}
+// whether the CPU path's running sum `sum` lies between the boundaries (the kernels evaluate both in lanes of their own)
+OFA_HD bool lse5_proven(float sum, Lse5Bounds b, const double *ec) {
+    return (double)sum > exp_ldexp((double)b.lower, ec, kProofLowerUnit) && !((double)sum > exp_ldexp((double)b.upper, ec, kProofUpperUnit));
+}
+
+// The scan update in two tiers, as the kernels take it: the estimate where it is settled or proven, the logarithm of the
+// CPU path's running sum elsewhere.
+OFA_HD float lse5_two_tier(float v0, float v1, float v2, float v3, float v4, float m, const LogCell *centred,
                            const double *series, const double *ec) {
     const Lse5Estimate e = lse5_estimate(v0, v1, v2, v3, v4, m);
     if (e.settled) return e.value;
-    return lse5_cpu_rounding_tab(v0, v1, v2, v3, v4, m, table, series, ec);
+    float s = (float)exp_nonpos_ldexp(v0 - m, ec);
+    s = (float)((double)s + exp_nonpos_ldexp(v1 - m, ec));
+    s = (float)((double)s + exp_nonpos_ldexp(v2 - m, ec));
+    s = (float)((double)s + exp_nonpos_ldexp(v3 - m, ec));
+    s = (float)((double)s + exp_nonpos_ldexp(v4 - m, ec));
+    if (lse5_proven(s, lse5_bounds(e.value, e.half, m), ec)) return e.value;
+    return (float)((double)m + log_centred(s, centred[log_centred_index(s)], series));
 }
 
 }  // namespace ofa

@@ -63,11 +63,11 @@ struct LogSeries {
     double c[6];
     double e[OFA_EXP_COEF_COUNT];  // exponential: polynomial, rounding shift, log2(e), -ln 2
 };
-// Unsettled updates are looked at eight lanes each (see certify): lanes 0 .. 4 evaluate the update's five
-// exponentials, lanes 5 and 6 those of the rounding boundaries, moved towards each other by about 2^-32.
+// Unsettled updates are looked at eight lanes each (settle_one, settle_eight): lanes 0 .. 4 evaluate the update's five
+// exponentials, lanes 5 and 6 those of the rounding boundaries, drawn in.
 __device__ __forceinline__ double certificate_unit() {
     const int k = threadIdx.x & 7;
-    return k == 5 ? 1.0 + 0x1p-32 : k == 6 ? 1.0 - 0x1p-32 : 1.0;
+    return k == 5 ? ofa::kProofLowerUnit : k == 6 ? ofa::kProofUpperUnit : 1.0;
 }
 struct LogArgs {
     const ofa::LogCell *cells;    // 32 cells, for the always-double arithmetic
@@ -84,13 +84,10 @@ struct LogArgs {
 //
 // Unsettled estimates are right all but one or two times in a hundred (counted over the sweeps of 64, 256 and 1024
 // states): the bound has to allow for roundings of the two running sums that never conspire.  So the second tier does not
-// work the result out again but proves the estimate r: with q = r - m and h half an ulp of r, both exact, r is what the
-// CPU path rounds m + ln s to if e^(q-h) < s < e^(q+h), s being the CPU path's fp32 running sum of the double
-// exponentials.  Seven exponentials side by side in seven lanes, the running sum, one comparison: no logarithm, and
-// nothing is handed back to the update's lane.  The boundaries are drawn in by 2^-32.5 or more (certificate_unit), which
-// covers the rounding of m + ln s to double on the CPU path, at most 2^-34 for h <= 2^-6, and the errors here; from
-// h = 2^-19 up q - h and q + h are exact in fp32.  Outside that range (|r| below 32 or above 2^19) and wherever the proof
-// fails, every lane takes the double arithmetic with the CPU path's roundings (`by_double`).
+// work the result out again but proves the estimate (dmath.h, lse5_bounds): seven exponentials side by side in seven lanes,
+// five of the update and two of the boundaries, the running sum, one comparison; no logarithm, and
+// nothing is handed back to the update's lane.  Where a proof fails, which it always does for |r| up to 32 or above 2^19, the
+// update takes the logarithm of the running sum that the proof has formed.
 //
 // An instruction costs a wave that is alone on its SIMD about four cycles whatever it does (fp64 and
 // dependent ones included), so a trip through this tier costs what it issues plus its LDS round trips.
@@ -98,7 +95,8 @@ struct LogArgs {
 //   one (two waves in three that have any, with one state per lane): its seven arguments are read into scalar
 //     registers and dealt to seven lanes, no LDS;
 //   several: handed through LDS to groups of eight lanes, eight updates at a time;
-//   many (only the first hundred time steps have them: values are small there and an ulp is tiny): by_double.
+//   many (only the first hundred time steps have them: values are small there and an ulp is tiny): no proof, every lane takes its
+//     update's five exponentials, running sum and logarithm in double.
 // Cycles of a lone wave for an update of 64 states with 0 | 1 | 2 to 8 | more of them unsettled: 250 | 620 | 780 | 890; when
 // the second tier worked the results out (and took the logarithm in every trip) 245 | 740 | 975 | 985.  Together with the order
 // of a step (see lse5_all) the backward sweep at T = 1666 went from 0.44 to 0.39 ms (1 chunk of 64 states), 0.68 to 0.58 (1 of
@@ -247,14 +245,12 @@ __device__ __forceinline__ bool resolve_unsettled(float (&value)[SPL], const flo
     int total = 0;
 #pragma unroll
     for (int i = 0; i < SPL; ++i) total += scalar(__builtin_popcountll(mask[i]));
-    // the boundaries, against m; a NaN where the proof does not hold, so that it fails
     float lower[SPL], upper[SPL];
 #pragma unroll
     for (int i = 0; i < SPL; ++i) {
-        const float q = value[i] - m[i];
-        const uint32_t h = __float_as_uint(half[i]);
-        lower[i] = h - 0x36000000u <= 0x3c800000u - 0x36000000u ? q - half[i] : __builtin_nanf("");  // h from 2^-19 to 2^-6
-        upper[i] = q + half[i];
+        const ofa::Lse5Bounds b = ofa::lse5_bounds(value[i], half[i], m[i]);
+        lower[i] = b.lower;
+        upper[i] = b.upper;
     }
     if (__builtin_expect(total == 1, 1)) {
         return settle_single<SPL>(value, mask, v, m, lower, upper, logtab);

@@ -79,8 +79,8 @@ long lse5_mismatches(const float *v, long n) {
 // taken as settled although it differs from the libm result (must be zero), stores the number of
 // unsettled estimates and the number of results of the whole two-tier update that differ
 long two_tier_wrongly_settled(const float *v, long n, long *unsettled, long *mismatches) {
-    ofa::LogCell table[32];
-    for (int i = 0; i < 32; ++i) table[i] = ofa::log_cell(i);
+    ofa::LogCell table[ofa::kLogCentredCells];
+    for (int i = 0; i < ofa::kLogCentredCells; ++i) table[i] = ofa::log_centred_cell(i);
     long wrong = 0, open = 0, bad = 0;
     for (long i = 0; i < n; ++i) {
         const float *p = v + 5 * i;
@@ -95,6 +95,31 @@ long two_tier_wrongly_settled(const float *v, long n, long *unsettled, long *mis
     }
     *unsettled = open;
     *mismatches = bad;
+    return wrong;
+}
+
+// The proof of an estimate, given the result that libm's arithmetic leads to and the floats `reach` ulps on either side of
+// it: how often it accepts another float than that one (must be zero); how often it accepts that one; and how often it
+// refuses although the result lies where proofs are meant to hold, |r| from 32 up to 2^19
+long proofs_of_wrong_values(const float *v, long n, int reach, long *accepted, long *refused) {
+    long wrong = 0, right = 0, open = 0;
+    for (long i = 0; i < n; ++i) {
+        const float *p = v + 5 * i;
+        float m = p[0];
+        for (int k = 1; k < 5; ++k) m = m > p[k] ? m : p[k];
+        float s = 0.0f;
+        for (int k = 0; k < 5; ++k) s = (float)((double)s + ofa::exp_nonpos_ldexp(p[k] - m, kExp));
+        const float want = lse5_libm(p, m);
+        for (int d = -reach; d <= reach; ++d) {
+            const float r = ofa::float_of(ofa::bits_of(want) + (uint32_t)d);
+            const bool proven = ofa::lse5_proven(s, ofa::lse5_bounds(r, ofa::lse5_binade(r) * 0x1p-24f, m), kExp);
+            if (d != 0) wrong += proven;
+            else if (proven) ++right;
+            else if (fabsf(r) > 32.0f && fabsf(r) <= 0x1p19f) ++open;
+        }
+    }
+    *accepted = right;
+    *refused = open;
     return wrong;
 }
 }

@@ -28,6 +28,8 @@ def lib(tmp_path_factory):
     L.max_abs_err_log_near.argtypes = [fp, C.c_long, C.c_int]
     L.two_tier_wrongly_settled.restype = C.c_long
     L.two_tier_wrongly_settled.argtypes = [fp, C.c_long, C.POINTER(C.c_long), C.POINTER(C.c_long)]
+    L.proofs_of_wrong_values.restype = C.c_long
+    L.proofs_of_wrong_values.argtypes = [fp, C.c_long, C.c_int, C.POINTER(C.c_long), C.POINTER(C.c_long)]
     return L
 
 
@@ -155,3 +157,58 @@ def test_two_tier_sums_next_to_a_binade_of_the_sum(lib, terms, centre):
     wrong = lib.two_tier_wrongly_settled(fptr(v), n, C.byref(unsettled), C.byref(mismatches))
     assert wrong == 0 and mismatches.value == 0
     assert unsettled.value < n
+
+
+def proofs(lib, v, reach=2):
+    accepted, refused = C.c_long(), C.c_long()
+    wrong = lib.proofs_of_wrong_values(fptr(v), v.shape[0], reach, C.byref(accepted), C.byref(refused))
+    return wrong, accepted.value, refused.value
+
+
+# both ends of the range of half ulps that proofs allow for (results of 32 and of 2^19 in magnitude), and between
+@pytest.mark.parametrize("sign", [1.0, -1.0])
+@pytest.mark.parametrize("centre,spread", [(0.0, 3.0), (33.0, 1.0), (32.0, 2.0), (40.0, 3.0), (63.0, 1.0), (700.0, 3.0), (5900.0, 40.0),
+                                           (262144.0, 3.0), (524280.0, 4.0), (524288.0, 1.0), (600000.0, 5.0)])
+def test_a_proof_accepts_the_libm_result_and_none_of_its_neighbours(lib, centre, spread, sign):
+    rng = np.random.default_rng(int(centre) + 23)
+    n = 400000
+    v = (sign * centre + spread * rng.standard_normal((n, 5))).astype(np.float32)
+    wrong, accepted, refused = proofs(lib, v)
+    assert wrong == 0
+    # a result is refused where the sum lies within 1.42 * 2^-32 of one of its two boundaries, an ulp of 2^-18 or more
+    # apart: 2^-13 of them at the smallest ulp, and powers of two beyond the nearer half ulp
+    assert refused <= 8 * n * 2.0 ** -13 + 16
+    if 34.0 <= centre <= 300000.0:
+        assert accepted > 0.9 * n
+    if centre == 600000.0:
+        assert accepted == 0
+
+
+@pytest.mark.parametrize("power", [32.0, 64.0, 512.0, 4096.0, 2.0 ** 18, 2.0 ** 19])
+@pytest.mark.parametrize("sign", [1.0, -1.0])
+def test_proofs_next_to_a_power_of_two(lib, power, sign):
+    """results scattered within three ulps of a power of two, and exactly on the boundaries beside it (see
+    test_two_tier_results_next_to_a_power_of_two for the inputs)"""
+    rng = np.random.default_rng(int(power) + 29)
+    n = 300000
+    ulp = np.spacing(np.float32(power))
+    gap = rng.uniform(1e-3 + 4.0 * ulp, np.log(2.0), n)
+    big = sign * power - gap
+    off = np.where(rng.random(n) < 0.5, rng.uniform(-3.0, 3.0, n), 0.25 * rng.integers(-8, 9, n))
+    other = big + np.log(np.expm1(gap + off * ulp))
+    v = np.stack([big, other, big - 200.0, big - 300.0, big - 400.0], axis=1).astype(np.float32)
+    wrong, accepted, _ = proofs(lib, v, reach=4)
+    assert wrong == 0
+    assert accepted > 0
+
+
+def test_proofs_of_sums_a_step_away_from_a_boundary(lib):
+    """two equal terms and a third far below: the sum is 2 or one of the floats next above it, and the result sits on every position
+    between two boundaries as the maximum runs through the floats of a range"""
+    m = np.arange(0, 400000, dtype=np.float32) * np.float32(2.0 ** -17) + np.float32(40.0)
+    v = np.stack([m, m, m - 15.0, m - 100.0, m - 100.0], axis=1).astype(np.float32)
+    wrong, accepted, _ = proofs(lib, v)
+    assert wrong == 0 and accepted > 0.5 * m.size
+    v = np.stack([m + 2.0 ** 17, m + 2.0 ** 17 - 0.7, m - 100.0, m - 100.0, m - 100.0], axis=1).astype(np.float32)
+    wrong, accepted, _ = proofs(lib, v)
+    assert wrong == 0 and accepted > 0.5 * m.size
