@@ -96,3 +96,41 @@ def test_backward_sweep_of_1024_states_on_either_side_of_a_chunk_per_unit(api, T
     ref_bwd, _, _ = O.scans(four.astype(np.float32), 5)
     bwd, _ = stage_scans(api, given, 5, 2.0, "two_tier", False)
     assert np.array_equal(bwd, ref_bwd)
+
+
+MAGNITUDES = [(-1.65, 0.5, -1.65, 150), (-21.0, 3.0, -19.0, 220), (2600.0, 3.0, 2600.0, 230), (30000.0, 2000.0, 30000.0, 40),
+              (-30000.0, 8.0, -30000.0, 40), (0.0, 12.0, 2.0, 120), (1.0, 0.2, 1.0, 300)]
+
+
+# how a decode is made to take each form of the two-tier update: states per lane (several of them share a proof's trip),
+# one kernel (four to a lane: one state after another, exponentials in a loop), sweep within the search, sweeps apart
+@pytest.mark.parametrize("state_len,N,form", [(sl, n, (split, spl)) for sl, n in ((3, 3), (4, 2), (5, 1)) for split in (False, True) for spl in (0, 1, 2, 4)] +
+                         [(4, 2, (2, 0)), (5, 2, (2, 0))])
+@pytest.mark.parametrize("mean,spread,stay,T", MAGNITUDES)
+def test_every_form_of_the_update_settles_estimates_right(api, state_len, N, form, mean, spread, stay, T):  # noqa: F811
+    """bwd bit for bit the oracle's.  Posteriors are compared with those of the always-double arithmetic in the same number of
+    kernels, which subtracts the same shift (another one would round the exponential's argument elsewhere: |x| 2^-24, 5e-6 for a
+    posterior of 1e-31) but may take the normalising sums in another order: at most 3 + 6 + 8 additions of 2^-24 each way, a reciprocal
+    of one ulp and a product, 2.5e-6 together.  A forward value that is an ulp off, |f| > 32, moves its posterior by
+    3.8e-6 or more."""
+    S = 4 ** state_len
+    split, spl = form
+    rng = np.random.default_rng(19 + T)
+    s16 = np.clip(rng.normal(mean, spread, (T, N, 4 * S)), -65000, 65000).astype(np.float16)
+    O.set_scan_stay(stay)
+    try:
+        ref_bwd, _, _ = O.scans(s16.astype(np.float32), state_len)
+    finally:
+        O.set_scan_stay()
+    _, precise = stage_scans(api, s16, state_len, stay, api.SCAN_PRECISE, split is False)
+    sc = api.upload_scores_to_hip(s16)
+    gb = api.GpuBuf(T, N, state_len)
+    gb.set_split_scans(split)
+    gb.set_scan_states_per_lane(spl)
+    api.lib().openfish_amd_memset(gb.handle.contents.post_NTC, 0xff, N * (T + 1) * S * 4)
+    api.openfish_decode_gpu(T, N, 4 * S, sc, state_len, api.DECODER_INIT(blank_score=stay), gb)
+    assert np.array_equal(gb.tensor("bwd_NTC"), ref_bwd)
+    post = gb.tensor("post_NTC")
+    finite = np.isfinite(precise)
+    assert np.array_equal(np.isfinite(post), finite)
+    np.testing.assert_allclose(post[finite], precise[finite], rtol=2.5e-6, atol=1.2e-38)
