@@ -1258,25 +1258,37 @@ __global__ __launch_bounds__((kBeamThreads<S, CPG, COLS, FWD>), (BeamCfg<S, FWD>
     }
 }
 
+// Chunks of a search that share a workgroup, and so a compute unit's LDS.  256 units: up to 512 chunks fit two to a unit; larger
+// batches go four to a group where the LDS of four chunks fits (64 and 256 states).  Few chunks have a unit each: two searches on one wait for
+// each other's LDS operations, and with the LDS to itself a chunk has an index so large that one step in forty (1024
+// states, with half the buckets, one in twenty) instead of one in ten meets two elements in a bucket.  Search, two to a unit | one,
+// T = 1666 (1024 states 833), ms: 64 states, 1 chunk 0.943 | 0.929, 16 1.033 | 0.936, 160 1.05 | 0.96; 256 states, 16
+// 1.024 | 0.941, 160 1.04 | 0.99; 1024 states, 37 0.565 | 0.490, 100 0.577 | 0.504, 160 (split: units are short) 0.74 | 1.0.
+//
+// Such a group leaves no room for a second on its unit.  So a search that is alone on the device takes units as long as those
+// it leaves hold a second decode of the same size that begins while it runs, two chunks (1024 states: one) to a unit: workgroups are dealt
+// round eight XCDs of 32 units, 20 and 10 of them with 160 chunks, 22 and 11 with 170.  Two callers whose calls begin at
+// random, a call's mean | 90th percentile, ms, two to a unit | one: 256 states, 160 chunks 1.98 2.19 | 2.02 2.30, 170 2.01 2.25 |
+// 2.12 2.50, 200 2.03 2.28 | 2.23 2.78; 64 states, 160 1.71 1.96 | 1.68 1.92, 170 1.72 1.96 | 1.74 2.16 (one caller: 256 states, 160
+// chunks 1.785 | 1.73, 200 1.80 | 1.755).  Where other decodes may be under way, three of them, a lane each, find units for all their chunks.
+int search_group(int S, int N, int flags) {
+    const bool alone = (flags & OFK_SEARCH_ALONE) != 0;
+    if (N <= (S >= 1024 ? (alone ? 128 : 32) : (alone ? 160 : 64))) return 1;
+    return S <= 256 && N > OFK_SPARSE_SEARCH_MAX_CHUNKS ? 4 : 2;
+}
+
 template <int S, int COLS>
 int launch_beam(const void *scores, const float *bwd, ofk_beam_slot_t *beam, int32_t *states,
                 uint8_t *moves, int T, int N, float log_cut, float stay, int flags, const double *lse_table,
                 hipStream_t st) {
-    // 256 compute units: up to 512 chunks fit two to a unit; larger batches go four to a group
-    // where the LDS of four chunks fits (64 and 256 states).  Few chunks have a unit each: two searches on one wait for each
-    // other's LDS operations, and with the LDS to itself a chunk has an index so large that one step in forty instead of
-    // one in ten meets two elements in a bucket.  Search, two to a unit | one, T = 1666 (1024 states 833), ms: 64 states, 1 chunk
-    // 0.943 | 0.929, 16 1.033 | 0.936, 200 1.051 | 0.974; 256 states, 16 1.024 | 0.941, 200 1.042 | 1.002; 1024 states, 37
-    // 0.565 | 0.490, 100 0.577 | 0.504, 160 (split: units are short) 0.74 | 1.0.  Such a group leaves no room for a second on its unit, hence
-    // the smaller bound where other decodes may be under way: three of them (a lane each) find units for all their chunks.
-    const int units = (flags & OFK_SEARCH_ALONE) ? 256 : 64;
-    if (N <= (S >= 1024 ? units / 2 : units)) {
+    const int group = search_group(S, N, flags);
+    if (group == 1) {
         hipLaunchKernelGGL((beam_kernel<S, 1, COLS, 0>), dim3(N), dim3(kBeamThreads<S, 1, COLS, 0>), 0, st, static_cast<const _Float16 *>(scores), bwd,
                            nullptr, beam, states, moves, T, N, log_cut, stay, flags, lse_table, LogSeries{});
         return (int)hipGetLastError();
     }
     if constexpr (S <= 256) {
-        if (N > OFK_SPARSE_SEARCH_MAX_CHUNKS) {
+        if (group == 4) {
             hipLaunchKernelGGL((beam_kernel<S, 4, COLS, 0>), dim3((N + 3) / 4), dim3(512), 0, st,
                                static_cast<const _Float16 *>(scores), bwd, nullptr, beam, states, moves, T, N, log_cut,
                                stay, flags, lse_table, LogSeries{});
@@ -1386,6 +1398,8 @@ extern "C" int ofk_beam_search_static(const void *scores, const float *bwd, int3
     return dispatch_beam(scores, bwd, beam, states, moves, T, N, state_len, columns, log_beam_cut, stay, flags,
                          lse_table, st);
 }
+
+extern "C" int ofk_search_chunks_per_group(int N, int state_len, int flags) { return search_group(1 << (2 * state_len), N, flags); }
 
 extern "C" int ofk_beam_search(const void *scores, const float *bwd, ofk_beam_slot_t *beam, int32_t *states,
                                uint8_t *moves, int T, int N, int state_len, int columns, float log_beam_cut,

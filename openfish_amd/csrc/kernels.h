@@ -82,9 +82,11 @@ int ofk_beam_search_static(const void *scores, const float *bwd, int32_t *states
  * otherwise taken only after a hash collision); results must not change.  Bit 1: seed hashes are
  * taken from (state & 15), so that different sequences share hashes and the search has to notice
  * the duplicates by itself; results then equal those of a CPU search seeded the same way. */
-/* Added to flags by a caller whose search shares the device with no other decode: up to a chunk per compute unit (half as many
- * of 1024 states, whose forward sweep wants a unit of its own) ofk_beam_search then gives every chunk the LDS of a unit. */
+/* Added to flags by a caller whose search shares the device with no other decode: ofk_beam_search then gives every chunk
+ * the LDS of a compute unit as long as the units left hold a decode of the same size that begins meanwhile. */
 #define OFK_SEARCH_ALONE 4
+/* The rule: how many chunks of a search share a workgroup (1: a chunk has a unit to itself).  Host-only. */
+int ofk_search_chunks_per_group(int N, int state_len, int flags);
 /* Phred characters run from '"' (34, q = 1) to 'S' (83, q = 50).  thr[j] is the smallest
  * miss probability x whose character is at most 82 - j (2.0f if no x in [0,1] reaches it),
  * so that char(x) = 83 - #{j : x >= thr[j]}. */

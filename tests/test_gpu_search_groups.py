@@ -12,8 +12,8 @@ from test_gpu_scan_options import api  # noqa: F401
 
 pytestmark = pytest.mark.gpu
 
-# 64 and 256 states: a chunk per unit up to 64, alone 256; two up to 512; then four.  1024 states: up to 32, alone 128; then two
-SIZES = [(3, 300, 8, n) for n in (8, 64, 65, 256, 257, 520)] + [(4, 240, 6, n) for n in (1, 64, 65, 256, 257)] + \
+# 64 and 256 states: a chunk per unit up to 64, alone 160; two up to 512; then four.  1024 states: up to 32, alone 128; then two
+SIZES = [(3, 300, 8, n) for n in (8, 64, 65, 160, 161, 256, 257, 520)] + [(4, 240, 6, n) for n in (1, 64, 65, 160, 161, 256, 257)] + \
         [(5, 90, 2, n) for n in (2, 32, 33, 128, 129)]
 
 
