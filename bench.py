@@ -58,7 +58,12 @@ def measured_traffic(workload, N, columns, kernel, arrangement):
 SCANS = ("one", "split", "merged")
 SCANS_TEXT = {"one": "both scans and the posterior as one kernel, then the beam search",
               "split": "backward scan, then forward scan + posterior on a second stream beside the beam search",
-              "merged": "backward scan, then forward scan + posterior within the beam search's kernel"}
+              "merged": "backward scan, then forward scan + posterior within the beam search's kernel",
+              "apart": "backward and forward scan side by side, then the posterior on a second stream beside the beam search"}
+
+
+def scans_text(ran, mean):
+    return SCANS_TEXT["apart" if mean["fwd_scan"] > 0 else ran]
 
 
 def arrangement_run(api, asked, mean, shape, scan_mode, states_per_lane):
@@ -84,6 +89,8 @@ def algorithmic_bytes(state_len, T, N, columns=4):
         "path_sums": N * 2 * T * S * 4,               # read the posteriors of T rows, write a sum per state
     }
     need["scan"] = need["bwd"] + need["fwd_post"]     # both scans + posterior as one kernel: the same minimum
+    need["fwd_scan"] = N * (scores + vec)             # the forward scan by itself: read scores, write fwd
+    need["posterior"] = N * 3 * vec                   # and the posteriors by themselves: read fwd + bwd, write post
     need["beam_merged"] = need["beam"] + N * vec      # search, forward scan and posterior over one reading of the rows
     return need
 
@@ -189,12 +196,41 @@ def timed_decodes(api, gpubuf, call_args, steps):
 
 
 def scan_stage(need, mean):
-    """scans + posterior: one kernel (`scan`) or the two split kernels (`bwd`, `fwd_post`); not for a forward scan
-    within the beam search's kernel, whose time is not the scans' alone"""
-    ms = mean["scan"] + mean["bwd"] + mean["fwd_post"]
+    """scans + posterior: one kernel (`scan`), the two split kernels (`bwd`, `fwd_post`), or both scans side by side
+    (`bwd`, `fwd_scan`) and then the posteriors (`fwd_post`); not for a forward scan within the beam search's kernel, whose
+    time is not the scans' alone"""
+    ms = mean["scan"] + max(mean["bwd"], mean["fwd_scan"]) + mean["fwd_post"]
     gbs = need["scan"] / 1e9 / (ms / 1e3)
     return {"ms": round(ms, 4), "algorithmic_GB": round(need["scan"] / 1e9, 4), "GBps": round(gbs, 1),
             "frac_of_hbm_peak": round(gbs / HBM_PEAK_GBS, 4)}
+
+
+def stage_table(need, mean, ran):
+    """every kernel's mean time with the bytes it has to move"""
+    mean, need = dict(mean), dict(need)
+    if ran == "merged":  # one kernel: its time is the beam search's, its bytes both stages'
+        mean["fwd_post"] = 0.0
+        need["beam"] = need["beam_merged"]
+    if mean["fwd_scan"] > 0:  # forward scan beside the backward one: what follows is the posteriors' pass
+        need["fwd_post"] = need["posterior"]
+    stages = {}
+    for k in ("scan", "bwd", "fwd_scan", "fwd_post", "beam", "sequence", "path_sums"):  # path_sums runs beside the beam search
+        if mean[k] > 0:
+            stages[k] = {"ms": round(mean[k], 4), "algorithmic_GB": round(need[k] / 1e9, 4),
+                         "GBps": round(need[k] / 1e9 / (mean[k] / 1e3), 1)}
+    stages["device_total_ms"] = round(mean["total"], 4)
+    # kernels that share the machine: the beam search starts together with the forward scan (split scans) or
+    # with the path sums (one scan kernel); their algorithmic bytes over the longer of the two
+    beside = "fwd_post" if mean["fwd_post"] > 0 else ("path_sums" if mean["path_sums"] > 0 else None)
+    if beside:
+        window_ms = max(mean["beam"], mean[beside])
+        gb = (need["beam"] + need[beside]) / 1e9
+        stages["beam_and_" + beside + "_side_by_side"] = {
+            "ms": round(window_ms, 4), "algorithmic_GB": round(gb, 4), "GBps": round(gb / (window_ms / 1e3), 1),
+            "frac_of_hbm_peak": round(gb / (window_ms / 1e3) / HBM_PEAK_GBS, 4)}
+    if ran != "merged":
+        stages["scan_plus_posterior"] = scan_stage(need, mean)
+    return stages
 
 
 def main():
@@ -279,27 +315,8 @@ def main():
 
     need = algorithmic_bytes(state_len, T, N, a.columns)
     ran = arrangement_run(api, asked, mean, (T, N, C, state_len), a.scan_mode, a.states_per_lane)
-    if ran == "merged":  # one kernel: its time is the beam search's, its bytes both stages'
-        mean["fwd_post"] = 0.0
-        need["beam"] = need["beam_merged"]
-    stages = {}
-    for k in ("scan", "bwd", "fwd_post", "beam", "sequence", "path_sums"):  # path_sums runs beside the beam search
-        if mean[k] > 0:
-            stages[k] = {"ms": round(mean[k], 4), "algorithmic_GB": round(need[k] / 1e9, 4),
-                         "GBps": round(need[k] / 1e9 / (mean[k] / 1e3), 1)}
-    stages["device_total_ms"] = round(mean["total"], 4)
-    # kernels that share the machine: the beam search starts together with the forward scan (split scans) or
-    # with the path sums (one scan kernel); their algorithmic bytes over the longer of the two
-    beside = "fwd_post" if mean["fwd_post"] > 0 else ("path_sums" if mean["path_sums"] > 0 else None)
-    if beside:
-        window_ms = max(mean["beam"], mean[beside])
-        gb = (need["beam"] + need[beside]) / 1e9
-        stages["beam_and_" + beside + "_side_by_side"] = {
-            "ms": round(window_ms, 4), "algorithmic_GB": round(gb, 4), "GBps": round(gb / (window_ms / 1e3), 1),
-            "frac_of_hbm_peak": round(gb / (window_ms / 1e3) / HBM_PEAK_GBS, 4)}
-    if ran != "merged":
-        stages["scan_plus_posterior"] = scan_stage(need, mean)
-    dominant = max((k for k in ("scan", "bwd", "fwd_post", "beam", "sequence") if k in stages), key=lambda k: stages[k]["ms"])
+    stages = stage_table(need, mean, ran)
+    dominant = max((k for k in ("scan", "bwd", "fwd_scan", "fwd_post", "beam", "sequence") if k in stages), key=lambda k: stages[k]["ms"])
     roofline = {"bound": "hbm", "kernel": dominant, "achieved": stages[dominant]["GBps"], "peak": HBM_PEAK_GBS,
                 "unit": "GB/s", "frac": round(stages[dominant]["GBps"] / HBM_PEAK_GBS, 4),
                 "traffic": measured_traffic(a.workload, N, a.columns, dominant, ran)}
@@ -340,7 +357,7 @@ def main():
         five_columns = {"C": 5 * S, "chunks_per_s": round(N / (ms5 / 1e3), 1), "ms_per_step": round(ms5, 4),
                         "stage_ms": {k: round(v, 4) for k, v in mn5.items() if v > 0},
                         "scan_plus_posterior": scan_stage(algorithmic_bytes(state_len, T, N, 5), mn5) if ran5 != "merged" else None,
-                        "scans": SCANS_TEXT[ran5],
+                        "scans": scans_text(ran5, mn5),
                         "note": "the same batch with five fp16 columns per state (blank first, never read), default settings"}
         scores5.free()
 
@@ -398,7 +415,7 @@ def main():
         "vs_baseline": None, "dtype": "f32" if a.scan_mode == "fast" else "f32+f64", "data": "synthetic",
         "config": {"workload": "%s: state_len %d, S=%d, C=%d fp16 TNC (%d columns per state), T=%d, N=%d, beam 32, "
                                "beam_cut 100, blank 2.0" % (a.workload, state_len, S, C, a.columns, T, N),
-                   "scan_mode": a.scan_mode, "scans": SCANS_TEXT[ran],
+                   "scan_mode": a.scan_mode, "scans": scans_text(ran, mean),
                    "seed": a.seed},
         "roofline": roofline, "stages": stages, "other_scan_arrangement": other_split, "fast_scan_mode": fast_mode,
         "five_columns": five_columns, "two_in_flight": overlap, "cpu_baseline": cpu, "cpu_baseline_config1": cpu1,

@@ -172,14 +172,17 @@ void openfish_amd_decode_wait(const openfish_gpubuf_t *gpubuf, const uint8_t **m
 enum openfish_amd_stage {
     OPENFISH_AMD_STAGE_BWD = 0,   /* backward scan kernel (0 when both scans ran as one kernel) */
     OPENFISH_AMD_STAGE_FWD = 1,   /* forward + posterior kernel (0 when both scans ran as one kernel; equal to the
-                                   * next where they ran within the beam search's kernel) */
+                                   * next where they ran within the beam search's kernel; the posteriors' pass alone
+                                   * where OPENFISH_AMD_STAGE_FWD_SCAN is not 0) */
     OPENFISH_AMD_STAGE_BEAM = 2,  /* beam search + traceback kernel */
     OPENFISH_AMD_STAGE_SEQ = 3,   /* quality + sequence kernel */
     OPENFISH_AMD_STAGE_TOTAL = 4, /* first launch to last kernel end, device side */
     OPENFISH_AMD_STAGE_SCAN = 5,  /* both scans + posterior as one kernel (0 when they ran split) */
     OPENFISH_AMD_STAGE_SUMS = 6,  /* per-state sums of posteriors for the quality stage, a kernel that runs beside the
                                    * beam search on a second stream (0 when the decode did without it) */
-    OPENFISH_AMD_STAGE_COUNT = 7
+    OPENFISH_AMD_STAGE_FWD_SCAN = 7, /* forward scan by itself, beside the backward one on a second stream (1024 states, few
+                                      * chunks; 0 in every other decode) */
+    OPENFISH_AMD_STAGE_COUNT = 8
 };
 
 /*

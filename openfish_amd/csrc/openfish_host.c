@@ -120,8 +120,9 @@ void openfish_amd_lse_table(double *out) { build_lse_table(out); }
 
 #define OFA_MAGIC 0x6f66616d64677075ull /* "ofamdgpu" */
 
-enum { EV_JOIN, EV_START, EV_BWD_END, EV_BEAM_START, EV_BEAM_END, EV_FWD_END, EV_SEQ_START, EV_SEQ_END, EV_SUMS_START, EV_SUMS_END, EV_MOVES, EV_COUNT };
-/* with both sweeps in one kernel EV_BWD_END marks its end and EV_FWD_END is not recorded */
+enum { EV_JOIN, EV_START, EV_BWD_END, EV_BEAM_START, EV_BEAM_END, EV_FWD_END, EV_FWD_SCAN_END, EV_SEQ_START, EV_SEQ_END, EV_SUMS_START, EV_SUMS_END, EV_MOVES, EV_COUNT };
+/* with both sweeps in one kernel EV_BWD_END marks its end and EV_FWD_END is not recorded; EV_FWD_SCAN_END only where the forward sweep runs
+ * beside the backward one */
 
 /* arrangements of the scans: both sweeps in one kernel; backward sweep, then forward sweep beside the beam search;
  * backward sweep, then forward sweep within the beam search's kernel */
@@ -146,6 +147,7 @@ typedef struct {
     int pend_T, pend_N, pend_sums;    /* its shape */
     int pend_copy;         /* its moves travel by a copy on the side lane */
     int pend_split;        /* how its scans were queued (which events were recorded): ARR_* */
+    int pend_apart;        /* split, with the forward sweep beside the backward one */
     int scan_mode;         /* OFK_SCAN_*: arithmetic of the scans of this gpubuf's decodes */
     int scan_spl;          /* states per lane of the scans, 0 = chosen from the batch size */
     int debug_flags;       /* bit 0: serial replay of the beam search's merges; bit 1: colliding seed hashes */
@@ -562,6 +564,7 @@ static void enqueue_decode(ofa_gpubuf_t *g, const int T, const int N, const int 
     const int others = take_main_lane(g), shared = others || enqueued;
     const int search_flags = g->debug_flags | (shared ? 0 : OFK_SEARCH_ALONE);
     g->pend_split = arrangement_of(g, T, N, C, state_len, shared);
+    g->pend_apart = 0;
     /* Sums only where the search leaves the machine idle, and not with 1024 states, whose search waits for
      * memory and was measured to take half as long again beside the extra kernel.
      * With split scans the posteriors are complete when the forward kernel ends.  With 64 states that is
@@ -613,13 +616,14 @@ static void enqueue_decode(ofa_gpubuf_t *g, const int T, const int N, const int 
          * Whole calls, ms, sweep and posterior beside the search | apart: 1 chunk, T = 33 0.171 | 0.160; 8, T = 100 0.317 | 0.264;
          * T = 833: 1 1.48 | 1.23, 37 1.51 | 1.27, 64 1.52 | 1.31, 96 1.53 | 1.33; five columns, T = 1666: 80 2.67 | 2.51,
          * 96 2.68 | 2.57, 112 2.72 | 2.73, 128 2.82 | 2.85. */
-        const int apart = state_len == 5 && N <= 96 && !shared && g->scan_mode == OFK_SCAN_TWO_TIER && g->scan_spl == 0;
+        const int apart = g->pend_apart = state_len == 5 && N <= 96 && !shared && g->scan_mode == OFK_SCAN_TWO_TIER && g->scan_spl == 0;
         launch_ok(ofk_bwd_scan(scores_TNC, g->pub.bwd_NTC, T, N, state_len, cols, stay, g->scan_mode, g->scan_spl, g->s_main),
                   "bwd_scan");
         HIP_OK(hipEventRecord(g->ev[EV_BWD_END], g->s_main));
         if (apart) {
             HIP_OK(hipStreamWaitEvent(g->s_side, g->ev[EV_START], 0));
             launch_ok(ofk_fwd_scan(scores_TNC, g->pub.post_NTC, T, N, state_len, cols, stay, g->s_side), "fwd_scan");
+            HIP_OK(hipEventRecord(g->ev[EV_FWD_SCAN_END], g->s_side));
         }
 
         /* The beam search is the longer of the two stages that follow and wants its workgroups (large
@@ -729,6 +733,14 @@ int openfish_amd_last_timings(const openfish_gpubuf_t *gpubuf, float *ms, int n)
     } else {
         g->ms[OPENFISH_AMD_STAGE_BWD] = g->ms[OPENFISH_AMD_STAGE_FWD] = 0.0f;
         HIP_OK(hipEventElapsedTime(&g->ms[OPENFISH_AMD_STAGE_SCAN], g->ev[EV_START], g->ev[EV_BWD_END]));
+    }
+    g->ms[OPENFISH_AMD_STAGE_FWD_SCAN] = 0.0f;
+    if (g->pend_split == ARR_SPLIT && g->pend_apart) {
+        /* the posteriors' pass begins with the later of the two sweeps' ends */
+        float behind = 0.0f;
+        HIP_OK(hipEventElapsedTime(&g->ms[OPENFISH_AMD_STAGE_FWD_SCAN], g->ev[EV_START], g->ev[EV_FWD_SCAN_END]));
+        HIP_OK(hipEventElapsedTime(&behind, g->ev[EV_FWD_SCAN_END], g->ev[EV_FWD_END]));
+        if (behind < g->ms[OPENFISH_AMD_STAGE_FWD]) g->ms[OPENFISH_AMD_STAGE_FWD] = behind;
     }
     HIP_OK(hipEventElapsedTime(&g->ms[OPENFISH_AMD_STAGE_BEAM], g->ev[EV_BEAM_START], g->ev[EV_BEAM_END]));
     HIP_OK(hipEventElapsedTime(&g->ms[OPENFISH_AMD_STAGE_SEQ], g->ev[EV_SEQ_START], g->ev[EV_SEQ_END]));

@@ -34,6 +34,7 @@ SQ2_COUNTERS = ["SQ_WAVE_CYCLES", "SQ_WAIT_ANY", "SQ_ACTIVE_INST_ANY", "SQ_ACTIV
 SCAN_MODES = {"0": "two_tier", "1": "precise", "2": "fast"}
 # kernel function -> the stage name bench.py uses
 STAGE_OF = {"scan_post_kernel": "scan", "bwd_scan_kernel": "bwd", "fwd_post_kernel": "fwd_post", "fwd_post_roles_kernel": "fwd_post",
+            "fwd_scan_kernel": "fwd_scan", "posterior_rows_kernel": "fwd_post",
             "beam_kernel": "beam", "sequence_kernel": "sequence", "path_sums_kernel": "path_sums"}
 
 
@@ -169,7 +170,7 @@ def main():
                 continue
             cells = [("%.3g" % d[n]) if n in d else "-" for n in SQ_COUNTERS]
             if a.updates:
-                sweeps = {"scan": 2, "bwd": 1, "fwd_post": 1}.get(stage_of(k))
+                sweeps = {"scan": 2, "bwd": 1, "fwd_post": 0 if k.startswith("posterior_rows") else 1, "fwd_scan": 1}.get(stage_of(k))
                 cells.append("%.1f" % (d.get("SQ_INSTS_VALU", 0.0) * 64 / (sweeps * a.updates)) if sweeps else "-")
             out.append("| %s | " % k + " | ".join(cells) + " |")
         if a.updates:
@@ -199,7 +200,7 @@ def main():
                 k, wc, d.get("SQ_WAIT_ANY", 0.0), d.get("SQ_ACTIVE_INST_ANY", 0.0), d.get("SQ_ACTIVE_INST_LDS", 0.0),
                 d.get("SQ_INSTS_VALU_FMA_F64", 0.0), d.get("SQ_INSTS_VALU_TRANS_F32", 0.0), d.get("SQ_INSTS_BRANCH", 0.0),
                 share, per_simd, min(1.0, share * per_simd),
-                ("%.2f" % (d.get("SQ_INSTS_VALU_FMA_F64", 0.0) / (waves * steps))) if (steps and waves and stage_of(k) in ("scan", "bwd", "fwd_post")) else "-"))
+                ("%.2f" % (d.get("SQ_INSTS_VALU_FMA_F64", 0.0) / (waves * steps))) if (steps and waves and stage_of(k) in ("scan", "bwd", "fwd_post", "fwd_scan")) else "-"))
         if a.steps_per_wave:
             out.append("\nfp64 FMA per wave and time step = SQ_INSTS_VALU_FMA_F64 / (waves x T): the second tier of the default "
                        "arithmetic is the only user of fp64 in the scans, but for the 32 warm-up steps of either sweep in the "

@@ -36,3 +36,23 @@ def test_both_sweeps_at_once_leave_what_the_stages_leave(api, T, N, stay, column
         ref = O.decode(s16[:, :base].astype(np.float32), 5, dict(q_scale=0.95, q_shift=-0.2), nthreads=4)
         assert np.array_equal(bwd[:base], ref["bwd"])
         close(post[:base], ref["post"], atol=1.2e-38)
+
+
+def test_the_timings_tell_the_forward_sweep_from_the_posteriors_pass(api):  # noqa: F811
+    T, N, S = 400, 8, 1024
+    s16 = synth.crf_scores(T, N, 5, seed=3)
+    sc, gb, opt = api.upload_scores_to_hip(s16), api.GpuBuf(T, N, 5), api.DECODER_INIT()
+    gb.set_split_scans(True)
+    for _ in range(2):
+        api.openfish_decode_gpu(T, N, 4 * S, sc, 5, opt, gb)
+    t = gb.timings()
+    assert t["scan"] == 0 and 0 < t["fwd_post"] < t["fwd_scan"] < t["total"]  # a pass over rows against T dependent steps
+    for change in (lambda: gb.set_scan_states_per_lane(2), lambda: gb.set_split_scans(False)):
+        change()
+        api.openfish_decode_gpu(T, N, 4 * S, sc, 5, opt, gb)
+        assert gb.timings()["fwd_scan"] == 0
+    gb.set_scan_states_per_lane(0)
+    gb.set_split_scans(True)
+    api.openfish_amd_decode_enqueue(T, N, 4 * S, sc, 5, opt, gb)  # may share the device: no units of its own
+    api.openfish_amd_decode_wait(gb)
+    assert gb.timings()["fwd_scan"] == 0 and gb.timings()["fwd_post"] > 0
