@@ -233,8 +233,8 @@ void openfish_amd_gpubuf_set_debug_flags(const openfish_gpubuf_t *gpubuf, int fl
  *   64 states: 1 up to 2048 chunks, 0 beyond.
  *   256 states: alone 1 up to 512 chunks (five columns: 463), 2 for five columns up to 512, 1 up to 768,
  *     2 beyond; shared 2 up to 512, 1 up to 640, 2 beyond.
- *   1024 states: alone 1 up to 160 chunks and from 257 to 320, 2 elsewhere; shared 2; but 0 for fewer than 16, and
- *     alone for more than 320, chunks shorter than 128 steps.
+ *   1024 states: alone 1 up to 160 chunks and from 257 to 320, 2 elsewhere, but 0 for more than 320 chunks shorter than
+ *     128 steps and for fewer than 16 shorter than 6; shared 2, but 0 for fewer than 16 chunks shorter than 128 steps.
  */
 int openfish_amd_scan_arrangement(int T, int N, int C, int state_len, int shared);
 

@@ -490,36 +490,36 @@ static void join_null_stream(ofa_gpubuf_t *g) {
  *           the search's alone (256 states by 5 %, 1024 by 16 to 40 %), twice that with two rounds of workgroups;
  *   one     both sweeps of a chunk side by side from its two ends, then the search: the longest, with the fewest launches.
  * Whole blocking calls, ms, one | split | merged, T = 1666 unless stated, inputs and arrangements in turn; in all of them
- * the forward sweep of the split decodes was seen to run beside the search.
- *   1024 states: 16 chunks, T = 833 1.95 | 1.69 | 1.80;  37, T = 833 1.98 | 1.71 | 1.82;  128 3.76 | 3.15 | 3.34;
- *                160 3.81 | 3.19 | 3.38;  168 3.81 | 4.26 | 3.40;  192 3.87 | 4.28 | 3.39;  256 4.26 | 4.34 | 3.46;
- *                257 6.91 | 5.10 | 5.69;  320 6.95 | 5.63 | 5.79;  336 7.03 | 5.82 | 5.86;  400 7.28 | 7.74 | 6.03;
- *                five columns: 160 3.90 | 3.18 | 3.40;  256 4.55 | 4.80 | 3.54;  257 7.15 | 5.44 | 5.72;
- *                288 7.27 | 5.78 | 5.89;  304 7.30 | 5.95 | 5.90;  320 7.36 | 6.11 | 5.88;
- *                T = 833: 320 3.80 | 3.11 | 3.11;  T = 400: 320 1.89 | 1.58 | 1.67;
- *                T = 100: 16 0.352 | 0.363 | 0.380;  256 0.392 | 0.467 | 0.401;  352 0.621 | 0.643 | 0.613;  512 0.648 | 0.829 | 0.708;
- *                T = 128: 16 0.425 | 0.422 | 0.440;  512 0.797 | 0.971 | 0.823;  T = 200: 16 0.586 | 0.563 | 0.593
- *    256 states: 403 2.63 | 2.14 | 2.20;  512 2.77 | 2.26 | 2.31;  520 3.77 | 2.64 | 3.93;  700 4.09 | 3.71 | 4.25;
- *                768 4.18 | 3.79 | 4.31;  800 4.62 | 4.41 | 4.52;  1024 4.84 | 5.03 | 4.84;
- *                five columns: 456 2.77 | 2.24 | 2.27;  472 2.80 | 2.30 | 2.28;  488 2.83 | 2.42 | 2.33;  512 2.90 | 2.57 | 2.34;
- *                768 4.34 | 4.15 | 4.42;  784 4.70 | 4.63 | 4.51;  1024 5.03 | 5.54 | 4.93
- *     64 states: 16 1.83 | 1.58;  512 2.03 | 1.76;  2048 4.37 | 3.61
- * Hence the lines: up to 160 chunks of 1024 states the search (two chunks to a unit) and the forward sweep (one) find
+ * the forward sweep of the split decodes was seen to run beside the search (up to 96 chunks of 1024 states beside the backward sweep, see
+ * enqueue_decode).
+ *   1024 states: 16 chunks, T = 833 1.79 | 1.21 | 1.57;  96, T = 833 1.85 | 1.34 | 1.59;  97, T = 833 1.85 | 1.50 | 1.59;
+ *                128 3.49 | 2.69 | 2.83;  160 3.69 | 2.76 | 2.85;  168 3.71 | 3.51 | 2.85;  192 3.75 | 3.53 | 2.87;
+ *                256 4.10 | 3.92 | 3.00;  257 6.61 | 4.77 | 5.32;  320 6.70 | 5.32 | 5.38;  400 6.97 | 7.35 | 5.53;
+ *                five columns: 160 3.81 | 2.78 | 2.88;  256 4.42 | 4.37 | 3.21;  257 6.93 | 5.12 | 5.45;
+ *                288 7.04 | 5.44 | 5.52;  304 7.05 | 5.63 | 5.53;  320 7.07 | 5.79 | 5.56;
+ *                T = 833: 320 3.71 | 2.96 | 2.94;  T = 400: 320 1.86 | 1.48 | 1.58;
+ *                T = 1: 1 0.079 | 0.090 | 0.077;  T = 6: 8 0.099 | 0.098 | 0.092;  T = 33: 1 0.170 | 0.136 | 0.162;  T = 64: 8 0.241 | 0.188 | 0.235;
+ *                T = 100: 16 0.330 | 0.244 | 0.314;  256 0.376 | 0.377 | 0.341;  352 0.585 | 0.581 | 0.562;  512 0.598 | 0.691 | 0.613;
+ *                T = 128: 16 0.391 | 0.288 | 0.370;  512 0.740 | 0.843 | 0.736;  T = 200: 16 0.544 | 0.391 | 0.509
+ *    256 states: 403, T = 1201 1.88 | 1.47 | 1.50;  512 2.63 | 2.01 | 2.04;  513 3.59 | 3.03 | 3.44;  700 3.74 | 3.55 | 3.65;
+ *                768 3.83 | 3.68 | 3.72;  800 4.16 | 4.19 | 3.87;  1024 4.45 | 4.69 | 4.15;
+ *                five columns: 456 2.63 | 2.00 | 2.03;  472 2.67 | 2.05 | 2.06;  488 2.68 | 2.06 | 2.06;  512 2.77 | 2.12 | 2.10;
+ *                640 3.81 | 3.71 | 3.67;  768 3.97 | 3.88 | 3.78;  784 4.29 | 4.42 | 3.96;  1024 4.69 | 4.83 | 4.20
+ *     64 states: 16 1.68 | 1.41;  512 1.97 | 1.66;  2048 4.19 | 3.55
+ * Hence the lines: up to 160 chunks of 1024 states the search and the forward sweep find
  * compute units of their own; above 256 merged takes a second round of workgroups, split does so only above 320; chunks
- * shorter than 128 steps are decided by launches and set-up (up to 256 of them no arrangement was ahead by more than
- * 0.03 ms, and they take that of longer ones).  The figures are from before up to 96 chunks of 1024 states had their sweeps apart,
- * see enqueue_decode, which only split gains from (8 chunks, T = 100 0.345 | 0.264); up to 64 steps fewer than 16 of them keep the
- * one kernel because that choice is part of what is tested (1 chunk, T = 33 0.20 | 0.16).  Up to 512 chunks of 256 states the chain of split is
+ * shorter than 128 steps are decided by launches and set-up: split is ahead where it has its sweeps apart, but for the very
+ * shortest of few chunks, and one kernel above 320.  Up to 512 chunks of 256 states the chain of split is
  * shorter, while its bytes fit beneath the chain, 3.8 MB a step; above, the search's workgroups hold four chunks, a unit
- * that has one of them in the merged kernel takes 2.5 ms whatever the others do, and split has units left for the
+ * that has one of them in the merged kernel takes 2.3 ms whatever the others do, and split has units left for the
  * forward sweep up to three chunks to a unit.
  *
  * A decode that is enqueued, or finds another one under way, shares the machine; two at a time, one | split | merged:
- *   1024 states: 16, T = 833 1.99 | 2.48 | 1.84;  128 4.32 | 5.01 | 3.89;  256 five columns 8.44 | 8.55 | 6.40;
- *                320 10.27 | 10.07 | 8.16;  16, T = 100 0.38 | 0.50 | 0.41
- *    256 states: 128 2.64 | 2.35 | 2.07;  512 5.34 | 4.65 | 3.78;  520 5.69 | 4.78 | 5.70;  640 five columns 6.77 | 6.03 | 6.17;
- *                700 6.60 | 6.21 | 6.13 (one alone 3.83 | 3.24 | 4.05);  704 five columns 6.93 | 6.73 | 6.41;  768 five columns 7.45 | 7.07 | 6.57
- *     64 states: 512 3.19 | 2.75;  2048 8.10 | 6.91
+ *   1024 states: 16, T = 833 1.84 | 2.22 | 1.61;  128 3.87 | 4.14 | 2.96;  256 five columns 8.17 | 8.66 | 6.27;
+ *                320 9.85 | 9.73 | 7.40;  8, T = 64 0.28 | 0.33 | 0.27;  16, T = 100 0.36 | 0.44 | 0.35
+ *    256 states: 128 2.55 | 2.13 | 1.88;  512 5.30 | 4.42 | 3.60;  520 5.35 | 4.63 | 5.11;  640 five columns 6.47 | 5.57 | 5.62;
+ *                700 6.37 | 6.13 | 5.72;  704 five columns 6.63 | 6.30 | 5.91;  768 five columns 7.16 | 7.04 | 6.05
+ *     64 states: 512 3.13 | 2.71;  2048 7.66 | 6.49
  *
  * The merged kernel exists for 256 and 1024 states with the default arithmetic and its own states per lane; without it
  * (can_merge = 0) 1024 states keep the one kernel and 256 states the split sweeps where they are ahead of it. */
@@ -533,7 +533,7 @@ static int arrangement_by_default(int T, int N, int C, int state_len, int shared
             return N <= (shared ? 640 : 768) ? ARR_SPLIT : ARR_MERGED;
         default:
             if (!can_merge) return ARR_ONE;
-            if (T < 128 && ((N < 16 && (shared || T <= 64)) || (N > 320 && !shared))) return ARR_ONE;
+            if (T < 128 && ((N < 16 && (shared || T < 6)) || (N > 320 && !shared))) return ARR_ONE;
             if (shared) return ARR_MERGED;
             return N <= 160 || (N > 256 && N <= 320) ? ARR_SPLIT : ARR_MERGED;
     }

@@ -162,8 +162,8 @@ def test_whole_decode_on_golden(api, name):
             assert t["bwd"] > 0 and t["fwd_post"] > 0 and (t["path_sums"] > 0) == (sl == 3 and N <= 512)
         else:
             assert t["bwd"] == 0 and t["fwd_post"] == 0 and (t["path_sums"] > 0) == (sl <= 4 and N <= 512)
-        if split is None:  # small batches of up to 256 states run split
-            assert ran_split == (sl <= 4 and N * 4 ** sl <= 512 * 256)
+        if split is None:
+            assert ran_split == (api.scan_arrangement(T, N, C, sl) == 1)
         else:
             assert ran_split == split
 
