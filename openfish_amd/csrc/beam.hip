@@ -377,7 +377,7 @@ struct __attribute__((aligned(16))) FwdLds {
 template <int S>
 struct FwdLds<S, 0> {};
 struct FwdTables {
-    ofa::LogCell cells[32], centred[ofa::kLogCentredCells];
+    ofa::LogCell centred[ofa::kLogCentredCells];
 };
 struct NoTables {};
 template <int S, int COLS, int FWD>
@@ -507,11 +507,7 @@ __global__ __launch_bounds__((kBeamThreads<S, CPG, COLS, FWD>), (BeamCfg<S, FWD>
             lds[member].fwd.taken = 0;
         }
     }
-    if constexpr (FWD > 0) {
-        static_assert(kBeamThreads<S, CPG, COLS, FWD> >= 160, "the tables are filled by the first 160 threads");
-        fill_log_tables<OFK_SCAN_TWO_TIER>(all.logs.cells, all.logs.centred);
-        static_assert(ofa::kLogCentredCells <= 160, "one cell per thread");
-    }
+    if constexpr (FWD > 0) fill_log_tables<OFK_SCAN_TWO_TIER, kBeamThreads<S, CPG, COLS, FWD>>(nullptr, all.logs.centred);
     for (int x = (int)threadIdx.x; x < OFK_LSE_DOUBLES; x += kBeamThreads<S, CPG, COLS, FWD>) lse[x] = lse_table[x];
     // the hash index starts empty: no entry may look like one of a real generation (tags start at 1 << 5)
     for (int x = (int)threadIdx.x; x < kGroupChunks * BeamIdx<S, CPG, FWD>::kBuckets / 2; x += kBeamThreads<S, CPG, COLS, FWD>)
@@ -534,7 +530,7 @@ __global__ __launch_bounds__((kBeamThreads<S, CPG, COLS, FWD>), (BeamCfg<S, FWD>
             constexpr int SPL = S / (64 * FWD), Q = S / 4;
             const int w = (wave - kFirstFwd) % FWD;
             const int s0 = SPL * (64 * w + lane), q = s0 >> 2;
-            const LogArgs logtab{all.logs.cells, all.logs.centred, series.c, series.e, fw.tier_lanes + 64 * w, 3, 2};
+            const LogArgs logtab{nullptr, all.logs.centred, series.c, series.e, fw.tier_lanes + 64 * w, 3, 2};
             __builtin_amdgcn_s_setprio(2);
             float f[SPL];
 #pragma unroll
@@ -1096,7 +1092,7 @@ __global__ __launch_bounds__((kBeamThreads<S, CPG, COLS, FWD>), (BeamCfg<S, FWD>
                 next.rest1 = c1;
                 next.rests = cs;
             }
-                        auto put = [&](int slot, uint32_t hsh, uint32_t inf, float rst) {
+            auto put = [&](int slot, uint32_t hsh, uint32_t inf, float rst) {
                 uint32_t at_elem;
                 asm("v_lshl_add_u32 %0, %1, 4, %2" : "=v"(at_elem) : "v"(slot), "v"(elem_base));
                 u32x3 rec;

@@ -70,7 +70,7 @@ __device__ __forceinline__ double certificate_unit() {
     return k == 5 ? ofa::kProofLowerUnit : k == 6 ? ofa::kProofUpperUnit : 1.0;
 }
 struct LogArgs {
-    const ofa::LogCell *cells;    // 32 cells, for the always-double arithmetic
+    const ofa::LogCell *cells;    // 32 cells, for the always-double arithmetic; null in a kernel that never takes it
     const ofa::LogCell *centred;  // ofa::kLogCentredCells cells, for the two-tier updates
     const double *series;
     const double *expc;
@@ -101,11 +101,14 @@ struct LogArgs {
 // the second tier worked the results out (and took the logarithm in every trip) 245 | 740 | 975 | 985.  Together with the order
 // of a step (see lse5_all) the backward sweep at T = 1666 went from 0.44 to 0.39 ms (1 chunk of 64 states), 0.68 to 0.58 (1 of
 // 256), 0.85 to 0.74 (512 of 256), 1.54 to 1.43 (256 of 1024), the merged kernel of 1024 chunks of 256 states from 2.60 to 2.42.
-template <int MODE, bool WITH_PRECISE = false>
+// The tables that a kernel of THREADS threads reads, one cell a thread.
+template <int MODE, int THREADS, bool WITH_PRECISE = false>
 __device__ __forceinline__ void fill_log_tables(ofa::LogCell *cells, ofa::LogCell *centred) {
+    constexpr bool kCells = MODE == OFK_SCAN_PRECISE || WITH_PRECISE, kCentred = MODE == OFK_SCAN_TWO_TIER;
+    static_assert(THREADS >= (kCentred ? ofa::kLogCentredCells : 0) && (!kCells || THREADS >= 160), "a thread for every cell");
     const int tid = threadIdx.x;
-    if ((MODE == OFK_SCAN_PRECISE || WITH_PRECISE) && tid >= 128 && tid < 160) cells[tid - 128] = ofa::log_cell(tid - 128);
-    if (MODE == OFK_SCAN_TWO_TIER && tid < ofa::kLogCentredCells) centred[tid] = ofa::log_centred_cell(tid);
+    if (kCells && tid >= 128 && tid < 160) cells[tid - 128] = ofa::log_cell(tid - 128);
+    if (kCentred && tid < ofa::kLogCentredCells) centred[tid] = ofa::log_centred_cell(tid);
 }
 
 // lane k of the result: x_k of lane `lane`, for k = 0 .. 6 (x_0 in the other lanes).  v_readlane may read a

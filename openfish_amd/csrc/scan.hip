@@ -328,12 +328,13 @@ __global__ __launch_bounds__((Shape<S, SPL>::kThreads)) void bwd_scan_kernel(
     constexpr int H = 4 / SPL;  // lanes sharing one quad
     using Vec = BwdVec<S>;
     __shared__ __attribute__((aligned(16))) float vec[Sh::kChunks][2][Vec::kLen];
-    __shared__ __attribute__((aligned(16))) ofa::LogCell logcells[32], centred[ofa::kLogCentredCells];
+    __shared__ __attribute__((aligned(16))) ofa::LogCell logcells[MODE == OFK_SCAN_PRECISE ? 32 : 1], centred[ofa::kLogCentredCells];
     __shared__ __attribute__((aligned(16))) float tier_lanes[MODE == OFK_SCAN_TWO_TIER ? Sh::kThreads : 64];
     const int tid = threadIdx.x;
-    const LogArgs logtab{logcells, centred, series.c, series.e, tier_lanes + (MODE == OFK_SCAN_TWO_TIER ? (tid & ~63) : 0)};
+    const LogArgs logtab{MODE == OFK_SCAN_PRECISE ? logcells : nullptr, centred, series.c, series.e,
+                         tier_lanes + (MODE == OFK_SCAN_TWO_TIER ? (tid & ~63) : 0)};
 
-    fill_log_tables<MODE>(logcells, centred);
+    fill_log_tables<MODE, Sh::kThreads>(logcells, centred);
     const int g = tid / L, l = tid % L;
     const int r = l / H, c0 = (l % H) * SPL;  // own states: r + (c0 + i) * Q
     int n = blockIdx.x * Sh::kChunks + g;
@@ -426,14 +427,15 @@ __global__ __launch_bounds__((Shape<S, SPL>::kThreads)) void fwd_post_kernel(
     constexpr int Q = Sh::kQuarter;
     __shared__ __attribute__((aligned(16))) float vec[Sh::kChunks][2][S];
     __shared__ float part[2][Sh::kChunks][Sh::kChunkWaves];
-    __shared__ __attribute__((aligned(16))) ofa::LogCell logcells[32], centred[ofa::kLogCentredCells];
+    __shared__ __attribute__((aligned(16))) ofa::LogCell logcells[MODE == OFK_SCAN_PRECISE ? 32 : 1], centred[ofa::kLogCentredCells];
     __shared__ __attribute__((aligned(16))) float tier_lanes[MODE == OFK_SCAN_TWO_TIER ? Sh::kThreads : 64];
     const int tid = threadIdx.x;
     // this sweep runs beside the beam search, whose waves run at priority 3: trips through the second tier
     // at 1 leave that search alone (2048 chunks of 64 states: search 2.50 ms against 2.59 with 3 here)
-    const LogArgs logtab{logcells, centred, series.c, series.e, tier_lanes + (MODE == OFK_SCAN_TWO_TIER ? (tid & ~63) : 0), 1};
+    const LogArgs logtab{MODE == OFK_SCAN_PRECISE ? logcells : nullptr, centred, series.c, series.e,
+                         tier_lanes + (MODE == OFK_SCAN_TWO_TIER ? (tid & ~63) : 0), 1};
 
-    fill_log_tables<MODE>(logcells, centred);
+    fill_log_tables<MODE, Sh::kThreads>(logcells, centred);
     const int g = tid / L, l = tid % L;
     const int s0 = SPL * l, q = s0 >> 2;  // own states s0 .. s0+SPL-1, all in quad q
     const int wave = l / 64;  // wave within the chunk
@@ -567,7 +569,7 @@ __global__ __launch_bounds__((2 * (S / SPL))) void fwd_post_roles_kernel(
     static_assert(L % 64 == 0 && RW > 1, "either job owns several whole waves");
     __shared__ __attribute__((aligned(16))) float vec[2][S];
     __shared__ float part[2][RW];
-    __shared__ __attribute__((aligned(16))) ofa::LogCell logcells[32], centred[ofa::kLogCentredCells];
+    __shared__ __attribute__((aligned(16))) ofa::LogCell centred[ofa::kLogCentredCells];
     __shared__ __attribute__((aligned(16))) float tier_lanes[L];
     const int tid = threadIdx.x;
     const int posterior = __builtin_amdgcn_readfirstlane(tid / L);
@@ -575,9 +577,9 @@ __global__ __launch_bounds__((2 * (S / SPL))) void fwd_post_roles_kernel(
     // This kernel runs beside the beam search, whose waves run at priority 3, which trips through the second tier leave
     // alone.  The recursion, which is the chain, goes before the posterior (512 chunks of 256 states: 1.02 ms against 1.14
     // with both at 0, search beside it 1.09 against 1.11).
-    const LogArgs logtab{logcells, centred, series.c, series.e, tier_lanes + (l & ~63), 2, 1};
+    const LogArgs logtab{nullptr, centred, series.c, series.e, tier_lanes + (l & ~63), 2, 1};
     if (!posterior) __builtin_amdgcn_s_setprio(1);
-    fill_log_tables<OFK_SCAN_TWO_TIER>(logcells, centred);
+    fill_log_tables<OFK_SCAN_TWO_TIER, 2 * (S / SPL)>(nullptr, centred);
     const int s0 = SPL * l, q = s0 >> 2;  // own states s0 .. s0+SPL-1, all in quad q
     const int n = blockIdx.x;            // one chunk per workgroup
     const ptrdiff_t row_stride = (ptrdiff_t)N * kCols * S;
@@ -692,11 +694,11 @@ __global__ __launch_bounds__(S) void fwd_scan_kernel(const _Float16 *__restrict_
     constexpr int Q = S / 4;
     static_assert(S > 64, "a state to a lane, and several waves");
     __shared__ __attribute__((aligned(16))) float vec[2][S];
-    __shared__ __attribute__((aligned(16))) ofa::LogCell logcells[32], centred[ofa::kLogCentredCells];
+    __shared__ __attribute__((aligned(16))) ofa::LogCell centred[ofa::kLogCentredCells];
     __shared__ __attribute__((aligned(16))) float tier_lanes[S];
     const int s = threadIdx.x, q = s >> 2;
-    const LogArgs logtab{logcells, centred, series.c, series.e, tier_lanes + (s & ~63)};
-    fill_log_tables<OFK_SCAN_TWO_TIER>(logcells, centred);
+    const LogArgs logtab{nullptr, centred, series.c, series.e, tier_lanes + (s & ~63)};
+    fill_log_tables<OFK_SCAN_TWO_TIER, S>(nullptr, centred);
     const ptrdiff_t row_stride = (ptrdiff_t)N * kCols * S;
     const _Float16 *pre = scores + (size_t)blockIdx.x * kCols * S;
     float *frow = fwd + (size_t)blockIdx.x * (size_t)(T + 1) * S;
@@ -838,7 +840,7 @@ __global__ __launch_bounds__((FusedShape<S, SPL>::kThreads), 4) void scan_post_k
     const int tid = threadIdx.x;
     const LogArgs logtab{logcells, centred, series.c, series.e, tier_lanes + (MODE == OFK_SCAN_TWO_TIER ? (tid & ~63) : 0)};
 
-    fill_log_tables<MODE, MODE == OFK_SCAN_TWO_TIER>(logcells, centred);  // the first steps of either sweep take the always-double arithmetic
+    fill_log_tables<MODE, Sh::kThreads, MODE == OFK_SCAN_TWO_TIER>(logcells, centred);  // the first steps of either sweep take the always-double arithmetic
     const int g = tid / Sh::kChunkThreads, u = tid % Sh::kChunkThreads;
     const int forward = __builtin_amdgcn_readfirstlane(u / L);
     const int l = u % L, wave = l / 64;
