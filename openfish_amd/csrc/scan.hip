@@ -24,8 +24,9 @@
 //             sequence of roundings (fp64 FMA issues at the fp32 rate on gfx950);
 //   fast    : v_exp_f32 / v_log_f32, within an ulp or two of the precise result;
 //   two-tier: the fast value wherever it provably rounds like the precise one (its
-//             distance to a rounding boundary exceeds a bound on its error), the
-//             precise arithmetic for the remaining lanes.  Same bits as precise.
+//             distance to a rounding boundary exceeds a bound on its error, or the CPU
+//             path's running sum lies between its two boundaries), the logarithm of that
+//             sum for the rest.  Same bits as precise.
 // State values reach several thousand, where one fp32 ulp is already 5e-4, and
 // the posterior is exp(fwd + bwd - const): a last-bit difference in a scan shows
 // up as a 5e-4 relative difference of a posterior.  Two-tier is the default for
@@ -33,7 +34,8 @@
 //
 // Kernels: bwd_scan_kernel is the backward sweep; fwd_post_kernel and fwd_post_roles_kernel are the
 // forward sweep with the posterior, for a decode that runs it beside the beam search (the third place
-// for it, within the search's kernel, is in beam.hip); scan_post_kernel runs both sweeps of a chunk in one
+// for it, within the search's kernel, is in beam.hip); fwd_scan_kernel and posterior_rows_kernel are the same in two
+// steps, for few chunks of 1024 states; scan_post_kernel runs both sweeps of a chunk in one
 // workgroup, from both ends of the chunk towards the middle and on to the other end.  Which of them a
 // decode uses is decided by its shape (openfish_host.c).
 #include <hip/hip_runtime.h>
@@ -276,10 +278,10 @@ __device__ __forceinline__ void fwd_terms(float (&v)[SPL][5], const float (&f)[S
 
 // A step of the kernel that holds both sweeps and is capped at 128 registers.  Of four states to a lane the terms are
 // not kept for a common second tier (as in the separate sweeps, which may use 256 registers): that spilled inside the
-// loops.  One state after another in the backward sweep and two and two in the forward one needs no scratch with 256
+// loops.  One state after another needs no scratch with 256
 // states, and with 1024 only between the phases.  Scans of 2048 chunks of 256 states, T = 1666: 6.87 ms all four
-// together, 5.8 now (five columns 7.87, 5.8); 512 chunks of 1024 states 6.14, 5.4; with the batch spread over twice the
-// lanes 6.07, 6.15 and 5.82.
+// together, 5.7 now (five columns 7.87, 6.05); 512 chunks of 1024 states 6.14, 5.45; with the batch spread over twice the
+// lanes 5.65, 6.0 and 5.75.
 // `publish` writes the new values to LDS (lse5_all says when; with four states to a lane once all of them are there).
 template <int SPL, int MODE, typename Publish>
 __device__ __forceinline__ void bwd_update(float (&a)[SPL], const float4 &nx, const BwdRow<SPL> &row, float stay, const LogArgs &logtab,

@@ -204,7 +204,7 @@ __global__ __launch_bounds__(kThreads) void sequence_kernel(
 
 // ---------------------------------------------------------------------------------------------
 // For every chunk, time step and state: the posterior of the k-mer plus that of its distinct
-// one-base shifts, summed in the CPU path's order -- what step 1 of sequence_kernel gathers for
+// one-base shifts, summed in the CPU path's order -- what step 3 of sequence_kernel gathers for
 // the one state on the path.  Those nine scattered reads per time step fetch about half of the
 // posteriors, 64 bytes for every 4 wanted, and made up most of that kernel's time; they come
 // after the beam search, which leaves most of the machine idle for a millisecond.  This kernel
@@ -342,8 +342,8 @@ template <int S>
 int launch_sequence(const float *post, int32_t *states, const uint8_t *moves, float *qual_data,
                     float *base_probs, float *total_probs, char *sequence, char *qstring, int T, int N,
                     const ofk_phred_table_t &phred, const float *path_sums, uint8_t *moves_out, hipStream_t st) {
-    // Up to a chunk per compute unit a time step has a lane of its own, or two share one: the rounds of memory accesses are what
-    // is waited for.  Beyond, two workgroups of half the size fill a unit and one's gathers run beside the other's characters.
+    // Up to a chunk per compute unit, 960 gathering lanes (two time steps each at T = 1666, nine at 8192): the rounds of memory accesses
+    // are what is waited for.  Beyond, two workgroups of half the size fill a unit and one's gathers run beside the other's characters.
     // 1024 | 512 | 256 lanes, us: 16 chunks of 64 states 14 | 17 | 25, 256 of 1024 84 | 86 | 92, 512 of 256 131 | 129 | 145, 1024 of 256
     // 270 | 263 | 283.
     if (N <= 256)

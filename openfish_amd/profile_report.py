@@ -204,9 +204,9 @@ def main():
         if a.steps_per_wave:
             out.append("\nfp64 FMA per wave and time step = SQ_INSTS_VALU_FMA_F64 / (waves x T): the second tier of the default "
                        "arithmetic is the only user of fp64 in the scans, but for the 32 warm-up steps of either sweep in the "
-                       "kernel that holds both (70 fp64 FMA per wave, state of a lane and step).  A trip through it is 25 fp64 "
-                       "FMA with one state to a lane and 21 with more; where many lanes need it (the first few hundred steps) "
-                       "it takes 70 for every state of a lane at once.")
+                       "kernel that holds both (70 fp64 FMA per wave, state of a lane and step).  A trip through it is 16 fp64 "
+                       "FMA for a single unsettled update and 12 for up to eight, 9 more where a proof fails; where many lanes need "
+                       "it (the first hundred steps) it takes 69 for every state of a lane at once.")
 
     log = first(os.path.join(base, "trace.log"))
     if log:
