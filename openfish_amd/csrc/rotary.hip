@@ -7,7 +7,7 @@
 // sums are separate fp32 operations (no fused multiply-add), the result is rounded
 // to half once.  The op is pure streaming; what bounds it is how whole the pieces are
 // that a wave asks memory for:
-//   rows    rotary_half a power of two from 8 to 256: a wave's loads and stores are whole lines;
+//   rows    rotary_half a power of two from 8 to 64: a wave's loads and stores are whole lines;
 //   vec8    other multiples of 8, single and short batches: 8 pairs per thread with 128-bit loads and stores;
 //   narrow  everything else: 4, 2 or 1 pairs per thread.
 #include <hip/hip_runtime.h>
@@ -64,7 +64,7 @@ struct __attribute__((aligned(16))) Table8 {
 // 2 rotary_half bytes.  Two batches to a lane share the sines and cosines, which are twice what it reads of x, and keep as
 // much in flight as a lane of rotary_vec8_kernel does.  500 x 833 x 8 heads of 64: 165 us -> 144 (5.9 TB/s; one batch to a
 // lane 150, four 149); heads of 32, 500 x 400 x 8: 41 -> 36; 31 x 833 x 8 heads of 64: 13.1 -> 12.1;
-// 1000 x 833 heads of 256: 162 -> 150; heads of 128, whose pieces are lines already: 144 -> 143.
+// heads of 128, whose pieces are lines already: 144 -> 143.
 __global__ __launch_bounds__(256) void rotary_rows_kernel(_Float16 *__restrict__ x, const float *__restrict__ sin_buf,
                                                           const float *__restrict__ cos_buf, unsigned per_batch, int batch,
                                                           unsigned nheads, int log_lanes, int rotary_half, long stride_batch,
@@ -161,11 +161,13 @@ extern "C" int ofk_rotary_emb(void *x, const float *sin_buf, const float *cos_bu
     const unsigned long apart = (unsigned long)rotary_half | (unsigned long)stride_batch | (unsigned long)stride_seq | (unsigned long)stride_head;
     const uintptr_t data = reinterpret_cast<uintptr_t>(x), tables = reinterpret_cast<uintptr_t>(sin_buf) | reinterpret_cast<uintptr_t>(cos_buf);
     if (apart % 8 == 0 && data % 16 == 0 && tables % 16 == 0) {
-        // Rows: heads that divide a wave, batches for every lane to have two (3 x 1700 x 12 heads of 64: 5.2 us | 5.3), and batches whose last workgroup's idle lanes are few
-        // beside the rest (500 x 1700 heads of 16, 14 workgroups for 3400 lanes a batch: 15.3 us | 13.2; 70000 batches of
-        // 2 lanes 3.5 | 17.8).  Batches that fit the launch's own time take the same either way.
+        // Rows: heads of up to 128, batches for every lane to have two (3 x 1700 x 12 heads of 64: 5.2 us | 5.3), and batches whose last
+        // workgroup's idle lanes are few beside the rest (500 x 1700 heads of 16, 14 workgroups for 3400 lanes a batch: 15.3 us | 13.2;
+        // 70000 batches of 2 lanes 3.5 | 17.8).  Batches that fit the launch's own time take the same either way.  Larger heads gain
+        // nothing in general: whole calls, us, vec8 | rows, heads of 256: 100 x 833 x 4 61.5 | 65.0, 500 x 833 71.8 | 74.4, 500 x 833 x 4 300 | 308,
+        // 16 x 1700 x 12 63.9 | 63.1, 1000 x 833 174 | 161; heads of 512: 64 x 833 x 8 158.8 | 162.9, 500 x 833 175 | 160.
         const unsigned __int128 per_batch = (unsigned __int128)((unsigned long)seqlen * (unsigned long)nheads) * (unsigned)(rotary_half / 4);
-        if (rotary_half >= 8 && rotary_half <= 256 && (rotary_half & (rotary_half - 1)) == 0 && batch >= 4 && per_batch >= 2048 && per_batch <= 0xffffff00u) {
+        if (rotary_half >= 8 && rotary_half <= 64 && (rotary_half & (rotary_half - 1)) == 0 && batch >= 4 && per_batch >= 2048 && per_batch <= 0xffffff00u) {
             const unsigned n = (unsigned)per_batch;
             const long pairs = ((long)batch + 1) / 2;
             hipLaunchKernelGGL(rotary_rows_kernel, dim3((n + 255) / 256, (unsigned)(pairs < 65535 ? pairs : 65535)), dim3(256), 0, st,
