@@ -196,7 +196,7 @@ typedef float f32x2 __attribute__((ext_vector_type(2)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 #define LDS_AS __attribute__((address_space(3)))
 __device__ __forceinline__ f32x2 lds_load_f2(uint32_t at) { return *(const LDS_AS f32x2 *)(uintptr_t)at; }
-__device__ __forceinline__ u32x2 lds_load_u2(uint32_t at) { return *(const LDS_AS u32x2 *)(uintptr_t)at; }
+
 __device__ __forceinline__ float lds_load_f(uint32_t at) { return *(const LDS_AS float *)(uintptr_t)at; }
 __device__ __forceinline__ void lds_store_f2(uint32_t at, float a, float b) {
     f32x2 v;
@@ -266,17 +266,22 @@ __device__ __forceinline__ float log_sum_exp(float x, float y, const double *tab
 // the fused multiply-add, taken exactly with a second one).  Half an ulp is 2^-24 of the binade of the
 // float below r in magnitude (r (1 - 2^-24), rounded: for a power of two it lies in the binade below, where its nearer
 // boundary is; every other float stays in its own); results below 2^-102 in magnitude never count as settled.
-__device__ __forceinline__ float log_sum_exp_estimate(float x, float y, bool &settled) {
+struct FoldValue {
+    float value, top, l2;
+};
+__device__ __forceinline__ FoldValue log_sum_exp_value(float x, float y) {
     const float gap = fabsf(x - y);
-    const float top = x > y ? x : y;
+    FoldValue f;
+    f.top = x > y ? x : y;
     const float e = __builtin_amdgcn_exp2f(gap * -1.44269504088896340736f);
-    const float l2 = __builtin_amdgcn_logf(1.0f + e);
-    const float kLn2 = 0.69314718055994530942f;
-    const float r = __builtin_fmaf(l2, kLn2, top);
-    const float rho = __builtin_fmaf(l2, kLn2, -(r - top));
-    const float binade = __uint_as_float(__float_as_uint(r * 0x1.fffffep-1f) & 0x7f800000u);
-    settled = __builtin_fmaf(binade, 0x1p-24f, -fabsf(rho)) > 4.0f * 0x1p-24f;
-    return r;
+    f.l2 = __builtin_amdgcn_logf(1.0f + e);
+    f.value = __builtin_fmaf(f.l2, 0.69314718055994530942f, f.top);
+    return f;
+}
+__device__ __forceinline__ bool log_sum_exp_settled(FoldValue f) {
+    const float rho = __builtin_fmaf(f.l2, 0.69314718055994530942f, -(f.value - f.top));
+    const float binade = __uint_as_float(__float_as_uint(f.value * 0x1.fffffep-1f) & 0x7f800000u);
+    return __builtin_fmaf(binade, 0x1p-24f, -fabsf(rho)) > 4.0f * 0x1p-24f;
 }
 
 __device__ __forceinline__ uint32_t float_key(float f) {
@@ -285,6 +290,14 @@ __device__ __forceinline__ uint32_t float_key(float f) {
 }
 __device__ __forceinline__ float key_float(uint32_t k) {
     return __uint_as_float(k ^ ((k >> 31) ? 0x80000000u : 0xFFFFFFFFu));
+}
+
+template <int N, int FIRST = 0, typename F>
+__device__ __forceinline__ void static_for_upwards(F &&f) {
+    if constexpr (FIRST < N) {
+        f(std::integral_constant<int, FIRST>{});
+        static_for_upwards<N, FIRST + 1>(f);
+    }
 }
 
 template <int BYTES>
@@ -323,12 +336,15 @@ struct RowRegs {
 
 
 // FWD is the number of waves per chunk that run the forward recursion beside the search (0: the search alone).
-template <int S, int FWD>
+template <int S, int CPG, int FWD>
 struct BeamCfg {
     static constexpr int kBits = S == 64 ? 6 : S == 256 ? 8 : 10;
     // two waves of recursion at 256 states is the choice for two workgroups per compute unit: 80 KB of LDS each
     static constexpr bool kDense = FWD == 2;
-    static constexpr int kLdsRows = FWD == 0 ? (S >= 1024 ? 3 : S >= 256 ? 4 : 6) : (kDense ? 3 : 4);  // LDS ring depth
+    // LDS ring depth, which is also how many time steps of the search are written out one after another.  Four, but for two chunks of
+    // 1024 states to a unit that they share with the forward sweep, and where two workgroups share it.
+    static constexpr int kLdsRows = kDense || (S >= 1024 && CPG > 1) ? 3 : 4;
+    static constexpr int kHandBack = FWD == 0 && kLdsRows == 4 ? 2 : 1;  // rows the search asks for and gives back at a time
     static constexpr int kRegRows = S >= 1024 ? (FWD == 0 ? 3 : 2) : (kDense ? 3 : 6);  // rows in flight in registers (2, 3 or 6)
 };
 
@@ -344,7 +360,6 @@ struct __attribute__((aligned(16))) Elem {
 
 struct BeamShared {
     Elem elem[kW + 64];           // slots 0 .. kW-1; entry kW + lane is lane's dump slot for candidates that are not kept
-    float cand[4 * kW + 64];      // scores of the step candidates 4i+b while stays merge into them; then dump slots
     float stay_score[kW];         // only used by the serial replay of merges
     uint32_t claim[4 * kW + 64];  // only used when the hash index was not conclusive: who claimed step candidate 4j+b
     int ready;                    // rows stored by the loader wave
@@ -353,17 +368,26 @@ struct BeamShared {
 
 // LDS of one chunk.  Score rows are kept as the caller lays them out: COLS = 4 transitions per
 // state, or 5 with an unused blank first.
-template <int S, int COLS, int FWD>
+template <int S, int CPG, int COLS, int FWD>
 struct __attribute__((aligned(16))) BeamRing {
-    _Float16 row_s[BeamCfg<S, FWD>::kLdsRows][COLS * S];
-    float row_b[BeamCfg<S, FWD>::kLdsRows][S];
+    _Float16 row_s[BeamCfg<S, CPG, FWD>::kLdsRows][COLS * S];
+    float row_b[BeamCfg<S, CPG, FWD>::kLdsRows][S];
 };
-// Buckets of the hash index of one chunk (8 bytes each: hash, generation << 5 | slot).  With w
-// live elements two of them share a bucket in about w^2 / (2 * buckets) of the time steps.
+// Hash index of one chunk: 2^kBits buckets of one word.  Hash bits 2 .. kBits + 1 are the bucket's byte address; in the entry
+// their place is free for the element's slot (bits 4 .. 8) and the generation (bits 2, 3 and 9 .. kBits + 1), so that one word
+// holds all that a look-up has to compare, and what is left of the comparison with the entry looked for is the partner's slot.
+// (Two words an entry, hash and generation << 5 | slot, took half the buckets, two more comparisons and 12 more LDS cycles a step.)
+// Low two bits of the generation: the ring slot of the time step; the rest counts ring rounds from 1, and when it is
+// used up the search's wave clears the table (about 6 cycles a step).  With w live elements two of them share a bucket in about
+// w^2 / (2 * buckets) of the time steps.
 template <int S, int CPG, int FWD>
 struct BeamIdx {
     static constexpr bool kLone = CPG == 1 && FWD == 0;  // a compute unit's LDS for one chunk
-    static constexpr int kBuckets = kLone ? (S >= 1024 ? 8192 : 16384) : (S >= 1024 || CPG > 2 || BeamCfg<S, FWD>::kDense) ? 2048 : 4096;
+    static constexpr int kBits = kLone ? 14 : (BeamCfg<S, CPG, FWD>::kDense || CPG > 2 || (S >= 1024 && FWD == 0)) ? 12 : 13;
+    static constexpr int kBuckets = 1 << kBits;
+    static constexpr uint32_t kAddress = (uint32_t)(kBuckets - 1) << 2;  // hash bits that address a bucket
+    static constexpr uint32_t kSlot = 31u << 4;
+    static constexpr uint32_t kRound = 1u << 9, kRoundEnd = 1u << (kBits + 2);
 };
 // What the forward recursion and the posterior of a chunk share.
 constexpr int kVecRows = 4;  // two would do (see beam_kernel); four let the posterior lag (1024 chunks of 256 states: 2.66 ms against 2.78)
@@ -380,19 +404,26 @@ struct FwdTables {
     ofa::LogCell centred[ofa::kLogCentredCells];
 };
 struct NoTables {};
-template <int S, int COLS, int FWD>
+template <int S, int CPG, int COLS, int FWD>
 struct __attribute__((aligned(16))) BeamLds {
-    BeamRing<S, COLS, FWD> ring;
+    BeamRing<S, CPG, COLS, FWD> ring;
     BeamShared sh;
-    uint2 idx_dump[64];  // where a dead lane files its leftovers instead of a bucket of the index
+    uint32_t idx_dump[64];  // where a dead lane files its leftovers instead of a bucket of the index
     FwdLds<S, FWD> fwd;
+};
+// scores of the step candidates 4i+b while stays merge into them, aligned so that a candidate's address is put together by `or`;
+// then a slot for every lane whose stay has no partner to write to
+struct __attribute__((aligned(512))) BeamCand {
+    float step[4 * kW];
+    float dump[64];
 };
 // All LDS of a workgroup, one object: the index tables come first and each is aligned to its
 // size, so that a bucket's address is (hash & bits) | table, one instruction.
 template <int S, int CPG, int COLS, int FWD>
 struct __attribute__((aligned(16))) BeamGroupLds {
-    uint2 idx[CPG][BeamIdx<S, CPG, FWD>::kBuckets];
-    BeamLds<S, COLS, FWD> chunk[CPG];
+    uint32_t idx[CPG][BeamIdx<S, CPG, FWD>::kBuckets];
+    BeamCand cand[CPG];
+    BeamLds<S, CPG, COLS, FWD> chunk[CPG];
     double lse[OFK_LSE_DOUBLES];  // coefficient table of the folds, one copy per workgroup
     typename std::conditional<FWD == 0, NoTables, FwdTables>::type logs;
 };
@@ -466,20 +497,21 @@ struct LdsRow {
 template <int S, int CPG, int COLS, int FWD>
 constexpr int kBeamThreads = BeamIdx<S, CPG, FWD>::kLone ? 256 : 64 * CPG * (FWD == 0 ? 2 : FWD + 3);  // a lone chunk: two waves more for the set-up
 template <int S, int CPG, int COLS, int FWD>
-__global__ __launch_bounds__((kBeamThreads<S, CPG, COLS, FWD>), (BeamCfg<S, FWD>::kDense ? 5 : 1)) void beam_kernel(const _Float16 *__restrict__ scores,
+__global__ __launch_bounds__((kBeamThreads<S, CPG, COLS, FWD>), (BeamCfg<S, CPG, FWD>::kDense ? 5 : 1)) void beam_kernel(const _Float16 *__restrict__ scores,
                                                    const float *__restrict__ bwd, float *__restrict__ post,
                                                    ofk_beam_slot_t *__restrict__ beam,
                                                    int32_t *__restrict__ states, uint8_t *__restrict__ moves,
                                                    int T, int N, float log_cut, float stay, int flags,
                                                    const double *__restrict__ lse_table, LogSeries series) {
-    using Cfg = BeamCfg<S, FWD>;
+    using Cfg = BeamCfg<S, CPG, FWD>;
+    using Idx = BeamIdx<S, CPG, FWD>;
     constexpr int BITS = Cfg::kBits;
     constexpr int LR = Cfg::kLdsRows;
     constexpr int RR = Cfg::kRegRows;
 
     constexpr int kGroupChunks = CPG;
     // bytes, so that the size is not rounded up to the alignment the index tables want
-    __shared__ __attribute__((aligned(BeamIdx<S, CPG, FWD>::kBuckets * 8))) unsigned char
+    __shared__ __attribute__((aligned(Idx::kBuckets * 4))) unsigned char
         lds_bytes[sizeof(BeamGroupLds<S, CPG, COLS, FWD>)];
     auto &all = *reinterpret_cast<BeamGroupLds<S, CPG, COLS, FWD> *>(lds_bytes);
     auto &lds = all.chunk;
@@ -509,12 +541,12 @@ __global__ __launch_bounds__((kBeamThreads<S, CPG, COLS, FWD>), (BeamCfg<S, FWD>
     }
     if constexpr (FWD > 0) fill_log_tables<OFK_SCAN_TWO_TIER, kBeamThreads<S, CPG, COLS, FWD>>(nullptr, all.logs.centred);
     for (int x = (int)threadIdx.x; x < OFK_LSE_DOUBLES; x += kBeamThreads<S, CPG, COLS, FWD>) lse[x] = lse_table[x];
-    // the hash index starts empty: no entry may look like one of a real generation (tags start at 1 << 5)
-    for (int x = (int)threadIdx.x; x < kGroupChunks * BeamIdx<S, CPG, FWD>::kBuckets / 2; x += kBeamThreads<S, CPG, COLS, FWD>)
+    // the hash index starts empty: no entry may look like one of a real generation (their rounds start at 1)
+    for (int x = (int)threadIdx.x; x < kGroupChunks * Idx::kBuckets / 4; x += kBeamThreads<S, CPG, COLS, FWD>)
         reinterpret_cast<uint4 *>(&all.idx[0][0])[x] = make_uint4(0u, 0u, 0u, 0u);
     __syncthreads();
     if (n >= N) return;  // odd batch: the last group has one chunk
-    if (BeamIdx<S, CPG, FWD>::kLone && wave > kFirstLoader) return;
+    if (Idx::kLone && wave > kFirstLoader) return;
 
     static_assert((FWD & (FWD - 1)) == 0 && FWD <= 64, "a lane reads one wave's counter");
     if constexpr (FWD > 0) {
@@ -684,8 +716,6 @@ __global__ __launch_bounds__((kBeamThreads<S, CPG, COLS, FWD>), (BeamCfg<S, FWD>
     // ---- search wave ----
     const int i = lane >> 1;  // lanes 2i and 2i+1 hold element i; candidate order is lane order
     const int h = lane & 1;
-    constexpr int kBuckets = BeamIdx<S, CPG, FWD>::kBuckets;
-    constexpr uint32_t kBucketBits = (uint32_t)(kBuckets - 1) << 3;  // hash bits that address an 8-byte bucket
     typedef __attribute__((address_space(3))) uint32_t lds_u32;
     // LDS addresses of this chunk's index table (a multiple of its size) and of this lane's spare entry
     const uint32_t idx_base = lds_address(&all.idx[member][0]);
@@ -751,7 +781,7 @@ __global__ __launch_bounds__((kBeamThreads<S, CPG, COLS, FWD>), (BeamCfg<S, FWD>
     const uint32_t from = (uint32_t)i << 10, from_stay = from | (1u << 15);  // the element's index as "prev" of its candidates
     int rows_ready = 0;  // last value seen of the loader's counter; it is usually several rows ahead
     const int b0 = 2 * h;
-    const uint32_t cand_base = lds_address(&sh.cand[0]);
+    const uint32_t cand_base = lds_address(&all.cand[member].step[0]);
     const uint32_t elem_base = lds_address(&sh.elem[0]);
     const uint32_t cand_mine = cand_base + 8u * (uint32_t)lane;           // candidates 4i+b0, 4i+b0+1
     const uint32_t cand_dump = cand_base + 4u * (uint32_t)(4 * kW + lane);  // where a stay without a partner writes
@@ -762,45 +792,65 @@ __global__ __launch_bounds__((kBeamThreads<S, CPG, COLS, FWD>), (BeamCfg<S, FWD>
     uint32_t r0h, r1h;  // fp16 scores of the lane's two step candidates, each in the low half of a word
     f32x2 g01;
     float gst;
-    u32x2 probe;     // index entry found under `want`
-    uint32_t mine_back;  // tag found under the element's own hash
-    uint32_t tagv;   // generation << 5 | slot of this element (generation = time step + 1)
-    uint64_t vm = ~0ull;  // lanes of live elements
+    uint32_t probe;      // index entry found under `want`
+    uint32_t expected;   // what it is if a partner is there, but for the partner's slot
+    uint32_t entry, mine_back;  // the element's own entry, as written and as found again
+    uint64_t vm = ~0ull, vs = 0x5555555555555555ull;  // lanes of live elements; of their stay candidates, which sit on the even lanes
+    const int i_stay = h == 0 ? i : kW;  // of an odd lane never below the beam's width
+    uint32_t hash_keep = ~Idx::kAddress, slot_bits = Idx::kSlot;
+    asm volatile("" : "+v"(hash_keep), "+v"(slot_bits));  // a vector instruction takes one scalar operand
+    const uint32_t slot_tag = (uint32_t)i << 4;
+    uint32_t round = 0;  // generation of the present ring round
     // ring addresses: the same in every lane, kept in scalar registers
     const uint32_t ring_s = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uintptr_t)(lds_u32 *)&row_s[0][0]);
     const uint32_t ring_b = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uintptr_t)(lds_u32 *)&row_b[0][0]);
-    auto wait_row = [&](int tt) {
-        while (__builtin_expect(rows_ready <= tt, 0)) {  // the counter is one LDS word: the same value in every lane
+    // The ring slot of a time step's row is known where steps are written out (K), elsewhere (K < 0) it is worked out.
+    auto ring_slot = [&](int tt, auto k_tag) {
+        constexpr int K = decltype(k_tag)::value;
+        return K >= 0 ? (uint32_t)K : (uint32_t)tt % (uint32_t)LR;
+    };
+    auto wait_row = [&](int tt, auto k_tag) {
+        constexpr int K = decltype(k_tag)::value;
+        if constexpr (K >= 0 && K % Cfg::kHandBack != 0) return;
+        int rows = tt + (K >= 0 ? Cfg::kHandBack : 1);
+        rows = rows < T ? rows : T;
+        while (__builtin_expect(rows_ready < rows, 0)) {  // the counter is one LDS word: the same value in every lane
             rows_ready = __builtin_amdgcn_readfirstlane(observe(&sh.ready));
-            if (rows_ready <= tt) __builtin_amdgcn_s_sleep(1);
+            if (rows_ready < rows) __builtin_amdgcn_s_sleep(1);
         }
     };
-    // ring addresses of row tt, worked out ahead of the wait for the beam they are used with
-    uint32_t rs, rb;
-    auto locate_row = [&](int tt) {
-        const uint32_t slot = (uint32_t)tt % (uint32_t)LR;
-        rs = ring_s + slot * (uint32_t)(2 * COLS * S);
-        rb = ring_b + slot * (uint32_t)(4 * S);
-        asm volatile("" : "+s"(rs), "+s"(rb));
+    auto next_round = [&](uint32_t slot) {
+        if (slot != 0) return;
+        round += Idx::kRound;
+        if (__builtin_expect(round == Idx::kRoundEnd, 0)) {
+            round = Idx::kRound;
+            typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+            u32x4 none;
+            none.x = none.y = none.z = none.w = 0u;
+#pragma unroll 1
+            for (uint32_t at = 0; at < 4u * Idx::kBuckets; at += 1024u) *(LDS_AS u32x4 *)(uintptr_t)(idx_base + at + 16u * (uint32_t)lane) = none;
+            wave_fence();
+        }
     };
-    auto fetch_row = [&](int tt) {
+    auto fetch_row = [&](int tt, auto k_tag) {
+        const uint32_t slot = ring_slot(tt, k_tag);
+        const uint32_t gen = round | (slot << 2);
         // hash index of the beam this step starts from; dead lanes file their leftovers apart
-        tagv = ((uint32_t)(tt + 1) << 5) | (uint32_t)i;
-        const uint32_t own = (uint32_t)pick_by_bit(vm, (int)and_or(hash, kBucketBits, idx_base), (int)idx_dump);
+        const uint32_t own = (uint32_t)pick_by_bit(vm, (int)and_or(hash, Idx::kAddress, idx_base), (int)idx_dump);
+        entry = and_or(hash, hash_keep, slot_tag | gen);
         lds_u32 *own_p = (lds_u32 *)(uintptr_t)own;
-        own_p[0] = hash;
-        own_p[1] = tagv;
+        own_p[0] = entry;
         __builtin_amdgcn_sched_barrier(0);  // the entries go out first, the row is asked for next: `want` takes a while
         wave_fence();  // one wave's LDS operations are carried out in order: the reads below see every lane's entry
         // scores of the candidates with bases b0, b0 + 1: rs[COLS * (lo4 + b0 + {0,1}) + (COLS - 4) + top];
         // guide terms rb[lo4 + b0 + {0,1}] and rb[state]
         const uint32_t st4 = (uint32_t)state << 2;
         const uint32_t cand = and_or(st4, (uint32_t)(S - 1), (uint32_t)b0);  // lo4 + b0
-        const uint32_t top = ((uint32_t)state >> (BITS - 2)) << 1;  // byte offset of the dropped base's column
+        const uint32_t top = (uint32_t)state >> (BITS - 2);                    // column of the dropped base
+        const uint32_t rs = ring_s + slot * (uint32_t)(2 * COLS * S), rb = ring_b + slot * (uint32_t)(4 * S);
         uint32_t at_s;
-        if constexpr (COLS == 4) at_s = (cand << 3) + rs;
-        else at_s = cand * 10u + rs;
-        at_s += top;
+        if constexpr (COLS == 4) at_s = (((cand << 2) | top) << 1) + rs;
+        else at_s = cand * 10u + (top << 1) + rs;
         typedef __attribute__((address_space(3))) uint16_t lds_u16;
         r0h = *(const lds_u16 *)(uintptr_t)(at_s + 2u * (COLS - 4));
         r1h = *(const lds_u16 *)(uintptr_t)(at_s + 2u * (COLS - 4) + 2u * COLS);
@@ -808,12 +858,14 @@ __global__ __launch_bounds__((kBeamThreads<S, CPG, COLS, FWD>), (BeamCfg<S, FWD>
         gst = lds_load_f(st4 + rb);
         __builtin_amdgcn_sched_barrier(0);
         want = crc2_inverse(hash, (uint32_t)state & 3u);
-        probe = lds_load_u2(and_or(want, kBucketBits, idx_base));
-        mine_back = own_p[1];
+        probe = *(const lds_u32 *)(uintptr_t)and_or(want, Idx::kAddress, idx_base);
+        mine_back = own_p[0];
+        expected = and_or(want, hash_keep, gen);
     };
-    wait_row(0);
-    locate_row(0);
-    fetch_row(0);
+    typedef std::integral_constant<int, -1> AnySlot;
+    wait_row(0, AnySlot{});
+    next_round(0);
+    fetch_row(0, AnySlot{});
     const uint64_t replay_all = (flags & 1) ? ~0ull : 0ull;
     ofk_beam_slot_t *bv_row = bv;  // row t of the persisted slots
     // One time step.  The last one (LAST) differs in what it hands on (nothing is fetched for a next
@@ -825,24 +877,25 @@ __global__ __launch_bounds__((kBeamThreads<S, CPG, COLS, FWD>), (BeamCfg<S, FWD>
     // nothing is placed into (about 1310 cycles for 1 chunk of 64 or 256 states: 0.94 ms at T = 1666; in the order of the
     // text, with every wait where its value is first needed, 1.02 ms).  Hence the order below: what does not depend on a round trip is issued
     // while it is under way, comparisons are issued in groups whose masks are read afterwards.
-    auto step = [&](const int next_t, auto last_tag) {  // next_t - 1 is the time step
+    auto step = [&](const int next_t, auto k_tag, auto last_tag) {  // next_t - 1 is the time step, K the ring slot of row next_t
+        constexpr int K = decltype(k_tag)::value;
         constexpr bool LAST = decltype(last_tag)::value;
-        const uint64_t vs = vm & 0x5555555555555555ull;  // the stay candidates sit on the even lanes
         // (score + transition) + guide, the CPU path's order of additions; the fp16 transition is
         // converted inside the first addition
         float c0 = add_half(r0h, score) + g01.x;
         float c1 = add_half(r1h, score) + g01.y;
-        float cs = (score + stay_h) + gst;
+        float cs0 = (score + stay_h) + gst;
         lds_store_f2(cand_mine, c0, c1);  // for the merges below
-        const uint32_t gen = (uint32_t)next_t << 5;
+        const uint32_t step_at = and_or((uint32_t)state << 2, 12u, cand_base);  // the partner is step candidate 4j + last base of this element
 
         // which previous element j has hash_j == want_i: off the index if every live element found its
         // own entry intact, else by comparing with every hash
-        const uint32_t d = probe.y - gen;  // below 32: an entry of this generation, and d is its slot
-        const uint64_t moved = ballot(mine_back != tagv), recent = ballot(d < 32u), equal = ballot(probe.x == want);
-        uint32_t j = d & 31u;
-        uint64_t mine_mask = recent & equal & vs;  // live even lanes whose stay has a partner
-        if (__builtin_expect(((moved & vm) | replay_all) != 0, 0)) {
+        const uint32_t d = probe ^ expected;  // the partner's slot and nothing else, if there is a partner
+        uint32_t at = and_or(d, slot_bits, step_at);
+        uint64_t moved = ballot(mine_back != entry);
+        if constexpr (K < 0) moved |= replay_all;
+        uint64_t mine_mask = ballot((d & ~Idx::kSlot) == 0u) & vs;  // live even lanes whose stay has a partner
+        if (__builtin_expect(moved != 0, 0)) {
             // Two live elements in one bucket (or with one hash).  Bit k of m says whether hash k of this
             // half of the beam equals `want`: each comparison is shifted into an accumulator with an
             // add-with-carry (a = 2a + equal), two accumulators so that no instruction waits for the one
@@ -903,7 +956,8 @@ __global__ __launch_bounds__((kBeamThreads<S, CPG, COLS, FWD>), (BeamCfg<S, FWD>
             const uint32_t live = w >= 32 ? 0xFFFFFFFFu : ((1u << w) - 1u);
             const uint32_t match = m & live;
             mine_mask = ballot(match != 0u) & vs;
-            j = (uint32_t)__builtin_ctz(match | 0x80000000u) & 31u;
+            const uint32_t j = (uint32_t)__builtin_ctz(match | 0x80000000u) & 31u;
+            at = step_at + 16u * j;
             // Merges in parallel need every stay to have one partner and every step candidate one claimant.
             // Otherwise (only possible after a CRC collision; flags bit 0 forces it) the merges are
             // replayed one by one in the CPU path's order, from the scores as they were before any merge.
@@ -913,7 +967,7 @@ __global__ __launch_bounds__((kBeamThreads<S, CPG, COLS, FWD>), (BeamCfg<S, FWD>
             const uint32_t claimed = sh.claim[claim_at];
             const uint32_t odd = (match & (match - 1u)) | (claimed ^ (uint32_t)i);
             if ((ballot(odd != 0u) & mine_mask) != 0 || (flags & 1)) {
-                if (h == 0) sh.stay_score[i] = cs;
+                if (h == 0) sh.stay_score[i] = cs0;
                 wave_fence();
                 if (lane == 0) {
                     for (int a = 0; a < w; ++a) {
@@ -921,7 +975,7 @@ __global__ __launch_bounds__((kBeamThreads<S, CPG, COLS, FWD>), (BeamCfg<S, FWD>
                         const uint32_t base = sh.elem[a].info & 3u;
                         for (int b = 0; b < w; ++b) {
                             if (crc2(sh.elem[b].hash, base) != ha) continue;
-                            float *st = &sh.cand[4 * b + (int)base];
+                            float *st = &all.cand[member].step[4 * b + (int)base];
                             const float both = log_sum_exp(sh.stay_score[a], *st, lse);
                             if (sh.stay_score[a] > *st) {
                                 sh.stay_score[a] = both;
@@ -937,7 +991,7 @@ __global__ __launch_bounds__((kBeamThreads<S, CPG, COLS, FWD>), (BeamCfg<S, FWD>
                 const f32x2 c01 = lds_load_f2(cand_mine);
                 c0 = c01.x;
                 c1 = c01.y;
-                if (h == 0) cs = sh.stay_score[i];
+                if (h == 0) cs0 = sh.stay_score[i];
                 mine_mask = 0;
             }
         }
@@ -949,55 +1003,58 @@ __global__ __launch_bounds__((kBeamThreads<S, CPG, COLS, FWD>), (BeamCfg<S, FWD>
         // instructions with whatever their registers hold and a dump slot as target: no exec
         // masking on the way.  Conditions are kept as wave-wide masks in scalar registers and combined
         // there; a select takes its mask as it is.
-        uint32_t at;  // the partner: step candidate 4j + last base of this element
-        asm("v_lshl_add_u32 %0, %1, 4, %2" : "=v"(at) : "v"(j), "v"(cand_base + (((uint32_t)state & 3u) << 2)));
         wave_fence();
         const float other = lds_load_f(at);
         // meanwhile: everything this step needs of row t is in registers; and the slot the traceback
         // reads is persisted (src/beam_search.c:417-427).  Both halves hold the same element and store the
         // same slot; slots past the width are never followed by the traceback.
-        bv_row[i] = (ofk_beam_slot_t)info;
-        bv_row += kW;
+        if constexpr (K < 0) {
+            bv_row[i] = (ofk_beam_slot_t)info;
+            bv_row += kW;
+        } else {
+            bv_row[(K + LR - 1) % LR * kW + i] = (ofk_beam_slot_t)info;
+            if constexpr (K == 0) bv_row += LR * kW;
+        }
         // no wait before this store: the wave's reads of row t are ahead of it in the LDS queue
-        __hip_atomic_store(&sh.consumed, next_t, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-        const uint64_t stay_wins = ballot(cs > other) & mine_mask;
+        if constexpr (K < 0 || K % Cfg::kHandBack == 0)
+            __hip_atomic_store(&sh.consumed, next_t, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        const uint64_t stay_wins = ballot(cs0 > other) & mine_mask;
         const uint64_t step_wins = mine_mask & ~stay_wins;
         const uint32_t target = (uint32_t)pick_by_bit(mine_mask, (int)at, (int)cand_dump);
-        // the fold from hardware exp/log where that provably rounds like the CPU path's double
-        // arithmetic (all but a few merges in a thousand at usual score magnitudes)
-        bool settled;
-        float folded = log_sum_exp_estimate(cs, other, settled);
+        // The fold from hardware exp/log, which the step goes on with.  Whether it rounds like the CPU path's double
+        // arithmetic (all but a few merges in a thousand at usual score magnitudes) is looked at while the new beam is on its
+        // way; if not, the step is done again from here with the double fold.
+        const FoldValue estimate = log_sum_exp_value(cs0, other);
+        uint32_t hash_again = hash;  // for the stay's record, in registers side by side with the rest of it
+        asm volatile("" : "+v"(hash_again));
+        typedef uint32_t u32x3 __attribute__((ext_vector_type(3)));
+        u32x3 e;
+        auto finish = [&](const float folded) {
         lds_store_f(target, pick_by_bit(step_wins, folded, -FLT_MAX));
         wave_fence();
-        f32x2 c01 = lds_load_f2(cand_mine);
-        if (__builtin_expect((ballot(!settled) & mine_mask) != 0, 0)) {
-            folded = log_sum_exp(cs, other, lse);
-            lds_store_f(target, pick_by_bit(step_wins, folded, -FLT_MAX));
-            wave_fence();
-            c01 = lds_load_f2(cand_mine);
-        }
+        const f32x2 c01 = lds_load_f2(cand_mine);
 
         // cut-off (src/beam_search.c:320-381)
         // Dead lanes carry -FLT_MAX as their score, which absorbs whatever is added: their candidates
         // are -FLT_MAX exactly (the stay of an odd lane: -FLT_MAX or -inf, see stay_h).
         // The best score does not wait for the step candidates to come back: a fold is not below either of
         // the two scores it joins, so the maximum of the scores before the merges and of the folds is that after them.
-        const float stay_or_fold = pick_by_bit(mine_mask, folded, cs);
+        const float stay_or_fold = pick_by_bit(mine_mask, folded, cs0);
         NextRecords next;
+        float cs;
         const float best = wave_max_beside_records(c0, c1, stay_or_fold, next, cs, hash, (uint32_t)b0, (uint32_t)state, from_stay,
                                                    (uint32_t)state << 2, (uint32_t)(S - 1), from, step_wins, -FLT_MAX, gst);
-        c0 = c01.x;
-        c1 = c01.y;
-        next.rest0 = c0 - g01.x;
-        next.rest1 = c1 - g01.y;
+        const float s0 = c01.x, s1 = c01.y;  // the steps' scores after the merges
+        next.rest0 = s0 - g01.x;
+        next.rest1 = s1 - g01.y;
 
         // Nearly every step has more candidates above the first cut than the width, and goes on to the cut
         // halfway to the best score: both are counted at once.
         float lo = best - log_cut;  // may be -FLT_MAX (no cut at all): mask the dead lanes
         float hi = best;
         float cut = (lo + hi) / 2.0f;
-        const uint64_t a0 = ballot(c0 >= lo), a1 = ballot(c1 >= lo), as = ballot(cs >= lo);
-        uint64_t k0 = ballot(c0 >= cut), k1 = ballot(c1 >= cut), ks = ballot(cs >= cut);
+        const uint64_t a0 = ballot(s0 >= lo), a1 = ballot(s1 >= lo), as = ballot(cs >= lo);
+        uint64_t k0 = ballot(s0 >= cut), k1 = ballot(s1 >= cut), ks = ballot(cs >= cut);
         int kept = popc64(a0 & vm) + popc64(a1 & vm) + popc64(as & vs);
         // kept candidates on lower lanes: masked bit counts
         auto lower = [&](uint64_t mask, int start) {
@@ -1029,8 +1086,8 @@ __global__ __launch_bounds__((kBeamThreads<S, CPG, COLS, FWD>), (BeamCfg<S, FWD>
                 cut = up ? next_up : next_down;
             };
             auto count = [&] {
-                k0 = ballot(c0 >= cut);
-                k1 = ballot(c1 >= cut);
+                k0 = ballot(s0 >= cut);
+                k1 = ballot(s1 >= cut);
                 ks = ballot(cs >= cut);
                 look_ahead();
                 steps_kept = popc64(k0) + popc64(k1);
@@ -1072,8 +1129,6 @@ __global__ __launch_bounds__((kBeamThreads<S, CPG, COLS, FWD>), (BeamCfg<S, FWD>
         }
 
         // survivors in candidate order: steps (i, b) by i then b, then stays by i
-        typedef uint32_t u32x3 __attribute__((ext_vector_type(3)));
-        u32x3 e;
         {
             // k0, k1 and ks hold this lane's own verdicts at its bit (dead lanes and the stays of the odd
             // lanes never pass): the masks select directly, nothing is compared again
@@ -1088,8 +1143,8 @@ __global__ __launch_bounds__((kBeamThreads<S, CPG, COLS, FWD>), (BeamCfg<S, FWD>
             const int slots = pick_by_bit(ks, ranks, dump);
             if constexpr (LAST) {
                 // the last beam is ranked by its candidate scores (src/beam_search.c:398-414)
-                next.rest0 = c0;
-                next.rest1 = c1;
+                next.rest0 = s0;
+                next.rest1 = s1;
                 next.rests = cs;
             }
             auto put = [&](int slot, uint32_t hsh, uint32_t inf, float rst) {
@@ -1103,7 +1158,7 @@ __global__ __launch_bounds__((kBeamThreads<S, CPG, COLS, FWD>), (BeamCfg<S, FWD>
             };
             put(slot0, next.h0, next.info0, next.rest0);
             put(slot1, next.h1, next.info1, next.rest1);
-            put(slots, hash, next.infos, next.rests);
+            put(slots, hash_again, next.infos, next.rests);
             wave_fence();
             // every lane reads its slot; slots past the new width hold leftovers: they count as dead through
             // their score and persist as zero, which is what the CPU path's untouched slots hold (a beam
@@ -1111,17 +1166,32 @@ __global__ __launch_bounds__((kBeamThreads<S, CPG, COLS, FWD>), (BeamCfg<S, FWD>
             e = *(const LDS_AS u32x3 *)(uintptr_t)(elem_base + 16u * (uint32_t)i);
         }
         w = kept;
-        vm = w > 0 ? ~0ull >> (64 - 2 * w) : 0ull;  // (the best candidate is always kept: w is zero only after NaN scores)
+        };
+        finish(estimate.value);
+        // while the beam is on its way: are the folds proven, and who is alive (the best candidate is always kept: w is zero only
+        // after NaN scores)
+        __builtin_amdgcn_sched_barrier(0);
+        uint64_t open = ballot(!log_sum_exp_settled(estimate));
+        asm volatile("" : "+s"(open));  // compared here, looked at further down
+        uint64_t vm_next = ballot(i < w), vs_next = ballot(i_stay < w);
+        asm volatile("" : "+s"(vm_next), "+s"(vs_next));
+        if (__builtin_expect((open & mine_mask) != 0, 0)) {
+            finish(log_sum_exp(cs0, other, lse));  // of the same beam: vm and vs are still its masks
+            vm_next = ballot(i < w);
+            vs_next = ballot(i_stay < w);
+        }
+        vm = vm_next;
+        vs = vs_next;
         if constexpr (!LAST) {
-            wait_row(next_t);
-            locate_row(next_t);
+            next_round(ring_slot(next_t, k_tag));
+            wait_row(next_t, k_tag);
             __builtin_amdgcn_sched_barrier(0);
         }
         hash = e.x;
         info = (uint32_t)pick_by_bit(vm, (int)e.z, 0);
         score = pick_by_bit(vm, __uint_as_float(e.y), -FLT_MAX);
         state = (int)(info & 1023u);
-        if constexpr (!LAST) fetch_row(next_t);
+        if constexpr (!LAST) fetch_row(next_t, k_tag);
 
         // last block: the best survivor goes to slot 0 (src/beam_search.c:398-414)
         if constexpr (LAST) {
@@ -1138,8 +1208,18 @@ __global__ __launch_bounds__((kBeamThreads<S, CPG, COLS, FWD>), (BeamCfg<S, FWD>
             bv_row[i] = (ofk_beam_slot_t)info;
         }
     };
-    for (int next_t = 1; next_t < T; ++next_t) step(next_t, std::false_type{});
-    step(T, std::true_type{});
+    // LR steps at a time: what goes by the ring slot, the parity of hand-overs and the row of persisted slots is then
+    // part of the instructions.  (Serial replay of the merges, for tests: one step at a time.)
+    int next_t = 1;
+    if (replay_all == 0) {
+        for (; next_t + LR <= T; next_t += LR)
+            static_for_upwards<LR>([&](auto k) {
+                constexpr int K = (decltype(k)::value + 1) % LR;
+                step(next_t + decltype(k)::value, std::integral_constant<int, K>{}, std::false_type{});
+            });
+    }
+    for (; next_t < T; ++next_t) step(next_t, AnySlot{}, std::false_type{});
+    step(T, AnySlot{}, std::true_type{});
 
     // ---- traceback from slot 0 of the last block (src/beam_search.c:432-439) ----
     // Followed one row at a time the walk is a chain of T dependent LDS reads.  It is done per block
@@ -1156,7 +1236,7 @@ __global__ __launch_bounds__((kBeamThreads<S, CPG, COLS, FWD>), (BeamCfg<S, FWD>
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
     {
         constexpr int RB = 128;  // rows per block
-        static_assert(2 * RB * kW * (int)sizeof(ofk_beam_slot_t) <= BeamIdx<S, CPG, FWD>::kBuckets * 8, "two blocks fit the index");
+        static_assert(2 * RB * kW * (int)sizeof(ofk_beam_slot_t) <= Idx::kBuckets * 4, "two blocks fit the index");
         int32_t *st_out = states + (size_t)n * T;
         uint8_t *mv_out = moves + (size_t)n * T;
         const uint32_t buf0 = idx_base;  // two buffers of RB rows of 64 bytes, row 127 the newest of a block

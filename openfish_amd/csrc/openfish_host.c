@@ -529,7 +529,7 @@ static int arrangement_by_default(int T, int N, int C, int state_len, int shared
         case 3: return N <= 2048 ? ARR_SPLIT : ARR_ONE;
         case 4:
             if (!can_merge) return N <= 768 ? ARR_SPLIT : ARR_ONE;
-            if (N <= 512) return shared || step_bytes > 3800000 ? ARR_MERGED : ARR_SPLIT;
+            if (N <= 512) return shared || step_bytes > 3300000 ? ARR_MERGED : ARR_SPLIT;
             return N <= (shared ? 640 : 768) ? ARR_SPLIT : ARR_MERGED;
         default:
             if (!can_merge) return ARR_ONE;
