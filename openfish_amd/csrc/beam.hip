@@ -863,7 +863,7 @@ __global__ __launch_bounds__((kBeamThreads<S, CPG, COLS, FWD>), (BeamCfg<S, CPG,
         expected = and_or(want, hash_keep, gen);
     };
     typedef std::integral_constant<int, -1> AnySlot;
-    wait_row(0, AnySlot{});
+    wait_row(0, std::integral_constant<int, 0>{});  // as many rows as the steps written out expect to find, not row 0 alone
     next_round(0);
     fetch_row(0, AnySlot{});
     const uint64_t replay_all = (flags & 1) ? ~0ull : 0ull;
