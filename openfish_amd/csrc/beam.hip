@@ -183,14 +183,6 @@ __device__ __forceinline__ int add_bit_of(int x, uint64_t mask) {
     return r;
 }
 __device__ __forceinline__ int popc64(uint64_t x) { return __builtin_popcountll(x); }
-// x + (float)h for the fp16 value h in the low half of a word, in one instruction: v_fma_mix_f32
-// converts the half operand on the fly and the product with 1.0 is exact, so the result is the
-// correctly rounded fp32 sum, bit for bit what a conversion followed by an addition gives
-__device__ __forceinline__ float add_half(uint32_t word, float x) {
-    float r;
-    asm("v_fma_mix_f32 %0, %1, 1.0, %2 op_sel_hi:[1,0,0]" : "=v"(r) : "v"(word), "v"(x));
-    return r;
-}
 // LDS accesses through a 32-bit LDS address
 typedef float f32x2 __attribute__((ext_vector_type(2)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
@@ -334,6 +326,48 @@ struct RowRegs {
     }
 };
 
+// A row of scores on its way to a ring slot that only the search reads: four planes of S values, one for every dropped base, a blank
+// column left out.  An element's four steps then lie side by side at 8 * state, whatever the layout of the caller's scores: one address
+// instruction and one LDS read instead of four and two.  A lane owns pairs of neighbouring states, COLS words each.
+template <int S, int COLS>
+struct PlaneRow {
+    static constexpr int kPairs = S / 2, kCnt = (kPairs + 63) / 64;
+    typedef uint32_t u32x4 __attribute__((ext_vector_type(4), aligned(4)));
+    u32x4 w[kCnt];
+    uint32_t w4[COLS == 5 ? kCnt : 1];  // the fifth word
+    static __device__ __forceinline__ bool mine(int i, int lane) { return (i + 1) * 64 <= kPairs || i * 64 + lane < kPairs; }
+    __device__ __forceinline__ void load(const char *row, int lane) {
+#pragma unroll
+        for (int i = 0; i < kCnt; ++i)
+            if (mine(i, lane)) {
+                const uint32_t *p = reinterpret_cast<const uint32_t *>(row) + COLS * (i * 64 + lane);
+                w[i] = *reinterpret_cast<const u32x4 *>(p);
+                if constexpr (COLS == 5) w4[i] = p[4];
+            }
+    }
+    static __device__ __forceinline__ uint32_t low_halves(uint32_t a, uint32_t b) { return __builtin_amdgcn_perm(b, a, 0x05040100u); }
+    static __device__ __forceinline__ uint32_t high_halves(uint32_t a, uint32_t b) { return __builtin_amdgcn_perm(b, a, 0x07060302u); }
+    static __device__ __forceinline__ uint32_t high_low(uint32_t a, uint32_t b) { return __builtin_amdgcn_perm(b, a, 0x05040302u); }
+    static __device__ __forceinline__ uint32_t low_high(uint32_t a, uint32_t b) { return __builtin_amdgcn_perm(b, a, 0x07060100u); }
+    __device__ __forceinline__ void store(char *row, int lane) const {
+#pragma unroll
+        for (int i = 0; i < kCnt; ++i)
+            if (mine(i, lane)) {
+                uint32_t *p = reinterpret_cast<uint32_t *>(row) + i * 64 + lane;
+                if constexpr (COLS == 4) {  // t0 t1 | t2 t3 of one state, then of the next
+                    p[0 * kPairs] = low_halves(w[i].x, w[i].z);
+                    p[1 * kPairs] = high_halves(w[i].x, w[i].z);
+                    p[2 * kPairs] = low_halves(w[i].y, w[i].w);
+                    p[3 * kPairs] = high_halves(w[i].y, w[i].w);
+                } else {  // blank t0 | t1 t2 | t3 blank | t0 t1 | t2 t3
+                    p[0 * kPairs] = high_low(w[i].x, w[i].w);
+                    p[1 * kPairs] = low_high(w[i].y, w[i].w);
+                    p[2 * kPairs] = high_low(w[i].y, w4[i]);
+                    p[3 * kPairs] = low_high(w[i].z, w4[i]);
+                }
+            }
+    }
+};
 
 // FWD is the number of waves per chunk that run the forward recursion beside the search (0: the search alone).
 template <int S, int CPG, int FWD>
@@ -366,11 +400,17 @@ struct BeamShared {
     int consumed;                 // rows the search wave is done with
 };
 
-// LDS of one chunk.  Score rows are kept as the caller lays them out: COLS = 4 transitions per
-// state, or 5 with an unused blank first.
+// LDS of one chunk.  Score rows are kept in planes for the search alone; where the recursion reads them too, as the caller lays them
+// out: COLS = 4 transitions per state, or 5 with an unused blank first.
+template <int S, int COLS, int FWD>
+struct ScoreRow {
+    static constexpr int kHalves = (FWD == 0 ? 4 : COLS) * S;
+    typedef RowRegs<2 * COLS * S> AsIs;
+    typedef typename std::conditional<FWD == 0, PlaneRow<S, COLS>, AsIs>::type Regs;
+};
 template <int S, int CPG, int COLS, int FWD>
 struct __attribute__((aligned(16))) BeamRing {
-    _Float16 row_s[BeamCfg<S, CPG, FWD>::kLdsRows][COLS * S];
+    _Float16 row_s[BeamCfg<S, CPG, FWD>::kLdsRows][ScoreRow<S, COLS, FWD>::kHalves];
     float row_b[BeamCfg<S, CPG, FWD>::kLdsRows][S];
 };
 // Hash index of one chunk: 2^kBits buckets of one word.  Hash bits 2 .. kBits + 1 are the bucket's byte address; in the entry
@@ -654,15 +694,16 @@ __global__ __launch_bounds__((kBeamThreads<S, CPG, COLS, FWD>), (BeamCfg<S, CPG,
         // ---- loader wave: row t = (scores[t], bwd[t+1]) into ring slot t % LR ----
         // The ring is spelled out as named registers (not an array indexed by a loop that
         // also contains the spin wait) so that every row stays in VGPRs.
-        RowRegs<2 * COLS * S> s0, s1, s2, s3, s4, s5;
+        typedef typename ScoreRow<S, COLS, FWD>::Regs Scores;
+        Scores s0, s1, s2, s3, s4, s5;
         RowRegs<4 * S> g0, g1, g2, g3, g4, g5;
-        auto fetch = [&](RowRegs<2 * COLS * S> &rs, RowRegs<4 * S> &rb, int t) {
+        auto fetch = [&](Scores &rs, RowRegs<4 * S> &rb, int t) {
             if (t < T) {
                 rs.load(reinterpret_cast<const char *>(sc_n + (size_t)t * row_stride), lane);
                 rb.load(reinterpret_cast<const char *>(bw_n + (size_t)(t + 1) * S), lane);
             }
         };
-        auto hand_over = [&](RowRegs<2 * COLS * S> &rs, RowRegs<4 * S> &rb, int t) {
+        auto hand_over = [&](Scores &rs, RowRegs<4 * S> &rb, int t) {
             if (t < T) {
                 // the ring is full most of the time (a search step takes about 3000 cycles): poll
                 // seldom, the rows in registers and in the ring leave ample slack for waking up late
@@ -789,7 +830,9 @@ __global__ __launch_bounds__((kBeamThreads<S, CPG, COLS, FWD>), (BeamCfg<S, CPG,
     // fetched as soon as that beam is known (at the end of the previous step): the row
     // entries of the lane's candidates, and the hash index: the element's own entry goes in, is
     // read back, and the entry filed under `want` is read.
-    uint32_t r0h, r1h;  // fp16 scores of the lane's two step candidates, each in the low half of a word
+    // fp16 scores of the lane's two step candidates: both in one word (planes), or each in the low half of a word
+    constexpr bool kPlanes = FWD == 0;
+    uint32_t r0h, r1h;
     f32x2 g01;
     float gst;
     uint32_t probe;      // index entry found under `want`
@@ -804,6 +847,8 @@ __global__ __launch_bounds__((kBeamThreads<S, CPG, COLS, FWD>), (BeamCfg<S, CPG,
     // ring addresses: the same in every lane, kept in scalar registers
     const uint32_t ring_s = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uintptr_t)(lds_u32 *)&row_s[0][0]);
     const uint32_t ring_b = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uintptr_t)(lds_u32 *)&row_b[0][0]);
+    uint32_t step_row = ring_s + 4u * (uint32_t)h;  // the lane's two of an element's four steps, less 8 * state
+    asm volatile("" : "+v"(step_row));
     // The ring slot of a time step's row is known where steps are written out (K), elsewhere (K < 0) it is worked out.
     auto ring_slot = [&](int tt, auto k_tag) {
         constexpr int K = decltype(k_tag)::value;
@@ -842,18 +887,22 @@ __global__ __launch_bounds__((kBeamThreads<S, CPG, COLS, FWD>), (BeamCfg<S, CPG,
         own_p[0] = entry;
         __builtin_amdgcn_sched_barrier(0);  // the entries go out first, the row is asked for next: `want` takes a while
         wave_fence();  // one wave's LDS operations are carried out in order: the reads below see every lane's entry
-        // scores of the candidates with bases b0, b0 + 1: rs[COLS * (lo4 + b0 + {0,1}) + (COLS - 4) + top];
-        // guide terms rb[lo4 + b0 + {0,1}] and rb[state]
+        // scores of the candidates with bases b0, b0 + 1, which lie in the column of the dropped base; guide terms rb[lo4 + b0 + {0,1}]
+        // and rb[state]
         const uint32_t st4 = (uint32_t)state << 2;
         const uint32_t cand = and_or(st4, (uint32_t)(S - 1), (uint32_t)b0);  // lo4 + b0
-        const uint32_t top = (uint32_t)state >> (BITS - 2);                    // column of the dropped base
-        const uint32_t rs = ring_s + slot * (uint32_t)(2 * COLS * S), rb = ring_b + slot * (uint32_t)(4 * S);
-        uint32_t at_s;
-        if constexpr (COLS == 4) at_s = (((cand << 2) | top) << 1) + rs;
-        else at_s = cand * 10u + (top << 1) + rs;
-        typedef __attribute__((address_space(3))) uint16_t lds_u16;
-        r0h = *(const lds_u16 *)(uintptr_t)(at_s + 2u * (COLS - 4));
-        r1h = *(const lds_u16 *)(uintptr_t)(at_s + 2u * (COLS - 4) + 2u * COLS);
+        const uint32_t rs = ring_s + slot * (uint32_t)sizeof(row_s[0]), rb = ring_b + slot * (uint32_t)sizeof(row_b[0]);
+        if constexpr (kPlanes) {
+            r0h = *(const lds_u32 *)(uintptr_t)(((uint32_t)state << 3) + step_row + slot * (uint32_t)sizeof(row_s[0]));
+        } else {
+            const uint32_t top = (uint32_t)state >> (BITS - 2);  // the dropped base
+            uint32_t at_s;  // rs[COLS * (lo4 + b0 + {0,1}) + (COLS - 4) + top]
+            if constexpr (COLS == 4) at_s = (((cand << 2) | top) << 1) + rs;
+            else at_s = cand * 10u + (top << 1) + rs;
+            typedef __attribute__((address_space(3))) uint16_t lds_u16;
+            r0h = *(const lds_u16 *)(uintptr_t)(at_s + 2u * (COLS - 4));
+            r1h = *(const lds_u16 *)(uintptr_t)(at_s + 2u * (COLS - 4) + 2u * COLS);
+        }
         g01 = lds_load_f2((cand << 2) + rb);
         gst = lds_load_f(st4 + rb);
         __builtin_amdgcn_sched_barrier(0);
@@ -882,8 +931,8 @@ __global__ __launch_bounds__((kBeamThreads<S, CPG, COLS, FWD>), (BeamCfg<S, CPG,
         constexpr bool LAST = decltype(last_tag)::value;
         // (score + transition) + guide, the CPU path's order of additions; the fp16 transition is
         // converted inside the first addition
-        float c0 = add_half(r0h, score) + g01.x;
-        float c1 = add_half(r1h, score) + g01.y;
+        float c0 = ::add_half<0>(r0h, score) + g01.x;
+        float c1 = ::add_half<kPlanes ? 1 : 0>(kPlanes ? r0h : r1h, score) + g01.y;
         float cs0 = (score + stay_h) + gst;
         lds_store_f2(cand_mine, c0, c1);  // for the merges below
         const uint32_t step_at = and_or((uint32_t)state << 2, 12u, cand_base);  // the partner is step candidate 4j + last base of this element
