@@ -28,12 +28,12 @@ C_OBJ   := $(BUILD)/openfish_host.o
 
 all: lib/libopenfish.a openfish_amd/libopenfish_amd.so openfish
 
-$(BUILD)/%.o: $(SRC)/%.hip $(SRC)/kernels.h $(SRC)/dmath.h $(SRC)/lse5.h
+$(BUILD)/%.o: $(SRC)/%.hip $(SRC)/kernels.h $(SRC)/dmath.h $(SRC)/lse5.h $(SRC)/queue.h
 	@mkdir -p $(BUILD)
 	$(HIPCC) $(HIPFLAGS) -c $< -o $@
 
 # the scans once more for scores with five columns per state (a blank first), read in place
-$(BUILD)/scan_five.o: $(SRC)/scan.hip $(SRC)/kernels.h $(SRC)/dmath.h $(SRC)/lse5.h
+$(BUILD)/scan_five.o: $(SRC)/scan.hip $(SRC)/kernels.h $(SRC)/dmath.h $(SRC)/lse5.h $(SRC)/queue.h
 	@mkdir -p $(BUILD)
 	$(HIPCC) $(HIPFLAGS) -DOFK_COLS=5 -c $< -o $@
 

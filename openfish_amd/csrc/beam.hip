@@ -37,6 +37,7 @@
 #include <type_traits>
 
 #include "kernels.h"
+#include "queue.h"
 #include "lse5.h"
 
 namespace {
@@ -1405,22 +1406,22 @@ int search_group(int S, int N, int flags) {
 template <int S, int COLS>
 int launch_beam(const void *scores, const float *bwd, ofk_beam_slot_t *beam, int32_t *states,
                 uint8_t *moves, int T, int N, float log_cut, float stay, int flags, const double *lse_table,
-                hipStream_t st) {
+                Queue st) {
     const int group = search_group(S, N, flags);
     if (group == 1) {
-        hipLaunchKernelGGL((beam_kernel<S, 1, COLS, 0>), dim3(N), dim3(kBeamThreads<S, 1, COLS, 0>), 0, st, static_cast<const _Float16 *>(scores), bwd,
+        queue_kernel((beam_kernel<S, 1, COLS, 0>), dim3(N), dim3(kBeamThreads<S, 1, COLS, 0>), 0, st, static_cast<const _Float16 *>(scores), bwd,
                            nullptr, beam, states, moves, T, N, log_cut, stay, flags, lse_table, LogSeries{});
         return (int)hipGetLastError();
     }
     if constexpr (S <= 256) {
         if (group == 4) {
-            hipLaunchKernelGGL((beam_kernel<S, 4, COLS, 0>), dim3((N + 3) / 4), dim3(512), 0, st,
+            queue_kernel((beam_kernel<S, 4, COLS, 0>), dim3((N + 3) / 4), dim3(512), 0, st,
                                static_cast<const _Float16 *>(scores), bwd, nullptr, beam, states, moves, T, N, log_cut,
                                stay, flags, lse_table, LogSeries{});
             return (int)hipGetLastError();
         }
     }
-    hipLaunchKernelGGL((beam_kernel<S, 2, COLS, 0>), dim3((N + 1) / 2), dim3(256), 0, st,
+    queue_kernel((beam_kernel<S, 2, COLS, 0>), dim3((N + 1) / 2), dim3(256), 0, st,
                        static_cast<const _Float16 *>(scores), bwd, nullptr, beam, states, moves, T, N, log_cut, stay,
                        flags, lse_table, LogSeries{});
     return (int)hipGetLastError();
@@ -1432,8 +1433,8 @@ const LogSeries kSeries = {OFA_LOG_SERIES, OFA_EXP_COEFS};
 template <int S, int CPG, int COLS, int FWD>
 int launch_beam_forward(const void *scores, const float *bwd, float *post, ofk_beam_slot_t *beam, int32_t *states,
                         uint8_t *moves, int T, int N, float log_cut, float stay, int flags, const double *lse_table,
-                        hipStream_t st) {
-    hipLaunchKernelGGL((beam_kernel<S, CPG, COLS, FWD>), dim3((N + CPG - 1) / CPG), dim3(kBeamThreads<S, CPG, COLS, FWD>), 0, st,
+                        Queue st) {
+    queue_kernel((beam_kernel<S, CPG, COLS, FWD>), dim3((N + CPG - 1) / CPG), dim3(kBeamThreads<S, CPG, COLS, FWD>), 0, st,
                        static_cast<const _Float16 *>(scores), bwd, post, beam, states, moves, T, N, log_cut, stay, flags,
                        lse_table, kSeries);
     return (int)hipGetLastError();
@@ -1441,7 +1442,7 @@ int launch_beam_forward(const void *scores, const float *bwd, float *post, ofk_b
 
 int dispatch_beam(const void *scores, const float *bwd, ofk_beam_slot_t *beam, int32_t *states, uint8_t *moves,
                   int T, int N, int state_len, int columns, float log_cut, float stay, int flags,
-                  const double *lse_table, hipStream_t st) {
+                  const double *lse_table, Queue st) {
     switch (state_len * 8 + columns) {
         case 3 * 8 + 4: return launch_beam<64, 4>(scores, bwd, beam, states, moves, T, N, log_cut, stay, flags, lse_table, st);
         case 4 * 8 + 4: return launch_beam<256, 4>(scores, bwd, beam, states, moves, T, N, log_cut, stay, flags, lse_table, st);
@@ -1519,7 +1520,7 @@ extern "C" int ofk_beam_search_static(const void *scores, const float *bwd, int3
     // nothing in the array has to start at zero: the search writes every slot the traceback reads
     ofk_beam_slot_t *beam = reinterpret_cast<ofk_beam_slot_t *>(base + kStaticTableBytes);
     const double *lse_table = reinterpret_cast<const double *>(base);
-    hipStream_t st = static_cast<hipStream_t>(stream);
+    const Queue st{static_cast<hipStream_t>(stream), nullptr};
     return dispatch_beam(scores, bwd, beam, states, moves, T, N, state_len, columns, log_beam_cut, stay, flags,
                          lse_table, st);
 }
@@ -1528,23 +1529,23 @@ extern "C" int ofk_search_chunks_per_group(int N, int state_len, int flags) { re
 
 extern "C" int ofk_beam_search(const void *scores, const float *bwd, ofk_beam_slot_t *beam, int32_t *states,
                                uint8_t *moves, int T, int N, int state_len, int columns, float log_beam_cut,
-                               float stay, const double *lse_table, int flags, void *stream) {
+                               float stay, const double *lse_table, int flags, void *stream, void *done) {
     if (!scores || !bwd || !beam || !states || !moves || !lse_table || T < 1 || N < 1) return OFK_BAD_ARGS;
     if ((reinterpret_cast<uintptr_t>(scores) | reinterpret_cast<uintptr_t>(bwd) | reinterpret_cast<uintptr_t>(beam)) & 15u)
         return OFK_BAD_ARGS;
-    hipStream_t st = static_cast<hipStream_t>(stream);
+    const Queue st{static_cast<hipStream_t>(stream), static_cast<hipEvent_t>(done)};
     return dispatch_beam(scores, bwd, beam, states, moves, T, N, state_len, columns, log_beam_cut, stay, flags,
                          lse_table, st);
 }
 
 extern "C" int ofk_beam_search_forward(const void *scores, const float *bwd, float *post, ofk_beam_slot_t *beam,
                                        int32_t *states, uint8_t *moves, int T, int N, int state_len, int columns,
-                                       float log_beam_cut, float stay, const double *lse_table, int flags, void *stream) {
+                                       float log_beam_cut, float stay, const double *lse_table, int flags, void *stream, void *done) {
     if (!scores || !bwd || !post || !beam || !states || !moves || !lse_table || T < 1 || N < 1) return OFK_BAD_ARGS;
     if ((reinterpret_cast<uintptr_t>(scores) | reinterpret_cast<uintptr_t>(bwd) | reinterpret_cast<uintptr_t>(post) |
          reinterpret_cast<uintptr_t>(beam)) & 15u)
         return OFK_BAD_ARGS;
-    hipStream_t st = static_cast<hipStream_t>(stream);
+    const Queue st{static_cast<hipStream_t>(stream), static_cast<hipEvent_t>(done)};
 #define OFK_FORWARD(S, CPG, COLS, FWD) \
     return launch_beam_forward<S, CPG, COLS, FWD>(scores, bwd, post, beam, states, moves, T, N, log_beam_cut, stay, flags, lse_table, st)
     const bool dense = N > OFK_SPARSE_SEARCH_MAX_CHUNKS;

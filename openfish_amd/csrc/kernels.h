@@ -2,6 +2,7 @@
  * Launchers of the gfx950 kernels, callable from C.  Each returns 0 on success,
  * a hipError_t value if the launch failed, or OFK_BAD_ARGS if the arguments do
  * not fit what the kernel assumes (nothing is launched in that case).
+ * stream: a hipStream_t; done: NULL, or a hipEvent_t that is complete when the kernel has ended.
  */
 #ifndef OPENFISH_AMD_KERNELS_H
 #define OPENFISH_AMD_KERNELS_H
@@ -35,19 +36,19 @@ typedef uint16_t ofk_beam_slot_t;
 #define OFK_SCAN_PRECISE 1
 #define OFK_SCAN_FAST 2
 int ofk_bwd_scan(const void *scores, float *bwd, int T, int N, int state_len, int columns, float stay, int mode,
-                 int spl, void *stream);
+                 int spl, void *stream, void *done);
 int ofk_fwd_post_scan(const void *scores, const float *bwd, float *post, int T, int N, int state_len,
-                      int columns, float stay, int mode, int spl, void *stream);
+                      int columns, float stay, int mode, int spl, void *stream, void *done);
 /* The same in two steps, 1024 states and the two-tier arithmetic only: the forward recursion by itself, which needs no bwd and can
  * run beside the backward sweep, and then the posteriors of its rows, in place. */
-int ofk_fwd_scan(const void *scores, float *fwd, int T, int N, int state_len, int columns, float stay, void *stream);
-int ofk_posterior_rows(const float *bwd, float *post, int T, int N, int state_len, void *stream);
+int ofk_fwd_scan(const void *scores, float *fwd, int T, int N, int state_len, int columns, float stay, void *stream, void *done);
+int ofk_posterior_rows(const float *bwd, float *post, int T, int N, int state_len, void *stream, void *done);
 /* Both sweeps and the posterior in one kernel: the forward and backward recursions of a chunk run
  * side by side in one workgroup and meet in the middle of the chunk (same tensors as
  * ofk_bwd_scan followed by ofk_fwd_post_scan).  Rows 0 .. T/2-1 of post hold forward values
  * while the kernel runs. */
 int ofk_scan_posterior(const void *scores, float *bwd, float *post, int T, int N, int state_len,
-                       int columns, float stay, int mode, int spl, void *stream);
+                       int columns, float stay, int mode, int spl, void *stream, void *done);
 /* Table behind log(1 + e^-gap), the correction of a pairwise log-sum-exp, for gap in
  * [0, 17): OFK_LSE_CELLS cells of width 1/4, each a degree-8 polynomial in
  * s = 8 * (gap - centre) in [-1, 1], coefficients lowest degree first.  Built on the
@@ -58,13 +59,13 @@ int ofk_scan_posterior(const void *scores, float *bwd, float *post, int T, int N
 
 int ofk_beam_search(const void *scores, const float *bwd, ofk_beam_slot_t *beam, int32_t *states,
                     uint8_t *moves, int T, int N, int state_len, int columns, float log_beam_cut, float stay,
-                    const double *lse_table, int flags, void *stream);
+                    const double *lse_table, int flags, void *stream, void *done);
 /* The search together with the forward sweep and the posterior of the same chunks, one kernel that reads
  * scores and bwd once for both (256 and 1024 states): the results of ofk_beam_search and of
  * ofk_fwd_post_scan with the two-tier arithmetic. */
 int ofk_beam_search_forward(const void *scores, const float *bwd, float *post, ofk_beam_slot_t *beam, int32_t *states,
                             uint8_t *moves, int T, int N, int state_len, int columns, float log_beam_cut, float stay,
-                            const double *lse_table, int flags, void *stream);
+                            const double *lse_table, int flags, void *stream, void *done);
 /* The same search with the beam slots and the table in a static device array of the library
  * (OFK_STATIC_SLOT_BYTES of slots: N * (T + 1) * 64 bytes must fit, else OFK_TOO_LARGE and nothing
  * is launched).  ofk_beam_search_static_prepare sets the array up on the current device (looks up
@@ -99,11 +100,11 @@ typedef struct {
  * moves_out: NULL, or N * T bytes (pinned host memory) that get a copy of moves. */
 int ofk_sequence(const float *post, int32_t *states, const uint8_t *moves, float *qual_data,
                  float *base_probs, float *total_probs, char *sequence, char *qstring, int T, int N,
-                 int state_len, const ofk_phred_table_t *phred, const float *path_sums, uint8_t *moves_out, void *stream);
+                 int state_len, const ofk_phred_table_t *phred, const float *path_sums, uint8_t *moves_out, void *stream, void *done);
 /* sums[n][t][s], N x T x states floats: posterior of state s at row t + 1 of chunk n plus that of its
  * distinct one-base shifts, fp32 sums in the CPU path's order (src/beam_search.c:441-463), for every
  * state: the input of a block's quality whichever state the path then takes. */
-int ofk_path_sums(const float *post, float *sums, int T, int N, int state_len, void *stream);
+int ofk_path_sums(const float *post, float *sums, int T, int N, int state_len, void *stream, void *done);
 /* Batches up to this size put at most two chunks of the beam search on a compute unit (one wave
  * each): the search then leaves room for ofk_path_sums beside it.  Larger batches fill the units
  * with search waves, and the extra kernel was measured to cost the search more than it saves the

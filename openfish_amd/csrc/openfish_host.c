@@ -120,9 +120,9 @@ void openfish_amd_lse_table(double *out) { build_lse_table(out); }
 
 #define OFA_MAGIC 0x6f66616d64677075ull /* "ofamdgpu" */
 
-enum { EV_JOIN, EV_START, EV_BWD_END, EV_BEAM_START, EV_BEAM_END, EV_FWD_END, EV_FWD_SCAN_END, EV_SEQ_START, EV_SEQ_END, EV_SUMS_START, EV_SUMS_END, EV_MOVES, EV_COUNT };
-/* with both sweeps in one kernel EV_BWD_END marks its end and EV_FWD_END is not recorded; EV_FWD_SCAN_END only where the forward sweep runs
- * beside the backward one */
+enum { EV_JOIN, EV_START, EV_BWD_END, EV_BEAM_END, EV_FWD_END, EV_FWD_SCAN_END, EV_SEQ_END, EV_SUMS_END, EV_MOVES, EV_COUNT };
+/* The events between kernels are carried by the kernels whose end they mark (queue.h); with both sweeps in one kernel EV_BWD_END is its
+ * end and EV_FWD_END is not used, EV_FWD_SCAN_END only where the forward sweep runs beside the backward one. */
 
 /* arrangements of the scans: both sweeps in one kernel; backward sweep, then forward sweep beside the beam search;
  * backward sweep, then forward sweep within the beam search's kernel */
@@ -477,8 +477,12 @@ static void fetch_outputs(ofa_gpubuf_t *g, int T, int N, uint8_t **moves, char *
     memcpy(*qstring, g->h_out + 2 * nt, nt);
 }
 
-/* order the library's streams after everything already queued on the null stream */
+/* Order the library's streams after everything already queued on the null stream (and on the streams that wait for it).  Where that
+ * has ended already, which the query tells in 0.2 us, there is nothing to wait for: the event and the wait for it in another hardware
+ * queue put 20 us before a decode's first kernel. */
 static void join_null_stream(ofa_gpubuf_t *g) {
+    if (hipStreamQuery(0) == hipSuccess) return;
+    (void)hipGetLastError(); /* the query's answer; what is wrong, if anything, the calls below say */
     HIP_OK(hipEventRecord(g->ev[EV_JOIN], 0));
     HIP_OK(hipStreamWaitEvent(g->s_main, g->ev[EV_JOIN], 0));
 }
@@ -581,33 +585,25 @@ static void enqueue_decode(ofa_gpubuf_t *g, const int T, const int N, const int 
     HIP_OK(hipEventRecord(g->ev[EV_START], g->s_main));
     if (g->pend_split == ARR_MERGED) {
         /* backward sweep, then the search with the forward sweep and the posterior in its workgroups */
-        launch_ok(ofk_bwd_scan(scores_TNC, g->pub.bwd_NTC, T, N, state_len, cols, stay, g->scan_mode, g->scan_spl, g->s_main),
-                  "bwd_scan");
-        HIP_OK(hipEventRecord(g->ev[EV_BWD_END], g->s_main));
-        HIP_OK(hipEventRecord(g->ev[EV_BEAM_START], g->s_main));
+        launch_ok(ofk_bwd_scan(scores_TNC, g->pub.bwd_NTC, T, N, state_len, cols, stay, g->scan_mode, g->scan_spl, g->s_main,
+                               g->ev[EV_BWD_END]), "bwd_scan");
         launch_ok(ofk_beam_search_forward(scores_TNC, g->pub.bwd_NTC, g->pub.post_NTC, (ofk_beam_slot_t *)g->pub.beam_vector,
                                           (int32_t *)g->pub.states, g->pub.moves, T, N, state_len, cols,
-                                          log_beam_cut(options), stay, g->lse_table, g->debug_flags, g->s_main),
+                                          log_beam_cut(options), stay, g->lse_table, g->debug_flags, g->s_main, g->ev[EV_BEAM_END]),
                   "beam_search_forward");
-        HIP_OK(hipEventRecord(g->ev[EV_BEAM_END], g->s_main));
     } else if (g->pend_split == ARR_ONE) {
         /* both sweeps and the posterior in one kernel, then the beam search, all on one stream */
         launch_ok(ofk_scan_posterior(scores_TNC, g->pub.bwd_NTC, g->pub.post_NTC, T, N, state_len, cols, stay, g->scan_mode,
-                                     g->scan_spl, g->s_main), "scan_posterior");
-        HIP_OK(hipEventRecord(g->ev[EV_BWD_END], g->s_main));
-        HIP_OK(hipEventRecord(g->ev[EV_BEAM_START], g->s_main));
+                                     g->scan_spl, g->s_main, g->ev[EV_BWD_END]), "scan_posterior");
         launch_ok(ofk_beam_search(scores_TNC, g->pub.bwd_NTC, (ofk_beam_slot_t *)g->pub.beam_vector,
                                   (int32_t *)g->pub.states, g->pub.moves, T, N, state_len, cols, log_beam_cut(options),
-                                  stay, g->lse_table, search_flags, g->s_main), "beam_search");
-        HIP_OK(hipEventRecord(g->ev[EV_BEAM_END], g->s_main));
+                                  stay, g->lse_table, search_flags, g->s_main, g->ev[EV_BEAM_END]), "beam_search");
         /* The search keeps one wave per chunk busy and leaves the rest of the machine idle: beside
          * it, on the second stream, the posteriors that a block's quality is made of are summed for
          * every state, so that the sequence stage reads one value per time step instead of nine. */
         if (use_sums) {
             HIP_OK(hipStreamWaitEvent(g->s_side, g->ev[EV_BWD_END], 0));
-            HIP_OK(hipEventRecord(g->ev[EV_SUMS_START], g->s_side));
-            launch_ok(ofk_path_sums(g->pub.post_NTC, g->path_sums, T, N, state_len, g->s_side), "path_sums");
-            HIP_OK(hipEventRecord(g->ev[EV_SUMS_END], g->s_side));
+            launch_ok(ofk_path_sums(g->pub.post_NTC, g->path_sums, T, N, state_len, g->s_side, g->ev[EV_SUMS_END]), "path_sums");
         }
     } else {
         /* A sweep of 1024 states has a compute unit to a chunk.  A batch that leaves half of the units idle, and shares them
@@ -617,35 +613,30 @@ static void enqueue_decode(ofa_gpubuf_t *g, const int T, const int N, const int 
          * T = 833: 1 1.48 | 1.23, 37 1.51 | 1.27, 64 1.52 | 1.31, 96 1.53 | 1.33; five columns, T = 1666: 80 2.67 | 2.51,
          * 96 2.68 | 2.57, 112 2.72 | 2.73, 128 2.82 | 2.85. */
         const int apart = g->pend_apart = state_len == 5 && N <= 96 && !shared && g->scan_mode == OFK_SCAN_TWO_TIER && g->scan_spl == 0;
-        launch_ok(ofk_bwd_scan(scores_TNC, g->pub.bwd_NTC, T, N, state_len, cols, stay, g->scan_mode, g->scan_spl, g->s_main),
-                  "bwd_scan");
-        HIP_OK(hipEventRecord(g->ev[EV_BWD_END], g->s_main));
+        launch_ok(ofk_bwd_scan(scores_TNC, g->pub.bwd_NTC, T, N, state_len, cols, stay, g->scan_mode, g->scan_spl, g->s_main,
+                               g->ev[EV_BWD_END]), "bwd_scan");
         if (apart) {
             HIP_OK(hipStreamWaitEvent(g->s_side, g->ev[EV_START], 0));
-            launch_ok(ofk_fwd_scan(scores_TNC, g->pub.post_NTC, T, N, state_len, cols, stay, g->s_side), "fwd_scan");
-            HIP_OK(hipEventRecord(g->ev[EV_FWD_SCAN_END], g->s_side));
+            launch_ok(ofk_fwd_scan(scores_TNC, g->pub.post_NTC, T, N, state_len, cols, stay, g->s_side, g->ev[EV_FWD_SCAN_END]),
+                      "fwd_scan");
         }
 
         /* The beam search is the longer of the two stages that follow and wants its workgroups (large
          * LDS blocks) resident before the forward sweep fills the compute units: it stays on the stream
          * the backward sweep ran on and so starts first; the forward sweep follows through an event. */
-        HIP_OK(hipEventRecord(g->ev[EV_BEAM_START], g->s_main));
         launch_ok(ofk_beam_search(scores_TNC, g->pub.bwd_NTC, (ofk_beam_slot_t *)g->pub.beam_vector,
                                   (int32_t *)g->pub.states, g->pub.moves, T, N, state_len, cols, log_beam_cut(options),
-                                  stay, g->lse_table, search_flags, g->s_main), "beam_search");
-        HIP_OK(hipEventRecord(g->ev[EV_BEAM_END], g->s_main));
+                                  stay, g->lse_table, search_flags, g->s_main, g->ev[EV_BEAM_END]), "beam_search");
 
         HIP_OK(hipStreamWaitEvent(g->s_side, g->ev[EV_BWD_END], 0));
         if (apart)
-            launch_ok(ofk_posterior_rows(g->pub.bwd_NTC, g->pub.post_NTC, T, N, state_len, g->s_side), "posterior_rows");
+            launch_ok(ofk_posterior_rows(g->pub.bwd_NTC, g->pub.post_NTC, T, N, state_len, g->s_side, g->ev[EV_FWD_END]),
+                      "posterior_rows");
         else
             launch_ok(ofk_fwd_post_scan(scores_TNC, g->pub.bwd_NTC, g->pub.post_NTC, T, N, state_len, cols, stay, g->scan_mode,
-                                        g->scan_spl, g->s_side), "fwd_post_scan");
-        HIP_OK(hipEventRecord(g->ev[EV_FWD_END], g->s_side));
+                                        g->scan_spl, g->s_side, g->ev[EV_FWD_END]), "fwd_post_scan");
         if (use_sums) {
-            HIP_OK(hipEventRecord(g->ev[EV_SUMS_START], g->s_side));
-            launch_ok(ofk_path_sums(g->pub.post_NTC, g->path_sums, T, N, state_len, g->s_side), "path_sums");
-            HIP_OK(hipEventRecord(g->ev[EV_SUMS_END], g->s_side));
+            launch_ok(ofk_path_sums(g->pub.post_NTC, g->path_sums, T, N, state_len, g->s_side, g->ev[EV_SUMS_END]), "path_sums");
         }
     }
 
@@ -661,7 +652,6 @@ static void enqueue_decode(ofa_gpubuf_t *g, const int T, const int N, const int 
     if (use_sums) HIP_OK(hipStreamWaitEvent(g->s_main, g->ev[EV_SUMS_END], 0));
     else if (g->pend_split == ARR_SPLIT) HIP_OK(hipStreamWaitEvent(g->s_main, g->ev[EV_FWD_END], 0));
 
-    HIP_OK(hipEventRecord(g->ev[EV_SEQ_START], g->s_main));
     /* The last kernel writes bases and qualities straight into the pinned host memory (N * T bytes
      * each, every byte once, 16 bytes a lane): they are in host memory when the
      * kernel ends and no copy follows it, which measured 0.05 ms less per call at 512 x 1666 than two
@@ -669,8 +659,8 @@ static void enqueue_decode(ofa_gpubuf_t *g, const int T, const int N, const int 
      * are filled by the stage-level entry points only. */
     launch_ok(ofk_sequence(g->pub.post_NTC, (int32_t *)g->pub.states, g->pub.moves, g->pub.qual_data,
                            g->pub.base_probs, g->pub.total_probs, (char *)g->d_out + nt, (char *)g->d_out + 2 * nt, T, N,
-                           state_len, phred_for(g, options), use_sums ? g->path_sums : NULL, g->pend_copy ? NULL : g->d_out, g->s_main), "sequence");
-    HIP_OK(hipEventRecord(g->ev[EV_SEQ_END], g->s_main));
+                           state_len, phred_for(g, options), use_sums ? g->path_sums : NULL, g->pend_copy ? NULL : g->d_out, g->s_main, NULL), "sequence");
+    HIP_OK(hipEventRecord(g->ev[EV_SEQ_END], g->s_main)); /* a marker, which makes what the kernel wrote to host memory visible there */
     g->pending = 1;
     g->pend_T = T;
     g->pend_N = N;
@@ -742,11 +732,18 @@ int openfish_amd_last_timings(const openfish_gpubuf_t *gpubuf, float *ms, int n)
         HIP_OK(hipEventElapsedTime(&behind, g->ev[EV_FWD_SCAN_END], g->ev[EV_FWD_END]));
         if (behind < g->ms[OPENFISH_AMD_STAGE_FWD]) g->ms[OPENFISH_AMD_STAGE_FWD] = behind;
     }
-    HIP_OK(hipEventElapsedTime(&g->ms[OPENFISH_AMD_STAGE_BEAM], g->ev[EV_BEAM_START], g->ev[EV_BEAM_END]));
-    HIP_OK(hipEventElapsedTime(&g->ms[OPENFISH_AMD_STAGE_SEQ], g->ev[EV_SEQ_START], g->ev[EV_SEQ_END]));
+    /* a stage begins where the last one that it waits for ends */
+    HIP_OK(hipEventElapsedTime(&g->ms[OPENFISH_AMD_STAGE_BEAM], g->ev[EV_BWD_END], g->ev[EV_BEAM_END]));
     HIP_OK(hipEventElapsedTime(&g->ms[OPENFISH_AMD_STAGE_TOTAL], g->ev[EV_START], g->ev[EV_SEQ_END]));
     g->ms[OPENFISH_AMD_STAGE_SUMS] = 0.0f;
-    if (g->pend_sums) HIP_OK(hipEventElapsedTime(&g->ms[OPENFISH_AMD_STAGE_SUMS], g->ev[EV_SUMS_START], g->ev[EV_SUMS_END]));
+    if (g->pend_sums)
+        HIP_OK(hipEventElapsedTime(&g->ms[OPENFISH_AMD_STAGE_SUMS], g->ev[g->pend_split == ARR_ONE ? EV_BWD_END : EV_FWD_END], g->ev[EV_SUMS_END]));
+    HIP_OK(hipEventElapsedTime(&g->ms[OPENFISH_AMD_STAGE_SEQ], g->ev[EV_BEAM_END], g->ev[EV_SEQ_END]));
+    if (g->pend_sums || g->pend_split == ARR_SPLIT) {
+        float behind = 0.0f;
+        HIP_OK(hipEventElapsedTime(&behind, g->ev[g->pend_sums ? EV_SUMS_END : EV_FWD_END], g->ev[EV_SEQ_END]));
+        if (behind < g->ms[OPENFISH_AMD_STAGE_SEQ]) g->ms[OPENFISH_AMD_STAGE_SEQ] = behind;
+    }
     if (n > OPENFISH_AMD_STAGE_COUNT) n = OPENFISH_AMD_STAGE_COUNT;
     memcpy(ms, g->ms, sizeof(float) * (size_t)n);
     return n;
@@ -764,7 +761,7 @@ void openfish_amd_bwd_scan(int T, int N, int C, const void *scores, int state_le
     openfish_opt_t o = DECODER_INIT;
     check_scores(T, N, C, scores, state_len, &o);
     check_scan_mode(scan_mode);
-    launch_ok(ofk_bwd_scan(scores, bwd, T, N, state_len, columns_of(C, state_len), stay_score, scan_mode, 0, NULL), "bwd_scan");
+    launch_ok(ofk_bwd_scan(scores, bwd, T, N, state_len, columns_of(C, state_len), stay_score, scan_mode, 0, NULL, NULL), "bwd_scan");
     HIP_OK(hipStreamSynchronize(0));
 }
 
@@ -773,7 +770,7 @@ void openfish_amd_fwd_post_scan(int T, int N, int C, const void *scores, int sta
     openfish_opt_t o = DECODER_INIT;
     check_scores(T, N, C, scores, state_len, &o);
     check_scan_mode(scan_mode);
-    launch_ok(ofk_fwd_post_scan(scores, bwd, post, T, N, state_len, columns_of(C, state_len), stay_score, scan_mode, 0, NULL), "fwd_post_scan");
+    launch_ok(ofk_fwd_post_scan(scores, bwd, post, T, N, state_len, columns_of(C, state_len), stay_score, scan_mode, 0, NULL, NULL), "fwd_post_scan");
     HIP_OK(hipStreamSynchronize(0));
 }
 
@@ -782,7 +779,7 @@ void openfish_amd_scan_posterior(int T, int N, int C, const void *scores, int st
     openfish_opt_t o = DECODER_INIT;
     check_scores(T, N, C, scores, state_len, &o);
     check_scan_mode(scan_mode);
-    launch_ok(ofk_scan_posterior(scores, bwd, post, T, N, state_len, columns_of(C, state_len), stay_score, scan_mode, 0, NULL), "scan_posterior");
+    launch_ok(ofk_scan_posterior(scores, bwd, post, T, N, state_len, columns_of(C, state_len), stay_score, scan_mode, 0, NULL, NULL), "scan_posterior");
     HIP_OK(hipStreamSynchronize(0));
 }
 
@@ -793,7 +790,7 @@ void openfish_amd_beam_search(int T, int N, int C, const void *scores, int state
     launch_ok(ofk_beam_search(scores, bwd, (ofk_beam_slot_t *)g->pub.beam_vector, (int32_t *)g->pub.states,
                               g->pub.moves, T, N, state_len, columns_of(C, state_len), log_beam_cut(options),
                               options->blank_score,
-                              g->lse_table, g->debug_flags, NULL),
+                              g->lse_table, g->debug_flags, NULL, NULL),
               "beam_search");
     HIP_OK(hipStreamSynchronize(0));
 }
@@ -835,7 +832,7 @@ void openfish_amd_sequence(int T, int N, int state_len, const openfish_opt_t *op
     ofa_gpubuf_t *g = checked(gpubuf, T, N, state_len);
     launch_ok(ofk_sequence(post, (int32_t *)g->pub.states, g->pub.moves, g->pub.qual_data, g->pub.base_probs,
                            g->pub.total_probs, g->pub.sequence, g->pub.qstring, T, N, state_len,
-                           phred_for(g, options), NULL, NULL, NULL), "sequence");
+                           phred_for(g, options), NULL, NULL, NULL, NULL), "sequence");
     HIP_OK(hipStreamSynchronize(0));
 }
 
@@ -851,16 +848,16 @@ void openfish_amd_decode_from_tensors(int T, int N, int C, const void *scores, i
     launch_ok(ofk_beam_search(scores, bwd, (ofk_beam_slot_t *)g->pub.beam_vector, (int32_t *)g->pub.states,
                               g->pub.moves, T, N, state_len, columns_of(C, state_len), log_beam_cut(options),
                               options->blank_score,
-                              g->lse_table, g->debug_flags, g->s_main), "beam_search");
+                              g->lse_table, g->debug_flags, g->s_main, NULL), "beam_search");
     /* the quality stage as a whole decode runs it: from per-state sums where the gpubuf holds room for them */
     const float *sums = NULL;
     if (g->path_sums != NULL && N <= OFK_SPARSE_SEARCH_MAX_CHUNKS) {
-        launch_ok(ofk_path_sums(post, g->path_sums, T, N, state_len, g->s_main), "path_sums");
+        launch_ok(ofk_path_sums(post, g->path_sums, T, N, state_len, g->s_main, NULL), "path_sums");
         sums = g->path_sums;
     }
     launch_ok(ofk_sequence(post, (int32_t *)g->pub.states, g->pub.moves, g->pub.qual_data, g->pub.base_probs,
                            g->pub.total_probs, g->pub.sequence, g->pub.qstring, T, N, state_len,
-                           phred_for(g, options), sums, NULL, g->s_main), "sequence");
+                           phred_for(g, options), sums, NULL, g->s_main, NULL), "sequence");
     fetch_outputs(g, T, N, moves, sequence, qstring);
 }
 

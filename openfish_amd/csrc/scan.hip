@@ -44,6 +44,7 @@
 
 #include "lse5.h"
 #include "kernels.h"
+#include "queue.h"
 
 namespace {
 
@@ -1136,23 +1137,23 @@ template <int S>
 constexpr int kPlainSpl = S >= 1024 ? 2 : 1;
 
 template <int S, int SPL, int DEPTH>
-int launch_bwd(int mode, const void *scores, float *bwd, int T, int N, float stay, hipStream_t st) {
+int launch_bwd(int mode, const void *scores, float *bwd, int T, int N, float stay, Queue st) {
     using Sh = Shape<S, SPL>;
     const dim3 grid((N + Sh::kChunks - 1) / Sh::kChunks), block(Sh::kThreads);
     const _Float16 *sc = static_cast<const _Float16 *>(scores);
     switch (mode) {
         case OFK_SCAN_TWO_TIER:
-            hipLaunchKernelGGL((bwd_scan_kernel<S, SPL, DEPTH, OFK_SCAN_TWO_TIER>), grid, block, 0, st, sc, bwd, T, N, stay, kSeries);
+            queue_kernel((bwd_scan_kernel<S, SPL, DEPTH, OFK_SCAN_TWO_TIER>), grid, block, 0, st, sc, bwd, T, N, stay, kSeries);
             break;
         case OFK_SCAN_PRECISE:
             if constexpr (SPL == kPlainSpl<S>)
-                hipLaunchKernelGGL((bwd_scan_kernel<S, SPL, DEPTH, OFK_SCAN_PRECISE>), grid, block, 0, st, sc, bwd, T, N, stay, kSeries);
+                queue_kernel((bwd_scan_kernel<S, SPL, DEPTH, OFK_SCAN_PRECISE>), grid, block, 0, st, sc, bwd, T, N, stay, kSeries);
             else
                 return OFK_BAD_ARGS;
             break;
         case OFK_SCAN_FAST:
             if constexpr (SPL == kPlainSpl<S>)
-                hipLaunchKernelGGL((bwd_scan_kernel<S, SPL, DEPTH, OFK_SCAN_FAST>), grid, block, 0, st, sc, bwd, T, N, stay, kSeries);
+                queue_kernel((bwd_scan_kernel<S, SPL, DEPTH, OFK_SCAN_FAST>), grid, block, 0, st, sc, bwd, T, N, stay, kSeries);
             else
                 return OFK_BAD_ARGS;
             break;
@@ -1162,7 +1163,7 @@ int launch_bwd(int mode, const void *scores, float *bwd, int T, int N, float sta
 }
 
 template <int S, int SPL, int DEPTH>
-int launch_fwd(int mode, const void *scores, const float *bwd, float *post, int T, int N, float stay, hipStream_t st) {
+int launch_fwd(int mode, const void *scores, const float *bwd, float *post, int T, int N, float stay, Queue st) {
     using Sh = Shape<S, SPL>;
     const dim3 grid((N + Sh::kChunks - 1) / Sh::kChunks), block(Sh::kThreads);
     const _Float16 *sc = static_cast<const _Float16 *>(scores);
@@ -1173,22 +1174,22 @@ int launch_fwd(int mode, const void *scores, const float *bwd, float *post, int 
             // 512 chunks 1.17 ms against 1.41 ms beside the beam search, 1024 chunks 3.5 against 3.1)
             if constexpr (Sh::kMultiWave && 2 * Sh::kLanes <= 1024) {
                 if ((long)N * (2 * Sh::kLanes / 64) <= 4096) {
-                    hipLaunchKernelGGL((fwd_post_roles_kernel<S, SPL, kRolesDepth>), dim3(N), dim3(2 * Sh::kLanes), 0, st, sc, bwd, post,
+                    queue_kernel((fwd_post_roles_kernel<S, SPL, kRolesDepth>), dim3(N), dim3(2 * Sh::kLanes), 0, st, sc, bwd, post,
                                        T, N, stay, kSeries);
                     break;
                 }
             }
-            hipLaunchKernelGGL((fwd_post_kernel<S, SPL, DEPTH, OFK_SCAN_TWO_TIER>), grid, block, 0, st, sc, bwd, post, T, N, stay, kSeries);
+            queue_kernel((fwd_post_kernel<S, SPL, DEPTH, OFK_SCAN_TWO_TIER>), grid, block, 0, st, sc, bwd, post, T, N, stay, kSeries);
             break;
         case OFK_SCAN_PRECISE:
             if constexpr (SPL == kPlainSpl<S>)
-                hipLaunchKernelGGL((fwd_post_kernel<S, SPL, DEPTH, OFK_SCAN_PRECISE>), grid, block, 0, st, sc, bwd, post, T, N, stay, kSeries);
+                queue_kernel((fwd_post_kernel<S, SPL, DEPTH, OFK_SCAN_PRECISE>), grid, block, 0, st, sc, bwd, post, T, N, stay, kSeries);
             else
                 return OFK_BAD_ARGS;
             break;
         case OFK_SCAN_FAST:
             if constexpr (SPL == kPlainSpl<S>)
-                hipLaunchKernelGGL((fwd_post_kernel<S, SPL, DEPTH, OFK_SCAN_FAST>), grid, block, 0, st, sc, bwd, post, T, N, stay, kSeries);
+                queue_kernel((fwd_post_kernel<S, SPL, DEPTH, OFK_SCAN_FAST>), grid, block, 0, st, sc, bwd, post, T, N, stay, kSeries);
             else
                 return OFK_BAD_ARGS;
             break;
@@ -1198,23 +1199,23 @@ int launch_fwd(int mode, const void *scores, const float *bwd, float *post, int 
 }
 
 template <int S, int SPL, int DEPTH>
-int launch_fused(int mode, const void *scores, float *bwd, float *post, int T, int N, float stay, hipStream_t st) {
+int launch_fused(int mode, const void *scores, float *bwd, float *post, int T, int N, float stay, Queue st) {
     using Sh = FusedShape<S, SPL>;
     const dim3 grid((N + Sh::kChunks - 1) / Sh::kChunks), block(Sh::kThreads);
     const _Float16 *sc = static_cast<const _Float16 *>(scores);
     switch (mode) {
         case OFK_SCAN_TWO_TIER:
-            hipLaunchKernelGGL((scan_post_kernel<S, SPL, DEPTH, OFK_SCAN_TWO_TIER>), grid, block, 0, st, sc, bwd, post, T, N, stay, kSeries);
+            queue_kernel((scan_post_kernel<S, SPL, DEPTH, OFK_SCAN_TWO_TIER>), grid, block, 0, st, sc, bwd, post, T, N, stay, kSeries);
             break;
         case OFK_SCAN_PRECISE:
             if constexpr (SPL == kPlainSpl<S>)
-                hipLaunchKernelGGL((scan_post_kernel<S, SPL, DEPTH, OFK_SCAN_PRECISE>), grid, block, 0, st, sc, bwd, post, T, N, stay, kSeries);
+                queue_kernel((scan_post_kernel<S, SPL, DEPTH, OFK_SCAN_PRECISE>), grid, block, 0, st, sc, bwd, post, T, N, stay, kSeries);
             else
                 return OFK_BAD_ARGS;
             break;
         case OFK_SCAN_FAST:
             if constexpr (SPL == kPlainSpl<S>)
-                hipLaunchKernelGGL((scan_post_kernel<S, SPL, DEPTH, OFK_SCAN_FAST>), grid, block, 0, st, sc, bwd, post, T, N, stay, kSeries);
+                queue_kernel((scan_post_kernel<S, SPL, DEPTH, OFK_SCAN_FAST>), grid, block, 0, st, sc, bwd, post, T, N, stay, kSeries);
             else
                 return OFK_BAD_ARGS;
             break;
@@ -1299,10 +1300,10 @@ static int fused_states_per_lane(int S, int N, int forced) {
 static int lanes_asked(int mode, int spl) { return mode == OFK_SCAN_TWO_TIER ? spl : 1; }
 
 static int scan_posterior(const void *scores, float *bwd, float *post, int T, int N, int state_len, float stay,
-                          int mode, int spl, void *stream) {
+                          int mode, int spl, void *stream, void *done) {
     if (!scores || !bwd || !post || T < 1 || N < 1 || !aligned16(scores) || !aligned16(bwd) || !aligned16(post))
         return OFK_BAD_ARGS;
-    hipStream_t st = static_cast<hipStream_t>(stream);
+    const Queue st{static_cast<hipStream_t>(stream), static_cast<hipEvent_t>(done)};
     const int S = 1 << (2 * state_len);
     switch (state_len * 8 + (state_len >= 3 && state_len <= 5 ? fused_states_per_lane(S, N, lanes_asked(mode, spl)) : 0)) {
         case 3 * 8 + 1:  // 64 states: latency-bound, the deeper prefetch pays until the rows are 4 MiB apart
@@ -1319,10 +1320,10 @@ static int scan_posterior(const void *scores, float *bwd, float *post, int T, in
 }
 
 static int bwd_scan(const void *scores, float *bwd, int T, int N, int state_len, float stay, int mode, int spl,
-                    void *stream) {
+                    void *stream, void *done) {
     if (!scores || !bwd || T < 1 || N < 1 || !aligned16(scores) || !aligned16(bwd)) return OFK_BAD_ARGS;
     if (state_len < 3 || state_len > 5) return OFK_BAD_ARGS;
-    hipStream_t st = static_cast<hipStream_t>(stream);
+    const Queue st{static_cast<hipStream_t>(stream), static_cast<hipEvent_t>(done)};
     // Up to a chunk for every compute unit, 1024 states take one state to a lane, sixteen waves: four waves on a SIMD fill each
     // other's waits, and a wave with half as many updates has the second tier's single trip more often (ms, two states to a
     // lane | one: 37 chunks, T = 833 0.76 | 0.67; 256, T = 1666 1.45 | 1.32; 9, T = 64 0.091 | 0.078).  Two such workgroups do
@@ -1333,17 +1334,17 @@ static int bwd_scan(const void *scores, float *bwd, int T, int N, int state_len,
 }
 
 static int fwd_post_scan(const void *scores, const float *bwd, float *post, int T, int N, int state_len,
-                         float stay, int mode, int spl, void *stream) {
+                         float stay, int mode, int spl, void *stream, void *done) {
     if (!scores || !bwd || !post || T < 1 || N < 1 || !aligned16(scores) || !aligned16(bwd) || !aligned16(post))
         return OFK_BAD_ARGS;
     if (state_len < 3 || state_len > 5) return OFK_BAD_ARGS;
-    hipStream_t st = static_cast<hipStream_t>(stream);
+    const Queue st{static_cast<hipStream_t>(stream), static_cast<hipEvent_t>(done)};
     OFK_DISPATCH(false, launch_fwd, mode, scores, bwd, post, T, N, stay, st)
 }
 
-static int fwd_scan(const void *scores, float *fwd, int T, int N, int state_len, float stay, void *stream) {
+static int fwd_scan(const void *scores, float *fwd, int T, int N, int state_len, float stay, void *stream, void *done) {
     if (!scores || !fwd || T < 1 || N < 1 || state_len != 5 || !aligned16(scores) || !aligned16(fwd)) return OFK_BAD_ARGS;
-    hipLaunchKernelGGL((fwd_scan_kernel<1024, OFK_DEPTH_1024>), dim3(N), dim3(1024), 0, static_cast<hipStream_t>(stream),
+    queue_kernel((fwd_scan_kernel<1024, OFK_DEPTH_1024>), dim3(N), dim3(1024), 0, Queue{static_cast<hipStream_t>(stream), static_cast<hipEvent_t>(done)},
                        static_cast<const _Float16 *>(scores), fwd, T, N, stay, kSeries);
     return (int)hipGetLastError();
 }
@@ -1352,61 +1353,61 @@ static int fwd_scan(const void *scores, float *fwd, int T, int N, int state_len,
 // with five, whose kernels the entry points reach through the three functions named *_five.
 #if OFK_COLS == 5
 extern "C" int ofk_scan_posterior_five(const void *scores, float *bwd, float *post, int T, int N, int state_len,
-                                       float stay, int mode, int spl, void *stream) {
-    return scan_posterior(scores, bwd, post, T, N, state_len, stay, mode, spl, stream);
+                                       float stay, int mode, int spl, void *stream, void *done) {
+    return scan_posterior(scores, bwd, post, T, N, state_len, stay, mode, spl, stream, done);
 }
 extern "C" int ofk_bwd_scan_five(const void *scores, float *bwd, int T, int N, int state_len, float stay, int mode,
-                                 int spl, void *stream) {
-    return bwd_scan(scores, bwd, T, N, state_len, stay, mode, spl, stream);
+                                 int spl, void *stream, void *done) {
+    return bwd_scan(scores, bwd, T, N, state_len, stay, mode, spl, stream, done);
 }
 extern "C" int ofk_fwd_post_scan_five(const void *scores, const float *bwd, float *post, int T, int N,
-                                      int state_len, float stay, int mode, int spl, void *stream) {
-    return fwd_post_scan(scores, bwd, post, T, N, state_len, stay, mode, spl, stream);
+                                      int state_len, float stay, int mode, int spl, void *stream, void *done) {
+    return fwd_post_scan(scores, bwd, post, T, N, state_len, stay, mode, spl, stream, done);
 }
-extern "C" int ofk_fwd_scan_five(const void *scores, float *fwd, int T, int N, int state_len, float stay, void *stream) {
-    return fwd_scan(scores, fwd, T, N, state_len, stay, stream);
+extern "C" int ofk_fwd_scan_five(const void *scores, float *fwd, int T, int N, int state_len, float stay, void *stream, void *done) {
+    return fwd_scan(scores, fwd, T, N, state_len, stay, stream, done);
 }
 #else
-extern "C" int ofk_scan_posterior_five(const void *, float *, float *, int, int, int, float, int, int, void *);
-extern "C" int ofk_bwd_scan_five(const void *, float *, int, int, int, float, int, int, void *);
-extern "C" int ofk_fwd_post_scan_five(const void *, const float *, float *, int, int, int, float, int, int, void *);
-extern "C" int ofk_fwd_scan_five(const void *, float *, int, int, int, float, void *);
+extern "C" int ofk_scan_posterior_five(const void *, float *, float *, int, int, int, float, int, int, void *, void *);
+extern "C" int ofk_bwd_scan_five(const void *, float *, int, int, int, float, int, int, void *, void *);
+extern "C" int ofk_fwd_post_scan_five(const void *, const float *, float *, int, int, int, float, int, int, void *, void *);
+extern "C" int ofk_fwd_scan_five(const void *, float *, int, int, int, float, void *, void *);
 
 extern "C" int ofk_scan_posterior(const void *scores, float *bwd, float *post, int T, int N, int state_len,
-                                  int columns, float stay, int mode, int spl, void *stream) {
-    if (columns == 5) return ofk_scan_posterior_five(scores, bwd, post, T, N, state_len, stay, mode, spl, stream);
+                                  int columns, float stay, int mode, int spl, void *stream, void *done) {
+    if (columns == 5) return ofk_scan_posterior_five(scores, bwd, post, T, N, state_len, stay, mode, spl, stream, done);
     if (columns != 4) return OFK_BAD_ARGS;
-    return scan_posterior(scores, bwd, post, T, N, state_len, stay, mode, spl, stream);
+    return scan_posterior(scores, bwd, post, T, N, state_len, stay, mode, spl, stream, done);
 }
 
 extern "C" int ofk_bwd_scan(const void *scores, float *bwd, int T, int N, int state_len, int columns, float stay,
-                            int mode, int spl, void *stream) {
-    if (columns == 5) return ofk_bwd_scan_five(scores, bwd, T, N, state_len, stay, mode, spl, stream);
+                            int mode, int spl, void *stream, void *done) {
+    if (columns == 5) return ofk_bwd_scan_five(scores, bwd, T, N, state_len, stay, mode, spl, stream, done);
     if (columns != 4) return OFK_BAD_ARGS;
-    return bwd_scan(scores, bwd, T, N, state_len, stay, mode, spl, stream);
+    return bwd_scan(scores, bwd, T, N, state_len, stay, mode, spl, stream, done);
 }
 
 extern "C" int ofk_fwd_post_scan(const void *scores, const float *bwd, float *post, int T, int N, int state_len,
-                                 int columns, float stay, int mode, int spl, void *stream) {
-    if (columns == 5) return ofk_fwd_post_scan_five(scores, bwd, post, T, N, state_len, stay, mode, spl, stream);
+                                 int columns, float stay, int mode, int spl, void *stream, void *done) {
+    if (columns == 5) return ofk_fwd_post_scan_five(scores, bwd, post, T, N, state_len, stay, mode, spl, stream, done);
     if (columns != 4) return OFK_BAD_ARGS;
-    return fwd_post_scan(scores, bwd, post, T, N, state_len, stay, mode, spl, stream);
+    return fwd_post_scan(scores, bwd, post, T, N, state_len, stay, mode, spl, stream, done);
 }
 
-extern "C" int ofk_fwd_scan(const void *scores, float *fwd, int T, int N, int state_len, int columns, float stay, void *stream) {
-    if (columns == 5) return ofk_fwd_scan_five(scores, fwd, T, N, state_len, stay, stream);
+extern "C" int ofk_fwd_scan(const void *scores, float *fwd, int T, int N, int state_len, int columns, float stay, void *stream, void *done) {
+    if (columns == 5) return ofk_fwd_scan_five(scores, fwd, T, N, state_len, stay, stream, done);
     if (columns != 4) return OFK_BAD_ARGS;
-    return fwd_scan(scores, fwd, T, N, state_len, stay, stream);
+    return fwd_scan(scores, fwd, T, N, state_len, stay, stream, done);
 }
 
-extern "C" int ofk_posterior_rows(const float *bwd, float *post, int T, int N, int state_len, void *stream) {
+extern "C" int ofk_posterior_rows(const float *bwd, float *post, int T, int N, int state_len, void *stream, void *done) {
     if (!bwd || !post || T < 1 || N < 1 || state_len != 5 || !aligned16(bwd) || !aligned16(post)) return OFK_BAD_ARGS;
     // Four rows to a workgroup, and few workgroups: the search beside this is longer, and more rows in flight only slow it down
     // (128 | 256 | 1024 workgroups, whole call, ms: 37 chunks, T = 833 1.27 | 1.27 | 1.29; 80, T = 1666 2.43 | 2.47 | 2.56).
     int parts = 128 / N;
     parts = parts < 1 ? 1 : parts;
     parts = parts < (T + 4) / 4 ? parts : (T + 4) / 4;
-    hipLaunchKernelGGL((posterior_rows_kernel<1024>), dim3(N * parts), dim3(256), 0, static_cast<hipStream_t>(stream), bwd, post, T, parts);
+    queue_kernel((posterior_rows_kernel<1024>), dim3(N * parts), dim3(256), 0, Queue{static_cast<hipStream_t>(stream), static_cast<hipEvent_t>(done)}, bwd, post, T, parts);
     return (int)hipGetLastError();
 }
 #endif

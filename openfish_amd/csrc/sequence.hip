@@ -15,6 +15,7 @@
 #include <hip/hip_runtime.h>
 
 #include "kernels.h"
+#include "queue.h"
 
 namespace {
 
@@ -311,7 +312,7 @@ __global__ __launch_bounds__(256) void path_sums_kernel(const float *__restrict_
 }
 
 template <int S>
-int launch_path_sums(const float *post, float *sums, int T, int N, hipStream_t st) {
+int launch_path_sums(const float *post, float *sums, int T, int N, Queue st) {
     const long rows = (long)N * T;
     // Half as many workgroups as chunks, up to one per compute unit (one wave per SIMD): with 512
     // chunks of 256 states the kernel then ends well inside the beam search it runs beside and does
@@ -319,21 +320,21 @@ int launch_path_sums(const float *post, float *sums, int T, int N, hipStream_t s
     // 1024 groups 1.27; 128 groups outlast the search).
     int wgs = N / 2;
     wgs = wgs < 64 ? 64 : (wgs > 256 ? 256 : wgs);
-    hipLaunchKernelGGL((path_sums_kernel<S>), dim3(wgs), dim3(256), 0, st, post, sums, T, rows);
+    queue_kernel((path_sums_kernel<S>), dim3(wgs), dim3(256), 0, st, post, sums, T, rows);
     return (int)hipGetLastError();
 }
 
 template <int S, int kThreads>
 int launch_sequence_with(const float *post, int32_t *states, const uint8_t *moves, float *qual_data,
                          float *base_probs, float *total_probs, char *sequence, char *qstring, int T, int N,
-                         const ofk_phred_table_t &phred, const float *path_sums, uint8_t *moves_out, hipStream_t st) {
+                         const ofk_phred_table_t &phred, const float *path_sums, uint8_t *moves_out, Queue st) {
     const size_t lds = sequence_lds(T);
     if (lds > 64 * 1024 - 1024) {  // beyond the default limit of dynamic LDS; the compute unit has 160 KB
         const hipError_t rc = hipFuncSetAttribute(reinterpret_cast<const void *>(&sequence_kernel<S, kThreads>),
                                                   hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
         if (rc != hipSuccess) return (int)rc;
     }
-    hipLaunchKernelGGL((sequence_kernel<S, kThreads>), dim3(N), dim3(kThreads), lds, st, post, states, moves, qual_data,
+    queue_kernel((sequence_kernel<S, kThreads>), dim3(N), dim3(kThreads), lds, st, post, states, moves, qual_data,
                        base_probs, total_probs, sequence, qstring, T, phred, path_sums, moves_out);
     return (int)hipGetLastError();
 }
@@ -341,7 +342,7 @@ int launch_sequence_with(const float *post, int32_t *states, const uint8_t *move
 template <int S>
 int launch_sequence(const float *post, int32_t *states, const uint8_t *moves, float *qual_data,
                     float *base_probs, float *total_probs, char *sequence, char *qstring, int T, int N,
-                    const ofk_phred_table_t &phred, const float *path_sums, uint8_t *moves_out, hipStream_t st) {
+                    const ofk_phred_table_t &phred, const float *path_sums, uint8_t *moves_out, Queue st) {
     // Up to a chunk per compute unit, 960 gathering lanes (two time steps each at T = 1666, nine at 8192): the rounds of memory accesses
     // are what is waited for.  Beyond, two workgroups of half the size fill a unit and one's gathers run beside the other's characters.
     // 1024 | 512 | 256 lanes, us: 16 chunks of 64 states 14 | 17 | 25, 256 of 1024 84 | 86 | 92, 512 of 256 131 | 129 | 145, 1024 of 256
@@ -355,10 +356,10 @@ int launch_sequence(const float *post, int32_t *states, const uint8_t *moves, fl
 
 }  // namespace
 
-extern "C" int ofk_path_sums(const float *post, float *sums, int T, int N, int state_len, void *stream) {
+extern "C" int ofk_path_sums(const float *post, float *sums, int T, int N, int state_len, void *stream, void *done) {
     if (!post || !sums || T < 1 || N < 1) return OFK_BAD_ARGS;
     if ((reinterpret_cast<uintptr_t>(post) | reinterpret_cast<uintptr_t>(sums)) & 15u) return OFK_BAD_ARGS;
-    hipStream_t st = static_cast<hipStream_t>(stream);
+    const Queue st{static_cast<hipStream_t>(stream), static_cast<hipEvent_t>(done)};
     switch (state_len) {
         case 3: return launch_path_sums<64>(post, sums, T, N, st);
         case 4: return launch_path_sums<256>(post, sums, T, N, st);
@@ -370,13 +371,13 @@ extern "C" int ofk_path_sums(const float *post, float *sums, int T, int N, int s
 extern "C" int ofk_sequence(const float *post, int32_t *states, const uint8_t *moves, float *qual_data,
                             float *base_probs, float *total_probs, char *sequence, char *qstring, int T, int N,
                             int state_len, const ofk_phred_table_t *phred, const float *path_sums, uint8_t *moves_out,
-                            void *stream) {
+                            void *stream, void *done) {
     // the per-chunk tables live in LDS: 13 bytes per time step
     if ((!post && !path_sums) || !states || !moves || !qual_data || !base_probs || !total_probs || !sequence || !qstring ||
         !phred || T < 1 || T > OFK_MAX_T || N < 1)
         return OFK_BAD_ARGS;
     if (reinterpret_cast<uintptr_t>(qual_data) & 15u) return OFK_BAD_ARGS;
-    hipStream_t st = static_cast<hipStream_t>(stream);
+    const Queue st{static_cast<hipStream_t>(stream), static_cast<hipEvent_t>(done)};
     switch (state_len) {
         case 3: return launch_sequence<64>(post, states, moves, qual_data, base_probs, total_probs, sequence, qstring, T, N, *phred, path_sums, moves_out, st);
         case 4: return launch_sequence<256>(post, states, moves, qual_data, base_probs, total_probs, sequence, qstring, T, N, *phred, path_sums, moves_out, st);
