@@ -208,6 +208,14 @@ __device__ __forceinline__ uint32_t lds_address(const void *p) {
     return at;
 }
 
+// The lane, worked out where it is wanted: for places off the search's way, so that no register holds it through the search (two
+// workgroups on a compute unit leave 96).
+__device__ __forceinline__ int lane_now() {
+    uint32_t none = 0;
+    asm volatile("" : "+v"(none));  // or the compiler takes it from elsewhere after all
+    return (int)__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, none));
+}
+
 __device__ __forceinline__ void wave_fence() {
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
@@ -397,8 +405,7 @@ struct BeamShared {
     Elem elem[kW + 64];           // slots 0 .. kW-1; entry kW + lane is lane's dump slot for candidates that are not kept
     float stay_score[kW];         // only used by the serial replay of merges
     uint32_t claim[4 * kW + 64];  // only used when the hash index was not conclusive: who claimed step candidate 4j+b
-    int ready;                    // rows stored by the loader wave
-    int consumed;                 // rows the search wave is done with
+    int ready, consumed;          // rows stored by the loader wave, rows the search wave is done with (with FWD > 0 in FwdLds)
 };
 
 // LDS of one chunk.  Score rows are kept in planes for the search alone; where the recursion reads them too, as the caller lays them
@@ -434,8 +441,11 @@ struct BeamIdx {
 constexpr int kVecRows = 4;  // two would do (see beam_kernel); four let the posterior lag (1024 chunks of 256 states: 2.66 ms against 2.78)
 template <int S, int FWD>
 struct __attribute__((aligned(16))) FwdLds {
-    int published[FWD];  // rows of the state vector each wave of the recursion has written
-    int taken;           // rows the posterior's wave has read
+    // Progress of the chunk's waves, side by side so that one LDS read of a wave, a lane to a counter, sees all of it: rows of the state
+    // vector that each wave of the recursion has written, rows that the posterior's wave has read, ring rows ready and consumed.
+    static constexpr int kTaken = FWD, kReady = FWD + 1, kConsumed = FWD + 2;
+    static constexpr int kCounters = FWD + 3 <= 8 ? 8 : 16;
+    int progress[kCounters];
     __attribute__((aligned(16))) float vec[kVecRows][S];  // row t in vec[t % kVecRows]
     float tier_lanes[64 * FWD];
 };
@@ -564,7 +574,7 @@ __global__ __launch_bounds__((kBeamThreads<S, CPG, COLS, FWD>), (BeamCfg<S, CPG,
     const bool recursion = FWD > 0 && wave >= kFirstFwd && wave < kFirstLoader;
     const int member = recursion ? (wave - kFirstFwd) / (FWD > 0 ? FWD : 1) : wave % kGroupChunks;
     const int n = blockIdx.x * kGroupChunks + member;
-    const int lane = threadIdx.x & 63;
+    const int lane = lane_now();
     auto &row_s = lds[member].ring.row_s;
     auto &row_b = lds[member].ring.row_b;
     BeamShared &sh = lds[member].sh;
@@ -572,13 +582,19 @@ __global__ __launch_bounds__((kBeamThreads<S, CPG, COLS, FWD>), (BeamCfg<S, CPG,
     const _Float16 *sc_n = scores + (size_t)n * COLS * S;
     const float *bw_n = bwd + (size_t)n * (size_t)(T + 1) * S;
 
+    int *ready, *consumed;  // rows stored by the loader wave, rows the search wave is done with
+    if constexpr (FWD == 0) {
+        ready = &sh.ready;
+        consumed = &sh.consumed;
+    } else {
+        ready = &lds[member].fwd.progress[FwdLds<S, FWD>::kReady];
+        consumed = &lds[member].fwd.progress[FwdLds<S, FWD>::kConsumed];
+    }
     if (wave < kGroupChunks && lane == 0) {
-        sh.ready = 0;
-        sh.consumed = 0;
-        if constexpr (FWD > 0) {
-            for (int x = 0; x < FWD; ++x) lds[member].fwd.published[x] = 0;
-            lds[member].fwd.taken = 0;
-        }
+        *ready = 0;
+        *consumed = 0;
+        if constexpr (FWD > 0)
+            for (int x = 0; x < FwdLds<S, FWD>::kCounters; ++x) lds[member].fwd.progress[x] = 0;
     }
     if constexpr (FWD > 0) fill_log_tables<OFK_SCAN_TWO_TIER, kBeamThreads<S, CPG, COLS, FWD>>(nullptr, all.logs.centred);
     for (int x = (int)threadIdx.x; x < OFK_LSE_DOUBLES; x += kBeamThreads<S, CPG, COLS, FWD>) lse[x] = lse_table[x];
@@ -589,17 +605,20 @@ __global__ __launch_bounds__((kBeamThreads<S, CPG, COLS, FWD>), (BeamCfg<S, CPG,
     if (n >= N) return;  // odd batch: the last group has one chunk
     if (Idx::kLone && wave > kFirstLoader) return;
 
-    static_assert((FWD & (FWD - 1)) == 0 && FWD <= 64, "a lane reads one wave's counter");
+    static_assert((FWD & (FWD - 1)) == 0 && FWD <= 8, "a lane reads one counter");
     if constexpr (FWD > 0) {
-        auto &fw = lds[member].fwd;
-        // whether every wave of the recursion has written row t of the state vector: a lane reads one counter
-        auto row_published = [&](int t) {
-            const int rows = __hip_atomic_load(&fw.published[lane & (FWD - 1)], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-            return ballot(rows <= t) == 0;
+        typedef FwdLds<S, FWD> Fwd;
+        Fwd &fw = lds[member].fwd;
+        // The counter of the lane, no wait included: what is read after it, in the order of the program, is from after it, because a
+        // wave's LDS operations are carried out in order (as are those of the wave that wrote rows first and its counter then).
+        auto progress = [&](int counter) {
+            const int rows = __hip_atomic_load(&fw.progress[counter], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+            wave_fence();
+            return rows;
         };
         if (recursion) {
             // ---- one wave of the forward recursion (same arithmetic as fwd_post_roles_kernel) ----
+            const int lane = lane_now();
             constexpr int SPL = S / (64 * FWD), Q = S / 4;
             const int w = (wave - kFirstFwd) % FWD;
             const int s0 = SPL * (64 * w + lane), q = s0 >> 2;
@@ -608,30 +627,29 @@ __global__ __launch_bounds__((kBeamThreads<S, CPG, COLS, FWD>), (BeamCfg<S, CPG,
             float f[SPL];
 #pragma unroll
             for (int k = 0; k < SPL; ++k) f[k] = 0.f;
-            int rows_ready = 0, rows_taken = 0, slot = 0;
+            int slot = 0;
             auto write_row = [&](int t) {
 #pragma unroll
                 for (int k = 0; k < SPL; ++k) fw.vec[t % kVecRows][s0 + k] = f[k];
             };
             auto publish_row = [&](int t) {
                 wave_fence();
-                __hip_atomic_store(&fw.published[w], t + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+                __hip_atomic_store(&fw.progress[w], t + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
             };
             write_row(0);
             publish_row(0);
+            // Step t needs row t of the vector from every wave, row t of the ring, and rows 0 .. t + 1 - kVecRows read by the posterior:
+            // row t + 1 goes where row t + 1 - kVecRows was.
+            const int counter = lane & (Fwd::kCounters - 1);
+            const int wanted = counter < FWD || counter == Fwd::kReady ? 1 : counter == Fwd::kTaken ? 2 - kVecRows : -(1 << 30);
             for (int t = 0; t < T; ++t) {
-                while (rows_ready <= t) {
-                    rows_ready = __builtin_amdgcn_readfirstlane(observe(&sh.ready));
-                    if (rows_ready <= t) __builtin_amdgcn_s_sleep(1);
-                }
+                // One look at all of that.  (The ring's counter, the posterior's and the other waves' polled one after another: 512 chunks
+                // of 256 states 1.041 | 1.008 ms, with five columns 1.060 | 1.036, 1024 of them 2.36 | 2.31.  The rows read together
+                // with the counters, again if it was too early: 1.037, 1.077, 2.28; 256 of 1024 states 1.76 instead of 1.68, and the
+                // clock lower for all that follows.)
+                while (ballot(progress(counter) < t + wanted) != 0) {}
                 LdsRow<SPL, COLS> row;
                 row.load(row_s[slot], s0);
-                slot = slot + 1 == LR ? 0 : slot + 1;
-                while (rows_taken < t + 2 - kVecRows) {  // rows 0 .. t - 1: row t + 1 goes where row t - 1 was
-                    rows_taken = __builtin_amdgcn_readfirstlane(observe(&fw.taken));
-                    if (rows_taken < t + 2 - kVecRows) __builtin_amdgcn_s_sleep(1);
-                }
-                while (!row_published(t)) {}
                 const float *vec = fw.vec[t % kVecRows];
                 const float p0 = vec[q], p1 = vec[q + Q], p2 = vec[q + 2 * Q], p3 = vec[q + 3 * Q];
                 float v[SPL][5];
@@ -643,6 +661,7 @@ __global__ __launch_bounds__((kBeamThreads<S, CPG, COLS, FWD>), (BeamCfg<S, CPG,
                     v[k][3] = ::add_half<0>(row.w[2 * k + 1], p2);
                     v[k][4] = ::add_half<1>(row.w[2 * k + 1], p3);
                 }
+                slot = slot + 1 == LR ? 0 : slot + 1;
                 lse5_all<SPL, OFK_SCAN_TWO_TIER>(f, v, logtab, [&] { write_row(t + 1); }, [](bool) {});
                 publish_row(t + 1);
             }
@@ -650,6 +669,7 @@ __global__ __launch_bounds__((kBeamThreads<S, CPG, COLS, FWD>), (BeamCfg<S, CPG,
         }
         if (wave >= kGroupChunks && wave < kFirstFwd) {
             // ---- posterior: softmax over the states of fwd[t] + bwd[t], t = 0 .. T ----
+            const int lane = lane_now();
             __builtin_amdgcn_s_setprio(1);
             constexpr int G = S / 256;  // pieces of four states per lane
             static_assert(G >= 1, "a lane holds at least four states");
@@ -663,8 +683,10 @@ __global__ __launch_bounds__((kBeamThreads<S, CPG, COLS, FWD>), (BeamCfg<S, CPG,
             const float shift = group_max<64>(top) - 10.0f;  // as in fwd_post_kernel
             float *prow = post + (size_t)n * (size_t)(T + 1) * S + 4 * lane;
             int slot = 0;
+            const int counter = lane & (Fwd::kCounters - 1);
+            const int wanted = counter < FWD ? 1 : -(1 << 30);
             for (int t = 0; t <= T; ++t) {
-                while (!row_published(t)) __builtin_amdgcn_s_sleep(2);
+                while (ballot(progress(counter) < t + wanted) != 0) __builtin_amdgcn_s_sleep(2);
                 float4 e[G];
 #pragma unroll
                 for (int g = 0; g < G; ++g) {
@@ -672,7 +694,7 @@ __global__ __launch_bounds__((kBeamThreads<S, CPG, COLS, FWD>), (BeamCfg<S, CPG,
                     if (t > 0) b[g] = *reinterpret_cast<const float4 *>(&row_b[slot][256 * g + 4 * lane]);
                 }
                 if (t > 0) slot = slot + 1 == LR ? 0 : slot + 1;
-                publish(&fw.taken, t + 1);
+                publish(&fw.progress[Fwd::kTaken], t + 1);
                 float total = 0.f;
 #pragma unroll
                 for (int g = 0; g < G; ++g) {
@@ -693,6 +715,7 @@ __global__ __launch_bounds__((kBeamThreads<S, CPG, COLS, FWD>), (BeamCfg<S, CPG,
     }
     if (wave >= kGroupChunks) {
         // ---- loader wave: row t = (scores[t], bwd[t+1]) into ring slot t % LR ----
+        const int lane = lane_now();
         // The ring is spelled out as named registers (not an array indexed by a loop that
         // also contains the spin wait) so that every row stays in VGPRs.
         typedef typename ScoreRow<S, COLS, FWD>::Regs Scores;
@@ -709,29 +732,20 @@ __global__ __launch_bounds__((kBeamThreads<S, CPG, COLS, FWD>), (BeamCfg<S, CPG,
                 // the ring is full most of the time (a search step takes about 3000 cycles): poll
                 // seldom, the rows in registers and in the ring leave ample slack for waking up late
                 if constexpr (FWD == 0) {
-                    while (t - observe(&sh.consumed) >= LR) __builtin_amdgcn_s_sleep(8);
+                    while (t - observe(consumed) >= LR) __builtin_amdgcn_s_sleep(8);
                 } else {
                     // the recursion is done with row p of scores once it has published row p + 1 of its vector,
                     // the posterior with row p of bwd (bwd[p + 1]) once it has taken row p + 1
-                    auto slots_free = [&] {
-                        int low = observe(&sh.consumed);
-                        const auto &fw = lds[member].fwd;
-                        const int taken = observe(const_cast<int *>(&fw.taken)) - 1;
-                        low = low < taken ? low : taken;
-#pragma unroll
-                        for (int x = 0; x < FWD; ++x) {
-                            const int done = observe(const_cast<int *>(&fw.published[x])) - 1;
-                            low = low < done ? low : done;
-                        }
-                        return low;
-                    };
-                    while (t >= LR && t - slots_free() >= LR) __builtin_amdgcn_s_sleep(2);
+                    typedef FwdLds<S, FWD> Fwd;
+                    const int counter = lane & (Fwd::kCounters - 1);
+                    const int wanted = counter <= Fwd::kTaken ? 2 - LR : counter == Fwd::kConsumed ? 1 - LR : -(1 << 30);
+                    while (t >= LR && ballot(observe(&lds[member].fwd.progress[counter]) < t + wanted) != 0) __builtin_amdgcn_s_sleep(2);
                 }
                 const int slot = t % LR;
                 rs.store(reinterpret_cast<char *>(row_s[slot]), lane);
                 rb.store(reinterpret_cast<char *>(row_b[slot]), lane);
                 fetch(rs, rb, t + RR);
-                publish(&sh.ready, t + 1);
+                publish(ready, t + 1);
             }
         };
         fetch(s0, g0, 0);
@@ -861,7 +875,7 @@ __global__ __launch_bounds__((kBeamThreads<S, CPG, COLS, FWD>), (BeamCfg<S, CPG,
         int rows = tt + (K >= 0 ? Cfg::kHandBack : 1);
         rows = rows < T ? rows : T;
         while (__builtin_expect(rows_ready < rows, 0)) {  // the counter is one LDS word: the same value in every lane
-            rows_ready = __builtin_amdgcn_readfirstlane(observe(&sh.ready));
+            rows_ready = __builtin_amdgcn_readfirstlane(observe(ready));
             if (rows_ready < rows) __builtin_amdgcn_s_sleep(1);
         }
     };
@@ -871,10 +885,12 @@ __global__ __launch_bounds__((kBeamThreads<S, CPG, COLS, FWD>), (BeamCfg<S, CPG,
         if (__builtin_expect(round == Idx::kRoundEnd, 0)) {
             round = Idx::kRound;
             typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+            uint32_t zero;
+            asm volatile("v_mov_b32 %0, 0" : "=v"(zero));  // here, not in registers through the search
             u32x4 none;
-            none.x = none.y = none.z = none.w = 0u;
+            none.x = none.y = none.z = none.w = zero;
 #pragma unroll 1
-            for (uint32_t at = 0; at < 4u * Idx::kBuckets; at += 1024u) *(LDS_AS u32x4 *)(uintptr_t)(idx_base + at + 16u * (uint32_t)lane) = none;
+            for (uint32_t at = 0; at < 4u * Idx::kBuckets; at += 1024u) *(LDS_AS u32x4 *)(uintptr_t)(idx_base + at + 16u * (uint32_t)lane_now()) = none;
             wave_fence();
         }
     };
@@ -1011,7 +1027,7 @@ __global__ __launch_bounds__((kBeamThreads<S, CPG, COLS, FWD>), (BeamCfg<S, CPG,
             // Merges in parallel need every stay to have one partner and every step candidate one claimant.
             // Otherwise (only possible after a CRC collision; flags bit 0 forces it) the merges are
             // replayed one by one in the CPU path's order, from the scores as they were before any merge.
-            const uint32_t claim_at = (uint32_t)pick_by_bit(mine_mask, (int)(4u * j + ((uint32_t)state & 3u)), 4 * kW + lane);
+            const uint32_t claim_at = (uint32_t)pick_by_bit(mine_mask, (int)(4u * j + ((uint32_t)state & 3u)), 4 * kW + lane_now());
             sh.claim[claim_at] = (uint32_t)i;
             wave_fence();
             const uint32_t claimed = sh.claim[claim_at];
@@ -1019,7 +1035,7 @@ __global__ __launch_bounds__((kBeamThreads<S, CPG, COLS, FWD>), (BeamCfg<S, CPG,
             if ((ballot(odd != 0u) & mine_mask) != 0 || (flags & 1)) {
                 if (h == 0) sh.stay_score[i] = cs0;
                 wave_fence();
-                if (lane == 0) {
+                if (lane_now() == 0) {
                     for (int a = 0; a < w; ++a) {
                         const uint32_t ha = sh.elem[a].hash;
                         const uint32_t base = sh.elem[a].info & 3u;
@@ -1067,7 +1083,7 @@ __global__ __launch_bounds__((kBeamThreads<S, CPG, COLS, FWD>), (BeamCfg<S, CPG,
         }
         // no wait before this store: the wave's reads of row t are ahead of it in the LDS queue
         if constexpr (K < 0 || K % Cfg::kHandBack == 0)
-            __hip_atomic_store(&sh.consumed, next_t, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+            __hip_atomic_store(consumed, next_t, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
         const uint64_t stay_wins = ballot(cs0 > other) & mine_mask;
         const uint64_t step_wins = mine_mask & ~stay_wins;
         const uint32_t target = (uint32_t)pick_by_bit(mine_mask, (int)at, (int)cand_dump);
@@ -1165,7 +1181,7 @@ __global__ __launch_bounds__((kBeamThreads<S, CPG, COLS, FWD>), (BeamCfg<S, CPG,
                         }
                         if (kept > kW) {
                             const int rank0 = lower(k1, lower(k0, 0));
-                            const int rank1 = rank0 + (int)((k0 >> lane) & 1);
+                            const int rank1 = add_bit_of(rank0, k0);
                             const int ranks = lower(ks, steps_kept);
                             k0 &= ballot(rank0 < kW);
                             k1 &= ballot(rank1 < kW);
@@ -1286,6 +1302,7 @@ __global__ __launch_bounds__((kBeamThreads<S, CPG, COLS, FWD>), (BeamCfg<S, CPG,
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
     {
         constexpr int RB = 128;  // rows per block
+        const int lane = lane_now();
         static_assert(2 * RB * kW * (int)sizeof(ofk_beam_slot_t) <= Idx::kBuckets * 4, "two blocks fit the index");
         int32_t *st_out = states + (size_t)n * T;
         uint8_t *mv_out = moves + (size_t)n * T;
