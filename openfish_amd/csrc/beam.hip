@@ -68,10 +68,15 @@ __device__ __forceinline__ uint32_t crc_tab(uint32_t x) {
 __device__ __forceinline__ uint32_t crc2(uint32_t crc, uint32_t base) {
     return (crc >> 2) ^ crc_tab((crc ^ base) & 3u);
 }
-// the hash h with crc2(h, base) == crc
+// (a & b) ^ c in one instruction (in the order that the compiler finds by itself the inverse below takes two more)
+__device__ __forceinline__ uint32_t and_xor(uint32_t a, uint32_t b, uint32_t c) { return __builtin_amdgcn_bitop3_b32(a, b, c, 0x6a); }
+// the hash h with crc2(h, base & 3) == crc: ((crc ^ entry k) << 2) | (k ^ base), k the two top bits.  With the entries' top bits
+// left out those of crc stay, and come round to the bottom.
 __device__ __forceinline__ uint32_t crc2_inverse(uint32_t crc, uint32_t base) {
-    const uint32_t k = crc >> 30;
-    return ((crc ^ crc_tab(k)) << 2) | (k ^ base);
+    const uint32_t bit0 = (uint32_t)((int32_t)(crc << 1) >> 31), bit1 = (uint32_t)((int32_t)crc >> 31);
+    uint32_t x = and_xor(bit0, kTab1 & 0x3fffffffu, crc);
+    x = and_xor(bit1, kTab2 & 0x3fffffffu, x);
+    return and_xor(base, 3u, __builtin_amdgcn_alignbit(x, x, 30));
 }
 __device__ __forceinline__ uint32_t crc32_word(uint32_t crc, uint32_t word) {
     for (int i = 0; i < 16; ++i) {
@@ -924,9 +929,10 @@ __global__ __launch_bounds__((kBeamThreads<S, CPG, COLS, FWD>), (BeamCfg<S, CPG,
         g01 = lds_load_f2((cand << 2) + rb);
         gst = lds_load_f(st4 + rb);
         __builtin_amdgcn_sched_barrier(0);
-        want = crc2_inverse(hash, (uint32_t)state & 3u);
+        want = crc2_inverse(hash, info);  // the last base: the two lowest bits
         probe = *(const lds_u32 *)(uintptr_t)and_or(want, Idx::kAddress, idx_base);
         mine_back = own_p[0];
+        __builtin_amdgcn_sched_barrier(0);  // nothing that waits for the row goes before the look-up
         expected = and_or(want, hash_keep, gen);
     };
     typedef std::integral_constant<int, -1> AnySlot;
