@@ -34,6 +34,15 @@ __device__ __forceinline__ void copy_out(unsigned char *dst, const unsigned char
     for (int i = tail + lane; i < hi + skew; i += lanes) d[i] = l[i];
 }
 
+// A posterior that is gathered.  Rows of 256 and 1024 states give a line or two for several values each and none of them again: they
+// pass by the caches.  Rows of 64 states are two lines, which nine values share.  Stage inside decodes, us, kept | passed by: 256 chunks
+// of 1024 states 84 | 70, 512 of 256 states 131 | 130, 403 of them (T = 1201) 81 | 79, 1024 of 64 states 125 | 182.
+template <int S>
+__device__ __forceinline__ float gathered(const float *p) {
+    if constexpr (S >= 256) return __builtin_nontemporal_load(p);
+    else return *p;
+}
+
 // LDS of a chunk: two 4-byte tables, a 2-byte one and three of bytes with room for their skews.
 constexpr size_t sequence_lds(int T) {
     const size_t t16 = ((size_t)T + 15) & ~(size_t)15;
@@ -45,7 +54,7 @@ constexpr size_t sequence_lds(int T) {
 // the posteriors comes first: base positions, the characters of the sequence and the zeros behind both strings, which one wave
 // then writes to their place (host memory, in a decode) while the others gather.  What is left after the gathers is a base's
 // character.  Inside decodes, ms, against gathers first, bytes last and one at a time, 256 lanes: 1 chunk of 64 states 0.021 ->
-// 0.014; 512 of 256 states 0.167 -> 0.130, 1024 of them 0.328 -> 0.263; 256 of 1024 0.103 -> 0.084.
+// 0.014; 512 of 256 states 0.167 -> 0.130, 1024 of them 0.328 -> 0.263; 256 of 1024 0.103 -> 0.084 (0.070 past the caches).
 template <int S, int kThreads>
 __global__ __launch_bounds__(kThreads) void sequence_kernel(
     const float *__restrict__ post, int32_t *__restrict__ states, const uint8_t *__restrict__ moves,
@@ -136,7 +145,7 @@ __global__ __launch_bounds__(kThreads) void sequence_kernel(
                 prob = path_sums[(first + t) * S + st];
             } else {
                 const float *p = post_n + (size_t)(t + 1) * S;
-                prob = p[st];
+                prob = gathered<S>(p + st);
                 int nb[8];
 #pragma unroll
                 for (int b = 0; b < 4; ++b) {
@@ -145,7 +154,7 @@ __global__ __launch_bounds__(kThreads) void sequence_kernel(
                 }
                 float x[8];  // all in flight together
 #pragma unroll
-                for (int k = 0; k < 8; ++k) x[k] = p[nb[k]];
+                for (int k = 0; k < 8; ++k) x[k] = gathered<S>(p + nb[k]);
 #pragma unroll
                 for (int k = 0; k < 8; ++k) {
                     bool fresh = nb[k] != st;
