@@ -1139,11 +1139,16 @@ constexpr int kPlainSpl = S >= 1024 ? 2 : 1;
 template <int S, int SPL, int DEPTH>
 int launch_bwd(int mode, const void *scores, float *bwd, int T, int N, float stay, Queue st) {
     using Sh = Shape<S, SPL>;
+    // Rows in flight where the memory's latency shows, which is with one state to a lane: 8 (1024 states: 6) | 12 (8) | 16 (10) | 20 (12)
+    // rows, ms, T = 1666: 512 chunks of 64 states 0.432 | 0.414 | 0.399 | 0.393, 512 of 256 states 0.733 | 0.711 | 0.700 | 0.694, 256 of
+    // 1024 states 1.262 | 1.235 | 1.25 | 1.227; 20 take so many registers that 1000 chunks of 256 states find no room (T = 1000: 0.70, 0.88).
+    // Several states to a lane fill the machine with fewer rows (1024 chunks of 256 states: 1.26 with 5, 8 or 12).
+    constexpr int kDeep = SPL > 1 ? DEPTH : S >= 1024 ? 8 : 16;
     const dim3 grid((N + Sh::kChunks - 1) / Sh::kChunks), block(Sh::kThreads);
     const _Float16 *sc = static_cast<const _Float16 *>(scores);
     switch (mode) {
         case OFK_SCAN_TWO_TIER:
-            queue_kernel((bwd_scan_kernel<S, SPL, DEPTH, OFK_SCAN_TWO_TIER>), grid, block, 0, st, sc, bwd, T, N, stay, kSeries);
+            queue_kernel((bwd_scan_kernel<S, SPL, kDeep, OFK_SCAN_TWO_TIER>), grid, block, 0, st, sc, bwd, T, N, stay, kSeries);
             break;
         case OFK_SCAN_PRECISE:
             if constexpr (SPL == kPlainSpl<S>)
