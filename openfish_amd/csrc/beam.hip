@@ -24,11 +24,11 @@
 // of the element's sequence without its last base.  Every beam element carries both
 // words (a candidate's `want` is its parent's hash, or its parent's `want` for a stay), and
 // the element j is found through a hash index in LDS: every live element files
-// {hash, generation << 5 | slot} under some bits of its hash, reads its own entry back, and
-// looks up the entry filed under the same bits of `want`.  If every element finds its own
+// one word (the hash, with generation and slot in place of the bits that choose the bucket) under
+// those bits of its hash, reads its own entry back, and looks up the entry filed under the same bits of `want`.  If every element finds its own
 // entry intact, all hashes are pairwise distinct and every existing partner is found by
 // exactly one probe (the full 32 bits are compared); otherwise (two elements in one
-// bucket, about one step in ten; equal hashes, only after a CRC collision) the step
+// bucket, one step in twenty to forty; equal hashes, only after a CRC collision) the step
 // falls back to comparing `want` with all 32 hashes.
 #include <hip/hip_runtime.h>
 
@@ -947,9 +947,10 @@ __global__ __launch_bounds__((kBeamThreads<S, CPG, COLS, FWD>), (BeamCfg<S, CPG,
     //
     // The wave is alone on its SIMD: a step costs its instructions, about four cycles each, plus the
     // LDS round trips and the reads of comparison masks by the scalar unit (about twenty cycles) that
-    // nothing is placed into (about 1310 cycles for 1 chunk of 64 or 256 states: 0.94 ms at T = 1666; in the order of the
-    // text, with every wait where its value is first needed, 1.02 ms).  Hence the order below: what does not depend on a round trip is issued
-    // while it is under way, comparisons are issued in groups whose masks are read afterwards.
+    // nothing is placed into (about 1210 cycles for 1 chunk of 64 or 256 states: 0.87 ms at T = 1666; before steps were written out and
+    // rows kept in planes 0.93; in the order of the text, with every wait where its value is first needed, 1.02).  Hence the order
+    // below: what does not depend on a round trip is issued while it is under way, comparisons are issued in groups whose masks are
+    // read afterwards.
     auto step = [&](const int next_t, auto k_tag, auto last_tag) {  // next_t - 1 is the time step, K the ring slot of row next_t
         constexpr int K = decltype(k_tag)::value;
         constexpr bool LAST = decltype(last_tag)::value;

@@ -514,7 +514,7 @@ static void join_null_stream(ofa_gpubuf_t *g) {
  * compute units of their own; above 256 merged takes a second round of workgroups, split does so only above 320; chunks
  * shorter than 128 steps are decided by launches and set-up: split is ahead where it has its sweeps apart, but for the very
  * shortest of few chunks, and one kernel above 320.  Up to 512 chunks of 256 states the chain of split is
- * shorter, while its bytes fit beneath the chain, 3.8 MB a step; above, the search's workgroups hold four chunks, a unit
+ * shorter, while its bytes fit beneath the chain, 3.3 MB a step; above, the search's workgroups hold four chunks, a unit
  * that has one of them in the merged kernel takes 2.3 ms whatever the others do, and split has units left for the
  * forward sweep up to three chunks to a unit.
  *
