@@ -1,6 +1,7 @@
 """The streams of the gpubufs: whichever hardware queues the runtime deals them to, a split decode has to run its
 forward sweep beside the beam search, and two batches in flight have to run side by side, with one gpubuf in the
 process and with several."""
+import ctypes as C
 import threading
 import time
 
@@ -91,3 +92,33 @@ def test_gpubufs_made_used_and_freed_by_several_threads(api, scores):  # noqa: F
     for th in threads:
         th.join()
     assert not wrong, wrong
+
+
+@pytest.mark.parametrize("producer", ["null stream", "stream that waits for the null stream"])
+def test_a_decode_waits_for_scores_that_are_still_on_their_way(api, producer):  # noqa: F811
+    """scores copied into place behind 10 ms of other copies, by the null stream or by one ordered with it: the decode, which looks whether
+    the null stream is idle, has to see the new ones"""
+    hip = api.lib()  # the runtime's functions, through the library that is linked against it
+    stream = C.c_void_p()
+    if producer != "null stream":
+        assert hip.hipStreamCreate(C.byref(stream)) == 0
+    old, new = (synth.crf_scores(200, 16, STATE_LEN, seed=s) for s in (11, 12))
+    at, source = api.DeviceBuffer.from_host(old), api.DeviceBuffer.from_host(new)
+    busy = [api.DeviceBuffer(1 << 28) for _ in range(2)]
+    gb, opt = api.GpuBuf(200, 16, STATE_LEN), api.DECODER_INIT()
+    want = api.openfish_decode_gpu(200, 16, 4 * S, source.ptr, STATE_LEN, opt, gb)
+    hip.hipDeviceSynchronize()
+
+    def copy(to, from_, nbytes):  # 3: device to device
+        assert hip.hipMemcpyAsync(C.c_void_p(to), C.c_void_p(from_), C.c_size_t(nbytes), 3, stream) == 0
+
+    for _ in range(80):
+        copy(busy[0].ptr, busy[1].ptr, 1 << 28)
+    copy(at.ptr, source.ptr, new.nbytes)
+    got = api.openfish_decode_gpu(200, 16, 4 * S, at.ptr, STATE_LEN, opt, gb)
+    hip.hipDeviceSynchronize()
+    if stream:
+        assert hip.hipStreamDestroy(stream) == 0
+    for b in busy + [at, source]:
+        b.free()
+    assert all(np.array_equal(a, b) for a, b in zip(got, want))
