@@ -479,8 +479,12 @@ static void fetch_outputs(ofa_gpubuf_t *g, int T, int N, uint8_t **moves, char *
 
 /* Order the library's streams after everything already queued on the null stream (and on the streams that wait for it).  Where that
  * has ended already, which the query tells in 0.2 us, there is nothing to wait for: the event and the wait for it in another hardware
- * queue put 20 us before a decode's first kernel. */
+ * queue put 20 us before a decode's first kernel.  It is the current device's null stream: a gpubuf of another device is refused, as
+ * recording its event there is by the runtime. */
 static void join_null_stream(ofa_gpubuf_t *g) {
+    int device;
+    HIP_OK(hipGetDevice(&device));
+    if (device != g->device) die("the gpubuf belongs to another device than the current one");
     if (hipStreamQuery(0) == hipSuccess) return;
     (void)hipGetLastError(); /* the query's answer; what is wrong, if anything, the calls below say */
     HIP_OK(hipEventRecord(g->ev[EV_JOIN], 0));

@@ -1,0 +1,67 @@
+"""What the host code refuses and what it asks of the runtime before a decode's first kernel: openfish_host.c against a HIP runtime
+of two devices that executes nothing (host_stub.c), a process per case, because a refusal ends the process."""
+import os
+import subprocess
+import sys
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+CSRC = os.path.join(ROOT, "openfish_amd", "csrc")
+
+DRIVER = """
+import ctypes as C, sys
+L = C.CDLL(sys.argv[1])
+L.openfish_gpubuf_init.restype = C.c_void_p
+class Opt(C.Structure):
+    _fields_ = [("w", C.c_size_t), ("f", C.c_float * 5), ("pad", C.c_bool)]
+opt = Opt(32, (C.c_float * 5)(100.0, 2.0, 0.0, 1.0, 1.0), False)
+T, N, SL = 8, 2, 3
+scores = C.create_string_buffer(2 * T * N * 4 * 64)
+tensor = C.create_string_buffer(4 * N * (T + 1) * 64)
+busy = (C.c_int * 2).in_dll(L, "stub_null_busy")
+out = [C.c_void_p() for _ in range(3)]
+refs = [C.byref(p) for p in out]
+def buf():
+    return C.c_void_p(L.openfish_gpubuf_init(T, N, SL))
+def decode(g):
+    L.openfish_decode_gpu(T, N, 256, scores, SL, C.byref(opt), g, *refs)
+def enqueue(g):
+    L.openfish_amd_decode_enqueue(T, N, 256, scores, SL, C.byref(opt), g)
+    L.openfish_amd_decode_wait(g, *refs)
+def from_tensors(g):
+    L.openfish_amd_decode_from_tensors(T, N, 256, scores, SL, C.byref(opt), tensor, tensor, g, *refs)
+def seen(name):
+    return C.c_int.in_dll(L, name).value
+"""
+
+
+@pytest.fixture(scope="module")
+def run(tmp_path_factory):
+    so = str(tmp_path_factory.mktemp("host") / "host.so")
+    subprocess.check_call(["gcc", "-O1", "-shared", "-fPIC", "-std=gnu11", "-D__HIP_PLATFORM_AMD__", "-Wl,-Bsymbolic",
+                           "-I", os.path.join(ROOT, "include"), "-I", CSRC, "-I", "/opt/rocm/include",
+                           os.path.join(CSRC, "openfish_host.c"), os.path.join(ROOT, "tests", "host_stub.c"), "-o", so, "-lm", "-lpthread"])
+
+    def go(code):
+        return subprocess.run([sys.executable, "-c", DRIVER + code, so], capture_output=True, text=True)
+    return go
+
+
+CALLS = ["decode", "enqueue", "from_tensors"]
+
+
+@pytest.mark.parametrize("busy", [0, 1])
+@pytest.mark.parametrize("call", CALLS)
+def test_a_decode_on_its_own_device_goes_through(run, call, busy):
+    """and waits for the null stream where that has work left"""
+    done = run("L.set_device_hip(1); g = buf(); busy[1] = %d; %s(g); print('joins', seen('stub_null_joins'))" % (busy, call))
+    assert done.returncode == 0 and done.stdout == "joins %d\n" % busy, done
+
+
+@pytest.mark.parametrize("busy", [0, 1])
+@pytest.mark.parametrize("call", CALLS)
+def test_a_gpubuf_of_another_device_is_refused(run, call, busy):
+    """whatever the null stream of the present device is doing: it is not the one that the scores may still be on their way on"""
+    done = run("g = buf(); L.set_device_hip(1); busy[0] = 1; busy[1] = %d; %s(g); print('went on')" % (busy, call))
+    assert done.returncode == 1 and "went on" not in done.stdout, done
