@@ -486,7 +486,7 @@ static void join_null_stream(ofa_gpubuf_t *g) {
     HIP_OK(hipGetDevice(&device));
     if (device != g->device) die("the gpubuf belongs to another device than the current one");
     if (hipStreamQuery(0) == hipSuccess) return;
-    (void)hipGetLastError(); /* the query's answer; what is wrong, if anything, the calls below say */
+    if (hipPeekAtLastError() == hipErrorNotReady) (void)hipGetLastError(); /* the query's answer, but no error that the caller left behind */
     HIP_OK(hipEventRecord(g->ev[EV_JOIN], 0));
     HIP_OK(hipStreamWaitEvent(g->s_main, g->ev[EV_JOIN], 0));
 }

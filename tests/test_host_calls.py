@@ -65,3 +65,11 @@ def test_a_gpubuf_of_another_device_is_refused(run, call, busy):
     """whatever the null stream of the present device is doing: it is not the one that the scores may still be on their way on"""
     done = run("g = buf(); L.set_device_hip(1); busy[0] = 1; busy[1] = %d; %s(g); print('went on')" % (busy, call))
     assert done.returncode == 1 and "went on" not in done.stdout, done
+
+
+@pytest.mark.parametrize("busy", [0, 1])
+@pytest.mark.parametrize("call", CALLS)
+def test_an_error_that_the_caller_left_behind_is_still_reported(run, call, busy):
+    """the launch of the kernel that was to make the scores, say: the first launch of the decode finds it"""
+    done = run("g = buf(); busy[0] = %d; L.stub_fail(); %s(g); print('went on')" % (busy, call))
+    assert done.returncode == 1 and "invalid configuration" in done.stderr and "went on" not in done.stdout, done
