@@ -479,8 +479,9 @@ static void fetch_outputs(ofa_gpubuf_t *g, int T, int N, uint8_t **moves, char *
 
 /* Order the library's streams after everything already queued on the null stream (and on the streams that wait for it).  Where that
  * has ended already, which the query tells in 0.2 us, there is nothing to wait for: the event and the wait for it in another hardware
- * queue put 20 us before a decode's first kernel.  It is the current device's null stream: a gpubuf of another device is refused, as
- * recording its event there is by the runtime. */
+ * queue put 20 us before a decode's first kernel.  That the query answers for the streams ordered with the null stream too is this
+ * runtime's doing, and tested for copies and kernels of both.  It is the current device's null stream: a gpubuf of another device is
+ * refused, as recording its event there is by the runtime. */
 static void join_null_stream(ofa_gpubuf_t *g) {
     int device;
     HIP_OK(hipGetDevice(&device));

@@ -94,10 +94,11 @@ def test_gpubufs_made_used_and_freed_by_several_threads(api, scores):  # noqa: F
     assert not wrong, wrong
 
 
+@pytest.mark.parametrize("work", ["copies", "kernels"])
 @pytest.mark.parametrize("producer", ["null stream", "stream that waits for the null stream"])
-def test_a_decode_waits_for_scores_that_are_still_on_their_way(api, producer):  # noqa: F811
-    """scores copied into place behind 10 ms of other copies, by the null stream or by one ordered with it: the decode, which looks whether
-    the null stream is idle, has to see the new ones"""
+def test_a_decode_waits_for_scores_that_are_still_on_their_way(api, producer, work):  # noqa: F811
+    """scores copied into place behind 10 ms of other copies, by the null stream or by one ordered with it, by the runtime's copies or by
+    kernels: the decode, which looks whether the null stream is idle, has to see the new ones"""
     hip = api.lib()  # the runtime's functions, through the library that is linked against it
     stream = C.c_void_p()
     if producer != "null stream":
@@ -109,7 +110,11 @@ def test_a_decode_waits_for_scores_that_are_still_on_their_way(api, producer):  
     want = api.openfish_decode_gpu(200, 16, 4 * S, source.ptr, STATE_LEN, opt, gb)
     hip.hipDeviceSynchronize()
 
-    def copy(to, from_, nbytes):  # 3: device to device
+    def copy(to, from_, nbytes):
+        if work == "kernels":
+            assert hip.ofk_copy(C.c_void_p(to), C.c_void_p(from_), C.c_size_t(nbytes), stream) == 0
+            return
+        # 3: device to device
         assert hip.hipMemcpyAsync(C.c_void_p(to), C.c_void_p(from_), C.c_size_t(nbytes), 3, stream) == 0
 
     for _ in range(80):
