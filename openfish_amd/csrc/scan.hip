@@ -1136,18 +1136,46 @@ const LogSeries kSeries = {OFA_LOG_SERIES, OFA_EXP_COEFS};
 template <int S>
 constexpr int kPlainSpl = S >= 1024 ? 2 : 1;
 
+// Rows that the backward sweep keeps in flight with one state to a lane and the default arithmetic: 8 (1024 states: 6) | 12 (8) | 16 (10) |
+// 20 (12) rows, ms, T = 1666: 512 chunks of 64 states 0.432 | 0.414 | 0.399 | 0.393, 512 of 256 states 0.733 | 0.711 | 0.700 | 0.694, 256 of
+// 1024 states 1.262 | 1.235 | 1.25 | 1.227; 20 take so many registers that 1000 chunks of 256 states find no room (T = 1000: 0.70, 0.88).
+// Several states to a lane fill the machine with fewer rows (1024 chunks of 256 states: 1.26 with 5, 8 or 12).
+#ifndef OFK_DEPTH_DEEP
+#define OFK_DEPTH_DEEP 16
+#endif
+#ifndef OFK_DEPTH_DEEP_1024
+#define OFK_DEPTH_DEEP_1024 8
+#endif
+
+// Where sixteen rows, 120 registers, cost more than they give, and eight, 88 to 90 registers, are kept instead.
+// More than four waves for every SIMD of 256 compute units, which only states per lane that were asked for bring about: 256 states, one to a
+// lane, T = 300, ms, 8 | 16 rows: 1024 chunks 0.249 | 0.251, 1100 0.296 | 0.347, 2048 0.468 | 0.487, 2100 0.515 | 0.553; 8192 of 64 0.443 | 0.454.
+// Beside another decode's merged kernel of 256 states, whose waves of 104 registers, up to four on a SIMD, leave room for the one but not for
+// the other, as soon as that kernel leaves too few units free.  Two decodes in flight, ms, 8 | 16 rows, T = 1666: 335 chunks 2.956 | 2.944,
+// 375 2.997 | 2.984, 385 3.010 | 3.061, 395 3.075 | 3.173, 512 3.350 | 3.416; T = 600: 375 1.204 | 1.206, 385 1.209 | 1.213, 395 1.233 | 1.274;
+// T = 1000: 704 3.38 | 3.47, 900 4.32 | 4.43.  Its waves of 114 registers with five columns leave room for neither, T = 1201: 403 2.456 | 2.459,
+// 512 2.637 | 2.651.  Smaller models and batches are ahead with sixteen (128 chunks 1.769 | 1.745, 512 of 64 states 2.579 | 2.540).
+constexpr long kWavesOfDepth16 = 4096;
+constexpr int kChunksBesideMerged = 384;
+template <int S>
+bool eight_rows(int N, int beside_merged) {
+    return (long)N * (S / 64) > kWavesOfDepth16 || (S == 256 && beside_merged && N > kChunksBesideMerged);
+}
+
 template <int S, int SPL, int DEPTH>
-int launch_bwd(int mode, const void *scores, float *bwd, int T, int N, float stay, Queue st) {
+int launch_bwd(int mode, const void *scores, float *bwd, int T, int N, float stay, int beside_merged, Queue st) {
     using Sh = Shape<S, SPL>;
-    // Rows in flight where the memory's latency shows, which is with one state to a lane: 8 (1024 states: 6) | 12 (8) | 16 (10) | 20 (12)
-    // rows, ms, T = 1666: 512 chunks of 64 states 0.432 | 0.414 | 0.399 | 0.393, 512 of 256 states 0.733 | 0.711 | 0.700 | 0.694, 256 of
-    // 1024 states 1.262 | 1.235 | 1.25 | 1.227; 20 take so many registers that 1000 chunks of 256 states find no room (T = 1000: 0.70, 0.88).
-    // Several states to a lane fill the machine with fewer rows (1024 chunks of 256 states: 1.26 with 5, 8 or 12).
-    constexpr int kDeep = SPL > 1 ? DEPTH : S >= 1024 ? 8 : 16;
+    constexpr int kDeep = SPL > 1 ? DEPTH : S >= 1024 ? OFK_DEPTH_DEEP_1024 : OFK_DEPTH_DEEP;
     const dim3 grid((N + Sh::kChunks - 1) / Sh::kChunks), block(Sh::kThreads);
     const _Float16 *sc = static_cast<const _Float16 *>(scores);
     switch (mode) {
         case OFK_SCAN_TWO_TIER:
+            if constexpr (SPL == 1 && S <= 256) {
+                if (eight_rows<S>(N, beside_merged)) {
+                    queue_kernel((bwd_scan_kernel<S, SPL, DEPTH, OFK_SCAN_TWO_TIER>), grid, block, 0, st, sc, bwd, T, N, stay, kSeries);
+                    break;
+                }
+            }
             queue_kernel((bwd_scan_kernel<S, SPL, kDeep, OFK_SCAN_TWO_TIER>), grid, block, 0, st, sc, bwd, T, N, stay, kSeries);
             break;
         case OFK_SCAN_PRECISE:
@@ -1263,8 +1291,9 @@ int states_per_lane(int S, int N, bool backward, int forced) {
 // apart; when that is a multiple of 4 MiB (2048 chunks of 256 states, 512 of 1024) all rows in
 // flight fall onto the same DRAM banks, and with sixteen of them (eight per sweep) the kernel ran
 // at half its rate and below (measured, 256 states, 2048 chunks: 8.97 ms; with four rows per sweep
-// 5.69 ms, the rate of smaller batches; at 512 chunks both depths take 1.59 ms).  The separate
-// sweeps, eight rows in flight altogether, never showed it.  Hence half the depth here.
+// 5.69 ms, the rate of smaller batches; at 512 chunks both depths take 1.59 ms).  Hence half the depth
+// here.  The separate sweeps, one row stored for every row read, do not show it, with sixteen rows either (backward, one state to a
+// lane, T = 300, eight | sixteen rows: 2000 chunks 0.471 | 0.484, 2048 0.468 | 0.487).
 #ifndef OFK_DEPTH_FUSED
 #define OFK_DEPTH_FUSED 4
 #endif
@@ -1325,7 +1354,7 @@ static int scan_posterior(const void *scores, float *bwd, float *post, int T, in
 }
 
 static int bwd_scan(const void *scores, float *bwd, int T, int N, int state_len, float stay, int mode, int spl,
-                    void *stream, void *done) {
+                    int beside_merged, void *stream, void *done) {
     if (!scores || !bwd || T < 1 || N < 1 || !aligned16(scores) || !aligned16(bwd)) return OFK_BAD_ARGS;
     if (state_len < 3 || state_len > 5) return OFK_BAD_ARGS;
     const Queue st{static_cast<hipStream_t>(stream), static_cast<hipEvent_t>(done)};
@@ -1334,8 +1363,8 @@ static int bwd_scan(const void *scores, float *bwd, int T, int N, int state_len,
     // lane | one: 37 chunks, T = 833 0.76 | 0.67; 256, T = 1666 1.45 | 1.32; 9, T = 64 0.091 | 0.078).  Two such workgroups do
     // not fit a unit (257 chunks, T = 400 0.55 | 0.71; 512 0.68 | 0.75; 1024, T = 300 1.05 | 1.15).
     if (state_len == 5 && mode == OFK_SCAN_TWO_TIER && spl == 0 && N <= 256)
-        return launch_bwd<1024, 1, OFK_DEPTH_1024>(mode, scores, bwd, T, N, stay, st);
-    OFK_DISPATCH(true, launch_bwd, mode, scores, bwd, T, N, stay, st)
+        return launch_bwd<1024, 1, OFK_DEPTH_1024>(mode, scores, bwd, T, N, stay, beside_merged, st);
+    OFK_DISPATCH(true, launch_bwd, mode, scores, bwd, T, N, stay, beside_merged, st)
 }
 
 static int fwd_post_scan(const void *scores, const float *bwd, float *post, int T, int N, int state_len,
@@ -1362,8 +1391,8 @@ extern "C" int ofk_scan_posterior_five(const void *scores, float *bwd, float *po
     return scan_posterior(scores, bwd, post, T, N, state_len, stay, mode, spl, stream, done);
 }
 extern "C" int ofk_bwd_scan_five(const void *scores, float *bwd, int T, int N, int state_len, float stay, int mode,
-                                 int spl, void *stream, void *done) {
-    return bwd_scan(scores, bwd, T, N, state_len, stay, mode, spl, stream, done);
+                                 int spl, int beside_merged, void *stream, void *done) {
+    return bwd_scan(scores, bwd, T, N, state_len, stay, mode, spl, beside_merged, stream, done);
 }
 extern "C" int ofk_fwd_post_scan_five(const void *scores, const float *bwd, float *post, int T, int N,
                                       int state_len, float stay, int mode, int spl, void *stream, void *done) {
@@ -1374,7 +1403,7 @@ extern "C" int ofk_fwd_scan_five(const void *scores, float *fwd, int T, int N, i
 }
 #else
 extern "C" int ofk_scan_posterior_five(const void *, float *, float *, int, int, int, float, int, int, void *, void *);
-extern "C" int ofk_bwd_scan_five(const void *, float *, int, int, int, float, int, int, void *, void *);
+extern "C" int ofk_bwd_scan_five(const void *, float *, int, int, int, float, int, int, int, void *, void *);
 extern "C" int ofk_fwd_post_scan_five(const void *, const float *, float *, int, int, int, float, int, int, void *, void *);
 extern "C" int ofk_fwd_scan_five(const void *, float *, int, int, int, float, void *, void *);
 
@@ -1386,10 +1415,10 @@ extern "C" int ofk_scan_posterior(const void *scores, float *bwd, float *post, i
 }
 
 extern "C" int ofk_bwd_scan(const void *scores, float *bwd, int T, int N, int state_len, int columns, float stay,
-                            int mode, int spl, void *stream, void *done) {
-    if (columns == 5) return ofk_bwd_scan_five(scores, bwd, T, N, state_len, stay, mode, spl, stream, done);
+                            int mode, int spl, int beside_merged, void *stream, void *done) {
+    if (columns == 5) return ofk_bwd_scan_five(scores, bwd, T, N, state_len, stay, mode, spl, beside_merged, stream, done);
     if (columns != 4) return OFK_BAD_ARGS;
-    return bwd_scan(scores, bwd, T, N, state_len, stay, mode, spl, stream, done);
+    return bwd_scan(scores, bwd, T, N, state_len, stay, mode, spl, beside_merged, stream, done);
 }
 
 extern "C" int ofk_fwd_post_scan(const void *scores, const float *bwd, float *post, int T, int N, int state_len,

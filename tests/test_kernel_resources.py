@@ -34,19 +34,33 @@ def code_objects(blob):
         at = blob.find(BUNDLE, at + 1)
 
 
-def test_no_kernel_keeps_registers_in_scratch(tmp_path):
+def most_of(field, tmp_path):
+    """the largest value of a field of the kernels' notes, by name (the scans are built twice, for both layouts of the scores)"""
     if not os.path.exists(READELF):
         pytest.skip("no llvm-readelf")
     blob = open(os.path.join(ROOT, "openfish_amd", "libopenfish_amd.so"), "rb").read()
-    scratch = {}
+    most = {}
     for i, code in enumerate(code_objects(blob)):
         path = tmp_path / ("%d.co" % i)
         path.write_bytes(code)
         notes = subprocess.run([READELF, "--notes", str(path)], capture_output=True, text=True, check=True).stdout
         for kernel in re.split(r"\n\s+- \.agpr_count", notes)[1:]:
             name = re.search(r"\.name:\s+(\S+)", kernel).group(1)
-            used = int(re.search(r"\.private_segment_fixed_size:\s+(\d+)", kernel).group(1))
-            scratch[name] = max(scratch.get(name, 0), used)
+            most[name] = max(most.get(name, 0), int(re.search(r"\.%s:\s+(\d+)" % field, kernel).group(1)))
+    return most
+
+
+def test_a_backward_sweep_finds_room_beside_another_decode_s_merged_kernel(tmp_path):
+    """256 states, four columns: two chunks of the merged kernel are 14 waves on the four SIMDs of a unit, and a SIMD's 512 registers, given
+    out by eights, are to hold four of them and a wave of the backward sweep that keeps eight rows in flight"""
+    registers = {k: (v + 7) // 8 * 8 for k, v in most_of("vgpr_count", tmp_path).items()}
+    merged, = [v for k, v in registers.items() if "beam_kernelILi256ELi2ELi4ELi4E" in k]
+    backward, = [v for k, v in registers.items() if "bwd_scan_kernelILi256ELi1ELi8ELi0E" in k]
+    assert 4 * merged + backward <= 512, (merged, backward)
+
+
+def test_no_kernel_keeps_registers_in_scratch(tmp_path):
+    scratch = most_of("private_segment_fixed_size", tmp_path)
     assert any("scan_post_kernel" in k for k in scratch) and any("beam_kernel" in k for k in scratch)
     # both sweeps of 1024 states with four states to a lane keep a few values there between their phases
     allowed = {k: 32 for k in scratch if "scan_post_kernelILi1024ELi4E" in k}
