@@ -231,10 +231,12 @@ void openfish_amd_gpubuf_set_debug_flags(const openfish_gpubuf_t *gpubuf, int fl
  * moves a quality character by one step now and then (up to three in ten thousand).  Callers that decode from several
  * threads and want the same characters every time fix the arrangement.  Host-only.
  *   64 states: 1 up to 2048 chunks, 0 beyond.
- *   256 states: alone 1 up to 512 chunks (five columns: 463), 2 for five columns up to 512, 1 up to 768,
- *     2 beyond; shared 2 up to 512, 1 up to 640, 2 beyond.
- *   1024 states: alone 1 up to 160 chunks and from 257 to 320, 2 elsewhere, but 0 for more than 320 chunks shorter than
- *     128 steps and for fewer than 16 shorter than 6; shared 2, but 0 for fewer than 16 chunks shorter than 128 steps.
+ *   256 states: alone 1 up to 446 chunks (five columns: 390), 2 up to 512, 1 up to 640 and, while T * C is at most
+ *     1250000, up to 768, 2 beyond; shared 2 up to 512, then up to 608 chunks 0 if they have at most 400 steps, 1 if T * C is at most 950000,
+ *     1 up to 548 if it is at most 1900000, 2 in all other cases.
+ *   1024 states: alone 1 up to 168 chunks, but 2 for chunks shorter than 12 steps (above 96 chunks: 4); 2 up to 256; 1 up to 340 while
+ *     N * (4 * C + 12288) + 1300 * T is at most 11550000; 2 elsewhere, but 0 for more than 340 chunks shorter than 48 steps and for 512 and
+ *     more of at most 100; shared 2, but 0 for fewer than 16 chunks shorter than 128 steps.
  */
 int openfish_amd_scan_arrangement(int T, int N, int C, int state_len, int shared);
 

@@ -498,53 +498,60 @@ static void join_null_stream(ofa_gpubuf_t *g) {
  *   merged  the chain of the kernel that holds both, three quarters of those bytes or less; the chain is longer than
  *           the search's alone (256 states by 5 %, 1024 by 16 to 40 %), twice that with two rounds of workgroups;
  *   one     both sweeps of a chunk side by side from its two ends, then the search: the longest, with the fewest launches.
- * Whole blocking calls, ms, one | split | merged, T = 1666 unless stated, inputs and arrangements in turn; in all of them
- * the forward sweep of the split decodes was seen to run beside the search (up to 96 chunks of 1024 states beside the backward sweep, see
- * enqueue_decode).
- *   1024 states: 16 chunks, T = 833 1.79 | 1.21 | 1.57;  96, T = 833 1.85 | 1.34 | 1.59;  97, T = 833 1.85 | 1.50 | 1.59;
- *                128 3.49 | 2.69 | 2.83;  160 3.69 | 2.76 | 2.85;  168 3.71 | 3.51 | 2.85;  192 3.75 | 3.53 | 2.87;
- *                256 4.10 | 3.92 | 3.00;  257 6.61 | 4.77 | 5.32;  320 6.70 | 5.32 | 5.38;  400 6.97 | 7.35 | 5.53;
- *                five columns: 160 3.81 | 2.78 | 2.88;  256 4.42 | 4.37 | 3.21;  257 6.93 | 5.12 | 5.45;
- *                288 7.04 | 5.44 | 5.52;  304 7.05 | 5.63 | 5.53;  320 7.07 | 5.79 | 5.56;
- *                T = 833: 320 3.71 | 2.96 | 2.94;  T = 400: 320 1.86 | 1.48 | 1.58;
- *                T = 1: 1 0.079 | 0.090 | 0.077;  T = 6: 8 0.099 | 0.098 | 0.092;  T = 33: 1 0.170 | 0.136 | 0.162;  T = 64: 8 0.241 | 0.188 | 0.235;
- *                T = 100: 16 0.330 | 0.244 | 0.314;  256 0.376 | 0.377 | 0.341;  352 0.585 | 0.581 | 0.562;  512 0.598 | 0.691 | 0.613;
- *                T = 128: 16 0.391 | 0.288 | 0.370;  512 0.740 | 0.843 | 0.736;  T = 200: 16 0.544 | 0.391 | 0.509
- *    256 states: 403, T = 1201 1.88 | 1.47 | 1.50;  512 2.63 | 2.01 | 2.04;  513 3.59 | 3.03 | 3.44;  700 3.74 | 3.55 | 3.65;
- *                768 3.83 | 3.68 | 3.72;  800 4.16 | 4.19 | 3.87;  1024 4.45 | 4.69 | 4.15;
- *                five columns: 456 2.63 | 2.00 | 2.03;  472 2.67 | 2.05 | 2.06;  488 2.68 | 2.06 | 2.06;  512 2.77 | 2.12 | 2.10;
- *                640 3.81 | 3.71 | 3.67;  768 3.97 | 3.88 | 3.78;  784 4.29 | 4.42 | 3.96;  1024 4.69 | 4.83 | 4.20
- *     64 states: 16 1.68 | 1.41;  512 1.97 | 1.66;  2048 4.19 | 3.55
- * Hence the lines: up to 160 chunks of 1024 states the search and the forward sweep find
- * compute units of their own; above 256 merged takes a second round of workgroups, split does so only above 320; chunks
- * shorter than 128 steps are decided by launches and set-up: split is ahead where it has its sweeps apart, but for the very
- * shortest of few chunks, and one kernel above 320.  Up to 512 chunks of 256 states the chain of split is
- * shorter, while its bytes fit beneath the chain, 3.3 MB a step; above, the search's workgroups hold four chunks, a unit
- * that has one of them in the merged kernel takes 2.3 ms whatever the others do, and split has units left for the
- * forward sweep up to three chunks to a unit.
+ * Whole blocking calls, ms, one | split | merged, T = 1666 unless stated, inputs and arrangements in turn (more of them in
+ * tests/test_arrangement.py):
+ *   1024 states: 128 3.39 | 2.65 | 2.78;  168 3.60 | 2.70 | 2.81;  172 3.64 | 3.37 | 2.84;  256 4.05 | 3.83 | 2.94;  257 6.55 | 4.74 | 5.37;
+ *                320 6.63 | 5.29 | 5.34;  328 6.64 | 5.36 | 5.35;  five columns: 290 6.97 | 5.50 | 5.52;  300 6.95 | 5.59 | 5.49;
+ *                T = 833: 336 3.47 | 2.78 | 2.88;  five columns 320 3.64 | 2.94 | 2.94;  T = 250: 340 1.17 | 0.93 | 1.05;  352 1.18 | 1.21 | 1.05;
+ *                T = 2000: 320 7.89 | 6.34 | 6.30;  five columns 280 8.28 | 6.48 | 6.52;
+ *                T = 1: 64 0.060 | 0.073 | 0.059;  T = 8: 64 0.086 | 0.086 | 0.078;  T = 12: 64 0.098 | 0.092 | 0.089;  T = 16: 0.111 | 0.099 | 0.100;
+ *                T = 4: 97 0.070 | 0.070 | 0.067;  T = 32: 360 0.244 | 0.237 | 0.250;  T = 64: 360 0.396 | 0.401 | 0.401;  T = 100: 450 0.595 | 0.596 | 0.547;
+ *                512 0.568 | 0.643 | 0.586;  T = 128: 512 0.718 | 0.824 | 0.709
+ *    256 states: 400 2.40 | 1.81 | 1.84;  440 2.42 | 1.85 | 1.87;  460 2.47 | 1.90 | 1.87;  512 2.56 | 2.15 | 1.95;
+ *                five columns: 360 2.41 | 1.82 | 1.83;  380 2.42 | 1.84 | 1.84;  400 2.44 | 1.89 | 1.87;  512 2.69 | 2.34 | 1.95;
+ *                T = 1201: 440 1.80 | 1.39 | 1.39;  460 1.81 | 1.42 | 1.41;  five columns 400 1.79 | 1.38 | 1.39;  420 1.81 | 1.42 | 1.40;
+ *                T = 400: 340 0.66 | 0.54 | 0.54;  420 0.67 | 0.56 | 0.55;  512 0.69 | 0.57 | 0.56;  T = 96: 256 0.190 | 0.176 | 0.182;  340 0.219 | 0.202 | 0.193;
+ *                513 3.39 | 2.42 | 3.19;  640 3.57 | 2.97 | 3.41;  660 3.58 | 3.41 | 3.40;  768 3.68 | 3.52 | 3.46;  1024 4.33 | 4.71 | 3.96;
+ *                five columns: 640 3.70 | 3.22 | 3.46;  660 3.74 | 3.65 | 3.51;  T = 1201: 768 2.69 | 2.60 | 2.60;  five columns 660 2.70 | 2.66 | 2.63;
+ *                T = 800: 768 1.79 | 1.76 | 1.81;  five columns 768 1.86 | 1.83 | 1.85;  T = 1000: five columns 680 2.25 | 2.23 | 2.22
+ *     64 states: 16 1.59 | 1.31;  512 1.87 | 1.54;  2048 4.11 | 3.41
+ * Hence the lines.  Up to 168 chunks of 1024 states the search and the forward sweep find compute units of their own (21 and 11 of an
+ * XCD's 32); up to 340, in two rounds, split is ahead while its bytes fit beneath the chain, and short chunks allow more of them:
+ * 11.55 MB a step, less 1300 bytes for every step of a chunk.  Chunks shorter than 12 steps are decided by launches and
+ * set-up, batches above 340 of chunks up to 100 steps by the rounds.  Up to 512 chunks of 256 states the chain of split is
+ * shorter, while its bytes fit beneath the chain, 3.2 MB a step (short chunks of 280 to 446 are ahead merged by up to 0.01 ms: left); above,
+ * the search's workgroups hold four chunks, a unit that has one of them in the merged kernel takes as long as one that has four,
+ * and split has units left for the forward sweep up to 640 chunks, with shorter chunks up to 768.
  *
  * A decode that is enqueued, or finds another one under way, shares the machine; two at a time, one | split | merged:
- *   1024 states: 16, T = 833 1.84 | 2.22 | 1.61;  128 3.87 | 4.14 | 2.96;  256 five columns 8.17 | 8.66 | 6.27;
- *                320 9.85 | 9.73 | 7.40;  8, T = 64 0.28 | 0.33 | 0.27;  16, T = 100 0.36 | 0.44 | 0.35
- *    256 states: 128 2.55 | 2.13 | 1.88;  512 5.30 | 4.42 | 3.60;  520 5.35 | 4.63 | 5.11;  640 five columns 6.47 | 5.57 | 5.62;
- *                700 6.37 | 6.13 | 5.72;  704 five columns 6.63 | 6.30 | 5.91;  768 five columns 7.16 | 7.04 | 6.05
- *     64 states: 512 3.13 | 2.71;  2048 7.66 | 6.49
+ *   1024 states: 16, T = 833 1.77 | 2.18 | 1.56;  128 4.08 | 4.87 | 3.04;  256 five columns 8.37 | 8.73 | 6.29;
+ *                320 9.81 | 9.37 | 7.36;  8, T = 64 0.228 | 0.295 | 0.231;  16, T = 100 0.309 | 0.413 | 0.300
+ *    256 states: 128 2.50 | 2.09 | 1.75;  512 5.20 | 4.44 | 3.52;  513 5.17 | 4.71 | 4.84;  530 5.29 | 4.91 | 4.93;  560 5.32 | 5.12 | 4.99;
+ *                five columns: 516 5.46 | 5.12 | 5.12;  545 5.55 | 5.47 | 5.15;  640 6.58 | 6.03 | 5.50;  T = 2000: 516 6.28 | 5.77 | 5.79;  540 6.37 | 5.91 | 5.86;
+ *                T = 1201: 545 3.82 | 3.61 | 3.66;  560 3.87 | 3.72 | 3.71;  T = 800: 600 2.65 | 2.65 | 2.67;  620 3.04 | 2.71 | 2.70;
+ *                T = 400: 530 1.32 | 1.34 | 1.41;  600 1.37 | 1.43 | 1.44;  620 1.55 | 1.45 | 1.45
+ *     64 states: 512 3.00 | 2.55;  2048 7.75 | 6.68
  *
  * The merged kernel exists for 256 and 1024 states with the default arithmetic and its own states per lane; without it
  * (can_merge = 0) 1024 states keep the one kernel and 256 states the split sweeps where they are ahead of it. */
 static int arrangement_by_default(int T, int N, int C, int state_len, int shared, int can_merge) {
-    const size_t step_bytes = (size_t)N * (4 * (size_t)C + 12 * (size_t)states_of(state_len)); /* of split */
+    const long step_bytes = (long)N * (4L * C + 12L * states_of(state_len)); /* of split */
+    const long chunk_scores = (long)T * C;
     switch (state_len) {
         case 3: return N <= 2048 ? ARR_SPLIT : ARR_ONE;
         case 4:
             if (!can_merge) return N <= 768 ? ARR_SPLIT : ARR_ONE;
-            if (N <= 512) return shared || step_bytes > 3300000 ? ARR_MERGED : ARR_SPLIT;
-            return N <= (shared ? 640 : 768) ? ARR_SPLIT : ARR_MERGED;
+            if (N <= 512) return shared || step_bytes > 3200000 ? ARR_MERGED : ARR_SPLIT;
+            if (!shared) return N <= 640 || (N <= 768 && chunk_scores <= 1250000) ? ARR_SPLIT : ARR_MERGED;
+            if (T <= 400 && N <= 608) return ARR_ONE;
+            return chunk_scores <= 1900000 && N <= (chunk_scores <= 950000 ? 608 : 548) ? ARR_SPLIT : ARR_MERGED;
         default:
             if (!can_merge) return ARR_ONE;
-            if (T < 128 && ((N < 16 && (shared || T < 6)) || (N > 320 && !shared))) return ARR_ONE;
-            if (shared) return ARR_MERGED;
-            return N <= 160 || (N > 256 && N <= 320) ? ARR_SPLIT : ARR_MERGED;
+            if (shared) return T < 128 && N < 16 ? ARR_ONE : ARR_MERGED;
+            if (N <= 168) return T < (N <= 96 ? 12 : 4) ? ARR_MERGED : ARR_SPLIT;
+            if (N <= 256) return ARR_MERGED;
+            if (N <= 340) return step_bytes + 1300L * T <= 11550000 ? ARR_SPLIT : ARR_MERGED;
+            return T < 48 || (N >= 512 && T <= 100) ? ARR_ONE : ARR_MERGED;
     }
 }
 
