@@ -12,7 +12,8 @@ Prints ONE JSON line:
   value      chunks decoded per second (wall clock around the K timed calls)
   roofline   the longest-running kernel: algorithmic bytes / mean device time
              (HIP events recorded by the library on the kernel's own stream)
-  stages     every kernel's mean device time and algorithmic GB/s
+  stages     every stage's mean device time, from the end of what it waits for to its kernel's end (the queue's gap, 5 to 10 us where
+             another stream is waited for, included), and algorithmic GB/s over that time
   cpu_baseline  the CPU path timed on this host on a bounded sample of the same tensor
 """
 import argparse

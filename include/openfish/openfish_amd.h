@@ -176,7 +176,7 @@ enum openfish_amd_stage {
                                    * where OPENFISH_AMD_STAGE_FWD_SCAN is not 0) */
     OPENFISH_AMD_STAGE_BEAM = 2,  /* beam search + traceback kernel */
     OPENFISH_AMD_STAGE_SEQ = 3,   /* quality + sequence kernel */
-    OPENFISH_AMD_STAGE_TOTAL = 4, /* first launch to last kernel end, device side */
+    OPENFISH_AMD_STAGE_TOTAL = 4, /* first stage's start to last kernel's end */
     OPENFISH_AMD_STAGE_SCAN = 5,  /* both scans + posterior as one kernel (0 when they ran split) */
     OPENFISH_AMD_STAGE_SUMS = 6,  /* per-state sums of posteriors for the quality stage, a kernel that runs beside the
                                    * beam search on a second stream (0 when the decode did without it) */
@@ -186,9 +186,13 @@ enum openfish_amd_stage {
 };
 
 /*
- * Device-side durations in milliseconds (HIP events on the streams the kernels
- * ran on) of the most recent openfish_decode_gpu call on this gpubuf.  Writes
- * min(n, OPENFISH_AMD_STAGE_COUNT) values and returns that count.
+ * Device-side durations in milliseconds (HIP events, completed by the kernels' own ends) of the
+ * most recent decode on this gpubuf.  A stage counts from the end of the last one that it waits
+ * for to the end of its kernel, so the queue's gap before the kernel, 5 to 10 us where another stream
+ * is waited for, is part of it; the first counts from the decode's start on its stream, and where the
+ * device is shared, whatever another decode's kernels hold up between the two ends counts as well.
+ * (Events at the start of every kernel would cost each 3 to 5 us.)  For kernels by themselves use
+ * a profiler.  Writes min(n, OPENFISH_AMD_STAGE_COUNT) values and returns that count.
  */
 int openfish_amd_last_timings(const openfish_gpubuf_t *gpubuf, float *ms, int n);
 
