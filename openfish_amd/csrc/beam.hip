@@ -28,7 +28,7 @@
 // those bits of its hash, reads its own entry back, and looks up the entry filed under the same bits of `want`.  If every element finds its own
 // entry intact, all hashes are pairwise distinct and every existing partner is found by
 // exactly one probe (the full 32 bits are compared); otherwise (two elements in one
-// bucket, one step in twenty to forty; equal hashes, only after a CRC collision) the step
+// bucket, one step in ten, twenty or forty by the size of the index; equal hashes, only after a CRC collision) the step
 // falls back to comparing `want` with all 32 hashes.
 #include <hip/hip_runtime.h>
 
@@ -311,17 +311,15 @@ struct Vec;
 template <>
 struct Vec<4> { typedef uint32_t type; };
 template <>
-struct Vec<8> { typedef uint32_t type __attribute__((ext_vector_type(2))); };
-template <>
 struct Vec<16> { typedef uint32_t type __attribute__((ext_vector_type(4))); };
 
 // one wave's share of a row of ROW_BYTES bytes: lane l owns vectors (i*64 + l).  Rows of 256
-// and 512 bytes are split into 4- and 8-byte vectors, one per lane; all others into 16-byte
+// bytes are split into 4-byte vectors, one per lane; all others into 16-byte
 // vectors, of which the last round may cover only the lower lanes (rows of five-column scores
-// are 640, 2560 or 10240 bytes).
+// are 2560 or 10240 bytes).
 template <int ROW_BYTES>
 struct RowRegs {
-    static constexpr int kVec = ROW_BYTES == 256 ? 4 : ROW_BYTES == 512 ? 8 : 16;
+    static constexpr int kVec = ROW_BYTES == 256 ? 4 : 16;
     static constexpr int kVecs = ROW_BYTES / kVec;
     static constexpr int kCnt = (kVecs + 63) / 64;
     static_assert(ROW_BYTES % kVec == 0, "rows are whole vectors");
@@ -433,7 +431,7 @@ struct __attribute__((aligned(16))) BeamRing {
 // (Two words an entry, hash and generation << 5 | slot, took half the buckets, two more comparisons and 12 more LDS cycles a step.)
 // Low two bits of the generation: the ring slot of the time step; the rest counts ring rounds from 1, and when it is
 // used up the search's wave clears the table (about 6 cycles a step).  With w live elements two of them share a bucket in about
-// w^2 / (2 * buckets) of the time steps.
+// w^2 / (2 * buckets) of the time steps: with 25 to 32 of them one step in 8 to 13 of 4096 buckets, in 16 to 26 of 8192, in 32 to 52 of 16384.
 template <int S, int CPG, int FWD>
 struct BeamIdx {
     static constexpr bool kLone = CPG == 1 && FWD == 0;  // a compute unit's LDS for one chunk
@@ -735,7 +733,7 @@ __global__ __launch_bounds__((kBeamThreads<S, CPG, COLS, FWD>), (BeamCfg<S, CPG,
         };
         auto hand_over = [&](Scores &rs, RowRegs<4 * S> &rb, int t) {
             if (t < T) {
-                // the ring is full most of the time (a search step takes about 3000 cycles): poll
+                // the ring is full most of the time (a search step takes about 1200 cycles): poll
                 // seldom, the rows in registers and in the ring leave ample slack for waking up late
                 if constexpr (FWD == 0) {
                     while (t - observe(consumed) >= LR) __builtin_amdgcn_s_sleep(8);
@@ -1411,8 +1409,8 @@ __global__ __launch_bounds__((kBeamThreads<S, CPG, COLS, FWD>), (BeamCfg<S, CPG,
 
 // Chunks of a search that share a workgroup, and so a compute unit's LDS.  256 units: up to 512 chunks fit two to a unit; larger
 // batches go four to a group where the LDS of four chunks fits (64 and 256 states).  Few chunks have a unit each: two searches on one wait for
-// each other's LDS operations, and with the LDS to itself a chunk has an index so large that one step in forty (1024
-// states, with half the buckets, one in twenty) instead of one in ten meets two elements in a bucket.  Search, two to a unit | one,
+// each other's LDS operations, and with the LDS to itself a chunk has an index so large that one step in forty instead of one in
+// twenty (1024 states: in ten) meets two elements in a bucket.  Search, two to a unit | one,
 // T = 1666 (1024 states 833), ms: 64 states, 1 chunk 0.943 | 0.929, 16 1.033 | 0.936, 160 1.05 | 0.96; 256 states, 16
 // 1.024 | 0.941, 160 1.04 | 0.99; 1024 states, 37 0.565 | 0.490, 100 0.577 | 0.504, 160 (split: units are short) 0.74 | 1.0.
 //
