@@ -118,11 +118,16 @@ void openfish_amd_lse_table(double *out) { build_lse_table(out); }
 
 /* ---- gpubuf ---------------------------------------------------------------- */
 
+/* Bytes of moves from which they travel beside the sequence stage; fewer are not worth three calls and a launch more (whole calls, us, by a
+ * copy | by the stage: 5 chunks of 32 steps 80 | 75; 16 of 64 states, T = 1666 1298 | 1287; 64 1315 | 1307; 150 of 256 1602 | 1610). */
+#define OFA_COPY_MOVES ((size_t)131072)
+
 #define OFA_MAGIC 0x6f66616d64677075ull /* "ofamdgpu" */
 
-enum { EV_JOIN, EV_START, EV_BWD_END, EV_BEAM_END, EV_FWD_END, EV_FWD_SCAN_END, EV_SEQ_END, EV_SUMS_END, EV_MOVES, EV_COUNT };
+enum { EV_JOIN, EV_START, EV_BWD_END, EV_BEAM_END, EV_FWD_END, EV_FWD_SCAN_END, EV_SEQ_END, EV_SUMS_END, EV_MOVES, EV_TAIL, EV_SIDE_TAIL, EV_COUNT };
 /* The events between kernels are carried by the kernels whose end they mark (queue.h); with both sweeps in one kernel EV_BWD_END is its
- * end and EV_FWD_END is not used, EV_FWD_SCAN_END only where the forward sweep runs beside the backward one. */
+ * end and EV_FWD_END is not used, EV_FWD_SCAN_END only where the forward sweep runs beside the backward one.  EV_START, EV_MOVES and the
+ * two tails are markers. */
 
 /* arrangements of the scans: both sweeps in one kernel; backward sweep, then forward sweep beside the beam search;
  * backward sweep, then forward sweep within the beam search's kernel */
@@ -312,7 +317,8 @@ openfish_gpubuf_t *openfish_gpubuf_init(const int T, const int N, const int stat
         *field[i] = sz[i] ? p : NULL;
         p += round_up(sz[i]);
     }
-    HIP_OK(hipHostMalloc((void **)&g->h_out, 3 * nt < 64 ? 64 : 3 * nt, hipHostMallocDefault));
+    /* coherent: what kernels write there is in host memory when their end is seen, with no marker behind them */
+    HIP_OK(hipHostMalloc((void **)&g->h_out, 3 * nt < 64 ? 64 : 3 * nt, hipHostMallocCoherent));
     HIP_OK(hipHostGetDevicePointer((void **)&g->d_out, g->h_out, 0));
     {
         double tab[OFK_LSE_DOUBLES];
@@ -481,15 +487,16 @@ static void fetch_outputs(ofa_gpubuf_t *g, int T, int N, uint8_t **moves, char *
  * has ended already, which the query tells in 0.2 us, there is nothing to wait for: the event and the wait for it in another hardware
  * queue put 20 us before a decode's first kernel.  That the query answers for the streams ordered with the null stream too is this
  * runtime's doing, and tested for copies and kernels of both.  It is the current device's null stream: a gpubuf of another device is
- * refused, as recording its event there is by the runtime. */
-static void join_null_stream(ofa_gpubuf_t *g) {
+ * refused, as recording its event there is by the runtime.  Returns whether there was something to wait for: EV_JOIN then marks its end. */
+static int join_null_stream(ofa_gpubuf_t *g) {
     int device;
     HIP_OK(hipGetDevice(&device));
     if (device != g->device) die("the gpubuf belongs to another device than the current one");
-    if (hipStreamQuery(0) == hipSuccess) return;
+    if (hipStreamQuery(0) == hipSuccess) return 0;
     if (hipPeekAtLastError() == hipErrorNotReady) (void)hipGetLastError(); /* the query's answer, but no error that the caller left behind */
     HIP_OK(hipEventRecord(g->ev[EV_JOIN], 0));
     HIP_OK(hipStreamWaitEvent(g->s_main, g->ev[EV_JOIN], 0));
+    return 1;
 }
 
 /* Which arrangement of the scans a decode finishes soonest with.  What bounds them, after the backward sweep:
@@ -591,14 +598,18 @@ static void enqueue_decode(ofa_gpubuf_t *g, const int T, const int N, const int 
     const int sums_fit = g->path_sums != NULL && N <= OFK_SPARSE_SEARCH_MAX_CHUNKS;
     const int use_sums = sums_fit && (g->pend_split == ARR_ONE || (g->pend_split == ARR_SPLIT && state_len == 3 && !others));
     g->pend_sums = use_sums;
-    g->pend_copy = !shared;
+    g->pend_copy = !shared && nt >= OFA_COPY_MOVES;
     if (g->pend_split == ARR_SPLIT || use_sums || g->pend_copy) take_side_lane(g);
-    join_null_stream(g);
-    HIP_OK(hipEventRecord(g->ev[EV_START], g->s_main));
+    const int joined = join_null_stream(g);
+    /* The start is a marker, which holds up what is behind it by 3 us: where the side lane has nothing to do yet it goes there, once
+     * the first kernel is queued. */
+    const int start_beside = g->side_lane >= 0 && !shared && !joined;
+    if (!start_beside) HIP_OK(hipEventRecord(g->ev[EV_START], g->s_main));
     if (g->pend_split == ARR_MERGED) {
         /* backward sweep, then the search with the forward sweep and the posterior in its workgroups */
         launch_ok(ofk_bwd_scan(scores_TNC, g->pub.bwd_NTC, T, N, state_len, cols, stay, g->scan_mode, g->scan_spl, shared, g->s_main,
                                g->ev[EV_BWD_END]), "bwd_scan");
+        if (start_beside) HIP_OK(hipEventRecord(g->ev[EV_START], g->s_side));
         launch_ok(ofk_beam_search_forward(scores_TNC, g->pub.bwd_NTC, g->pub.post_NTC, (ofk_beam_slot_t *)g->pub.beam_vector,
                                           (int32_t *)g->pub.states, g->pub.moves, T, N, state_len, cols,
                                           log_beam_cut(options), stay, g->lse_table, g->debug_flags, g->s_main, g->ev[EV_BEAM_END]),
@@ -607,6 +618,7 @@ static void enqueue_decode(ofa_gpubuf_t *g, const int T, const int N, const int 
         /* both sweeps and the posterior in one kernel, then the beam search, all on one stream */
         launch_ok(ofk_scan_posterior(scores_TNC, g->pub.bwd_NTC, g->pub.post_NTC, T, N, state_len, cols, stay, g->scan_mode,
                                      g->scan_spl, g->s_main, g->ev[EV_BWD_END]), "scan_posterior");
+        if (start_beside) HIP_OK(hipEventRecord(g->ev[EV_START], g->s_side));
         launch_ok(ofk_beam_search(scores_TNC, g->pub.bwd_NTC, (ofk_beam_slot_t *)g->pub.beam_vector,
                                   (int32_t *)g->pub.states, g->pub.moves, T, N, state_len, cols, log_beam_cut(options),
                                   stay, g->lse_table, search_flags, g->s_main, g->ev[EV_BEAM_END]), "beam_search");
@@ -627,8 +639,9 @@ static void enqueue_decode(ofa_gpubuf_t *g, const int T, const int N, const int 
         const int apart = g->pend_apart = state_len == 5 && N <= 96 && !shared && g->scan_mode == OFK_SCAN_TWO_TIER && g->scan_spl == 0;
         launch_ok(ofk_bwd_scan(scores_TNC, g->pub.bwd_NTC, T, N, state_len, cols, stay, g->scan_mode, g->scan_spl, 0, g->s_main,
                                g->ev[EV_BWD_END]), "bwd_scan");
+        if (start_beside) HIP_OK(hipEventRecord(g->ev[EV_START], g->s_side));
         if (apart) {
-            HIP_OK(hipStreamWaitEvent(g->s_side, g->ev[EV_START], 0));
+            if (joined) HIP_OK(hipStreamWaitEvent(g->s_side, g->ev[EV_JOIN], 0));
             launch_ok(ofk_fwd_scan(scores_TNC, g->pub.post_NTC, T, N, state_len, cols, stay, g->s_side, g->ev[EV_FWD_SCAN_END]),
                       "fwd_scan");
         }
@@ -652,7 +665,7 @@ static void enqueue_decode(ofa_gpubuf_t *g, const int T, const int N, const int 
         }
     }
 
-    /* The moves are final once the beam search is.  Of a decode that has the device to itself they travel, and
+    /* The moves are final once the beam search is.  Of a decode that has the device to itself, and enough of them, they travel, and
      * the host takes them, while the sequence stage runs.  Otherwise that stage writes them to the host itself (0.02 ms),
      * because a copy that waits for the search would hold up another decode's forward sweep behind
      * it on the side lane (two batches of 16 chunks of 64 states in flight: 2.14 ms with the copies, 1.63 without). */
@@ -671,8 +684,12 @@ static void enqueue_decode(ofa_gpubuf_t *g, const int T, const int N, const int 
      * are filled by the stage-level entry points only. */
     launch_ok(ofk_sequence(g->pub.post_NTC, (int32_t *)g->pub.states, g->pub.moves, g->pub.qual_data,
                            g->pub.base_probs, g->pub.total_probs, (char *)g->d_out + nt, (char *)g->d_out + 2 * nt, T, N,
-                           state_len, phred_for(g, options), use_sums ? g->path_sums : NULL, g->pend_copy ? NULL : g->d_out, g->s_main, NULL), "sequence");
-    HIP_OK(hipEventRecord(g->ev[EV_SEQ_END], g->s_main)); /* a marker, which makes what the kernel wrote to host memory visible there */
+                           state_len, phred_for(g, options), use_sums ? g->path_sums : NULL, g->pend_copy ? NULL : g->d_out, g->s_main, g->ev[EV_SEQ_END]), "sequence");
+    /* The host waits for the end of that kernel, which it sees 3 us before the end of a marker behind it.  The markers are for the
+     * runtime: a stream that ends with one is known to be done, one that ends with a kernel gets a marker and a wait of its own, 5 us
+     * each, in the caller's next hipDeviceSynchronize. */
+    HIP_OK(hipEventRecord(g->ev[EV_TAIL], g->s_main));
+    if (g->side_lane >= 0 && !g->pend_copy) HIP_OK(hipEventRecord(g->ev[EV_SIDE_TAIL], g->s_side));
     g->pending = 1;
     g->pend_T = T;
     g->pend_N = N;
@@ -736,6 +753,9 @@ int openfish_amd_last_timings(const openfish_gpubuf_t *gpubuf, float *ms, int n)
         g->ms[OPENFISH_AMD_STAGE_BWD] = g->ms[OPENFISH_AMD_STAGE_FWD] = 0.0f;
         HIP_OK(hipEventElapsedTime(&g->ms[OPENFISH_AMD_STAGE_SCAN], g->ev[EV_START], g->ev[EV_BWD_END]));
     }
+    /* a start marked beside the first kernel can be behind the end of one of a few steps */
+    if (g->ms[OPENFISH_AMD_STAGE_BWD] < 0.0f) g->ms[OPENFISH_AMD_STAGE_BWD] = 0.0f;
+    if (g->ms[OPENFISH_AMD_STAGE_SCAN] < 0.0f) g->ms[OPENFISH_AMD_STAGE_SCAN] = 0.0f;
     g->ms[OPENFISH_AMD_STAGE_FWD_SCAN] = 0.0f;
     if (g->pend_split == ARR_SPLIT && g->pend_apart) {
         /* the posteriors' pass begins with the later of the two sweeps' ends */
