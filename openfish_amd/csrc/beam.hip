@@ -43,6 +43,7 @@
 namespace {
 
 constexpr int kW = OFK_BEAM_WIDTH;
+constexpr int kTraceRows = 128;  // rows that the traceback takes at a time
 constexpr uint32_t kPoly = 0x82f63b78u;
 constexpr uint32_t kSeed = 0x12345678u;
 
@@ -409,6 +410,7 @@ struct BeamShared {
     float stay_score[kW];         // only used by the serial replay of merges
     uint32_t claim[4 * kW + 64];  // only used when the hash index was not conclusive: who claimed step candidate 4j+b
     int ready, consumed;          // rows stored by the loader wave, rows the search wave is done with (with FWD > 0 in FwdLds)
+    int searched, mapped;         // the search has ended; waves of the traceback that have their blocks' maps in LDS
 };
 
 // LDS of one chunk.  Score rows are kept in planes for the search alone; where the recursion reads them too, as the caller lays them
@@ -440,6 +442,11 @@ struct BeamIdx {
     static constexpr uint32_t kAddress = (uint32_t)(kBuckets - 1) << 2;  // hash bits that address a bucket
     static constexpr uint32_t kSlot = 31u << 4;
     static constexpr uint32_t kRound = 1u << 9, kRoundEnd = 1u << (kBits + 2);
+    // Waves that trace a chunk's path back, each with a buffer of 8 KB in the index: the search's, the loader's and, of a lone chunk, the
+    // two that were there for the set-up, or two of the recursion's.  The maps they exchange, 16 KB, lie behind the buffers where there is
+    // room.  An index of 16 KB has two buffers and no maps: one wave.
+    static constexpr int kTeam = kLone || FWD >= 4 ? 4 : kBits == 13 ? 2 : 1;
+    static constexpr bool kMapsApart = FWD >= 4;
 };
 // What the forward recursion and the posterior of a chunk share.
 constexpr int kVecRows = 4;  // two would do (see beam_kernel); four let the posterior lag (1024 chunks of 256 states: 2.66 ms against 2.78)
@@ -459,12 +466,16 @@ struct FwdTables {
     ofa::LogCell centred[ofa::kLogCentredCells];
 };
 struct NoTables {};
+struct TraceMaps {
+    uint32_t map[(OFK_MAX_T + kTraceRows - 1) / kTraceRows][64];
+};
 template <int S, int CPG, int COLS, int FWD>
 struct __attribute__((aligned(16))) BeamLds {
     BeamRing<S, CPG, COLS, FWD> ring;
     BeamShared sh;
     uint32_t idx_dump[64];  // where a dead lane files its leftovers instead of a bucket of the index
     FwdLds<S, FWD> fwd;
+    typename std::conditional<BeamIdx<S, CPG, FWD>::kMapsApart, TraceMaps, NoTables>::type trace;
 };
 // scores of the step candidates 4i+b while stays merge into them, aligned so that a candidate's address is put together by `or`;
 // then a slot for every lane whose stay has no partner to write to
@@ -597,6 +608,8 @@ __global__ __launch_bounds__((kBeamThreads<S, CPG, COLS, FWD>), (BeamCfg<S, CPG,
     if (wave < kGroupChunks && lane == 0) {
         *ready = 0;
         *consumed = 0;
+        sh.searched = 0;
+        sh.mapped = 0;
         if constexpr (FWD > 0)
             for (int x = 0; x < FwdLds<S, FWD>::kCounters; ++x) lds[member].fwd.progress[x] = 0;
     }
@@ -607,9 +620,11 @@ __global__ __launch_bounds__((kBeamThreads<S, CPG, COLS, FWD>), (BeamCfg<S, CPG,
         reinterpret_cast<uint4 *>(&all.idx[0][0])[x] = make_uint4(0u, 0u, 0u, 0u);
     __syncthreads();
     if (n >= N) return;  // odd batch: the last group has one chunk
-    if (Idx::kLone && wave > kFirstLoader) return;
+    ofk_beam_slot_t *const bv = beam + (size_t)n * (size_t)(T + 1) * kW;
 
     static_assert((FWD & (FWD - 1)) == 0 && FWD <= 8, "a lane reads one counter");
+    constexpr int kTeam = Idx::kTeam;
+    int mate = 0;  // of those that trace this chunk's path back: the search's wave is the first
     if constexpr (FWD > 0) {
         typedef FwdLds<S, FWD> Fwd;
         Fwd &fw = lds[member].fwd;
@@ -669,7 +684,9 @@ __global__ __launch_bounds__((kBeamThreads<S, CPG, COLS, FWD>), (BeamCfg<S, CPG,
                 lse5_all<SPL, OFK_SCAN_TWO_TIER>(f, v, logtab, [&] { write_row(t + 1); }, [](bool) {});
                 publish_row(t + 1);
             }
-            return;
+            if (kTeam <= 2 || w + 2 >= kTeam) return;
+            mate = w + 2;
+            __builtin_amdgcn_s_setprio(0);
         }
         if (wave >= kGroupChunks && wave < kFirstFwd) {
             // ---- posterior: softmax over the states of fwd[t] + bwd[t], t = 0 .. T ----
@@ -717,7 +734,7 @@ __global__ __launch_bounds__((kBeamThreads<S, CPG, COLS, FWD>), (BeamCfg<S, CPG,
             return;
         }
     }
-    if (wave >= kGroupChunks) {
+    auto load_rows = [&]() __attribute__((always_inline)) {
         // ---- loader wave: row t = (scores[t], bwd[t+1]) into ring slot t % LR ----
         const int lane = lane_now();
         // The ring is spelled out as named registers (not an array indexed by a loop that
@@ -770,9 +787,9 @@ __global__ __launch_bounds__((kBeamThreads<S, CPG, COLS, FWD>), (BeamCfg<S, CPG,
                 hand_over(s5, g5, t0 + 5);
             }
         }
-        return;
-    }
+    };
 
+    auto search = [&]() __attribute__((always_inline)) {
     // ---- search wave ----
     const int i = lane >> 1;  // lanes 2i and 2i+1 hold element i; candidate order is lane order
     const int h = lane & 1;
@@ -828,7 +845,6 @@ __global__ __launch_bounds__((kBeamThreads<S, CPG, COLS, FWD>), (BeamCfg<S, CPG,
     }
     int state = (int)(info & 1023u);
     int w = kW;
-    ofk_beam_slot_t *bv = beam + (size_t)n * (size_t)(T + 1) * kW;
 
     // The search is a chain of dependent short instructions; when it shares a SIMD with
     // throughput-bound waves (the forward scan runs at the same time) it should win the
@@ -1292,6 +1308,23 @@ __global__ __launch_bounds__((kBeamThreads<S, CPG, COLS, FWD>), (BeamCfg<S, CPG,
     }
     for (; next_t < T; ++next_t) step(next_t, AnySlot{}, std::false_type{});
     step(T, AnySlot{}, std::true_type{});
+    };
+
+    if (wave < kGroupChunks) {
+        search();
+        // The slots are in memory, and what was done in LDS is done, before the other waves go on.
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+        if constexpr (kTeam > 1) __hip_atomic_store(&sh.searched, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    } else {
+        if (wave >= kFirstLoader) {
+            mate = 1 + (wave - kFirstLoader) / kGroupChunks;
+            if (mate == 1) load_rows();
+        }
+        if (kTeam == 1 || mate * kTraceRows >= T) return;  // no block to trace
+        while (__hip_atomic_load(&sh.searched, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) == 0) __builtin_amdgcn_s_sleep(16);
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+    }
 
     // ---- traceback from slot 0 of the last block (src/beam_search.c:432-439) ----
     // Followed one row at a time the walk is a chain of T dependent LDS reads.  It is done per block
@@ -1304,15 +1337,21 @@ __global__ __launch_bounds__((kBeamThreads<S, CPG, COLS, FWD>), (BeamCfg<S, CPG,
     // wave stores 128 states and moves side by side.  Rows that a block lacks at its old end are
     // staged as slots that point at themselves.  The next block's slots travel from global memory
     // while a block is walked.
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+    //
+    // Pass 1 needs nothing of another block.  Where the index has room the waves of the chunk deal the blocks round, leave each
+    // block's eight maps in LDS, a word a lane, and meet once; every wave then threads the entry through all blocks and walks its own
+    // again (kernels, T = 1666, one wave | with the others, us: 1 chunk of 64 states 880 | 862, 512, two waves, 985 | 978; 512 of 256 states
+    // merged 1001 | 993, 256 of 1024 1672 | 1666).  They wait for the search alone, and the search's wave for their maps only here, so all
+    // waits end.  The kernel's waves share a compute unit, whose first-level cache writes through: their fences need not write the second
+    // level back (which took 10 us of the merged kernel of 512 chunks of 256 states, 17 of 256 of 1024).
     {
-        constexpr int RB = 128;  // rows per block
+        constexpr int RB = kTraceRows;  // rows per block
         const int lane = lane_now();
-        static_assert(2 * RB * kW * (int)sizeof(ofk_beam_slot_t) <= Idx::kBuckets * 4, "two blocks fit the index");
+        constexpr int kStage = RB * kW * (int)sizeof(ofk_beam_slot_t);  // bytes of a staged block
+        static_assert((kTeam > 1 ? kTeam * kStage + (Idx::kMapsApart ? 0 : (int)sizeof(TraceMaps)) : 2 * kStage) <= Idx::kBuckets * 4, "the index has room");
         int32_t *st_out = states + (size_t)n * T;
         uint8_t *mv_out = moves + (size_t)n * T;
-        const uint32_t buf0 = idx_base;  // two buffers of RB rows of 64 bytes, row 127 the newest of a block
+        const uint32_t idx_base = lds_address(&all.idx[member][0]);
         typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
         u32x4 pre[8];  // a block on its way from global memory: 16-byte piece 64 k + lane in pre[k]
         // block b covers rows hi - rows + 1 .. hi with hi = T - RB b; piece x of the buffer holds
@@ -1345,16 +1384,9 @@ __global__ __launch_bounds__((kBeamThreads<S, CPG, COLS, FWD>), (BeamCfg<S, CPG,
             asm("v_lshl_add_u32 %0, %1, 1, %2" : "=v"(at) : "v"(cur), "v"(row_base));
             return (uint32_t) * (const LDS_AS uint16_t *)(uintptr_t)(at + 64u * (uint32_t)row);
         };
-        uint32_t cursor = 0;  // slot through which the walk enters the block: the same in every lane
-        load_block(T);
-        store_block(T, buf0);
-        int blk = 0;
-        for (int hi = T; hi > 0; hi -= RB, ++blk) {
-            const int rows = hi < RB ? hi : RB;
-            const uint32_t buf = buf0 + (uint32_t)(blk & 1) * (uint32_t)(RB * 64);
-            if (hi > RB) load_block(hi - RB);
-            wave_fence();
-            // pass 1: sub-block s = 4 (lane / 32) + k covers buffer rows 127 - 16 s down to 112 - 16 s
+        // pass 1: sub-block s = 4 (lane / 32) + k covers buffer rows 127 - 16 s down to 112 - 16 s; where entry lane % 32 leaves it is byte
+        // k of the lane's word
+        auto map_block = [&](uint32_t buf) {
             uint32_t cur[4];
             const uint32_t low1 = buf + 64u * (uint32_t)(112 - 64 * (lane >> 5));  // oldest row of this lane's sub-block k = 0
 #pragma unroll
@@ -1367,20 +1399,23 @@ __global__ __launch_bounds__((kBeamThreads<S, CPG, COLS, FWD>), (BeamCfg<S, CPG,
 #pragma unroll
                 for (int k = 0; k < 4; ++k) cur[k] = (e[k] >> 10) & 31u;
             }
-            // the real entry of every sub-block
-            uint32_t enter[8];
+            return cur[0] | cur[1] << 8 | cur[2] << 16 | cur[3] << 24;
+        };
+        // lanes 8 s .. 8 s + 7 walk sub-block s in pass 2; lane q of them keeps rows 2q, 2q+1 of the walk
+        const int sb2 = lane >> 3, q = lane & 7;
+        uint32_t cursor = 0;  // slot through which the walk enters the block: the same in every lane
+        auto thread_block = [&](uint32_t map) {  // and the slot through which it enters the lane's sub-block
+            uint32_t enter = 0;
 #pragma unroll
             for (int sb = 0; sb < 8; ++sb) {
-                enter[sb] = cursor;
-                cursor = (uint32_t)__builtin_amdgcn_readlane((int)cur[sb & 3], (int)(cursor + 32u * (uint32_t)(sb >> 2)));
+                enter = sb2 == sb ? cursor : enter;
+                cursor = ((uint32_t)__builtin_amdgcn_readlane((int)map, (int)(cursor + 32u * (uint32_t)(sb >> 2))) >> (8 * (sb & 3))) & 31u;
             }
-            // pass 2: lanes 8 s .. 8 s + 7 walk sub-block s from its real entry; lane q keeps rows 2q, 2q+1 of the walk
-            const int sb2 = lane >> 3, q = lane & 7;
-            uint32_t walk = enter[0];
-#pragma unroll
-            for (int sb = 1; sb < 8; ++sb) walk = sb2 == sb ? enter[sb] : walk;
+            return enter;
+        };
+        uint32_t newer = 0, older = 0;
+        auto walk_block = [&](uint32_t buf, uint32_t walk) {
             const uint32_t low2 = buf + 64u * (uint32_t)(112 - 16 * sb2);
-            uint32_t newer = 0, older = 0;
 #pragma unroll
             for (int r = 15; r >= 0; --r) {
                 const uint32_t e = slot_at(low2, walk, r);
@@ -1388,11 +1423,11 @@ __global__ __launch_bounds__((kBeamThreads<S, CPG, COLS, FWD>), (BeamCfg<S, CPG,
                 else older = q == (15 - r) / 2 ? e : older;
                 walk = (e >> 10) & 31u;
             }
-            // the next block goes into the other buffer before this block's results are stored: the wait
-            // for its loads then does not wait for those stores as well
-            if (hi > RB) store_block(hi - RB, buf0 + (uint32_t)((blk + 1) & 1) * (uint32_t)(RB * 64));
-            // buffer row of `newer`: 127 - 16 sb2 - 2 q; the block's rows start at buffer row RB - rows,
-            // which is row hi - rows + 1 of the chunk, i.e. time step hi - rows
+        };
+        // buffer row of `newer`: 127 - 16 sb2 - 2 q; the block's rows start at buffer row RB - rows,
+        // which is row hi - rows + 1 of the chunk, i.e. time step hi - rows
+        auto store_path = [&](int hi) {
+            const int rows = hi < RB ? hi : RB;
             const int p_new = 127 - 16 * sb2 - 2 * q;
             const int t_new = hi - rows + (p_new - (RB - rows));
             if (p_new >= RB - rows) {
@@ -1402,6 +1437,57 @@ __global__ __launch_bounds__((kBeamThreads<S, CPG, COLS, FWD>), (BeamCfg<S, CPG,
             if (p_new - 1 >= RB - rows) {
                 st_out[t_new - 1] = (int32_t)(older & 1023u);
                 mv_out[t_new - 1] = (t_new - 1 == 0 || !(older >> 15)) ? (uint8_t)1 : (uint8_t)0;
+            }
+        };
+        if constexpr (kTeam == 1) {
+            load_block(T);
+            store_block(T, idx_base);
+            int blk = 0;
+            for (int hi = T; hi > 0; hi -= RB, ++blk) {  // two buffers in turn
+                const uint32_t buf = idx_base + (uint32_t)(blk & 1) * (uint32_t)kStage;
+                if (hi > RB) load_block(hi - RB);
+                wave_fence();
+                walk_block(buf, thread_block(map_block(buf)));
+                // the next block goes into the other buffer before this block's results are stored: the wait
+                // for its loads then does not wait for those stores as well
+                if (hi > RB) store_block(hi - RB, idx_base + (uint32_t)((blk + 1) & 1) * (uint32_t)kStage);
+                store_path(hi);
+            }
+        } else {
+            // block b is wave b % kTeam's.  The newest of a wave's blocks comes last in pass 1, so that it is staged where pass 2 begins.
+            const int blocks = (T + RB - 1) / RB, waves = blocks < kTeam ? blocks : kTeam;
+            const uint32_t buf = idx_base + (uint32_t)(mate * kStage);
+            uint32_t maps = idx_base + (uint32_t)(kTeam * kStage);
+            if constexpr (Idx::kMapsApart) maps = lds_address(&lds[member].trace);
+            maps += 4u * (uint32_t)lane;
+            int b = blocks - 1 - (blocks - 1 - mate) % kTeam;  // the oldest of the wave's
+            load_block(T - RB * b);
+            for (; b >= 0; b -= kTeam) {
+                wave_fence();
+                store_block(T - RB * b, buf);
+                if (b >= kTeam) load_block(T - RB * (b - kTeam));
+                wave_fence();
+                *(LDS_AS uint32_t *)(uintptr_t)(maps + 256u * (uint32_t)b) = map_block(buf);
+            }
+            if (mate + kTeam < blocks) load_block(T - RB * (mate + kTeam));
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+            if (lane == 0) __hip_atomic_fetch_add(&sh.mapped, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+            while (observe(&sh.mapped) < waves) {}
+            uint32_t map = *(const LDS_AS uint32_t *)(uintptr_t)maps;
+            for (b = 0; b < blocks; ++b) {
+                const uint32_t here = map;
+                if (b + 1 < blocks) map = *(const LDS_AS uint32_t *)(uintptr_t)(maps + 256u * (uint32_t)(b + 1));
+                const uint32_t enter = thread_block(here);
+                if (b % kTeam != mate) continue;
+                const int hi = T - RB * b;
+                wave_fence();
+                walk_block(buf, enter);
+                wave_fence();
+                if (b + kTeam < blocks) {
+                    store_block(hi - RB * kTeam, buf);
+                    if (b + 2 * kTeam < blocks) load_block(hi - 2 * RB * kTeam);
+                }
+                store_path(hi);
             }
         }
     }
