@@ -18,8 +18,11 @@ SRC   := openfish_amd/csrc
 BUILD := build
 # -ffp-contract=off: every fp32 product and sum rounds separately, as on the CPU path.
 # packed fp32 instructions are disabled for the whole device build.
+# Blocks that are only jumped to begin at multiples of 32 bytes: a wave that is alone on its SIMD waits for every fetch after a jump
+# (search of 1 chunk of 64 states 866 us -> 858, backward sweep 367 -> 363, merged kernel of 512 chunks of 256 states 993 -> 981, of 1024
+# 2243 -> 2218; 64 bytes gave no more).
 HIPFLAGS := $(ROCM_ARCH) -O3 -fPIC -ffp-contract=off -Xclang -target-feature -Xclang -packed-fp32-ops \
-            -Wall -Wno-unused-command-line-argument -I include -I $(SRC)
+            -mllvm -align-all-nofallthru-blocks=5 -Wall -Wno-unused-command-line-argument -I include -I $(SRC)
 CFLAGS   := -O2 -g -Wall -fPIC -std=gnu11 -D__HIP_PLATFORM_AMD__ -I include -I $(SRC) -I $(ROCM_ROOT)/include
 LDLIBS   := -L$(ROCM_ROOT)/lib -Wl,-rpath,$(ROCM_ROOT)/lib -lamdhip64 -lm -lpthread
 
