@@ -496,38 +496,40 @@ struct __attribute__((aligned(16))) BeamGroupLds {
 
 // The scores of one lane's states for one step of the recursion, read from a row in LDS: fp16 pairs in
 // 32-bit words.  Five-column rows are read in aligned words (a state's transitions start at a word or in the
-// middle of one, by its parity) and shifted into place.
+// middle of one, by its parity) and shifted into place.  Addresses are plain numbers: where the compiler sees the object behind them
+// it puts the distance from LDS address 0 into every one anew, past what an instruction's offset holds.
 template <int SPL, int COLS>
 struct LdsRow {
+    typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
     uint32_t w[2 * SPL];
-    __device__ __forceinline__ void load(const _Float16 *row, int s0) {
-        const uint32_t *p = reinterpret_cast<const uint32_t *>(row);
+    static __device__ __forceinline__ uint32_t word(uint32_t at) { return *(const LDS_AS uint32_t *)(uintptr_t)at; }
+    static __device__ __forceinline__ uint32_t first(int s0) {  // bytes from the row's start; s0 is even where a lane has two states or more
+        return COLS == 4 ? 8u * (uint32_t)s0 : SPL == 1 ? ((5u * (uint32_t)s0 + 1u) >> 1) << 2 : 10u * (uint32_t)s0;
+    }
+    __device__ __forceinline__ void load(uint32_t at, int s0) {
         if constexpr (COLS == 4) {
-            p += 2 * s0;
             if constexpr (SPL == 1) {
-                const uint2 x = *reinterpret_cast<const uint2 *>(p);
+                const u32x2 x = *(const LDS_AS u32x2 *)(uintptr_t)at;
                 w[0] = x.x; w[1] = x.y;
             } else {
 #pragma unroll
                 for (int i = 0; i < SPL / 2; ++i) {
-                    const uint4 x = reinterpret_cast<const uint4 *>(p)[i];
+                    const u32x4 x = *(const LDS_AS u32x4 *)(uintptr_t)(at + 16u * (uint32_t)i);
                     w[4 * i] = x.x; w[4 * i + 1] = x.y; w[4 * i + 2] = x.z; w[4 * i + 3] = x.w;
                 }
             }
         } else if constexpr (SPL == 1) {
-            p += (5 * s0 + 1) >> 1;
-            const uint32_t a = p[0], b = p[1], c = p[s0 & 1 ? 1 : 2], by = s0 & 1 ? 0u : 16u;
+            const uint32_t a = word(at), b = word(at + 4), c = word(at + (s0 & 1 ? 4u : 8u)), by = s0 & 1 ? 0u : 16u;
             w[0] = __builtin_amdgcn_alignbit(b, a, by);
             w[1] = __builtin_amdgcn_alignbit(c, b, by);
         } else {
-            p += (5 * s0) >> 1;  // s0 is even
 #pragma unroll
             for (int i = 0; i < SPL / 2; ++i) {
-                const uint32_t a = p[5 * i], b = p[5 * i + 1], c = p[5 * i + 2];
+                const uint32_t p = at + 20u * (uint32_t)i, a = word(p), b = word(p + 4), c = word(p + 8);
                 w[4 * i] = __builtin_amdgcn_alignbit(b, a, 16);
                 w[4 * i + 1] = __builtin_amdgcn_alignbit(c, b, 16);
-                w[4 * i + 2] = p[5 * i + 3];
-                w[4 * i + 3] = p[5 * i + 4];
+                w[4 * i + 2] = word(p + 12);
+                w[4 * i + 3] = word(p + 16);
             }
         }
     }
@@ -646,14 +648,25 @@ __global__ __launch_bounds__((kBeamThreads<S, CPG, COLS, FWD>), (BeamCfg<S, CPG,
             float f[SPL];
 #pragma unroll
             for (int k = 0; k < SPL; ++k) f[k] = 0.f;
-            int slot = 0;
+            // what the lane reads and writes of a row: its scores in the ring, its predecessors and its own places in the vector
+            const uint32_t vec_at = lds_address(&fw.vec[0][q]), own_at = lds_address(&fw.vec[0][s0]);
+            uint32_t row_at = lds_address(&row_s[0][0]) + LdsRow<SPL, COLS>::first(s0);
+            asm volatile("" : "+v"(row_at));
+            uint32_t slot = 0;  // bytes
+            const uint32_t mark_at = lds_address(&fw.progress[w]);
+            auto vec_row = [](int t) { return (uint32_t)(t % kVecRows) * (uint32_t)(4 * S); };
             auto write_row = [&](int t) {
+                const uint32_t at = own_at + vec_row(t);
+                if constexpr (SPL == 1) {
+                    lds_store_f(at, f[0]);
+                } else {
 #pragma unroll
-                for (int k = 0; k < SPL; ++k) fw.vec[t % kVecRows][s0 + k] = f[k];
+                    for (int k = 0; k < SPL; k += 2) lds_store_f2(at + 4u * (uint32_t)k, f[k], f[k + 1]);
+                }
             };
             auto publish_row = [&](int t) {
                 wave_fence();
-                __hip_atomic_store(&fw.progress[w], t + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+                __hip_atomic_store((LDS_AS int *)(uintptr_t)mark_at, t + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
             };
             write_row(0);
             publish_row(0);
@@ -668,9 +681,9 @@ __global__ __launch_bounds__((kBeamThreads<S, CPG, COLS, FWD>), (BeamCfg<S, CPG,
                 // clock lower for all that follows.)
                 while (ballot(progress(counter) < t + wanted) != 0) {}
                 LdsRow<SPL, COLS> row;
-                row.load(row_s[slot], s0);
-                const float *vec = fw.vec[t % kVecRows];
-                const float p0 = vec[q], p1 = vec[q + Q], p2 = vec[q + 2 * Q], p3 = vec[q + 3 * Q];
+                row.load(row_at + slot, s0);
+                const uint32_t vec = vec_at + vec_row(t);
+                const float p0 = lds_load_f(vec), p1 = lds_load_f(vec + 4 * Q), p2 = lds_load_f(vec + 8 * Q), p3 = lds_load_f(vec + 12 * Q);
                 float v[SPL][5];
 #pragma unroll
                 for (int k = 0; k < SPL; ++k) {
@@ -680,7 +693,7 @@ __global__ __launch_bounds__((kBeamThreads<S, CPG, COLS, FWD>), (BeamCfg<S, CPG,
                     v[k][3] = ::add_half<0>(row.w[2 * k + 1], p2);
                     v[k][4] = ::add_half<1>(row.w[2 * k + 1], p3);
                 }
-                slot = slot + 1 == LR ? 0 : slot + 1;
+                slot = slot == (uint32_t)((LR - 1) * sizeof(row_s[0])) ? 0u : slot + (uint32_t)sizeof(row_s[0]);
                 lse5_all<SPL, OFK_SCAN_TWO_TIER>(f, v, logtab, [&] { write_row(t + 1); }, [](bool) {});
                 publish_row(t + 1);
             }
