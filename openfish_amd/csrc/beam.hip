@@ -125,15 +125,21 @@ __device__ __forceinline__ float wave_max(float x) {
 //   cs = the stay's score after the merges, rests = cs minus its guide term (the steps' scores are still on their way from LDS)
 // The lane maximum of x0, x1 and the stay's (one v_max3) opens the block; the read of lane 63, where the six steps leave the
 // wave's maximum, wants one instruction between itself and the last of them, and the vector unit two before it uses what was read.
+// The first two cuts come out of it as well, lo = best - log_cut (-FLT_MAX at least), cut = (lo + best) / 2 with the halves of both bounds: behind
+// inline assembly whose results it reads at once the compiler idles an instruction.
 struct NextRecords {
     uint32_t h0, h1, info0, info1, infos;
     float rest0, rest1, rests;
 };
-__device__ __forceinline__ float wave_max_beside_records(float x0, float x1, float stay_or_fold, NextRecords &n, float &cs, uint32_t hash,
-                                                         uint32_t b0, uint32_t state, uint32_t from_stay, uint32_t st4,
-                                                         uint32_t state_mask, uint32_t from, uint64_t step_wins, float lowest, float gs) {
+struct Cuts {
+    float lo, half_lo, half_hi, cut;
+};
+__device__ __forceinline__ Cuts wave_max_beside_records(float x0, float x1, float stay_or_fold, NextRecords &n, float &cs, uint32_t hash,
+                                                        uint32_t b0, uint32_t state, uint32_t from_stay, uint32_t st4,
+                                                        uint32_t state_mask, uint32_t from, uint64_t step_wins, float lowest, float gs, float log_cut) {
     uint32_t t0, t1, best;
     float x;
+    Cuts c;
     asm volatile(
         "v_max3_f32 %[x], %[x0], %[x1], %[x2]\n\t"
         "v_xor_b32 %[t0], %[hash], %[b0]\n\t"
@@ -157,13 +163,18 @@ __device__ __forceinline__ float wave_max_beside_records(float x0, float x1, flo
         "v_cndmask_b32 %[cs], %[x2], %[lowest], %[wins]\n\t"
         "v_readlane_b32 %[best], %[x], 63\n\t"
         "v_or_b32 %[is], %[state], %[fromstay]\n\t"
-        "v_sub_f32 %[rs], %[cs], %[gs]"
-        : [x] "=&v"(x), [best] "=&s"(best), [t0] "=&v"(t0), [t1] "=&v"(t1), [h0] "=&v"(n.h0), [h1] "=&v"(n.h1),
+        "v_sub_f32 %[rs], %[cs], %[gs]\n\t"
+        "v_sub_f32 %[lo], %[best], %[logcut]\n\t"
+        "v_mul_f32 %[hh], %[best], 0.5\n\t"
+        "v_max_f32 %[lo], %[lowest], %[lo]\n\t"
+        "v_mul_f32 %[hl], 0.5, %[lo]\n\t"
+        "v_add_f32 %[cut], %[hl], %[hh]"
+        : [lo] "=&v"(c.lo), [hl] "=&v"(c.half_lo), [hh] "=&v"(c.half_hi), [cut] "=&v"(c.cut), [x] "=&v"(x), [best] "=&s"(best), [t0] "=&v"(t0), [t1] "=&v"(t1), [h0] "=&v"(n.h0), [h1] "=&v"(n.h1),
           [i0] "=&v"(n.info0), [i1] "=&v"(n.info1), [is] "=&v"(n.infos), [rs] "=&v"(n.rests), [cs] "=&v"(cs)
         : [hash] "v"(hash), [b0] "v"(b0), [tab1] "s"(kTab1), [tab2] "s"(kTab2), [st4] "v"(st4), [mask] "s"(state_mask),
           [from] "v"(from), [state] "v"(state), [fromstay] "v"(from_stay), [x0] "v"(x0), [x1] "v"(x1), [x2] "v"(stay_or_fold),
-          [wins] "s"(step_wins), [lowest] "v"(lowest), [gs] "v"(gs));
-    return __uint_as_float(best);
+          [wins] "s"(step_wins), [lowest] "v"(lowest), [gs] "v"(gs), [logcut] "v"(log_cut));
+    return c;
 }
 __device__ __forceinline__ int wave_sum_i(int x) {
     x += __builtin_amdgcn_update_dpp(0, x, 0x128, 0xF, 0xF, true);
@@ -863,10 +874,9 @@ __global__ __launch_bounds__((kBeamThreads<S, CPG, COLS, FWD>), (BeamCfg<S, CPG,
     // throughput-bound waves (the forward scan runs at the same time) it should win the
     // issue arbitration.
     __builtin_amdgcn_s_setprio(3);
-    // Only the even lane of a pair carries the element's stay.  The odd lane adds -FLT_MAX instead of
-    // the stay score, so that its stay candidate is -FLT_MAX (or -inf once the element is dead):
-    // it never passes a cut and never wins a maximum, without a select in every time step.
-    const float stay_h = h == 0 ? stay : -FLT_MAX;
+    // Only the even lane of a pair carries the element's stay.  The odd lane adds -inf instead of the stay score, so that its stay
+    // candidate, like all candidates of a dead element, whose score is -inf, never passes a cut and never wins a maximum, without a mask.
+    const float stay_h = h == 0 ? stay : -INFINITY;
     const uint32_t from = (uint32_t)i << 10, from_stay = from | (1u << 15);  // the element's index as "prev" of its candidates
     int rows_ready = 0;  // last value seen of the loader's counter; it is usually several rows ahead
     const int b0 = 2 * h;
@@ -886,6 +896,7 @@ __global__ __launch_bounds__((kBeamThreads<S, CPG, COLS, FWD>), (BeamCfg<S, CPG,
     uint32_t probe;      // index entry found under `want`
     uint32_t expected;   // what it is if a partner is there, but for the partner's slot
     uint32_t entry, mine_back;  // the element's own entry, as written and as found again
+    uint32_t step_at;           // a partner is step candidate 4j + last base of this element
     uint64_t vm = ~0ull, vs = 0x5555555555555555ull;  // lanes of live elements; of their stay candidates, which sit on the even lanes
     const int i_stay = h == 0 ? i : kW;  // of an odd lane never below the beam's width
     uint32_t hash_keep = ~Idx::kAddress, slot_bits = Idx::kSlot;
@@ -959,6 +970,8 @@ __global__ __launch_bounds__((kBeamThreads<S, CPG, COLS, FWD>), (BeamCfg<S, CPG,
         want = crc2_inverse(hash, info);  // the last base: the two lowest bits
         probe = *(const lds_u32 *)(uintptr_t)and_or(want, Idx::kAddress, idx_base);
         mine_back = own_p[0];
+        step_at = and_or(st4, 12u, cand_base);
+        asm volatile("" : "+v"(step_at));
         __builtin_amdgcn_sched_barrier(0);  // nothing that waits for the row goes before the look-up
         expected = and_or(want, hash_keep, gen);
     };
@@ -974,10 +987,12 @@ __global__ __launch_bounds__((kBeamThreads<S, CPG, COLS, FWD>), (BeamCfg<S, CPG,
     //
     // The wave is alone on its SIMD: a step costs its instructions, about four cycles each, plus the
     // LDS round trips and the reads of comparison masks by the scalar unit (about twenty cycles) that
-    // nothing is placed into (about 1210 cycles for 1 chunk of 64 or 256 states: 0.87 ms at T = 1666; before steps were written out and
+    // nothing is placed into (about 1110 cycles for 1 chunk of 64 or 256 states: 0.80 ms at T = 1666; before steps were written out and
     // rows kept in planes 0.93; in the order of the text, with every wait where its value is first needed, 1.02).  Hence the order
     // below: what does not depend on a round trip is issued while it is under way, comparisons are issued in groups whose masks are
-    // read afterwards.
+    // read afterwards.  That order is fenced where the compiler would count a mask as soon as it is compared: the counts of the cut-off behind all
+    // six comparisons, the fold's verdict behind the logarithm, the proof's behind the comparisons of the next masks (0.847 | 0.800 ms
+    // together; 512 chunks of 64 states 0.957 | 0.915).
     auto step = [&](const int next_t, auto k_tag, auto last_tag) {  // next_t - 1 is the time step, K the ring slot of row next_t
         constexpr int K = decltype(k_tag)::value;
         constexpr bool LAST = decltype(last_tag)::value;
@@ -987,15 +1002,14 @@ __global__ __launch_bounds__((kBeamThreads<S, CPG, COLS, FWD>), (BeamCfg<S, CPG,
         float c1 = ::add_half<kPlanes ? 1 : 0>(kPlanes ? r0h : r1h, score) + g01.y;
         float cs0 = (score + stay_h) + gst;
         lds_store_f2(cand_mine, c0, c1);  // for the merges below
-        const uint32_t step_at = and_or((uint32_t)state << 2, 12u, cand_base);  // the partner is step candidate 4j + last base of this element
 
         // which previous element j has hash_j == want_i: off the index if every live element found its
         // own entry intact, else by comparing with every hash
-        const uint32_t d = probe ^ expected;  // the partner's slot and nothing else, if there is a partner
-        uint32_t at = and_or(d, slot_bits, step_at);
+        uint32_t at = and_or(probe, slot_bits, step_at);
         uint64_t moved = ballot(mine_back != entry);
         if constexpr (K < 0) moved |= replay_all;
-        uint64_t mine_mask = ballot((d & ~Idx::kSlot) == 0u) & vs;  // live even lanes whose stay has a partner
+        // (probe ^ expected) & ~kSlot, which is nothing if there is a partner: live even lanes whose stay has one
+        uint64_t mine_mask = ballot(__builtin_amdgcn_bitop3_b32(probe, Idx::kSlot, expected, 0x12) == 0u) & vs;
         if (__builtin_expect(moved != 0, 0)) {
             // Two live elements in one bucket (or with one hash).  Bit k of m says whether hash k of this
             // half of the beam equals `want`: each comparison is shifted into an accumulator with an
@@ -1119,15 +1133,16 @@ __global__ __launch_bounds__((kBeamThreads<S, CPG, COLS, FWD>), (BeamCfg<S, CPG,
         // no wait before this store: the wave's reads of row t are ahead of it in the LDS queue
         if constexpr (K < 0 || K % Cfg::kHandBack == 0)
             __hip_atomic_store(consumed, next_t, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-        const uint64_t stay_wins = ballot(cs0 > other) & mine_mask;
-        const uint64_t step_wins = mine_mask & ~stay_wins;
+        uint32_t hash_again = hash;  // for the stay's record, in registers side by side with the rest of it
+        asm volatile("" : "+v"(hash_again));
+        const uint64_t stay_above = ballot(cs0 > other);  // its mask is not asked for before the fold is on its way
         const uint32_t target = (uint32_t)pick_by_bit(mine_mask, (int)at, (int)cand_dump);
         // The fold from hardware exp/log, which the step goes on with.  Whether it rounds like the CPU path's double
         // arithmetic (all but a few merges in a thousand at usual score magnitudes) is looked at while the new beam is on its
         // way; if not, the step is done again from here with the double fold.
         const FoldValue estimate = log_sum_exp_value(cs0, other);
-        uint32_t hash_again = hash;  // for the stay's record, in registers side by side with the rest of it
-        asm volatile("" : "+v"(hash_again));
+        __builtin_amdgcn_sched_barrier(0);
+        const uint64_t step_wins = mine_mask & ~stay_above;
         typedef uint32_t u32x3 __attribute__((ext_vector_type(3)));
         u32x3 e;
         auto finish = [&](const float folded) {
@@ -1136,27 +1151,29 @@ __global__ __launch_bounds__((kBeamThreads<S, CPG, COLS, FWD>), (BeamCfg<S, CPG,
         const f32x2 c01 = lds_load_f2(cand_mine);
 
         // cut-off (src/beam_search.c:320-381)
-        // Dead lanes carry -FLT_MAX as their score, which absorbs whatever is added: their candidates
-        // are -FLT_MAX exactly (the stay of an odd lane: -FLT_MAX or -inf, see stay_h).
+        // Dead lanes carry -inf as their score, and so do their candidates (and the stays of odd lanes, see stay_h): they pass no cut, while the
+        // losers of merges, -FLT_MAX, pass the one that keeps everything.
         // The best score does not wait for the step candidates to come back: a fold is not below either of
         // the two scores it joins, so the maximum of the scores before the merges and of the folds is that after them.
         const float stay_or_fold = pick_by_bit(mine_mask, folded, cs0);
         NextRecords next;
         float cs;
-        const float best = wave_max_beside_records(c0, c1, stay_or_fold, next, cs, hash, (uint32_t)b0, (uint32_t)state, from_stay,
-                                                   (uint32_t)state << 2, (uint32_t)(S - 1), from, step_wins, -FLT_MAX, gst);
+        const Cuts first = wave_max_beside_records(c0, c1, stay_or_fold, next, cs, hash, (uint32_t)b0, (uint32_t)state, from_stay,
+                                                   (uint32_t)state << 2, (uint32_t)(S - 1), from, step_wins, -FLT_MAX, gst, log_cut);
         const float s0 = c01.x, s1 = c01.y;  // the steps' scores after the merges
         next.rest0 = s0 - g01.x;
         next.rest1 = s1 - g01.y;
 
         // Nearly every step has more candidates above the first cut than the width, and goes on to the cut
         // halfway to the best score: both are counted at once.
-        float lo = best - log_cut;  // may be -FLT_MAX (no cut at all): mask the dead lanes
-        float hi = best;
-        float cut = (lo + hi) / 2.0f;
+        // Of the bounds of the bisection their halves are kept, which makes the cut between them, (lo + hi) / 2 on the CPU path, one
+        // addition and the two that can come next a fused multiply-add each: halving is exact (down to 2^-125) and changes no rounding.
+        const float lo = first.lo;  // -FLT_MAX: no cut at all, or nobody alive
+        float half_lo = first.half_lo, half_hi = first.half_hi, cut = first.cut;
         const uint64_t a0 = ballot(s0 >= lo), a1 = ballot(s1 >= lo), as = ballot(cs >= lo);
         uint64_t k0 = ballot(s0 >= cut), k1 = ballot(s1 >= cut), ks = ballot(cs >= cut);
-        int kept = popc64(a0 & vm) + popc64(a1 & vm) + popc64(as & vs);
+        __builtin_amdgcn_sched_barrier(0);  // all comparisons, then the first count: a mask takes its time to the scalar unit
+        int kept = popc64(a0) + popc64(a1) + popc64(as);
         // kept candidates on lower lanes: masked bit counts
         auto lower = [&](uint64_t mask, int start) {
             return (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32),
@@ -1164,26 +1181,26 @@ __global__ __launch_bounds__((kBeamThreads<S, CPG, COLS, FWD>), (BeamCfg<S, CPG,
         };
         int steps_kept = popc64(k0) + popc64(k1);  // of `kept` those that are steps
         if (__builtin_expect(kept <= kW, 0)) {
-            k0 = a0 & vm;
-            k1 = a1 & vm;
-            ks = as & vs;
+            k0 = a0;
+            k1 = a1;
+            ks = as;
             steps_kept = popc64(k0) + popc64(k1);
         } else {
             // Bisection between the cut and the best score.  Every cut tried in here lies above
-            // (-FLT_MAX + best) / 2, so dead lanes and dropped candidates never pass and the
-            // ballots need no mask.  (lo + hi) / 2 is the CPU path's (cut + hi) / 2 or
+            // (-FLT_MAX + best) / 2, so the losers of merges never pass.  The cut between the bounds is the CPU path's (cut + hi) / 2 or
             // (cut + lo) / 2: one of the two bounds is the cut just tried.  Two guesses in a row settle most steps; they
             // are nested and not left by jumps, for which the compiler builds a ladder of blocks that costs as much as a guess.
             float next_up, next_down;  // both cuts that can come next, worked out while the masks travel to the scalar unit
             auto look_ahead = [&] {
-                next_up = (cut + hi) / 2.0f;
-                next_down = (lo + cut) / 2.0f;
+                next_up = __builtin_fmaf(cut, 0.5f, half_hi);
+                next_down = __builtin_fmaf(cut, 0.5f, half_lo);
                 asm volatile("" : "+v"(next_up), "+v"(next_down));
             };
             auto next_guess = [&] {
                 const bool up = kept > kW;
-                lo = up ? cut : lo;
-                hi = up ? hi : cut;
+                const float half = 0.5f * cut;
+                half_lo = up ? half : half_lo;
+                half_hi = up ? half_hi : half;
                 cut = up ? next_up : next_down;
             };
             auto count = [&] {
@@ -1191,6 +1208,7 @@ __global__ __launch_bounds__((kBeamThreads<S, CPG, COLS, FWD>), (BeamCfg<S, CPG,
                 k1 = ballot(s1 >= cut);
                 ks = ballot(cs >= cut);
                 look_ahead();
+                __builtin_amdgcn_sched_barrier(0);
                 steps_kept = popc64(k0) + popc64(k1);
                 kept = steps_kept + popc64(ks);
             };
@@ -1210,7 +1228,7 @@ __global__ __launch_bounds__((kBeamThreads<S, CPG, COLS, FWD>), (BeamCfg<S, CPG,
 #pragma unroll 1
                         for (int guess = 5;; ++guess) {
                             next_guess();
-                            if (guess == 10) cut = hi;
+                            if (guess == 10) cut = 2.0f * half_hi;
                             count();
                             if (!too_many_or_few() || guess == 10) break;
                         }
@@ -1276,6 +1294,7 @@ __global__ __launch_bounds__((kBeamThreads<S, CPG, COLS, FWD>), (BeamCfg<S, CPG,
         asm volatile("" : "+s"(open));  // compared here, looked at further down
         uint64_t vm_next = ballot(i < w), vs_next = ballot(i_stay < w);
         asm volatile("" : "+s"(vm_next), "+s"(vs_next));
+        __builtin_amdgcn_sched_barrier(0);
         if (__builtin_expect((open & mine_mask) != 0, 0)) {
             finish(log_sum_exp(cs0, other, lse));  // of the same beam: vm and vs are still its masks
             vm_next = ballot(i < w);
@@ -1290,7 +1309,7 @@ __global__ __launch_bounds__((kBeamThreads<S, CPG, COLS, FWD>), (BeamCfg<S, CPG,
         }
         hash = e.x;
         info = (uint32_t)pick_by_bit(vm, (int)e.z, 0);
-        score = pick_by_bit(vm, __uint_as_float(e.y), -FLT_MAX);
+        score = pick_by_bit(vm, __uint_as_float(e.y), -INFINITY);
         state = (int)(info & 1023u);
         if constexpr (!LAST) fetch_row(next_t, k_tag);
 
