@@ -373,6 +373,29 @@ __device__ __forceinline__ void lse5_all(float (&out)[SPL], const float (&v)[SPL
     }
 }
 
+// The same with the double arithmetic for every lane and no estimate before it: where most updates would turn out unsettled.
+template <int SPL, typename Publish, typename Beside>
+__device__ __forceinline__ void lse5_all_double(float (&out)[SPL], const float (&v)[SPL][5], const LogArgs &logtab, Publish &&publish, Beside &&beside) {
+#pragma unroll
+    for (int i = 0; i < SPL; ++i) {
+        const float m = max5(v[i][0], v[i][1], v[i][2], v[i][3], v[i][4]);
+        float s = (float)ofa::exp_nonpos_ldexp(v[i][0] - m, logtab.expc);
+#pragma unroll
+        for (int k = 1; k < 5; ++k) {
+            __builtin_amdgcn_sched_barrier(0);  // an exponential at a time: side by side they take 60 registers more, and no less time
+            s = (float)((double)s + ofa::exp_nonpos_ldexp(v[i][k] - m, logtab.expc));
+        }
+        out[i] = from_sum(m, s, logtab);
+    }
+    publish();
+    beside(true);
+}
+
+// whether a wave's values are still below `bits` (of a float) in magnitude: those of a step lie close together, lane 0 speaks for all
+__device__ __forceinline__ bool values_below(float value, uint32_t bits) {
+    return ((uint32_t)__builtin_amdgcn_readfirstlane(__float_as_int(value)) & 0x7fffffffu) < bits;
+}
+
 // x + (float)h for the fp16 value h in the low (HI = 0) or high half of a 32-bit register, in one
 // instruction: v_fma_mix_f32 converts the half operand on the fly, the product with 1.0 is
 // exact, so the result is the correctly rounded fp32 sum, bit for bit what v_cvt_f32_f16

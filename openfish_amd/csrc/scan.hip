@@ -249,6 +249,24 @@ __device__ __forceinline__ void pipelined(int count, Step &&step) {
         });
 }
 
+// The same in two kinds of trips: while early() holds, asked once a trip, steps get a true_type as their fourth argument.
+template <int DEPTH, typename Early, typename Step>
+__device__ __forceinline__ void pipelined_from_early(int count, Early &&early, Step &&step) {
+    int j0 = 0;
+    for (; j0 + 2 * DEPTH <= count && early(); j0 += DEPTH)
+        static_for<DEPTH>([&](auto k) { step(k, j0 + (int)k, std::false_type{}, std::true_type{}); });
+    for (; j0 + 2 * DEPTH <= count; j0 += DEPTH)
+        static_for<DEPTH>([&](auto k) { step(k, j0 + (int)k, std::false_type{}, std::false_type{}); });
+    for (; j0 < count && early(); j0 += DEPTH)
+        static_for<DEPTH>([&](auto k) {
+            if (j0 + (int)k < count) step(k, j0 + (int)k, std::true_type{}, std::true_type{});
+        });
+    for (; j0 < count; j0 += DEPTH)
+        static_for<DEPTH>([&](auto k) {
+            if (j0 + (int)k < count) step(k, j0 + (int)k, std::true_type{}, std::false_type{});
+        });
+}
+
 // the five terms of one state of a lane, and of every one; the row's registers are free for the next load afterwards
 template <int I, int SPL>
 __device__ __forceinline__ void bwd_terms_of(float (&v)[5], const float (&a)[SPL], const float4 &nx, const BwdRow<SPL> &row, float stay) {
@@ -275,6 +293,13 @@ template <int SPL>
 __device__ __forceinline__ void fwd_terms(float (&v)[SPL][5], const float (&f)[SPL], float p0, float p1, float p2, float p3,
                                           const FwdRow<SPL> &row, float stay) {
     static_for<SPL>([&](auto i) { fwd_terms_of<i, SPL>(v[i], f, p0, p1, p2, p3, row, stay); });
+}
+
+// the update of a step of the separate sweeps; EARLY: in the double arithmetic at once
+template <int SPL, int MODE, bool EARLY, typename Publish, typename Beside>
+__device__ __forceinline__ void update(float (&out)[SPL], const float (&v)[SPL][5], const LogArgs &logtab, Publish &&publish, Beside &&beside) {
+    if constexpr (EARLY) lse5_all_double<SPL>(out, v, logtab, publish, beside);
+    else lse5_all<SPL, MODE>(out, v, logtab, publish, beside);
 }
 
 // A step of the kernel that holds both sweeps and is capped at 128 registers.  Of four states to a lane the terms are
@@ -324,7 +349,7 @@ __device__ __forceinline__ void fwd_update(float (&f)[SPL], float p0, float p1, 
 // ---------------------------------------------------------------------------
 template <int S, int SPL, int DEPTH, int MODE>
 __global__ __launch_bounds__((Shape<S, SPL>::kThreads)) void bwd_scan_kernel(
-    const _Float16 *__restrict__ scores, float *__restrict__ bwd, int T, int N, float stay, LogSeries series) {
+    const _Float16 *__restrict__ scores, float *__restrict__ bwd, int T, int N, float stay, uint32_t double_below, LogSeries series) {
     using Sh = Shape<S, SPL>;
     constexpr int L = Sh::kLanes;
     constexpr int Q = Sh::kQuarter;
@@ -361,14 +386,6 @@ __global__ __launch_bounds__((Shape<S, SPL>::kThreads)) void bwd_scan_kernel(
         vec[g][0][Vec::at(r, c0 + i)] = 0.f;
     }
 
-    // The first rows are fetched without a condition (of a chunk shorter than DEPTH the oldest row again):
-    // were they not, the compiler, which counts loads in flight, would have to assume that a row's load may
-    // be the latest one and let every trip round the loop below wait for all of them.
-    BwdRow<SPL> ring[DEPTH];
-    static_for<DEPTH>([&](auto k) {
-        ring[k].load(pre + sc_lane);
-        pre -= (int)k < T - 1 ? row_stride : 0;
-    });
     int buf = 0;
     __syncthreads();  // the log table is shared by the whole group
 
@@ -376,24 +393,19 @@ __global__ __launch_bounds__((Shape<S, SPL>::kThreads)) void bwd_scan_kernel(
     // while the write is under way, the row's store and the loads ahead are issued while the verdict's mask is (lse5_all);
     // where a chunk is one wave, the next step's read is asked for as soon as the values are written.
     auto neighbours = [&](int b) { return *reinterpret_cast<const float4 *>(&vec[g][b][Vec::of(4 * r)]); };
-    constexpr bool kBehindRead = SPL == 1;
     float4 nx;
     if constexpr (!Sh::kMultiWave) {
         chunk_sync<false>();
         nx = neighbours(0);
     }
-    pipelined<DEPTH>(T, [&](auto k, int j, auto checked) {
+    // one step; `load_ahead` fetches into the row's registers
+    auto step = [&](BwdRow<SPL> &next, auto early, auto &&load_ahead) {
+        constexpr bool kEarly = decltype(early)::value, kBehindRead = SPL == 1 && !kEarly;
         if constexpr (Sh::kMultiWave) {
             chunk_sync<true>();
             nx = neighbours(buf);
         }
-        const BwdRow<SPL> row = ring[k];
-        auto load_ahead = [&] {
-            if (!checked || j + DEPTH < T) {
-                ring[k].load(pre + sc_lane);
-                pre -= row_stride;
-            }
-        };
+        const BwdRow<SPL> row = next;
         if constexpr (kBehindRead) {
             __builtin_amdgcn_sched_barrier(0);
             load_ahead();
@@ -403,7 +415,7 @@ __global__ __launch_bounds__((Shape<S, SPL>::kThreads)) void bwd_scan_kernel(
         bwd_terms(v, a, nx, row, stay);
         buf ^= 1;
         orow -= S;
-        lse5_all<SPL, MODE>(a, v, logtab, [&] {
+        update<SPL, MODE, kEarly>(a, v, logtab, [&] {
 #pragma unroll
             for (int i = 0; i < SPL; ++i) vec[g][buf][Vec::at(r, c0 + i)] = a[i];
             if constexpr (!Sh::kMultiWave) {
@@ -415,6 +427,50 @@ __global__ __launch_bounds__((Shape<S, SPL>::kThreads)) void bwd_scan_kernel(
             for (int i = 0; i < SPL; ++i) orow[st_lane + i * Q] = a[i];
             if (!kBehindRead && first) load_ahead();
         });
+    };
+    // The first rows are fetched without a condition (of a chunk shorter than the ring the oldest row again):
+    // were they not, the compiler, which counts loads in flight, would have to assume that a row's load may
+    // be the latest one and let every trip round the loop below wait for all of them.
+    auto first_rows = [&](auto &ring, auto depth, int left) {
+        static_for<decltype(depth)::value>([&](auto k) {
+            ring[k].load(pre + sc_lane);
+            pre -= (int)k < left - 1 ? row_stride : 0;
+        });
+    };
+    int done = 0;
+    if constexpr (MODE == OFK_SCAN_TWO_TIER && SPL == 1) {
+        // The early steps, in double arithmetic (double_below in the launcher).  They have a ring of their own and fill the one below anew: with one
+        // ring for both the compiler kept every row twice, 164 registers instead of 120.
+        constexpr int kRows = 8;
+        BwdRow<SPL> ring[kRows];
+        first_rows(ring, std::integral_constant<int, kRows>{}, T);
+        auto trip = [&](auto checked) {
+            static_for<kRows>([&](auto k) {
+                const int j = done + (int)k;
+                if (checked && j >= T) return;
+                step(ring[k], std::true_type{}, [&] {
+                    if (!checked || j + kRows < T) {
+                        ring[k].load(pre + sc_lane);
+                        pre -= row_stride;
+                    }
+                });
+            });
+            done += kRows;
+        };
+        while (done + 2 * kRows <= T && values_below(a[0], double_below)) trip(std::false_type{});
+        while (done < T && values_below(a[0], double_below)) trip(std::true_type{});
+        if (done >= T) return;
+        pre = scores + (size_t)first_chunk * kCols * S + (ptrdiff_t)(T - 1 - done) * row_stride;
+    }
+    BwdRow<SPL> ring[DEPTH];
+    first_rows(ring, std::integral_constant<int, DEPTH>{}, T - done);
+    pipelined<DEPTH>(T - done, [&](auto k, int j, auto checked) {
+        step(ring[k], std::false_type{}, [&] {
+            if (!checked || done + j + DEPTH < T) {
+                ring[k].load(pre + sc_lane);
+                pre -= row_stride;
+            }
+        });
     });
 }
 
@@ -424,7 +480,7 @@ __global__ __launch_bounds__((Shape<S, SPL>::kThreads)) void bwd_scan_kernel(
 template <int S, int SPL, int DEPTH, int MODE>
 __global__ __launch_bounds__((Shape<S, SPL>::kThreads)) void fwd_post_kernel(
     const _Float16 *__restrict__ scores, const float *__restrict__ bwd, float *__restrict__ post, int T,
-    int N, float stay, LogSeries series) {
+    int N, float stay, uint32_t double_below, LogSeries series) {
     using Sh = Shape<S, SPL>;
     constexpr int L = Sh::kLanes;
     constexpr int Q = Sh::kQuarter;
@@ -519,7 +575,7 @@ __global__ __launch_bounds__((Shape<S, SPL>::kThreads)) void fwd_post_kernel(
         e.store(prow + st_lane);
         prow += S;
     };
-    pipelined<DEPTH>(T, [&](auto k, int j, auto checked) {
+    auto step = [&](auto k, int j, auto checked, auto early) {
         row(bring[k]);
         const float p0 = vec[g][buf][q], p1 = vec[g][buf][q + Q];
         const float p2 = vec[g][buf][q + 2 * Q], p3 = vec[g][buf][q + 3 * Q];
@@ -534,8 +590,12 @@ __global__ __launch_bounds__((Shape<S, SPL>::kThreads)) void fwd_post_kernel(
             bpre += S;
         }
         buf ^= 1;
-        lse5_all<SPL, MODE>(f, v, logtab, [&] { fv.store(&vec[g][buf][s0]); }, [](bool) {});
-    });
+        update<SPL, MODE, decltype(early)::value>(f, v, logtab, [&] { fv.store(&vec[g][buf][s0]); }, [](bool) {});
+    };
+    if constexpr (MODE == OFK_SCAN_TWO_TIER && SPL == 1)
+        pipelined_from_early<DEPTH>(T, [&] { return values_below(f[0], double_below); }, step);
+    else
+        pipelined<DEPTH>(T, [&](auto k, int j, auto checked) { step(k, j, checked, std::false_type{}); });
     static_for<DEPTH>([&](auto k) {
         if (T % DEPTH == (int)k) row(bring[k]);
     });
@@ -565,7 +625,7 @@ constexpr int kRolesDepth = 2;
 template <int S, int SPL, int DEPTH>
 __global__ __launch_bounds__((2 * (S / SPL))) void fwd_post_roles_kernel(
     const _Float16 *__restrict__ scores, const float *__restrict__ bwd, float *__restrict__ post, int T,
-    int N, float stay, LogSeries series) {
+    int N, float stay, uint32_t double_below, LogSeries series) {
     constexpr int L = S / SPL;  // lanes of either job
     constexpr int Q = S / 4;
     constexpr int RW = L / 64;  // waves of either job
@@ -605,20 +665,24 @@ __global__ __launch_bounds__((2 * (S / SPL))) void fwd_post_roles_kernel(
         barrier();  // the other half exchanges the maxima behind the shift
         barrier();
         __syncthreads();  // the log table
-        pipelined<DEPTH>(T, [&](auto k, int j, auto checked) {
+        auto step = [&](auto k, int j, auto checked, auto early) {
             barrier();
             const float p0 = vec[buf][q], p1 = vec[buf][q + Q];
             const float p2 = vec[buf][q + 2 * Q], p3 = vec[buf][q + 3 * Q];
             float v[SPL][5];
             fwd_terms(v, f, p0, p1, p2, p3, ring[k], stay);
             buf ^= 1;
-            lse5_all<SPL, OFK_SCAN_TWO_TIER>(f, v, logtab, [&] { fv.store(&vec[buf][s0]); }, [&](bool first) {  // row j + 1
+            update<SPL, OFK_SCAN_TWO_TIER, decltype(early)::value>(f, v, logtab, [&] { fv.store(&vec[buf][s0]); }, [&](bool first) {  // row j + 1
                 if (first && (!checked || j + DEPTH < T)) {
                     ring[k].load(pre + sc_lane);
                     pre += row_stride;
                 }
             });
-        });
+        };
+        if constexpr (SPL == 1)
+            pipelined_from_early<DEPTH>(T, [&] { return values_below(f[0], double_below); }, step);
+        else
+            pipelined<DEPTH>(T, [&](auto k, int j, auto checked) { step(k, j, checked, std::false_type{}); });
         barrier();
         barrier();  // the other half finishes row T
     } else {
@@ -693,7 +757,7 @@ __global__ __launch_bounds__((2 * (S / SPL))) void fwd_post_roles_kernel(
 // ---------------------------------------------------------------------------
 template <int S, int DEPTH>
 __global__ __launch_bounds__(S) void fwd_scan_kernel(const _Float16 *__restrict__ scores, float *__restrict__ fwd, int T, int N,
-                                                     float stay, LogSeries series) {
+                                                     float stay, uint32_t double_below, LogSeries series) {
     constexpr int Q = S / 4;
     static_assert(S > 64, "a state to a lane, and several waves");
     __shared__ __attribute__((aligned(16))) float vec[2][S];
@@ -716,7 +780,7 @@ __global__ __launch_bounds__(S) void fwd_scan_kernel(const _Float16 *__restrict_
     vec[0][s] = 0.f;
     frow[s] = 0.f;
     __syncthreads();  // the log table
-    pipelined<DEPTH>(T, [&](auto k, int j, auto checked) {
+    pipelined_from_early<DEPTH>(T, [&] { return values_below(f[0], double_below); }, [&](auto k, int j, auto checked, auto early) {
         chunk_sync<true>();
         const float p0 = vec[buf][q], p1 = vec[buf][q + Q], p2 = vec[buf][q + 2 * Q], p3 = vec[buf][q + 3 * Q];
         const FwdRow<1> row = ring[k];
@@ -730,7 +794,7 @@ __global__ __launch_bounds__(S) void fwd_scan_kernel(const _Float16 *__restrict_
         fwd_terms(v, f, p0, p1, p2, p3, row, stay);
         buf ^= 1;
         frow += S;
-        lse5_all<1, OFK_SCAN_TWO_TIER>(f, v, logtab, [&] { vec[buf][s] = f[0]; }, [&](bool) { frow[s] = f[0]; });
+        update<1, OFK_SCAN_TWO_TIER, decltype(early)::value>(f, v, logtab, [&] { vec[buf][s] = f[0]; }, [&](bool) { frow[s] = f[0]; });
     });
 }
 
@@ -1162,6 +1226,19 @@ bool eight_rows(int N, int beside_merged) {
     return (long)N * (S / 64) > kWavesOfDepth16 || (S == 256 && beside_merged && N > kChunksBesideMerged);
 }
 
+// Up to which magnitude of its values a sweep with one state to a lane takes the double arithmetic for every update at once.  An ulp of small
+// values is below or near the estimate's bound, most steps have several unsettled updates somewhere in a chunk, and the double arithmetic
+// behind an estimate and its verdict takes longer than by itself.  Values grow by about four a step; below 0 | 256 | 512 | 1024 | 2048 |
+// 4096, backward sweep, us: 5 chunks of 64 states, T = 512 154 | 142 | 137 | 133 | 139 | 140; 512 of them, T = 1666 386 | 376 | 369 | 369 |
+// 378 | 422; 16 of 256 states, T = 1666 577 | 565 | 558 | 548 | 538 | 555; 200, T = 600 258 | 246 | 239 | 228 | 216 | 217.  Where waves
+// share a SIMD the other waves' trips are hidden and instructions count: 400 of 256 states, T = 256 138 | 135 | 143 | 146; 37 of 1024, T = 833
+// 662 | 652 | 659 | 678.  The forward sweeps beside a search lose less time to unsettled updates (16 of 256 states 599 | 592 | 588 | 584 | 590 | 628).
+uint32_t double_below(int S, int N, bool backward) {
+    constexpr uint32_t k256 = 0x43800000u, k1024 = 0x44800000u, k2048 = 0x45000000u;  // as floats
+    if ((long)N * (S / 64) > 1024) return S == 256 && !backward ? 0u : k256;  // more than a wave for every SIMD, or sixteen waves to a chunk
+    return S == 1024 ? k256 : S == 256 && backward ? k2048 : k1024;
+}
+
 template <int S, int SPL, int DEPTH>
 int launch_bwd(int mode, const void *scores, float *bwd, int T, int N, float stay, int beside_merged, Queue st) {
     using Sh = Shape<S, SPL>;
@@ -1172,21 +1249,21 @@ int launch_bwd(int mode, const void *scores, float *bwd, int T, int N, float sta
         case OFK_SCAN_TWO_TIER:
             if constexpr (SPL == 1 && S <= 256) {
                 if (eight_rows<S>(N, beside_merged)) {
-                    queue_kernel((bwd_scan_kernel<S, SPL, DEPTH, OFK_SCAN_TWO_TIER>), grid, block, 0, st, sc, bwd, T, N, stay, kSeries);
+                    queue_kernel((bwd_scan_kernel<S, SPL, DEPTH, OFK_SCAN_TWO_TIER>), grid, block, 0, st, sc, bwd, T, N, stay, double_below(S, N, true), kSeries);
                     break;
                 }
             }
-            queue_kernel((bwd_scan_kernel<S, SPL, kDeep, OFK_SCAN_TWO_TIER>), grid, block, 0, st, sc, bwd, T, N, stay, kSeries);
+            queue_kernel((bwd_scan_kernel<S, SPL, kDeep, OFK_SCAN_TWO_TIER>), grid, block, 0, st, sc, bwd, T, N, stay, double_below(S, N, true), kSeries);
             break;
         case OFK_SCAN_PRECISE:
             if constexpr (SPL == kPlainSpl<S>)
-                queue_kernel((bwd_scan_kernel<S, SPL, DEPTH, OFK_SCAN_PRECISE>), grid, block, 0, st, sc, bwd, T, N, stay, kSeries);
+                queue_kernel((bwd_scan_kernel<S, SPL, DEPTH, OFK_SCAN_PRECISE>), grid, block, 0, st, sc, bwd, T, N, stay, double_below(S, N, true), kSeries);
             else
                 return OFK_BAD_ARGS;
             break;
         case OFK_SCAN_FAST:
             if constexpr (SPL == kPlainSpl<S>)
-                queue_kernel((bwd_scan_kernel<S, SPL, DEPTH, OFK_SCAN_FAST>), grid, block, 0, st, sc, bwd, T, N, stay, kSeries);
+                queue_kernel((bwd_scan_kernel<S, SPL, DEPTH, OFK_SCAN_FAST>), grid, block, 0, st, sc, bwd, T, N, stay, double_below(S, N, true), kSeries);
             else
                 return OFK_BAD_ARGS;
             break;
@@ -1208,21 +1285,21 @@ int launch_fwd(int mode, const void *scores, const float *bwd, float *post, int 
             if constexpr (Sh::kMultiWave && 2 * Sh::kLanes <= 1024) {
                 if ((long)N * (2 * Sh::kLanes / 64) <= 4096) {
                     queue_kernel((fwd_post_roles_kernel<S, SPL, kRolesDepth>), dim3(N), dim3(2 * Sh::kLanes), 0, st, sc, bwd, post,
-                                       T, N, stay, kSeries);
+                                       T, N, stay, double_below(S, N, false), kSeries);
                     break;
                 }
             }
-            queue_kernel((fwd_post_kernel<S, SPL, DEPTH, OFK_SCAN_TWO_TIER>), grid, block, 0, st, sc, bwd, post, T, N, stay, kSeries);
+            queue_kernel((fwd_post_kernel<S, SPL, DEPTH, OFK_SCAN_TWO_TIER>), grid, block, 0, st, sc, bwd, post, T, N, stay, double_below(S, N, false), kSeries);
             break;
         case OFK_SCAN_PRECISE:
             if constexpr (SPL == kPlainSpl<S>)
-                queue_kernel((fwd_post_kernel<S, SPL, DEPTH, OFK_SCAN_PRECISE>), grid, block, 0, st, sc, bwd, post, T, N, stay, kSeries);
+                queue_kernel((fwd_post_kernel<S, SPL, DEPTH, OFK_SCAN_PRECISE>), grid, block, 0, st, sc, bwd, post, T, N, stay, double_below(S, N, false), kSeries);
             else
                 return OFK_BAD_ARGS;
             break;
         case OFK_SCAN_FAST:
             if constexpr (SPL == kPlainSpl<S>)
-                queue_kernel((fwd_post_kernel<S, SPL, DEPTH, OFK_SCAN_FAST>), grid, block, 0, st, sc, bwd, post, T, N, stay, kSeries);
+                queue_kernel((fwd_post_kernel<S, SPL, DEPTH, OFK_SCAN_FAST>), grid, block, 0, st, sc, bwd, post, T, N, stay, double_below(S, N, false), kSeries);
             else
                 return OFK_BAD_ARGS;
             break;
@@ -1379,7 +1456,7 @@ static int fwd_post_scan(const void *scores, const float *bwd, float *post, int 
 static int fwd_scan(const void *scores, float *fwd, int T, int N, int state_len, float stay, void *stream, void *done) {
     if (!scores || !fwd || T < 1 || N < 1 || state_len != 5 || !aligned16(scores) || !aligned16(fwd)) return OFK_BAD_ARGS;
     queue_kernel((fwd_scan_kernel<1024, OFK_DEPTH_1024>), dim3(N), dim3(1024), 0, Queue{static_cast<hipStream_t>(stream), static_cast<hipEvent_t>(done)},
-                       static_cast<const _Float16 *>(scores), fwd, T, N, stay, kSeries);
+                       static_cast<const _Float16 *>(scores), fwd, T, N, stay, double_below(1024, N, false), kSeries);
     return (int)hipGetLastError();
 }
 
