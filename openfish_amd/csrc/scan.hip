@@ -347,7 +347,7 @@ __device__ __forceinline__ void fwd_update(float (&f)[SPL], float p0, float p1, 
 // ---------------------------------------------------------------------------
 // backward: bwd[n][t][s] for t = T..0
 // ---------------------------------------------------------------------------
-template <int S, int SPL, int DEPTH, int MODE>
+template <int S, int SPL, int DEPTH, int MODE, bool EARLY>  // EARLY: the first steps in double arithmetic, while values are small
 __global__ __launch_bounds__((Shape<S, SPL>::kThreads)) void bwd_scan_kernel(
     const _Float16 *__restrict__ scores, float *__restrict__ bwd, int T, int N, float stay, uint32_t double_below, LogSeries series) {
     using Sh = Shape<S, SPL>;
@@ -438,7 +438,8 @@ __global__ __launch_bounds__((Shape<S, SPL>::kThreads)) void bwd_scan_kernel(
         });
     };
     int done = 0;
-    if constexpr (MODE == OFK_SCAN_TWO_TIER && SPL == 1) {
+    if constexpr (EARLY) {
+        static_assert(MODE == OFK_SCAN_TWO_TIER && SPL == 1);
         // The early steps, in double arithmetic (double_below in the launcher).  They have a ring of their own and fill the one below anew: with one
         // ring for both the compiler kept every row twice, 164 registers instead of 120.
         constexpr int kRows = 8;
@@ -477,7 +478,7 @@ __global__ __launch_bounds__((Shape<S, SPL>::kThreads)) void bwd_scan_kernel(
 // ---------------------------------------------------------------------------
 // forward + posterior: post[n][t][s] = softmax_s(fwd[t][s] + bwd[n][t][s]), t = 0..T
 // ---------------------------------------------------------------------------
-template <int S, int SPL, int DEPTH, int MODE>
+template <int S, int SPL, int DEPTH, int MODE, bool EARLY>
 __global__ __launch_bounds__((Shape<S, SPL>::kThreads)) void fwd_post_kernel(
     const _Float16 *__restrict__ scores, const float *__restrict__ bwd, float *__restrict__ post, int T,
     int N, float stay, uint32_t double_below, LogSeries series) {
@@ -592,7 +593,7 @@ __global__ __launch_bounds__((Shape<S, SPL>::kThreads)) void fwd_post_kernel(
         buf ^= 1;
         update<SPL, MODE, decltype(early)::value>(f, v, logtab, [&] { fv.store(&vec[g][buf][s0]); }, [](bool) {});
     };
-    if constexpr (MODE == OFK_SCAN_TWO_TIER && SPL == 1)
+    if constexpr (EARLY)
         pipelined_from_early<DEPTH>(T, [&] { return values_below(f[0], double_below); }, step);
     else
         pipelined<DEPTH>(T, [&](auto k, int j, auto checked) { step(k, j, checked, std::false_type{}); });
@@ -1239,6 +1240,14 @@ uint32_t double_below(int S, int N, bool backward) {
     return S == 1024 ? k256 : S == 256 && backward ? k2048 : k1024;
 }
 
+// Where the kernels have these early steps.  What follows them in the same kernel is slower for it where waves share a SIMD.  Backward sweep of 256
+// states, us, without | with: 300 chunks, T = 96 59 | 55, 200 109 | 107, 300 156 | 155, 500 243 | 246; 512, T = 96 67 | 63, 200 118 | 115, 300 172 |
+// 172, 500 248 | 252, 1666 677 | 711, with five columns 695 | 732; of the other models the early steps are ahead at any size (1024 states, 160 chunks, T = 64
+// 74 | 63, 833 661 | 655; 2048 of 64, T = 1000 357 | 350).  Forward sweep of 64 states beside a search: 1024 chunks, T = 300 184 | 175, T = 1666 733 |
+// 685; 1500 234 | 315 and 1002 | 1324.
+bool early_backward(int S, int T, int N) { return S != 256 || N <= 256 || T <= 256; }
+constexpr int kEarlyForwardChunks = 1024;
+
 template <int S, int SPL, int DEPTH>
 int launch_bwd(int mode, const void *scores, float *bwd, int T, int N, float stay, int beside_merged, Queue st) {
     using Sh = Shape<S, SPL>;
@@ -1249,21 +1258,27 @@ int launch_bwd(int mode, const void *scores, float *bwd, int T, int N, float sta
         case OFK_SCAN_TWO_TIER:
             if constexpr (SPL == 1 && S <= 256) {
                 if (eight_rows<S>(N, beside_merged)) {
-                    queue_kernel((bwd_scan_kernel<S, SPL, DEPTH, OFK_SCAN_TWO_TIER>), grid, block, 0, st, sc, bwd, T, N, stay, double_below(S, N, true), kSeries);
+                    queue_kernel((bwd_scan_kernel<S, SPL, DEPTH, OFK_SCAN_TWO_TIER, false>), grid, block, 0, st, sc, bwd, T, N, stay, 0u, kSeries);
                     break;
                 }
             }
-            queue_kernel((bwd_scan_kernel<S, SPL, kDeep, OFK_SCAN_TWO_TIER>), grid, block, 0, st, sc, bwd, T, N, stay, double_below(S, N, true), kSeries);
+            if constexpr (SPL == 1) {
+                if (early_backward(S, T, N)) {
+                    queue_kernel((bwd_scan_kernel<S, SPL, kDeep, OFK_SCAN_TWO_TIER, true>), grid, block, 0, st, sc, bwd, T, N, stay, double_below(S, N, true), kSeries);
+                    break;
+                }
+            }
+            queue_kernel((bwd_scan_kernel<S, SPL, kDeep, OFK_SCAN_TWO_TIER, false>), grid, block, 0, st, sc, bwd, T, N, stay, 0u, kSeries);
             break;
         case OFK_SCAN_PRECISE:
             if constexpr (SPL == kPlainSpl<S>)
-                queue_kernel((bwd_scan_kernel<S, SPL, DEPTH, OFK_SCAN_PRECISE>), grid, block, 0, st, sc, bwd, T, N, stay, double_below(S, N, true), kSeries);
+                queue_kernel((bwd_scan_kernel<S, SPL, DEPTH, OFK_SCAN_PRECISE, false>), grid, block, 0, st, sc, bwd, T, N, stay, 0u, kSeries);
             else
                 return OFK_BAD_ARGS;
             break;
         case OFK_SCAN_FAST:
             if constexpr (SPL == kPlainSpl<S>)
-                queue_kernel((bwd_scan_kernel<S, SPL, DEPTH, OFK_SCAN_FAST>), grid, block, 0, st, sc, bwd, T, N, stay, double_below(S, N, true), kSeries);
+                queue_kernel((bwd_scan_kernel<S, SPL, DEPTH, OFK_SCAN_FAST, false>), grid, block, 0, st, sc, bwd, T, N, stay, 0u, kSeries);
             else
                 return OFK_BAD_ARGS;
             break;
@@ -1289,17 +1304,23 @@ int launch_fwd(int mode, const void *scores, const float *bwd, float *post, int 
                     break;
                 }
             }
-            queue_kernel((fwd_post_kernel<S, SPL, DEPTH, OFK_SCAN_TWO_TIER>), grid, block, 0, st, sc, bwd, post, T, N, stay, double_below(S, N, false), kSeries);
+            if constexpr (S == 64 && SPL == 1) {
+                if (N <= kEarlyForwardChunks) {
+                    queue_kernel((fwd_post_kernel<S, SPL, DEPTH, OFK_SCAN_TWO_TIER, true>), grid, block, 0, st, sc, bwd, post, T, N, stay, double_below(S, N, false), kSeries);
+                    break;
+                }
+            }
+            queue_kernel((fwd_post_kernel<S, SPL, DEPTH, OFK_SCAN_TWO_TIER, false>), grid, block, 0, st, sc, bwd, post, T, N, stay, 0u, kSeries);
             break;
         case OFK_SCAN_PRECISE:
             if constexpr (SPL == kPlainSpl<S>)
-                queue_kernel((fwd_post_kernel<S, SPL, DEPTH, OFK_SCAN_PRECISE>), grid, block, 0, st, sc, bwd, post, T, N, stay, double_below(S, N, false), kSeries);
+                queue_kernel((fwd_post_kernel<S, SPL, DEPTH, OFK_SCAN_PRECISE, false>), grid, block, 0, st, sc, bwd, post, T, N, stay, 0u, kSeries);
             else
                 return OFK_BAD_ARGS;
             break;
         case OFK_SCAN_FAST:
             if constexpr (SPL == kPlainSpl<S>)
-                queue_kernel((fwd_post_kernel<S, SPL, DEPTH, OFK_SCAN_FAST>), grid, block, 0, st, sc, bwd, post, T, N, stay, double_below(S, N, false), kSeries);
+                queue_kernel((fwd_post_kernel<S, SPL, DEPTH, OFK_SCAN_FAST, false>), grid, block, 0, st, sc, bwd, post, T, N, stay, 0u, kSeries);
             else
                 return OFK_BAD_ARGS;
             break;

@@ -59,3 +59,17 @@ def test_both_sweeps_of_1024_states_apart(api, T, kind):  # noqa: F811
         gb.free()
     assert np.array_equal(got[0][0], got[1][0])
     close(got[0][1], got[1][1])
+
+
+@pytest.mark.parametrize("state_len,N,T", [(4, 256, 257), (4, 257, 256), (4, 257, 257), (3, 1024, 40), (3, 1025, 40)])
+def test_either_side_of_the_sizes_that_have_early_steps(api, state_len, N, T):  # noqa: F811
+    """kernels with and without them, bwd bit for bit the oracle's, posteriors within the bar of the always-double arithmetic's"""
+    S = 4 ** state_len
+    s16 = scores_of("plain", T, 3, S, N + T)
+    ref, _, _ = O.scans(s16.astype(np.float32), state_len)
+    tiled = np.ascontiguousarray(np.tile(s16, (1, -(-N // 3), 1))[:, :N])
+    bwd, post = stage_scans(api, tiled, state_len, 2.0, "two_tier", False)
+    _, precise = stage_scans(api, s16, state_len, 2.0, "precise", False)
+    for n in (0, N // 2, N - 1):
+        assert np.array_equal(bwd[n], ref[n % 3]), n
+        close(post[n], precise[n % 3])
