@@ -520,13 +520,17 @@ static int join_null_stream(ofa_gpubuf_t *g) {
  *                T = 400: 340 0.66 | 0.54 | 0.54;  420 0.67 | 0.56 | 0.55;  512 0.69 | 0.57 | 0.56;  T = 96: 256 0.190 | 0.176 | 0.182;  340 0.219 | 0.202 | 0.193;
  *                513 3.39 | 2.42 | 3.19;  640 3.57 | 2.97 | 3.41;  660 3.58 | 3.41 | 3.40;  768 3.68 | 3.52 | 3.46;  1024 4.33 | 4.71 | 3.96;
  *                five columns: 640 3.70 | 3.22 | 3.46;  660 3.74 | 3.65 | 3.51;  T = 1201: 768 2.69 | 2.60 | 2.60;  five columns 660 2.70 | 2.66 | 2.63;
+ *                with the present search, split | merged: 256 1.56 | 1.62;  260 1.70 | 1.71;  300 1.72 | 1.73;  320 1.73 | 1.73;  340 1.74 | 1.74;  440 1.91 | 1.78;
+ *                512 2.15 | 1.82;  five columns: 280 1.72 | 1.74;  320 1.74 | 1.75;  512 2.34 | 1.86;  T = 1201: 260 1.29 | 1.29;  340 1.32 | 1.31;
+ *                five columns 320 1.32 | 1.33;  T = 600: 340 0.742 | 0.739;  T = 200: 280 0.296 | 0.291;
  *                T = 800: 768 1.79 | 1.76 | 1.81;  five columns 768 1.86 | 1.83 | 1.85;  T = 1000: five columns 680 2.25 | 2.23 | 2.22
  *     64 states: 16 1.59 | 1.31;  512 1.87 | 1.54;  2048 4.11 | 3.41
  * Hence the lines.  Up to 168 chunks of 1024 states the search and the forward sweep find compute units of their own (21 and 11 of an
  * XCD's 32); up to 340, in two rounds, split is ahead while its bytes fit beneath the chain, and short chunks allow more of them:
  * 11.55 MB a step, less 1300 bytes for every step of a chunk.  Chunks shorter than 12 steps are decided by launches and
  * set-up, batches above 340 of chunks up to 100 steps by the rounds.  Up to 512 chunks of 256 states the chain of split is
- * shorter, while its bytes fit beneath the chain, 3.2 MB a step (short chunks of 280 to 446 are ahead merged by up to 0.01 ms: left); above,
+ * shorter, while its bytes fit beneath the chain, 2.5 MB a step (348 chunks; 3.2 MB when a step of the search took a tenth longer, under which more
+ * bytes found time); above,
  * the search's workgroups hold four chunks, a unit that has one of them in the merged kernel takes as long as one that has four,
  * and split has units left for the forward sweep up to 640 chunks, with shorter chunks up to 768.
  *
@@ -548,7 +552,7 @@ static int arrangement_by_default(int T, int N, int C, int state_len, int shared
         case 3: return N <= 2048 ? ARR_SPLIT : ARR_ONE;
         case 4:
             if (!can_merge) return N <= 768 ? ARR_SPLIT : ARR_ONE;
-            if (N <= 512) return shared || step_bytes > 3200000 ? ARR_MERGED : ARR_SPLIT;
+            if (N <= 512) return shared || step_bytes > 2500000 ? ARR_MERGED : ARR_SPLIT;
             if (!shared) return N <= 640 || (N <= 768 && chunk_scores <= 1250000) ? ARR_SPLIT : ARR_MERGED;
             if (T <= 400 && N <= 608) return ARR_ONE;
             return chunk_scores <= 1900000 && N <= (chunk_scores <= 950000 ? 608 : 548) ? ARR_SPLIT : ARR_MERGED;
