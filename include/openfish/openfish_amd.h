@@ -189,8 +189,7 @@ enum openfish_amd_stage {
  * Device-side durations in milliseconds (HIP events, completed by the kernels' own ends) of the
  * most recent decode on this gpubuf.  A stage counts from the end of the last one that it waits
  * for to the end of its kernel, so the queue's gap before the kernel, 5 to 10 us where another stream
- * is waited for, is part of it; the first counts from the decode's start on its stream (a blocking
- * decode with the device to itself marks it beside its first kernel, up to 2 us late: never before 0), and where the
+ * is waited for, is part of it; the first counts from the decode's start on its stream, and where the
  * device is shared, whatever another decode's kernels hold up between the two ends counts as well.
  * (Events at the start of every kernel would cost each 3 to 5 us.)  For kernels by themselves use
  * a profiler.  Writes min(n, OPENFISH_AMD_STAGE_COUNT) values and returns that count.

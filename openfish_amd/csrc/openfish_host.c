@@ -487,16 +487,15 @@ static void fetch_outputs(ofa_gpubuf_t *g, int T, int N, uint8_t **moves, char *
  * has ended already, which the query tells in 0.2 us, there is nothing to wait for: the event and the wait for it in another hardware
  * queue put 20 us before a decode's first kernel.  That the query answers for the streams ordered with the null stream too is this
  * runtime's doing, and tested for copies and kernels of both.  It is the current device's null stream: a gpubuf of another device is
- * refused, as recording its event there is by the runtime.  Returns whether there was something to wait for: EV_JOIN then marks its end. */
-static int join_null_stream(ofa_gpubuf_t *g) {
+ * refused, as recording its event there is by the runtime. */
+static void join_null_stream(ofa_gpubuf_t *g) {
     int device;
     HIP_OK(hipGetDevice(&device));
     if (device != g->device) die("the gpubuf belongs to another device than the current one");
-    if (hipStreamQuery(0) == hipSuccess) return 0;
+    if (hipStreamQuery(0) == hipSuccess) return;
     if (hipPeekAtLastError() == hipErrorNotReady) (void)hipGetLastError(); /* the query's answer, but no error that the caller left behind */
     HIP_OK(hipEventRecord(g->ev[EV_JOIN], 0));
     HIP_OK(hipStreamWaitEvent(g->s_main, g->ev[EV_JOIN], 0));
-    return 1;
 }
 
 /* Which arrangement of the scans a decode finishes soonest with.  What bounds them, after the backward sweep:
@@ -604,16 +603,14 @@ static void enqueue_decode(ofa_gpubuf_t *g, const int T, const int N, const int 
     g->pend_sums = use_sums;
     g->pend_copy = !shared && nt >= OFA_COPY_MOVES;
     if (g->pend_split == ARR_SPLIT || use_sums || g->pend_copy) take_side_lane(g);
-    const int joined = join_null_stream(g);
-    /* The start is a marker, which holds up what is behind it by 3 us: where the side lane has nothing to do yet it goes there, once
-     * the first kernel is queued. */
-    const int start_beside = g->side_lane >= 0 && !shared && !joined;
-    if (!start_beside) HIP_OK(hipEventRecord(g->ev[EV_START], g->s_main));
+    join_null_stream(g);
+    /* A marker, which holds up the first kernel by 3 us.  It has to be ahead of that kernel on the same stream: on the side lane it would be
+     * behind whatever another thread's decode, or a stream of the caller's in the same hardware queue, has there meanwhile. */
+    HIP_OK(hipEventRecord(g->ev[EV_START], g->s_main));
     if (g->pend_split == ARR_MERGED) {
         /* backward sweep, then the search with the forward sweep and the posterior in its workgroups */
         launch_ok(ofk_bwd_scan(scores_TNC, g->pub.bwd_NTC, T, N, state_len, cols, stay, g->scan_mode, g->scan_spl, shared, g->s_main,
                                g->ev[EV_BWD_END]), "bwd_scan");
-        if (start_beside) HIP_OK(hipEventRecord(g->ev[EV_START], g->s_side));
         launch_ok(ofk_beam_search_forward(scores_TNC, g->pub.bwd_NTC, g->pub.post_NTC, (ofk_beam_slot_t *)g->pub.beam_vector,
                                           (int32_t *)g->pub.states, g->pub.moves, T, N, state_len, cols,
                                           log_beam_cut(options), stay, g->lse_table, g->debug_flags, g->s_main, g->ev[EV_BEAM_END]),
@@ -622,7 +619,6 @@ static void enqueue_decode(ofa_gpubuf_t *g, const int T, const int N, const int 
         /* both sweeps and the posterior in one kernel, then the beam search, all on one stream */
         launch_ok(ofk_scan_posterior(scores_TNC, g->pub.bwd_NTC, g->pub.post_NTC, T, N, state_len, cols, stay, g->scan_mode,
                                      g->scan_spl, g->s_main, g->ev[EV_BWD_END]), "scan_posterior");
-        if (start_beside) HIP_OK(hipEventRecord(g->ev[EV_START], g->s_side));
         launch_ok(ofk_beam_search(scores_TNC, g->pub.bwd_NTC, (ofk_beam_slot_t *)g->pub.beam_vector,
                                   (int32_t *)g->pub.states, g->pub.moves, T, N, state_len, cols, log_beam_cut(options),
                                   stay, g->lse_table, search_flags, g->s_main, g->ev[EV_BEAM_END]), "beam_search");
@@ -643,9 +639,8 @@ static void enqueue_decode(ofa_gpubuf_t *g, const int T, const int N, const int 
         const int apart = g->pend_apart = state_len == 5 && N <= 96 && !shared && g->scan_mode == OFK_SCAN_TWO_TIER && g->scan_spl == 0;
         launch_ok(ofk_bwd_scan(scores_TNC, g->pub.bwd_NTC, T, N, state_len, cols, stay, g->scan_mode, g->scan_spl, 0, g->s_main,
                                g->ev[EV_BWD_END]), "bwd_scan");
-        if (start_beside) HIP_OK(hipEventRecord(g->ev[EV_START], g->s_side));
         if (apart) {
-            if (joined) HIP_OK(hipStreamWaitEvent(g->s_side, g->ev[EV_JOIN], 0));
+            HIP_OK(hipStreamWaitEvent(g->s_side, g->ev[EV_START], 0));
             launch_ok(ofk_fwd_scan(scores_TNC, g->pub.post_NTC, T, N, state_len, cols, stay, g->s_side, g->ev[EV_FWD_SCAN_END]),
                       "fwd_scan");
         }
@@ -757,9 +752,6 @@ int openfish_amd_last_timings(const openfish_gpubuf_t *gpubuf, float *ms, int n)
         g->ms[OPENFISH_AMD_STAGE_BWD] = g->ms[OPENFISH_AMD_STAGE_FWD] = 0.0f;
         HIP_OK(hipEventElapsedTime(&g->ms[OPENFISH_AMD_STAGE_SCAN], g->ev[EV_START], g->ev[EV_BWD_END]));
     }
-    /* a start marked beside the first kernel can be behind the end of one of a few steps */
-    if (g->ms[OPENFISH_AMD_STAGE_BWD] < 0.0f) g->ms[OPENFISH_AMD_STAGE_BWD] = 0.0f;
-    if (g->ms[OPENFISH_AMD_STAGE_SCAN] < 0.0f) g->ms[OPENFISH_AMD_STAGE_SCAN] = 0.0f;
     g->ms[OPENFISH_AMD_STAGE_FWD_SCAN] = 0.0f;
     if (g->pend_split == ARR_SPLIT && g->pend_apart) {
         /* the posteriors' pass begins with the later of the two sweeps' ends */

@@ -73,3 +73,39 @@ def test_an_error_that_the_caller_left_behind_is_still_reported(run, call, busy)
     """the launch of the kernel that was to make the scores, say: the first launch of the decode finds it"""
     done = run("g = buf(); busy[0] = %d; L.stub_fail(); %s(g); print('went on')" % (busy, call))
     assert done.returncode == 1 and "invalid configuration" in done.stderr and "went on" not in done.stdout, done
+
+
+TIMED = """
+T, N, SL = %d, %d, %d
+scores = C.create_string_buffer(2 * T * N * 4 ** (SL + 1))
+g = buf()
+L.openfish_amd_gpubuf_set_split_scans(g, %d)
+ms = (C.c_float * 8)()
+def timed(intruder):
+    C.c_int.in_dll(L, "stub_intruder").value = intruder
+    L.openfish_decode_gpu(T, N, 4 ** (SL + 1), scores, SL, C.byref(opt), g, *refs)
+    assert L.openfish_amd_last_timings(g, ms, 8) == 8
+    print(*ms)
+"""
+
+
+# what the decode waits for on another lane: 64 states sweep and sums | sums; 256 states sweep | nothing but the copy of its moves | sums;
+# few of 1024 states a sweep from the decode's start, and the posteriors' pass
+@pytest.mark.parametrize("state_len,T,N,split,total", [(3, 8, 2, -1, 53), (3, 8, 2, 0, 52), (4, 8, 2, 1, 52), (4, 2048, 64, 2, 3), (4, 2048, 64, 0, 52),
+                                                       (5, 16, 2, -1, 53)])
+def test_a_decodes_times_begin_with_its_first_kernel_whatever_the_other_lanes_do(run, state_len, T, N, split, total):
+    """another thread's decode puts 50 ms of work on every other stream while this one's kernels, a millisecond each, are being queued"""
+    done = run(TIMED % (T, N, state_len, split) + "timed(50)")
+    assert done.returncode == 0, done
+    ms = dict(zip(("bwd", "fwd", "beam", "seq", "total", "scan", "sums", "fwd_scan"), map(float, done.stdout.split())))
+    assert (ms["bwd"], ms["scan"]) == ((0, 1) if split == 0 else (1, 0)) and ms["beam"] == 1 and ms["seq"] == 1 and ms["total"] == total
+    assert ms["fwd_scan"] == (51 if state_len == 5 else 0)
+
+
+def test_a_forward_sweep_beside_the_backward_one_does_not_end_before_its_decode_starts(run):
+    """decodes on lanes that are ahead of one another"""
+    done = run(TIMED % (16, 2, 5, -1) + "for x in range(6): timed(50 - 7 * x)")
+    assert done.returncode == 0, done
+    for line in done.stdout.splitlines():
+        bwd, fwd, beam, seq, total, scan, sums, fwd_scan = map(float, line.split())
+        assert bwd == 1 and 1 <= fwd_scan < total, done.stdout
