@@ -1645,7 +1645,7 @@ extern "C" int ofk_beam_search_static_ready(void) {
 extern "C" int ofk_beam_search_static(const void *scores, const float *bwd, int32_t *states, uint8_t *moves, int T,
                                       int N, int state_len, int columns, float log_beam_cut, float stay, int flags,
                                       void *stream) {
-    if (!scores || !bwd || !states || !moves || T < 1 || N < 1) return OFK_BAD_ARGS;
+    if (!scores || !bwd || !states || !moves || T < 1 || T > OFK_MAX_T || N < 1) return OFK_BAD_ARGS;
     if ((reinterpret_cast<uintptr_t>(scores) | reinterpret_cast<uintptr_t>(bwd)) & 15u) return OFK_BAD_ARGS;
     if ((size_t)N * (size_t)(T + 1) * kW * sizeof(ofk_beam_slot_t) > (size_t)OFK_STATIC_SLOT_BYTES) return OFK_TOO_LARGE;
     int dev = -1;
@@ -1671,7 +1671,7 @@ extern "C" int ofk_search_chunks_per_group(int N, int state_len, int flags) { re
 extern "C" int ofk_beam_search(const void *scores, const float *bwd, ofk_beam_slot_t *beam, int32_t *states,
                                uint8_t *moves, int T, int N, int state_len, int columns, float log_beam_cut,
                                float stay, const double *lse_table, int flags, void *stream, void *done) {
-    if (!scores || !bwd || !beam || !states || !moves || !lse_table || T < 1 || N < 1) return OFK_BAD_ARGS;
+    if (!scores || !bwd || !beam || !states || !moves || !lse_table || T < 1 || T > OFK_MAX_T || N < 1) return OFK_BAD_ARGS;
     if ((reinterpret_cast<uintptr_t>(scores) | reinterpret_cast<uintptr_t>(bwd) | reinterpret_cast<uintptr_t>(beam)) & 15u)
         return OFK_BAD_ARGS;
     const Queue st{static_cast<hipStream_t>(stream), static_cast<hipEvent_t>(done)};
@@ -1682,7 +1682,7 @@ extern "C" int ofk_beam_search(const void *scores, const float *bwd, ofk_beam_sl
 extern "C" int ofk_beam_search_forward(const void *scores, const float *bwd, float *post, ofk_beam_slot_t *beam,
                                        int32_t *states, uint8_t *moves, int T, int N, int state_len, int columns,
                                        float log_beam_cut, float stay, const double *lse_table, int flags, void *stream, void *done) {
-    if (!scores || !bwd || !post || !beam || !states || !moves || !lse_table || T < 1 || N < 1) return OFK_BAD_ARGS;
+    if (!scores || !bwd || !post || !beam || !states || !moves || !lse_table || T < 1 || T > OFK_MAX_T || N < 1) return OFK_BAD_ARGS;
     if ((reinterpret_cast<uintptr_t>(scores) | reinterpret_cast<uintptr_t>(bwd) | reinterpret_cast<uintptr_t>(post) |
          reinterpret_cast<uintptr_t>(beam)) & 15u)
         return OFK_BAD_ARGS;

@@ -14,7 +14,8 @@
 extern "C" {
 #endif
 
-/* longest chunk in time steps: the sequence stage keeps 13 bytes per step in LDS (160 KB) */
+/* longest chunk in time steps: the sequence stage keeps 13 bytes per step in LDS (160 KB), and the waves that trace a chunk's path back the
+ * maps of OFK_MAX_T / 128 blocks; both refuse longer ones */
 #define OFK_MAX_T 8192
 #define OFK_BAD_ARGS (-1)
 #define OFK_TOO_LARGE (-2)
