@@ -36,10 +36,8 @@ typedef uint16_t ofk_beam_slot_t;
 #define OFK_SCAN_TWO_TIER 0
 #define OFK_SCAN_PRECISE 1
 #define OFK_SCAN_FAST 2
-/* beside_merged: another decode's merged kernel (ofk_beam_search_forward) may be under way, for which the backward sweep then keeps to fewer
- * registers where that lets the two share compute units.  Same results. */
 int ofk_bwd_scan(const void *scores, float *bwd, int T, int N, int state_len, int columns, float stay, int mode,
-                 int spl, int beside_merged, void *stream, void *done);
+                 int spl, void *stream, void *done);
 int ofk_fwd_post_scan(const void *scores, const float *bwd, float *post, int T, int N, int state_len,
                       int columns, float stay, int mode, int spl, void *stream, void *done);
 /* The same in two steps, 1024 states and the two-tier arithmetic only: the forward recursion by itself, which needs no bwd and can

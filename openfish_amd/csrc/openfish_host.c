@@ -609,7 +609,7 @@ static void enqueue_decode(ofa_gpubuf_t *g, const int T, const int N, const int 
     HIP_OK(hipEventRecord(g->ev[EV_START], g->s_main));
     if (g->pend_split == ARR_MERGED) {
         /* backward sweep, then the search with the forward sweep and the posterior in its workgroups */
-        launch_ok(ofk_bwd_scan(scores_TNC, g->pub.bwd_NTC, T, N, state_len, cols, stay, g->scan_mode, g->scan_spl, shared, g->s_main,
+        launch_ok(ofk_bwd_scan(scores_TNC, g->pub.bwd_NTC, T, N, state_len, cols, stay, g->scan_mode, g->scan_spl, g->s_main,
                                g->ev[EV_BWD_END]), "bwd_scan");
         launch_ok(ofk_beam_search_forward(scores_TNC, g->pub.bwd_NTC, g->pub.post_NTC, (ofk_beam_slot_t *)g->pub.beam_vector,
                                           (int32_t *)g->pub.states, g->pub.moves, T, N, state_len, cols,
@@ -637,7 +637,7 @@ static void enqueue_decode(ofa_gpubuf_t *g, const int T, const int N, const int 
          * T = 833: 1 1.48 | 1.23, 37 1.51 | 1.27, 64 1.52 | 1.31, 96 1.53 | 1.33; five columns, T = 1666: 80 2.67 | 2.51,
          * 96 2.68 | 2.57, 112 2.72 | 2.73, 128 2.82 | 2.85. */
         const int apart = g->pend_apart = state_len == 5 && N <= 96 && !shared && g->scan_mode == OFK_SCAN_TWO_TIER && g->scan_spl == 0;
-        launch_ok(ofk_bwd_scan(scores_TNC, g->pub.bwd_NTC, T, N, state_len, cols, stay, g->scan_mode, g->scan_spl, 0, g->s_main,
+        launch_ok(ofk_bwd_scan(scores_TNC, g->pub.bwd_NTC, T, N, state_len, cols, stay, g->scan_mode, g->scan_spl, g->s_main,
                                g->ev[EV_BWD_END]), "bwd_scan");
         if (apart) {
             HIP_OK(hipStreamWaitEvent(g->s_side, g->ev[EV_START], 0));
@@ -789,7 +789,7 @@ void openfish_amd_bwd_scan(int T, int N, int C, const void *scores, int state_le
     openfish_opt_t o = DECODER_INIT;
     check_scores(T, N, C, scores, state_len, &o);
     check_scan_mode(scan_mode);
-    launch_ok(ofk_bwd_scan(scores, bwd, T, N, state_len, columns_of(C, state_len), stay_score, scan_mode, 0, 0, NULL, NULL), "bwd_scan");
+    launch_ok(ofk_bwd_scan(scores, bwd, T, N, state_len, columns_of(C, state_len), stay_score, scan_mode, 0, NULL, NULL), "bwd_scan");
     HIP_OK(hipStreamSynchronize(0));
 }
 

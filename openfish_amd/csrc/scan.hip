@@ -1212,19 +1212,18 @@ constexpr int kPlainSpl = S >= 1024 ? 2 : 1;
 #define OFK_DEPTH_DEEP_1024 8
 #endif
 
-// Where sixteen rows, 120 registers, cost more than they give, and eight, 88 to 90 registers, are kept instead.
-// More than four waves for every SIMD of 256 compute units, which only states per lane that were asked for bring about: 256 states, one to a
+// Where sixteen rows, 120 registers, cost more than they give, and eight, 88 to 90 registers, are kept instead: more than four waves for
+// every SIMD of 256 compute units, which only states per lane that were asked for bring about.  256 states, one to a
 // lane, T = 300, ms, 8 | 16 rows: 1024 chunks 0.249 | 0.251, 1100 0.296 | 0.347, 2048 0.468 | 0.487, 2100 0.515 | 0.553; 8192 of 64 0.443 | 0.454.
-// Beside another decode's merged kernel of 256 states, whose waves of 104 registers, up to four on a SIMD, leave room for the one but not for
-// the other, as soon as that kernel leaves too few units free.  Two decodes in flight, ms, 8 | 16 rows, T = 1666: 335 chunks 2.956 | 2.944,
-// 375 2.997 | 2.984, 385 3.010 | 3.061, 395 3.075 | 3.173, 512 3.350 | 3.416; T = 600: 375 1.204 | 1.206, 385 1.209 | 1.213, 395 1.233 | 1.274;
-// T = 1000: 704 3.38 | 3.47, 900 4.32 | 4.43.  Its waves of 114 registers with five columns leave room for neither, T = 1201: 403 2.456 | 2.459,
-// 512 2.637 | 2.651.  Smaller models and batches are ahead with sixteen (128 chunks 1.769 | 1.745, 512 of 64 states 2.579 | 2.540).
+// Beside another decode's merged kernel of 256 states sixteen are no dearer: four of its waves on a SIMD, of 96 registers (104 before, when
+// eight rows were 2 % ahead), leave room for a wave of either kind, and with five columns, 120 registers, for neither.  Two decodes in
+// flight, ms, 8 | 16 rows, T = 1666: 385 chunks 2.893 | 2.901, 450 3.126 | 3.132, 512 3.298 | 3.313 (runs differ by 3 %), 640 5.018 | 5.023,
+// 1024 7.348 | 7.354; T = 600: 395 1.244 | 1.244, 512 1.333 | 1.324; T = 1000: 800 4.261 | 4.255; five columns: 512 3.483 | 3.507, 1024 7.735 |
+// 7.731, T = 1201 2.570 | 2.573, T = 600 1.389 | 1.388.
 constexpr long kWavesOfDepth16 = 4096;
-constexpr int kChunksBesideMerged = 384;
 template <int S>
-bool eight_rows(int N, int beside_merged) {
-    return (long)N * (S / 64) > kWavesOfDepth16 || (S == 256 && beside_merged && N > kChunksBesideMerged);
+bool eight_rows(int N) {
+    return (long)N * (S / 64) > kWavesOfDepth16;
 }
 
 // Up to which magnitude of its values a sweep with one state to a lane takes the double arithmetic for every update at once.  An ulp of small
@@ -1249,7 +1248,7 @@ bool early_backward(int S, int T, int N) { return S != 256 || N <= 256 || T <= 2
 constexpr int kEarlyForwardChunks = 1024;
 
 template <int S, int SPL, int DEPTH>
-int launch_bwd(int mode, const void *scores, float *bwd, int T, int N, float stay, int beside_merged, Queue st) {
+int launch_bwd(int mode, const void *scores, float *bwd, int T, int N, float stay, Queue st) {
     using Sh = Shape<S, SPL>;
     constexpr int kDeep = SPL > 1 ? DEPTH : S >= 1024 ? OFK_DEPTH_DEEP_1024 : OFK_DEPTH_DEEP;
     const dim3 grid((N + Sh::kChunks - 1) / Sh::kChunks), block(Sh::kThreads);
@@ -1257,7 +1256,7 @@ int launch_bwd(int mode, const void *scores, float *bwd, int T, int N, float sta
     switch (mode) {
         case OFK_SCAN_TWO_TIER:
             if constexpr (SPL == 1 && S <= 256) {
-                if (eight_rows<S>(N, beside_merged)) {
+                if (eight_rows<S>(N)) {
                     queue_kernel((bwd_scan_kernel<S, SPL, DEPTH, OFK_SCAN_TWO_TIER, false>), grid, block, 0, st, sc, bwd, T, N, stay, 0u, kSeries);
                     break;
                 }
@@ -1452,7 +1451,7 @@ static int scan_posterior(const void *scores, float *bwd, float *post, int T, in
 }
 
 static int bwd_scan(const void *scores, float *bwd, int T, int N, int state_len, float stay, int mode, int spl,
-                    int beside_merged, void *stream, void *done) {
+                    void *stream, void *done) {
     if (!scores || !bwd || T < 1 || N < 1 || !aligned16(scores) || !aligned16(bwd)) return OFK_BAD_ARGS;
     if (state_len < 3 || state_len > 5) return OFK_BAD_ARGS;
     const Queue st{static_cast<hipStream_t>(stream), static_cast<hipEvent_t>(done)};
@@ -1461,8 +1460,8 @@ static int bwd_scan(const void *scores, float *bwd, int T, int N, int state_len,
     // lane | one: 37 chunks, T = 833 0.76 | 0.67; 256, T = 1666 1.45 | 1.32; 9, T = 64 0.091 | 0.078).  Two such workgroups do
     // not fit a unit (257 chunks, T = 400 0.55 | 0.71; 512 0.68 | 0.75; 1024, T = 300 1.05 | 1.15).
     if (state_len == 5 && mode == OFK_SCAN_TWO_TIER && spl == 0 && N <= 256)
-        return launch_bwd<1024, 1, OFK_DEPTH_1024>(mode, scores, bwd, T, N, stay, beside_merged, st);
-    OFK_DISPATCH(true, launch_bwd, mode, scores, bwd, T, N, stay, beside_merged, st)
+        return launch_bwd<1024, 1, OFK_DEPTH_1024>(mode, scores, bwd, T, N, stay, st);
+    OFK_DISPATCH(true, launch_bwd, mode, scores, bwd, T, N, stay, st)
 }
 
 static int fwd_post_scan(const void *scores, const float *bwd, float *post, int T, int N, int state_len,
@@ -1489,8 +1488,8 @@ extern "C" int ofk_scan_posterior_five(const void *scores, float *bwd, float *po
     return scan_posterior(scores, bwd, post, T, N, state_len, stay, mode, spl, stream, done);
 }
 extern "C" int ofk_bwd_scan_five(const void *scores, float *bwd, int T, int N, int state_len, float stay, int mode,
-                                 int spl, int beside_merged, void *stream, void *done) {
-    return bwd_scan(scores, bwd, T, N, state_len, stay, mode, spl, beside_merged, stream, done);
+                                 int spl, void *stream, void *done) {
+    return bwd_scan(scores, bwd, T, N, state_len, stay, mode, spl, stream, done);
 }
 extern "C" int ofk_fwd_post_scan_five(const void *scores, const float *bwd, float *post, int T, int N,
                                       int state_len, float stay, int mode, int spl, void *stream, void *done) {
@@ -1501,7 +1500,7 @@ extern "C" int ofk_fwd_scan_five(const void *scores, float *fwd, int T, int N, i
 }
 #else
 extern "C" int ofk_scan_posterior_five(const void *, float *, float *, int, int, int, float, int, int, void *, void *);
-extern "C" int ofk_bwd_scan_five(const void *, float *, int, int, int, float, int, int, int, void *, void *);
+extern "C" int ofk_bwd_scan_five(const void *, float *, int, int, int, float, int, int, void *, void *);
 extern "C" int ofk_fwd_post_scan_five(const void *, const float *, float *, int, int, int, float, int, int, void *, void *);
 extern "C" int ofk_fwd_scan_five(const void *, float *, int, int, int, float, void *, void *);
 
@@ -1513,10 +1512,10 @@ extern "C" int ofk_scan_posterior(const void *scores, float *bwd, float *post, i
 }
 
 extern "C" int ofk_bwd_scan(const void *scores, float *bwd, int T, int N, int state_len, int columns, float stay,
-                            int mode, int spl, int beside_merged, void *stream, void *done) {
-    if (columns == 5) return ofk_bwd_scan_five(scores, bwd, T, N, state_len, stay, mode, spl, beside_merged, stream, done);
+                            int mode, int spl, void *stream, void *done) {
+    if (columns == 5) return ofk_bwd_scan_five(scores, bwd, T, N, state_len, stay, mode, spl, stream, done);
     if (columns != 4) return OFK_BAD_ARGS;
-    return bwd_scan(scores, bwd, T, N, state_len, stay, mode, spl, beside_merged, stream, done);
+    return bwd_scan(scores, bwd, T, N, state_len, stay, mode, spl, stream, done);
 }
 
 extern "C" int ofk_fwd_post_scan(const void *scores, const float *bwd, float *post, int T, int N, int state_len,

@@ -101,7 +101,7 @@ int ofk_meet(int *mark, int waits, void *stream) {
 /* the others take no notice of their arguments */
 #define KERNEL { return launched(stream, done); }
 #define KERNEL_NO_EVENT { return launched(stream, NULL); }
-int ofk_bwd_scan(const void *scores, float *bwd, int T, int N, int state_len, int columns, float stay, int mode, int spl, int beside_merged,
+int ofk_bwd_scan(const void *scores, float *bwd, int T, int N, int state_len, int columns, float stay, int mode, int spl,
                  void *stream, void *done) { return launched_first(stream, done); }
 int ofk_scan_posterior(const void *scores, float *bwd, float *post, int T, int N, int state_len, int columns, float stay, int mode, int spl,
                        void *stream, void *done) { return launched_first(stream, done); }

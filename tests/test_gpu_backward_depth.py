@@ -1,5 +1,5 @@
-"""The backward sweep keeps eight rows in flight instead of sixteen where its registers are wanted by another decode's merged kernel, and
-where more waves than four to a SIMD are asked for: either side of both lines, the same bits."""
+"""The backward sweep keeps eight rows in flight instead of sixteen where more waves than four to a SIMD are asked for: either side of the
+line, the same bits; and the same beside another decode's merged kernel as alone, whether or not that leaves compute units free."""
 import numpy as np
 import pytest
 

@@ -52,11 +52,11 @@ def most_of(field, tmp_path):
 
 def test_a_backward_sweep_finds_room_beside_another_decode_s_merged_kernel(tmp_path):
     """256 states, four columns: two chunks of the merged kernel are 14 waves on the four SIMDs of a unit, and a SIMD's 512 registers, given
-    out by eights, are to hold four of them and a wave of the backward sweep that keeps eight rows in flight"""
+    out by eights, are to hold four of them and a wave of the backward sweep, which keeps sixteen rows in flight"""
     registers = {k: (v + 7) // 8 * 8 for k, v in most_of("vgpr_count", tmp_path).items()}
     merged, = [v for k, v in registers.items() if "beam_kernelILi256ELi2ELi4ELi4E" in k]
-    backward, = [v for k, v in registers.items() if "bwd_scan_kernelILi256ELi1ELi8ELi0E" in k]
-    assert 4 * merged + backward <= 512, (merged, backward)
+    backward = [v for k, v in registers.items() if "bwd_scan_kernelILi256ELi1ELi16ELi0E" in k]
+    assert len(backward) == 2 and 4 * merged + max(backward) <= 512, (merged, backward)  # with early steps and without
 
 
 def test_no_kernel_keeps_registers_in_scratch(tmp_path):
