@@ -1,5 +1,6 @@
-"""The beam search keeps the halves of the cut-off's bounds (beam.hip): the cuts that come of them are the CPU path's (lo + hi) / 2, bit for
-bit, whichever way the bisection goes, at usual scores, next to zero and next to the largest float."""
+"""The argument behind the halves that the beam search keeps of the cut-off's bounds (beam.hip), worked out here in exact fractions: the cuts
+that come of them are the CPU path's (lo + hi) / 2, bit for bit, whichever way the bisection goes, at usual scores, next to zero and
+next to the largest float.  This is arithmetic alone, no kernel runs: test_gpu_cut_options.py compares the kernels' cuts with the oracle's."""
 from fractions import Fraction
 
 import numpy as np
