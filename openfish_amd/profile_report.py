@@ -31,6 +31,8 @@ SQ_COUNTERS = ["SQ_WAVES", "SQ_BUSY_CYCLES", "SQ_INSTS_VALU", "SQ_INSTS_SALU", "
                "SQ_LDS_BANK_CONFLICT", "SQ_ACTIVE_INST_VALU"]
 SQ2_COUNTERS = ["SQ_WAVE_CYCLES", "SQ_WAIT_ANY", "SQ_ACTIVE_INST_ANY", "SQ_ACTIVE_INST_LDS", "SQ_INSTS_VALU_FMA_F64",
                 "SQ_INSTS_VALU_TRANS_F32", "SQ_INSTS_BRANCH", "SQ_WAIT_INST_ANY"]
+# of an MI355X: vector units, and the shader engines over which the SQ's counters are added up
+SIMDS, ENGINES = 1024, 32
 SCAN_MODES = {"0": "two_tier", "1": "precise", "2": "fast"}
 # kernel function -> the stage name bench.py uses
 STAGE_OF = {"scan_post_kernel": "scan", "bwd_scan_kernel": "bwd", "fwd_post_kernel": "fwd_post", "fwd_post_roles_kernel": "fwd_post",
@@ -39,12 +41,12 @@ STAGE_OF = {"scan_post_kernel": "scan", "bwd_scan_kernel": "bwd", "fwd_post_kern
 
 
 def template_ints(name):
-    """integer template arguments of a kernel name, mangled (ILi64ELi1E...) or demangled (<64, 1, ...>)"""
-    m = re.search(r"I((?:Li\d+E)+)", name)
+    """integer and truth-value template arguments of a kernel name, mangled (ILi64ELb1E...) or demangled (<64, true, ...>)"""
+    m = re.search(r"I((?:L[ib]\d+E)+)", name)
     if m:
-        return re.findall(r"Li(\d+)E", m.group(1))
-    m = re.search(r"<([0-9, ]+)>", name)
-    return [x.strip() for x in m.group(1).split(",")] if m else []
+        return re.findall(r"L[ib](\d+)E", m.group(1))
+    m = re.search(r"<((?:\d+|true|false|, ?)+)>", name)
+    return [{"true": "1", "false": "0"}.get(x.strip(), x.strip()) for x in m.group(1).split(",")] if m else []
 
 
 def short(name):
@@ -56,7 +58,8 @@ def short(name):
             if fn == "fwd_post_roles_kernel" and len(a) >= 3:
                 return "%s<S=%s,SPL=%s,DEPTH=%s>" % (fn, a[0], a[1], a[2])
             if fn in ("scan_post_kernel", "bwd_scan_kernel", "fwd_post_kernel") and len(a) >= 4:
-                return "%s<S=%s,SPL=%s,DEPTH=%s,%s>" % (fn, a[0], a[1], a[2], SCAN_MODES.get(a[3], a[3]))
+                early = ",early steps" if fn != "scan_post_kernel" and len(a) >= 5 and a[4] == "1" else ""
+                return "%s<S=%s,SPL=%s,DEPTH=%s,%s%s>" % (fn, a[0], a[1], a[2], SCAN_MODES.get(a[3], a[3]), early)
             if fn == "beam_kernel" and len(a) >= 3:
                 forward = ",forward waves=%s" % a[3] if len(a) >= 4 and a[3] != "0" else ""
                 return "beam_kernel<S=%s,chunks/group=%s,columns=%s%s>" % (a[0], a[1], a[2], forward)
@@ -80,6 +83,15 @@ def counters(path):
         for r in csv.DictReader(fh):
             agg[short(r["Kernel_Name"])][r["Counter_Name"]].append(float(r["Counter_Value"]))
     return {k: {c: sum(v) / len(v) for c, v in d.items()} for k, d in agg.items()}
+
+
+def use_of_simds(waves, busy_cycles, wave_cycles, active_valu):
+    """per SIMD of the device, over the kernel's length: waves launched, waves resident on average, fraction of time in which the vector ALU
+    is busy.  BUSY_CYCLES counts clocks, WAVE_CYCLES and ACTIVE_INST_VALU tick once per four."""
+    clocks = busy_cycles / ENGINES
+    if not clocks:
+        return waves / SIMDS, 0.0, 0.0
+    return waves / SIMDS, 4.0 * wave_cycles / (SIMDS * clocks), 4.0 * active_valu / (SIMDS * clocks)
 
 
 def main():
@@ -183,30 +195,32 @@ def main():
         c1, c2 = counters(sq), counters(sq2)
         out.append("\n## Where the waves' time goes (`--pmc %s`, with the table above)\n" % " ".join(SQ2_COUNTERS))
         out.append("Per launch. The SQ's time counters tick once per four clocks; WAVE_CYCLES adds up the lifetimes of all "
-                   "waves, ACTIVE_INST_VALU the time their vector instructions occupy a SIMD's ALU. `VALU share of wave "
-                   "time` x `waves per SIMD` is the fraction of time a SIMD's vector ALU is busy (1024 SIMDs; the waves of "
-                   "these kernels are all resident at once).\n")
+                   "waves, ACTIVE_INST_VALU the time their vector instructions occupy a SIMD's ALU, BUSY_CYCLES, in "
+                   "clocks, the length of the kernel on each of 32 shader engines (those that have a workgroup at all). Over that "
+                   "length, per SIMD of the device: the waves resident on average, beside those launched, and the fraction of time "
+                   "its vector ALU is busy. Fewer resident than launched: the rest waited for room.\n")
         out.append("| kernel | WAVE_CYCLES | WAIT_ANY | ACTIVE_INST_ANY | ACTIVE_INST_LDS | INSTS_VALU_FMA_F64 | INSTS_VALU_TRANS_F32 | "
-                   "INSTS_BRANCH | VALU share of wave time | waves per SIMD | SIMD vector ALU busy | fp64 FMA per wave and time step |"
-                   "\n|---|---|---|---|---|---|---|---|---|---|---|---|")
+                   "INSTS_BRANCH | VALU share of wave time | waves launched per SIMD | waves resident per SIMD | SIMD vector ALU busy | fp64 FMA per wave and time step |"
+                   "\n|---|---|---|---|---|---|---|---|---|---|---|---|---|")
         for k, d in c2.items():
             if k.startswith("__amd") or k not in c1:
                 continue
             wc, act, waves = d.get("SQ_WAVE_CYCLES", 0.0), c1[k].get("SQ_ACTIVE_INST_VALU", 0.0), c1[k].get("SQ_WAVES", 0.0)
             share = act / wc if wc else 0.0
-            per_simd = waves / 1024.0
+            launched, resident, busy = use_of_simds(waves, c1[k].get("SQ_BUSY_CYCLES", 0.0), wc, act)
             steps = a.steps_per_wave
-            out.append("| %s | %.3g | %.3g | %.3g | %.3g | %.3g | %.3g | %.3g | %.3f | %.2f | %.2f | %s |" % (
+            out.append("| %s | %.3g | %.3g | %.3g | %.3g | %.3g | %.3g | %.3g | %.3f | %.2f | %.2f | %.2f | %s |" % (
                 k, wc, d.get("SQ_WAIT_ANY", 0.0), d.get("SQ_ACTIVE_INST_ANY", 0.0), d.get("SQ_ACTIVE_INST_LDS", 0.0),
                 d.get("SQ_INSTS_VALU_FMA_F64", 0.0), d.get("SQ_INSTS_VALU_TRANS_F32", 0.0), d.get("SQ_INSTS_BRANCH", 0.0),
-                share, per_simd, min(1.0, share * per_simd),
+                share, launched, resident, busy,
                 ("%.2f" % (d.get("SQ_INSTS_VALU_FMA_F64", 0.0) / (waves * steps))) if (steps and waves and stage_of(k) in ("scan", "bwd", "fwd_post", "fwd_scan")) else "-"))
         if a.steps_per_wave:
-            out.append("\nfp64 FMA per wave and time step = SQ_INSTS_VALU_FMA_F64 / (waves x T): the second tier of the default "
-                       "arithmetic is the only user of fp64 in the scans, but for the 32 warm-up steps of either sweep in the "
-                       "kernel that holds both (70 fp64 FMA per wave, state of a lane and step).  A trip through it is 16 fp64 "
-                       "FMA for a single unsettled update and 12 for up to eight, 9 more where a proof fails; where many lanes need "
-                       "it (the first hundred steps) it takes 69 for every state of a lane at once.")
+            out.append("\nfp64 FMA per wave and time step = SQ_INSTS_VALU_FMA_F64 / (waves x T): besides the second tier of the default "
+                       "arithmetic, steps that are taken in double at once, 70 per state of a lane: the 32 warm-up steps of either sweep "
+                       "in the kernel that holds both, and in a kernel with early steps (forward sweeps apart and in roles, one state to a "
+                       "lane, have them too) those in which values are below 256 to 2048, four or so more a step.  A trip through the "
+                       "second tier is 16 for a single unsettled update and 12 for up to eight, 9 more where a proof fails; where many "
+                       "lanes need it (in other kernels the first hundred steps) it takes 69 for every state of a lane at once.")
 
     log = first(os.path.join(base, "trace.log"))
     if log:
