@@ -235,12 +235,13 @@ void openfish_amd_gpubuf_set_debug_flags(const openfish_gpubuf_t *gpubuf, int fl
  * moves a quality character by one step now and then (up to three in ten thousand).  Callers that decode from several
  * threads and want the same characters every time fix the arrangement.  Host-only.
  *   64 states: 1 up to 2048 chunks, 0 beyond.
- *   256 states: alone 1 up to 446 chunks (five columns: 390), 2 up to 512, 1 up to 640 and, while T * C is at most
- *     1250000, up to 768, 2 beyond; shared 2 up to 512, then up to 608 chunks 0 if they have at most 400 steps, 1 if T * C is at most 950000,
- *     1 up to 548 if it is at most 1900000, 2 in all other cases.
- *   1024 states: alone 1 up to 168 chunks, but 2 for chunks shorter than 12 steps (above 96 chunks: 4); 2 up to 256; 1 up to 340 while
- *     N * (4 * C + 12288) + 1300 * T is at most 11550000; 2 elsewhere, but 0 for more than 340 chunks shorter than 48 steps and for 512 and
- *     more of at most 100; shared 2, but 0 for fewer than 16 chunks shorter than 128 steps.
+ *   256 states: alone 1 up to 348 chunks (five columns: 305), 2 up to 512, 1 up to 640 and, while T * C is at most
+ *     1250000, up to 768, 2 beyond; shared 2 up to 512, then 0 up to 608 chunks of at most 400 steps; up to 660 chunks with T * C at most
+ *     525000 0 if they have at most 128 steps, else 1; 1 up to 608 chunks with T * C at most 950000, up to 530 (five columns: 518) of
+ *     at most 2400 steps, and up to 548 with T * C at most 1900000; 2 in all other cases.
+ *   1024 states: alone 1 up to 168 chunks, but 2 for chunks of at most 16 steps; 2 up to 256; 1 up to 338 while
+ *     N * (4 * C + 12288) + 1300 * T is at most 11650000; 2 elsewhere, but 0 for more than 338 chunks shorter than 72 steps and for 512 and
+ *     more of at most 100; shared 2.
  */
 int openfish_amd_scan_arrangement(int T, int N, int C, int state_len, int shared);
 

@@ -506,41 +506,44 @@ static void join_null_stream(ofa_gpubuf_t *g) {
  *   one     both sweeps of a chunk side by side from its two ends, then the search: the longest, with the fewest launches.
  * Whole blocking calls, ms, one | split | merged, T = 1666 unless stated, inputs and arrangements in turn (more of them in
  * tests/test_arrangement.py):
- *   1024 states: 128 3.39 | 2.65 | 2.78;  168 3.60 | 2.70 | 2.81;  172 3.64 | 3.37 | 2.84;  256 4.05 | 3.83 | 2.94;  257 6.55 | 4.74 | 5.37;
- *                320 6.63 | 5.29 | 5.34;  328 6.64 | 5.36 | 5.35;  five columns: 290 6.97 | 5.50 | 5.52;  300 6.95 | 5.59 | 5.49;
- *                T = 833: 336 3.47 | 2.78 | 2.88;  five columns 320 3.64 | 2.94 | 2.94;  T = 250: 340 1.17 | 0.93 | 1.05;  352 1.18 | 1.21 | 1.05;
- *                T = 2000: 320 7.89 | 6.34 | 6.30;  five columns 280 8.28 | 6.48 | 6.52;
- *                T = 1: 64 0.060 | 0.073 | 0.059;  T = 8: 64 0.086 | 0.086 | 0.078;  T = 12: 64 0.098 | 0.092 | 0.089;  T = 16: 0.111 | 0.099 | 0.100;
- *                T = 4: 97 0.070 | 0.070 | 0.067;  T = 32: 360 0.244 | 0.237 | 0.250;  T = 64: 360 0.396 | 0.401 | 0.401;  T = 100: 450 0.595 | 0.596 | 0.547;
- *                512 0.568 | 0.643 | 0.586;  T = 128: 512 0.718 | 0.824 | 0.709
- *    256 states: 400 2.40 | 1.81 | 1.84;  440 2.42 | 1.85 | 1.87;  460 2.47 | 1.90 | 1.87;  512 2.56 | 2.15 | 1.95;
- *                five columns: 360 2.41 | 1.82 | 1.83;  380 2.42 | 1.84 | 1.84;  400 2.44 | 1.89 | 1.87;  512 2.69 | 2.34 | 1.95;
- *                T = 1201: 440 1.80 | 1.39 | 1.39;  460 1.81 | 1.42 | 1.41;  five columns 400 1.79 | 1.38 | 1.39;  420 1.81 | 1.42 | 1.40;
- *                T = 400: 340 0.66 | 0.54 | 0.54;  420 0.67 | 0.56 | 0.55;  512 0.69 | 0.57 | 0.56;  T = 96: 256 0.190 | 0.176 | 0.182;  340 0.219 | 0.202 | 0.193;
- *                513 3.39 | 2.42 | 3.19;  640 3.57 | 2.97 | 3.41;  660 3.58 | 3.41 | 3.40;  768 3.68 | 3.52 | 3.46;  1024 4.33 | 4.71 | 3.96;
- *                five columns: 640 3.70 | 3.22 | 3.46;  660 3.74 | 3.65 | 3.51;  T = 1201: 768 2.69 | 2.60 | 2.60;  five columns 660 2.70 | 2.66 | 2.63;
- *                with the present search, split | merged: 256 1.56 | 1.62;  260 1.70 | 1.71;  300 1.72 | 1.73;  320 1.73 | 1.73;  340 1.74 | 1.74;  440 1.91 | 1.78;
- *                512 2.15 | 1.82;  five columns: 280 1.72 | 1.74;  320 1.74 | 1.75;  512 2.34 | 1.86;  T = 1201: 260 1.29 | 1.29;  340 1.32 | 1.31;
- *                five columns 320 1.32 | 1.33;  T = 600: 340 0.742 | 0.739;  T = 200: 280 0.296 | 0.291;
- *                T = 800: 768 1.79 | 1.76 | 1.81;  five columns 768 1.86 | 1.83 | 1.85;  T = 1000: five columns 680 2.25 | 2.23 | 2.22
- *     64 states: 16 1.59 | 1.31;  512 1.87 | 1.54;  2048 4.11 | 3.41
+ *   1024 states: 128 3.33 | 2.61 | 2.74;  168 3.56 | 2.66 | 2.77;  172 3.59 | 3.35 | 2.76;  256 3.99 | 3.81 | 2.87;  257 6.50 | 4.64 | 5.22;
+ *                320 6.60 | 5.15 | 5.24;  five columns: 288 6.95 | 5.39 | 5.48;  296 6.96 | 5.48 | 5.46;  304 6.95 | 5.56 | 5.49;
+ *                T = 833: five columns 320 3.65 | 2.90 | 2.88;  T = 1200: 338 4.97 | 3.92 | 3.95;  340 4.96 | 4.84 | 3.96;
+ *                T = 400: 338 1.75 | 1.39 | 1.52;  340 1.75 | 1.77 | 1.52;  five columns 338 1.83 | 1.48 | 1.54;
+ *                T = 2000: 320 7.88 | 6.19 | 6.24;  338 7.96 | 6.46 | 6.29;
+ *                T = 8: 64 0.068 | 0.072 | 0.057;  164 0.071 | 0.070 | 0.060;  T = 16: 16 0.091 | 0.077 | 0.076;  97 0.094 | 0.082 | 0.079;
+ *                T = 20: 16 0.101 | 0.079 | 0.086;  97 0.105 | 0.089 | 0.092;  T = 64: 338 0.359 | 0.332 | 0.377;  360 0.362 | 0.377 | 0.377;
+ *                450 0.380 | 0.399 | 0.381;  512 0.370 | 0.430 | 0.404;  T = 100: 360 0.535 | 0.536 | 0.513;  512 0.543 | 0.622 | 0.561
+ *    256 states: 256 1.99 | 1.56 | 1.61;  300 2.24 | 1.73 | 1.73;  340 2.26 | 1.74 | 1.75;  360 2.27 | 1.76 | 1.75;  440 2.34 | 1.90 | 1.78;
+ *                512 2.47 | 2.15 | 1.82;  five columns: 305 2.26 | 1.74 | 1.75;  320 2.28 | 1.75 | 1.76;  340 2.29 | 1.77 | 1.76;  512 2.70 | 2.34 | 1.86;
+ *                T = 1201: 260 1.64 | 1.29 | 1.29;  340 1.68 | 1.32 | 1.31;  five columns 320 1.68 | 1.32 | 1.32;  T = 400: 340 0.632 | 0.525 | 0.525;
+ *                five columns 340 0.636 | 0.526 | 0.532;  T = 96: 300 0.195 | 0.170 | 0.163;
+ *                513 3.37 | 2.35 | 3.15;  640 3.44 | 2.86 | 3.31;  680 3.47 | 3.34 | 3.33;  768 3.53 | 3.47 | 3.42;  1024 4.18 | 4.67 | 3.87;
+ *                five columns: 640 3.58 | 3.13 | 3.42;  680 3.62 | 3.78 | 3.48;  T = 1201: 768 2.55 | 2.52 | 2.54;  T = 1000: five columns 680
+ *                2.18 | 2.24 | 2.21;  768 2.26 | 2.26 | 2.24
+ *     64 states: 16 1.48 | 1.19;  512 1.78 | 1.43;  2048 3.83 | 3.21
  * Hence the lines.  Up to 168 chunks of 1024 states the search and the forward sweep find compute units of their own (21 and 11 of an
- * XCD's 32); up to 340, in two rounds, split is ahead while its bytes fit beneath the chain, and short chunks allow more of them:
- * 11.55 MB a step, less 1300 bytes for every step of a chunk.  Chunks shorter than 12 steps are decided by launches and
- * set-up, batches above 340 of chunks up to 100 steps by the rounds.  Up to 512 chunks of 256 states the chain of split is
- * shorter, while its bytes fit beneath the chain, 2.5 MB a step (348 chunks; 3.2 MB when a step of the search took a tenth longer, under which more
- * bytes found time); above,
+ * XCD's 32); up to 338, in two rounds, split is ahead while its bytes fit beneath the chain, and short chunks allow more of them:
+ * 11.65 MB a step, less 1300 bytes for every step of a chunk.  Chunks of up to 16 steps are decided by launches and
+ * set-up, batches above 338 of chunks up to 100 steps by the rounds.  Up to 512 chunks of 256 states the chain of split is
+ * shorter, while its bytes fit beneath the chain, 2.5 MB a step (348 chunks, five columns 305; between 2.5 and 2.8 MB the two are within 1 % of each
+ * other); above,
  * the search's workgroups hold four chunks, a unit that has one of them in the merged kernel takes as long as one that has four,
  * and split has units left for the forward sweep up to 640 chunks, with shorter chunks up to 768.
  *
  * A decode that is enqueued, or finds another one under way, shares the machine; two at a time, one | split | merged:
- *   1024 states: 16, T = 833 1.77 | 2.18 | 1.56;  128 4.08 | 4.87 | 3.04;  256 five columns 8.37 | 8.73 | 6.29;
- *                320 9.81 | 9.37 | 7.36;  8, T = 64 0.228 | 0.295 | 0.231;  16, T = 100 0.309 | 0.413 | 0.300
- *    256 states: 128 2.50 | 2.09 | 1.75;  512 5.20 | 4.44 | 3.52;  513 5.17 | 4.71 | 4.84;  530 5.29 | 4.91 | 4.93;  560 5.32 | 5.12 | 4.99;
- *                five columns: 516 5.46 | 5.12 | 5.12;  545 5.55 | 5.47 | 5.15;  640 6.58 | 6.03 | 5.50;  T = 2000: 516 6.28 | 5.77 | 5.79;  540 6.37 | 5.91 | 5.86;
- *                T = 1201: 545 3.82 | 3.61 | 3.66;  560 3.87 | 3.72 | 3.71;  T = 800: 600 2.65 | 2.65 | 2.67;  620 3.04 | 2.71 | 2.70;
- *                T = 400: 530 1.32 | 1.34 | 1.41;  600 1.37 | 1.43 | 1.44;  620 1.55 | 1.45 | 1.45
- *     64 states: 512 3.00 | 2.55;  2048 7.75 | 6.68
+ *   1024 states: 128 3.98 | 4.82 | 2.87;  320 9.75 | 9.31 | 7.02;  T = 8: 8 0.082 | 0.120 | 0.070;  T = 64: 8 0.219 | 0.286 | 0.203;
+ *                T = 127: 15 0.359 | 0.483 | 0.338
+ *    256 states: 128 2.50 | 2.11 | 1.74;  512 5.01 | 4.41 | 3.29;  513 4.91 | 4.51 | 4.83;  530 5.04 | 4.82 | 4.92;  548 5.05 | 4.90 | 4.94;  640 6.01 | 5.37 | 5.00;
+ *                five columns: 513 5.21 | 4.96 | 4.99;  530 5.32 | 5.24 | 5.07;  T = 2000: 513 5.86 | 5.44 | 5.66;  530 6.09 | 5.75 | 5.88;  548 6.08 | 5.91 | 5.82;
+ *                five columns 513 6.21 | 5.82 | 6.01;  T = 2400: 530 7.18 | 6.89 | 6.99;  T = 4000: 513 12.99 | 12.47 | 12.27;
+ *                T = 1201: 560 3.68 | 3.61 | 3.66;  T = 800: 600 2.51 | 2.56 | 2.56;  640 2.96 | 2.62 | 2.59;
+ *                T = 400: 608 1.29 | 1.37 | 1.41;  620 1.50 | 1.39 | 1.42;  660 1.49 | 1.42 | 1.43;  five columns 640 1.60 | 1.48 | 1.48;
+ *                T = 200: 660 0.782 | 0.755 | 0.796;  704 0.795 | 0.813 | 0.833;  T = 100: 620 0.420 | 0.423 | 0.449;  660 0.424 | 0.442 | 0.453
+ *     64 states: five columns 512 2.84 | 2.37;  2048 9.96 | 8.95
+ * The merged kernel is ahead with 1024 states at every size.  With 256 states split is ahead where a few chunks above 512 would leave merged
+ * workgroups half empty, up to 530 chunks of at most 2400 steps (five columns 518) or 548 of a shorter product of steps and scores,
+ * and short chunks go further, because the kernels of one batch end between those of the other.
  *
  * The merged kernel exists for 256 and 1024 states with the default arithmetic and its own states per lane; without it
  * (can_merge = 0) 1024 states keep the one kernel and 256 states the split sweeps where they are ahead of it. */
@@ -554,14 +557,17 @@ static int arrangement_by_default(int T, int N, int C, int state_len, int shared
             if (N <= 512) return shared || step_bytes > 2500000 ? ARR_MERGED : ARR_SPLIT;
             if (!shared) return N <= 640 || (N <= 768 && chunk_scores <= 1250000) ? ARR_SPLIT : ARR_MERGED;
             if (T <= 400 && N <= 608) return ARR_ONE;
-            return chunk_scores <= 1900000 && N <= (chunk_scores <= 950000 ? 608 : 548) ? ARR_SPLIT : ARR_MERGED;
+            if (chunk_scores <= 525000 && N <= 660) return T <= 128 ? ARR_ONE : ARR_SPLIT;
+            if (chunk_scores <= 950000 && N <= 608) return ARR_SPLIT;
+            if (T <= 2400 && N <= 530 && step_bytes <= 4250000) return ARR_SPLIT;
+            return chunk_scores <= 1900000 && N <= 548 ? ARR_SPLIT : ARR_MERGED;
         default:
             if (!can_merge) return ARR_ONE;
-            if (shared) return T < 128 && N < 16 ? ARR_ONE : ARR_MERGED;
-            if (N <= 168) return T < (N <= 96 ? 12 : 4) ? ARR_MERGED : ARR_SPLIT;
+            if (shared) return ARR_MERGED;
+            if (N <= 168) return T <= 16 ? ARR_MERGED : ARR_SPLIT;
             if (N <= 256) return ARR_MERGED;
-            if (N <= 340) return step_bytes + 1300L * T <= 11550000 ? ARR_SPLIT : ARR_MERGED;
-            return T < 48 || (N >= 512 && T <= 100) ? ARR_ONE : ARR_MERGED;
+            if (N <= 338) return step_bytes + 1300L * T <= 11650000 ? ARR_SPLIT : ARR_MERGED;
+            return T < 72 || (N >= 512 && T <= 100) ? ARR_ONE : ARR_MERGED;
     }
 }
 

@@ -92,7 +92,7 @@ def timed(intruder):
 # what the decode waits for on another lane: 64 states sweep and sums | sums; 256 states sweep | nothing but the copy of its moves | sums;
 # few of 1024 states a sweep from the decode's start, and the posteriors' pass
 @pytest.mark.parametrize("state_len,T,N,split,total", [(3, 8, 2, -1, 53), (3, 8, 2, 0, 52), (4, 8, 2, 1, 52), (4, 2048, 64, 2, 3), (4, 2048, 64, 0, 52),
-                                                       (5, 16, 2, -1, 53)])
+                                                       (5, 20, 2, -1, 53)])
 def test_a_decodes_times_begin_with_its_first_kernel_whatever_the_other_lanes_do(run, state_len, T, N, split, total):
     """another thread's decode puts 50 ms of work on every other stream while this one's kernels, a millisecond each, are being queued"""
     done = run(TIMED % (T, N, state_len, split) + "timed(50)")
@@ -104,7 +104,7 @@ def test_a_decodes_times_begin_with_its_first_kernel_whatever_the_other_lanes_do
 
 def test_a_forward_sweep_beside_the_backward_one_does_not_end_before_its_decode_starts(run):
     """decodes on lanes that are ahead of one another"""
-    done = run(TIMED % (16, 2, 5, -1) + "for x in range(6): timed(50 - 7 * x)")
+    done = run(TIMED % (20, 2, 5, -1) + "for x in range(6): timed(50 - 7 * x)")
     assert done.returncode == 0, done
     for line in done.stdout.splitlines():
         bwd, fwd, beam, seq, total, scan, sums, fwd_scan = map(float, line.split())
