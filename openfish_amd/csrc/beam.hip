@@ -225,8 +225,8 @@ __device__ __forceinline__ uint32_t lds_address(const void *p) {
     return at;
 }
 
-// The lane, worked out where it is wanted: for places off the search's way, so that no register holds it through the search (two
-// workgroups on a compute unit leave 96).
+// The lane, worked out where it is wanted: for places off the search's way, so that no register holds it through the search (the
+// merged kernel of large batches has 96).
 __device__ __forceinline__ int lane_now() {
     uint32_t none = 0;
     asm volatile("" : "+v"(none));  // or the compiler takes it from elsewhere after all
@@ -397,10 +397,11 @@ struct PlaneRow {
 template <int S, int CPG, int FWD>
 struct BeamCfg {
     static constexpr int kBits = S == 64 ? 6 : S == 256 ? 8 : 10;
-    // two waves of recursion at 256 states is the choice for two workgroups per compute unit: 80 KB of LDS each
+    // two waves of recursion at 256 states: the LDS (75 and 78 KB) and the registers of two workgroups fit a compute unit (see beam_kernel for
+    // what comes of it)
     static constexpr bool kDense = FWD == 2;
     // LDS ring depth, which is also how many time steps of the search are written out one after another.  Four, but for two chunks of
-    // 1024 states to a unit that they share with the forward sweep, and where two workgroups share it.
+    // 1024 states to a unit that they share with the forward sweep, and where two workgroups are to fit one.
     static constexpr int kLdsRows = kDense || (S >= 1024 && CPG > 1) ? 3 : 4;
     static constexpr int kHandBack = FWD == 0 && kLdsRows == 4 ? 2 : 1;  // rows the search asks for and gives back at a time
     static constexpr int kRegRows = S >= 1024 ? (FWD == 0 ? 3 : 2) : (kDense ? 3 : 6);  // rows in flight in registers (2, 3 or 6)
@@ -455,7 +456,9 @@ struct BeamIdx {
     static constexpr uint32_t kRound = 1u << 9, kRoundEnd = 1u << (kBits + 2);
     // Waves that trace a chunk's path back, each with a buffer of 8 KB in the index: the search's, the loader's and, of a lone chunk, the
     // two that were there for the set-up, or two of the recursion's.  The maps they exchange, 16 KB, lie behind the buffers where there is
-    // room.  An index of 16 KB has two buffers and no maps: one wave.
+    // room, and apart in the merged kernels of four and eight waves: 148 KB of LDS a workgroup of 256 states (five columns 152; 115 and 119
+    // without them), 127 (136) of 1024 states.  The 12 to 33 KB that are left of a unit take a workgroup of another decode's backward sweep,
+    // 6 or 15 KB, but of its sequence stage, 13 bytes a step, only with shorter chunks.  An index of 16 KB has two buffers and no maps: one wave.
     static constexpr int kTeam = kLone || FWD >= 4 ? 4 : kBits == 13 ? 2 : 1;
     static constexpr bool kMapsApart = FWD >= 4;
 };
@@ -557,7 +560,7 @@ struct LdsRow {
 // rows the loader has put into LDS, so that scores and bwd cross HBM once for both.  As two kernels side by
 // side they were bound by that traffic at large batches (1024 chunks of 256 states with five columns: 13.9 GB
 // in 2.98 ms, what a copy reaches; 256 of 1024 states the same in 2.84); here 7.9 GB take 2.54 and 1.74 ms,
-// bound by the vector ALUs and by a step's chain of round trips.
+// bound by the chain of a step and by its instructions.
 //   search | posterior | FWD waves of recursion | loader
 // There is no barrier after the set-up: the waves of a chunk hand rows over through counters in LDS.  A wave of
 // the recursion writes its part of row t + 1 of the state vector and then its counter (a wave's LDS operations
@@ -571,8 +574,10 @@ struct LdsRow {
 // more at large batches, with the search below the recursion 256 states lose 0.2 ms at 512 chunks.
 //
 // FWD: one state per lane (4 waves) with one workgroup of two chunks on a compute unit.  Above 512 chunks of 256
-// states two workgroups share a unit (80 KB of LDS, 96 registers per lane): two states per lane and smaller
-// rings.  1024 states: two per lane, one chunk per workgroup (four per lane: 2.15 ms against 1.74 at 256 chunks).
+// states two workgroups were to share a unit (78 KB of LDS, 96 registers per lane): two states per lane and smaller
+// rings.  They do not: by the counters 2.2 of the 5 waves launched for a SIMD are resident, which is one workgroup a unit at a time, and the vector
+// ALUs are busy 0.61 of 2.14 ms (1024 chunks).  A workgroup's ten waves lie 3 + 3 + 2 + 2 on SIMDs that hold five each, so a second one
+// fits only with its larger shares on the other two.  1024 states: two per lane, one chunk per workgroup (four per lane: 2.15 ms against 1.74 at 256 chunks).
 template <int S, int CPG, int COLS, int FWD>
 constexpr int kBeamThreads = BeamIdx<S, CPG, FWD>::kLone ? 256 : 64 * CPG * (FWD == 0 ? 2 : FWD + 3);  // a lone chunk: two waves more for the set-up
 template <int S, int CPG, int COLS, int FWD>

@@ -528,7 +528,7 @@ static void join_null_stream(ofa_gpubuf_t *g) {
  * set-up, batches above 338 of chunks up to 100 steps by the rounds.  Up to 512 chunks of 256 states the chain of split is
  * shorter, while its bytes fit beneath the chain, 2.5 MB a step (348 chunks, five columns 305; between 2.5 and 2.8 MB the two are within 1 % of each
  * other); above,
- * the search's workgroups hold four chunks, a unit that has one of them in the merged kernel takes as long as one that has four,
+ * the search's workgroups hold four chunks, the merged kernel's two, in a second round that takes as long with one chunk as with 512,
  * and split has units left for the forward sweep up to 640 chunks, with shorter chunks up to 768.
  *
  * A decode that is enqueued, or finds another one under way, shares the machine; two at a time, one | split | merged:

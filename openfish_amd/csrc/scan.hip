@@ -1243,7 +1243,8 @@ uint32_t double_below(int S, int N, bool backward) {
 // states, us, without | with: 300 chunks, T = 96 59 | 55, 200 109 | 107, 300 156 | 155, 500 243 | 246; 512, T = 96 67 | 63, 200 118 | 115, 300 172 |
 // 172, 500 248 | 252, 1666 677 | 711, with five columns 695 | 732; of the other models the early steps are ahead at any size (1024 states, 160 chunks, T = 64
 // 74 | 63, 833 661 | 655; 2048 of 64, T = 1000 357 | 350).  Forward sweep of 64 states beside a search: 1024 chunks, T = 300 184 | 175, T = 1666 733 |
-// 685; 1500 234 | 315 and 1002 | 1324.
+// 685; 1500 234 | 315 and 1002 | 1324.  Whole calls of 2048 chunks 614 | 711 at T = 300, but 3116 | 3034 at T = 1666, where the slower sweep leaves more
+// to the search beside it: the rule goes by chunks alone and gives that away.
 bool early_backward(int S, int T, int N) { return S != 256 || N <= 256 || T <= 256; }
 constexpr int kEarlyForwardChunks = 1024;
 

@@ -1,6 +1,6 @@
 """The search writes its steps out over the slots of its row ring and counts ring rounds in the entries of its hash index, which it
-clears when the count is used up: after 124 steps (two chunks of 1024 states to a compute unit, and merged kernels of 256 states two
-workgroups to a unit: 93), 252 or 508, by the size of the index.  Chunk lengths around a ring's length and around the first and second
+clears when the count is used up: after 124 steps (two chunks of 1024 states to a compute unit, and merged kernels of 256 states
+above 512 chunks: 93), 252 or 508, by the size of the index.  Chunk lengths around a ring's length and around the first and second
 clearing, every size of the index, both layouts: steps that end a chunk anywhere in a round, and nothing else overwritten.  (That what is to be
 cleared is cleared, test_search_index.py shows.)"""
 import numpy as np
